@@ -79,6 +79,7 @@ struct aspen_hip_graph_t
     uint32_t default_workgroups;    // grid of a dataflow run when the caller names none, see graph_parallelism
     double parallelism;             // average parallelism of the tile graph, see graph_parallelism
     int cached_loads;       // 1: no cache line of an activation is shared by two producer tiles
+    void **d_arranged;              // per layer: the graph's own arranged copy of its weights, or NULL (see graph_create)
     unsigned long long *d_trace;    // [2*tile] start, [2*tile+1] end time stamps (allocated on first traced run)
     uint32_t *h_abort;              // pinned host word the persistent kernel raises when it gives this graph's run up
 };
@@ -519,11 +520,7 @@ __device__ __forceinline__ void wait_until_ready ()
 }
 
 template <int COH, unsigned FEAT, bool ORDERED = false>
-// (The variant for transformer graphs is built for three workgroups per compute unit instead of four: those graphs never
-// fill the device (256 to 768 workgroups), and 168 instead of 128 registers per lane spare their attention and matmul loops
-// the spills the tighter budget forces.)
-#define DATAFLOW_WG_PER_CU(feat, ordered) ((feat) == TILES_TRANSFORMER ? WG_PER_CU - 1 : WG_PER_CU)
-__global__ void __launch_bounds__ (WG_THREADS, DATAFLOW_WG_PER_CU (FEAT, ORDERED)) dataflow_kernel (dataflow_args_t args)
+__global__ void __launch_bounds__ (WG_THREADS, WG_PER_CU) dataflow_kernel (dataflow_args_t args)
 {
     extern __shared__ __align__ (16) float smem[];
     if (threadIdx.x == 0)
@@ -677,7 +674,7 @@ extern "C" void aspen_hip_tile_shapes (uint32_t shapes[13])
 {
     shapes[11] = VAR4_BM; shapes[12] = VAR4_BN;
     shapes[0] = VAR0_BM; shapes[1] = VAR0_BN; shapes[2] = VAR1_BM; shapes[3] = VAR1_BN; shapes[4] = VAR2_BM; shapes[5] = VAR2_BN;
-    shapes[6] = KATTN_BN; shapes[7] = VATTN_BN; shapes[8] = WG_PER_CU; shapes[9] = VAR3_BM; shapes[10] = VAR3_BN;
+    shapes[6] = KATTN_BN; shapes[7] = VATTN_BN; shapes[8] = 2; shapes[9] = VAR3_BM; shapes[10] = VAR3_BN;
 }
 
 extern "C" int aspen_hip_device_info (int *num_cu, int *clock_khz, size_t *mem_bytes, char *name, int name_len)
@@ -855,6 +852,68 @@ extern "C" int aspen_hip_copy (void *dst, const void *src, size_t bytes)
     hipLaunchKernelGGL (copy_kernel, dim3 (grid), dim3 (WG_THREADS), 0, g_stream, (const float4 *)src, (float4 *)dst, n4);
     CHECK (hipGetLastError ());
     return 0;
+}
+
+// ------------------------------------------------------------------------------------------------
+// weights
+// ------------------------------------------------------------------------------------------------
+// Row-major floats -> the fragment order the contraction tiles read (WeightFragments): one thread per lane of a fragment.
+// Rows from M to the last whole block are written as zeros.
+template <bool RAW>
+__global__ void __launch_bounds__ (WG_THREADS) arrange_weights_kernel (const float *__restrict__ rows, uint32_t ld, uint32_t M, uint32_t slices, uint32_t blocks, char *__restrict__ dst)
+{
+    const size_t n = (size_t)blocks * slices * 128u, stride = (size_t)gridDim.x * blockDim.x;
+    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride)
+    {
+        const uint32_t lane = (uint32_t)i & 63u, step = (uint32_t)(i >> 6) & 1u;
+        const size_t bs = i >> 7, block = bs / slices;
+        const uint32_t slice = (uint32_t)(bs - block * slices), row = (uint32_t)block * WEIGHT_BLOCK_ROWS + (lane & 31u), unit = 2u * step + (lane >> 5);
+        float4 a = make_float4 (0.f, 0.f, 0.f, 0.f), b = a;
+        if (row < M)
+        {
+            const float *src = rows + (size_t)row * ld + (size_t)slice * SLICE_K + unit * 4u;
+            a = gld4 (src); b = gld4 (src + 16);
+        }
+        constexpr uint32_t SLICE = WeightFragments<RAW>::SLICE;
+        char *d = dst + bs * SLICE + step * (SLICE / 2) + lane * 16u;
+        if (RAW) { *reinterpret_cast<float4 *> (d) = a; *reinterpret_cast<float4 *> (d + 1024) = b; }
+        else
+        {
+            const split8_t f = split8 (a, b);
+            *reinterpret_cast<u32x4 *> (d) = f.h; *reinterpret_cast<u32x4 *> (d + 1024) = f.m; *reinterpret_cast<u32x4 *> (d + 2048) = f.l;
+        }
+    }
+}
+
+static size_t arranged_bytes (uint32_t M, uint32_t Kp, bool raw)
+{
+    return (size_t)((M + 127u) / 128u * 4u) * (Kp / SLICE_K) * (raw ? RAW_SLICE_BYTES : SPLIT_SLICE_BYTES);
+}
+// `rows`: M rows of Kp floats, `ld` apart, on the device; on the library's stream
+static int arrange_weights (void *dst, const float *rows, uint32_t ld, uint32_t M, uint32_t Kp, bool raw)
+{
+    const uint32_t slices = Kp / SLICE_K, blocks = (M + 127u) / 128u * 4u;
+    const dim3 grid (stream_grid ((size_t)blocks * slices * 128u));
+    if (raw) hipLaunchKernelGGL (arrange_weights_kernel<true>, grid, dim3 (WG_THREADS), 0, g_stream, rows, ld, M, slices, blocks, (char *)dst);
+    else hipLaunchKernelGGL (arrange_weights_kernel<false>, grid, dim3 (WG_THREADS), 0, g_stream, rows, ld, M, slices, blocks, (char *)dst);
+    CHECK (hipGetLastError ());
+    return 0;
+}
+
+extern "C" void *aspen_hip_upload_weights (const float *rows, uint32_t M, uint32_t Kp, int raw)
+{
+    if (aspen_hip_init ()) return nullptr;
+    if (!rows || M == 0 || Kp == 0 || Kp % SLICE_K) { snprintf (g_err, sizeof (g_err), "upload_weights: bad arguments"); return nullptr; }
+    const size_t bytes = (size_t)M * Kp * sizeof (float);
+    float *flat = (float *)aspen_hip_alloc (bytes);
+    void *arranged = aspen_hip_alloc (arranged_bytes (M, Kp, raw != 0));
+    if (!flat || !arranged || aspen_hip_h2d (flat, rows, bytes) || arrange_weights (arranged, flat, Kp, M, Kp, raw != 0) || aspen_hip_sync ())
+    {
+        aspen_hip_free (flat); aspen_hip_free (arranged);
+        return nullptr;
+    }
+    aspen_hip_free (flat);
+    return arranged;
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -1051,9 +1110,13 @@ static double graph_parallelism (const aspen_hip_layer_t *layers, const uint32_t
     return ordered && longest > 0.0 ? total / longest : 1e30;
 }
 
-extern "C" aspen_hip_graph_t *aspen_hip_graph_create (const aspen_hip_layer_t *layers, uint32_t num_layers,
+static bool is_contraction (const aspen_hip_layer_t &L) { return (L.type == CONV_LAYER || L.type == FC_LAYER || L.type == MATMUL_LAYER) && L.num_ninst != 0; }
+
+// prepared: the contraction layers' weights come from aspen_hip_upload_weights; else they are row-major floats, and the
+// graph makes and owns the arranged copies
+static aspen_hip_graph_t *graph_create (const aspen_hip_layer_t *layers, uint32_t num_layers,
     const uint32_t *ninst_layer, const uint32_t *num_parents, const uint32_t *child_off,
-    const uint32_t *child_idx, uint32_t num_ninst, const uint32_t *roots, uint32_t num_roots)
+    const uint32_t *child_idx, uint32_t num_ninst, const uint32_t *roots, uint32_t num_roots, bool prepared)
 {
     if (aspen_hip_init ()) return nullptr;
     if (num_ninst > QUEUE_ID_MASK) { snprintf (g_err, sizeof (g_err), "graph has more than %u tiles", QUEUE_ID_MASK); return nullptr; }
@@ -1124,6 +1187,21 @@ extern "C" aspen_hip_graph_t *aspen_hip_graph_create (const aspen_hip_layer_t *l
     if (!g->h_layers) { snprintf (g_err, sizeof (g_err), "out of host memory"); free (g); return nullptr; }
     memcpy (g->h_layers, layers, sizeof (aspen_hip_layer_t) * num_layers);
     for (uint32_t l = 0; l < num_layers; l++) fill_derived (g->h_layers[l]);
+    if (!prepared)
+    {
+        g->d_arranged = (void **)calloc (num_layers ? num_layers : 1, sizeof (void *));
+        bool ok = g->d_arranged != nullptr;
+        for (uint32_t l = 0; l < num_layers && ok; l++)
+        {
+            aspen_hip_layer_t &L = g->h_layers[l];
+            if (!is_contraction (L)) continue;
+            const bool raw = L.variant == ASPEN_HIP_GEMM_TALL;
+            g->d_arranged[l] = aspen_hip_alloc (arranged_bytes (L.M, L.Kp, raw));
+            ok = g->d_arranged[l] && arrange_weights (g->d_arranged[l], L.weight, L.Kp, L.M, L.Kp, raw) == 0;
+            L.weight = (const float *)g->d_arranged[l];
+        }
+        if (!ok) { aspen_hip_graph_destroy (g); return nullptr; }
+    }
     g->d_layers = upload (g->h_layers, num_layers);
     g->d_ninst_layer = upload (ninst_layer, num_ninst);
     g->d_num_parents = upload (num_parents, num_ninst);
@@ -1192,10 +1270,25 @@ extern "C" aspen_hip_graph_t *aspen_hip_graph_create (const aspen_hip_layer_t *l
     return g;
 }
 
+extern "C" aspen_hip_graph_t *aspen_hip_graph_create (const aspen_hip_layer_t *layers, uint32_t num_layers,
+    const uint32_t *ninst_layer, const uint32_t *num_parents, const uint32_t *child_off,
+    const uint32_t *child_idx, uint32_t num_ninst, const uint32_t *roots, uint32_t num_roots)
+{
+    return graph_create (layers, num_layers, ninst_layer, num_parents, child_off, child_idx, num_ninst, roots, num_roots, false);
+}
+extern "C" aspen_hip_graph_t *aspen_hip_graph_create_prepared (const aspen_hip_layer_t *layers, uint32_t num_layers,
+    const uint32_t *ninst_layer, const uint32_t *num_parents, const uint32_t *child_off,
+    const uint32_t *child_idx, uint32_t num_ninst, const uint32_t *roots, uint32_t num_roots)
+{
+    return graph_create (layers, num_layers, ninst_layer, num_parents, child_off, child_idx, num_ninst, roots, num_roots, true);
+}
+
 extern "C" void aspen_hip_graph_destroy (aspen_hip_graph_t *g)
 {
     if (!g) return;
     (void)hipStreamSynchronize (g_stream);
+    for (uint32_t l = 0; g->d_arranged && l < g->num_layers; l++) aspen_hip_free (g->d_arranged[l]);
+    free (g->d_arranged);
     aspen_hip_free (g->d_layers); aspen_hip_free (g->d_ninst_layer); aspen_hip_free (g->d_num_parents);
     aspen_hip_free (g->d_child_off); aspen_hip_free (g->d_child_idx); aspen_hip_free (g->d_roots); aspen_hip_free (g->d_ninst_home); aspen_hip_free (g->d_root_pos);
     aspen_hip_free (g->d_child_rec); aspen_hip_free (g->d_dep); aspen_hip_free (g->d_queue); aspen_hip_free (g->d_ran); aspen_hip_free (g->d_arrivals); aspen_hip_free (g->d_state); aspen_hip_free (g->d_prof); aspen_hip_free (g->d_trace); aspen_hip_free (g->d_group_sinks); aspen_hip_free (g->d_dep_spread);
@@ -1527,11 +1620,10 @@ extern "C" int aspen_hip_sgemm (uint32_t M, uint32_t N, uint32_t K, const float 
     if (aspen_hip_init ()) return -1;
     if (K == 0 || K % GEMM_BK || lda % 4 || ldb % 4 || ldc % 4 || lda < K || ldb < K || ldc < M)
     { snprintf (g_err, sizeof (g_err), "sgemm: K must be a multiple of 32, strides multiples of 4"); return -1; }
-    // weight rows are read in blocks of 64 without a row clamp: stage A into a zero-padded copy
-    const uint32_t Mp = (M + 127) / 128 * 128;
-    float *Ap = (float *)aspen_hip_alloc ((size_t)Mp * K * sizeof (float));
+    // A in the order the tiles read their weights, rows padded with zeros
+    float *Ap = (float *)aspen_hip_alloc (arranged_bytes (M, K, false));
     if (!Ap) return -1;
-    CHECK (hipMemcpy2DAsync (Ap, (size_t)K * 4, A, (size_t)lda * 4, (size_t)K * 4, M, hipMemcpyDeviceToDevice, g_stream));
+    if (arrange_weights (Ap, A, lda, M, K, false)) { aspen_hip_free (Ap); return -1; }
     aspen_hip_layer_t L;
     memset (&L, 0, sizeof (L));
     L.type = MATMUL_LAYER; L.act = act; L.variant = ASPEN_HIP_GEMM_SMALL; L.direct = 1;
@@ -1561,7 +1653,7 @@ extern "C" int aspen_hip_sgemm (uint32_t M, uint32_t N, uint32_t K, const float 
 // ------------------------------------------------------------------------------------------------
 #define SGEMM_SCRATCH_BYTES (8u << 20)
 #define MAX_DEVICES 16
-static __device__ __align__ (256) unsigned char scratch[SGEMM_SCRATCH_BYTES];
+static __device__ __align__ (256) unsigned char scratch[SGEMM_SCRATCH_BYTES / 2 * 3];    // (six bytes per float, see SPLIT_SLICE_BYTES)
 static float *g_scratch_ptr[MAX_DEVICES];           // device address of `scratch` per device, see scratch_for_current_device
 
 static float *scratch_for_current_device (void)
@@ -1576,19 +1668,6 @@ static float *scratch_for_current_device (void)
         g_scratch_ptr[dev] = (float *)p;
     }
     return g_scratch_ptr[dev];
-}
-
-// dst[r][0..K) = src[r][0..K) for r < M, zeros for M <= r < Mp; K % 4 == 0, lda % 4 == 0
-__global__ void __launch_bounds__ (WG_THREADS) pad_rows_kernel (const float *__restrict__ src, uint32_t lda, float *__restrict__ dst, uint32_t M, uint32_t Mp, uint32_t K)
-{
-    const uint32_t k4 = K >> 2;
-    const size_t n = (size_t)Mp * k4, step = (size_t)gridDim.x * blockDim.x;
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += step)
-    {
-        const uint32_t r = (uint32_t)(i / k4), c = (uint32_t)(i - (size_t)r * k4) * 4;
-        const float4 v = r < M ? gld4 (src + (size_t)r * lda + c) : make_float4 (0.f, 0.f, 0.f, 0.f);
-        st4 (dst + (size_t)r * K + c, v);
-    }
 }
 
 // one contraction tile per workgroup, the descriptor in the kernel-argument segment
@@ -1619,8 +1698,7 @@ extern "C" int aspen_hip_sgemm_static (uint32_t M, uint32_t N, uint32_t K, const
     if ((uint64_t)N * ldc * 4 >= 0xffffff00ull || (uint64_t)N * ldb * 4 >= 0xffffff00ull) { snprintf (g_err, sizeof (g_err), "sgemm_static: matrix larger than 4 GiB"); return -1; }
     float *Ap = scratch_for_current_device ();
     if (!Ap) return -1;
-    hipLaunchKernelGGL (pad_rows_kernel, dim3 (stream_grid ((size_t)Mp * (K / 4))), dim3 (WG_THREADS), 0, g_stream, A, lda, Ap, M, (uint32_t)Mp, K);
-    CHECK (hipGetLastError ());
+    if (arrange_weights (Ap, A, lda, M, K, false)) return -1;
     aspen_hip_layer_t L;
     memset (&L, 0, sizeof (L));
     L.type = MATMUL_LAYER; L.act = act; L.variant = ASPEN_HIP_GEMM_SMALL; L.direct = 1;

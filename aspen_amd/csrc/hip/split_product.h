@@ -1,0 +1,127 @@
+// Single-precision products on the bfloat16 matrix cores.
+//
+// A float has 24 significant bits, a bfloat16 eight: x = h + m + l with h = bf16 (x), m = bf16 (x - h), l = x - h - m, and
+// all three terms are exact (each rounding to nearest takes eight bits and a sign off the rest; the rest of the second
+// fits a bfloat16 whole).  A product of two floats is then nine products of bfloat16 terms, each of them exact in the
+// matrix core's single-precision sum.  Six are computed:
+//     a b = ah bh  +  (ah bm + am bh)  +  (ah bl + al bh + am bm)      left out: am bl + al bm + al bl < 2^-25 |a b|
+// i.e. less than half of what rounding ONE float product to a float may cost.  The leading products are summed in one
+// accumulator and the five small ones in another, added at the end: the large sum is then rounded once per 16 K positions
+// instead of once per two (v_mfma_f32_32x32x2_f32), the small sum's roundings do not count at its size, and the result is closer to the
+// exact one than the single-precision matrix instruction's (relative to a 64-bit sum, 2-norm over 128 x 128 results, inputs
+// normal / rectified normal: K = 64 4.8e-8 / 4.2e-8 against 1.4e-7 / 1.0e-7; K = 1024 1.8e-7 / 1.5e-7 against 5.7e-7 / 4.2e-7;
+// K = 4096 4.0e-7 / 3.2e-7 against 1.1e-6 / 8.1e-7; with one accumulator for all six products 1.0e-6 / 9.5e-7).
+// Speed: a v_mfma_f32_32x32x16_bf16 does eight times the work of a v_mfma_f32_32x32x2_f32 in half its cycles, so six of them take 3 / 8
+// of the time.  In practice both are limited by power: a large product reaches 154 TFLOP/s with the single-precision
+// instruction (98 % of its peak) and 205-212 with this scheme.
+// The range is float's own (bfloat16 has the same exponent): terms of inputs below 2^-110 lose low bits, inputs within 0.4 %
+// of the largest float round to infinity, and an infinite input makes its products NaN.
+#pragma once
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+typedef float floatx16 __attribute__ ((ext_vector_type (16)));
+typedef uint32_t u32x4 __attribute__ ((ext_vector_type (4)));
+typedef __bf16 bf16x2 __attribute__ ((ext_vector_type (2)));
+typedef __bf16 bf16x8 __attribute__ ((ext_vector_type (8)));
+typedef float floatx2 __attribute__ ((ext_vector_type (2)));
+
+// two floats rounded to bfloat16, the first in the low half (one v_cvt_pk_bf16_f32)
+__device__ __forceinline__ uint32_t bf16_pair (float a, float b)
+{
+    return __builtin_bit_cast (uint32_t, __builtin_convertvector ((floatx2){a, b}, bf16x2));
+}
+__device__ __forceinline__ float bf16_low (uint32_t p) { return __builtin_bit_cast (float, p << 16); }
+__device__ __forceinline__ float bf16_high (uint32_t p) { return __builtin_bit_cast (float, p & 0xffff0000u); }
+
+// the three terms of eight floats, as matrix-core operands (K positions 0 .. 7 of a lane)
+struct split8_t { u32x4 h, m, l; };
+__device__ __forceinline__ split8_t split8 (float4 a, float4 b)
+{
+    split8_t s;
+    const float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+    #pragma unroll
+    for (int q = 0; q < 4; q++)
+    {
+        float u = x[2 * q], v = x[2 * q + 1];
+        const uint32_t h = bf16_pair (u, v);
+        u -= bf16_low (h); v -= bf16_high (h);
+        const uint32_t m = bf16_pair (u, v);
+        u -= bf16_low (m); v -= bf16_high (m);
+        s.h[q] = h; s.m[q] = m; s.l[q] = bf16_pair (u, v);
+    }
+    return s;
+}
+
+// hi += leading products, lo += the five small ones, of 32 x 32 x 16: rows of the result = rows of `a`, columns = rows of `b`
+__device__ __forceinline__ void split_mfma (const split8_t &a, const split8_t &b, floatx16 &hi, floatx16 &lo)
+{
+    const bf16x8 ah = __builtin_bit_cast (bf16x8, a.h), am = __builtin_bit_cast (bf16x8, a.m), al = __builtin_bit_cast (bf16x8, a.l);
+    const bf16x8 bh = __builtin_bit_cast (bf16x8, b.h), bm = __builtin_bit_cast (bf16x8, b.m), bl = __builtin_bit_cast (bf16x8, b.l);
+    hi = __builtin_amdgcn_mfma_f32_32x32x16_bf16 (ah, bh, hi, 0, 0, 0);
+    lo = __builtin_amdgcn_mfma_f32_32x32x16_bf16 (al, bh, lo, 0, 0, 0);
+    lo = __builtin_amdgcn_mfma_f32_32x32x16_bf16 (ah, bl, lo, 0, 0, 0);
+    lo = __builtin_amdgcn_mfma_f32_32x32x16_bf16 (am, bm, lo, 0, 0, 0);
+    lo = __builtin_amdgcn_mfma_f32_32x32x16_bf16 (am, bh, lo, 0, 0, 0);
+    lo = __builtin_amdgcn_mfma_f32_32x32x16_bf16 (ah, bm, lo, 0, 0, 0);
+}
+
+// Order of the K axis inside a slice of 32 (both operands have to agree, the sum does not care): a lane of a matrix
+// instruction holds eight K positions of one row, "unit" u = 2 * step + lane / 32 (u = 0 .. 3, two instruction steps per
+// slice), and unit u stands for the slice's floats 4u .. 4u+3 and 16+4u .. 16+4u+3.  Four neighbouring threads that
+// fetch the four units of a row then read 64 contiguous bytes with each of their two 16-byte requests.
+#define SLICE_K 32
+
+// Weights on the device.  SPLIT: per block of 32 rows and slice, per step, the terms h, m, l, each as the 64 lanes' 16 bytes in a row (lane l: row
+// l % 32, unit 2 * step + l / 32): 6144 bytes that a wavefront fetches with six contiguous 1 KB requests straight into
+// the registers the matrix instructions read.  RAW: the same with the floats themselves, per step two rows of 64 x 16
+// bytes (floats 4u .. and 16+4u ..): 4096 bytes per block and slice, split in registers.  A weight belongs to one
+// wavefront of a tile (or is shared by two, from the compute unit's cache), so nothing is staged through LDS.
+// RAW is for layers that are bound by the weights' trip from memory.
+#define WEIGHT_BLOCK_ROWS 32
+#define SPLIT_SLICE_BYTES 6144u
+#define RAW_SLICE_BYTES 4096u
+
+template <bool RAW> struct WeightFragments
+{
+    static constexpr uint32_t SLICE = RAW ? RAW_SLICE_BYTES : SPLIT_SLICE_BYTES, PARTS = RAW ? 2 : 3;
+    typedef const char __attribute__ ((address_space (1))) *bytes_t;
+    bytes_t base;               // of the wavefront's row block (uniform)
+    uint32_t lane16;
+    u32x4 f[2][PARTS];          // [step]
+    __device__ __forceinline__ void init (const void *w, uint32_t block, uint32_t slices, uint32_t lane)
+    {
+        base = (bytes_t)w + (uint64_t)block * ((uint64_t)slices * SLICE);
+        lane16 = lane * 16u;
+    }
+    __device__ __forceinline__ void load (int it, int step)
+    {
+        const bytes_t p = base + ((uint32_t)it * SLICE + (uint32_t)step * (SLICE / 2));
+        #pragma unroll
+        for (uint32_t q = 0; q < PARTS; q++) f[step][q] = *(const u32x4 __attribute__ ((address_space (1))) *)(p + (lane16 + q * 1024u));
+    }
+    __device__ __forceinline__ split8_t operand (int step) const
+    {
+        if constexpr (RAW) return split8 (__builtin_bit_cast (float4, f[step][0]), __builtin_bit_cast (float4, f[step][1]));
+        else return {f[step][0], f[step][1], f[step][2]};
+    }
+};
+
+// LDS stage of the other operand, one slice of ROWS rows: three planes (h, m, l) of ROWS x 64 bytes, the four 16-byte units
+// of a row in the order unit ^ (row / 4 % 4): a fragment read (16 neighbouring rows, the same unit, at a time) and a write (four rows whole)
+// both touch every bank once.
+template <int ROWS> struct SplitStage
+{
+    static constexpr uint32_t PLANE = ROWS * 64u, BYTES = 3u * PLANE;
+    static __device__ __forceinline__ uint32_t offset (uint32_t row, uint32_t unit) { return row * 64u + ((unit ^ ((row >> 2) & 3u)) * 16u); }
+    static __device__ __forceinline__ void write (char *stage, uint32_t off, const split8_t &s)
+    {
+        *reinterpret_cast<u32x4 *> (stage + off) = s.h;
+        *reinterpret_cast<u32x4 *> (stage + off + PLANE) = s.m;
+        *reinterpret_cast<u32x4 *> (stage + off + 2 * PLANE) = s.l;
+    }
+    static __device__ __forceinline__ split8_t read (const char *stage, uint32_t off)
+    {
+        return {*reinterpret_cast<const u32x4 *> (stage + off), *reinterpret_cast<const u32x4 *> (stage + off + PLANE), *reinterpret_cast<const u32x4 *> (stage + off + 2 * PLANE)};
+    }
+};

@@ -14,8 +14,7 @@
 #include <type_traits>
 #include "aspen.h"
 #include "aspen_hip.h"
-
-typedef float floatx16 __attribute__ ((ext_vector_type (16)));
+#include "split_product.h"
 
 // Phase accounting of contraction tiles inside the persistent kernel (defined next to the kernel; costs one
 // LDS read per call when profiling is off): 8 = operand set-up and first loads, 9 = K loop, 10 = epilogue,
@@ -26,14 +25,12 @@ __device__ void tile_phase_lap (int which);
 #define GEMM_BK 32            // K floats staged per iteration: one 128-byte line per operand row
 #define LDS_ROW 36            // floats per staged row: 32 + 4 padding -> conflict-free 128-bit reads
 
-// Tiles of at most 128 x 64 outputs, 32 accumulator registers per lane, one LDS stage (the next K
-// slice waits in registers) -> <= 128 VGPRs and <= 40 KB LDS per workgroup, so FOUR workgroups (16
-// wavefronts) share a compute unit and one workgroup's load latency, epilogue and scheduling gaps are
-// covered by the other three.  (128 x 128 tiles with two LDS stages and two workgroups per compute
-// unit were measured too: better for very large GEMMs only, worse for every network here.)
+// Contraction tiles of at most 128 x 64 outputs, 64 accumulator registers per lane (two sums per output, see
+// split_product.h), two LDS stages -> <= 168 VGPRs and <= 50 KB LDS per workgroup, so THREE workgroups (12 wavefronts)
+// share a compute unit and one workgroup's load latency, epilogue and scheduling gaps are covered by the other two.
 #define VAR0_BM 128
 #define VAR0_BN 64
-#define WG_PER_CU 4
+#define WG_PER_CU 3
 #define KATTN_BN 32            // queries per K-attention tile
 #define VATTN_BN 64            // queries per V-attention tile
 #define VAR1_BM 64
@@ -42,25 +39,15 @@ __device__ void tile_phase_lap (int which);
 #define VAR2_BN 64
 // The tall shape, for layers that stream a large weight matrix past a handful of columns (a fully connected layer at
 // batch <= 32): four wavefronts, each 32 weight rows x the tile's 32 columns.  A 64 x 64 tile computes 32 columns of
-// padding there, which makes such a layer bound by the matrix pipeline at twice its useful work instead of by the
-// weights' trip from memory; this shape requests 16 KB of weights per K slice for the same number of MFMAs.
+// padding there.  Its weights stay floats in memory (WeightFragments<true>): such a layer is bound by their trip.
 #define VAR4_BM 128
 #define VAR4_BN 32
-#define VAR4_DEPTH 2            // two slices of weights in flight: memory latency is all such a tile waits for
-// K slices in flight from memory per tile shape (see gemm_core).  With two the larger shapes run out of registers
-// (measured: ResNet-50 batch 32 2.81 -> 2.89 ms, VGG-16 7.90 -> 8.83 ms).  The small shape takes two for the matmul
-// layers of transformer graphs, which run one or two workgroups per compute unit with nothing else to hide a slice's
-// memory latency (BERT-base 2.45 -> 2.24 ms), and one in the kernels for convolutional networks: there four workgroups
-// per compute unit hide it, and the second set of requests only lengthens the memory queues every tile's set-up
-// waits in (YOLO-v3 batch 8 4.90 -> 4.84 ms, ResNet-50 batch 1 with one launch per layer 0.62 -> 0.60).
-#define VAR0_DEPTH 1
-#define VAR1_DEPTH 1
-#define VAR2_DEPTH 2
 #define SPLITK_TILE_FLOATS (VAR2_BM * VAR2_BN)     // one slice's sums of one output tile: a block of its own in `partial` (the tall shape has as many)
 #define CMAX(a, b) ((a) > (b) ? (a) : (b))
-#define STAGE_FLOATS(bm, bn) (((bm) + (bn)) * LDS_ROW)
+#define STAGE_FLOATS(bm, bn) (((bm) + (bn)) * LDS_ROW)          // attention tiles
 #define EPI_FLOATS(bm, bn) ((bn) * ((bm) + 8))
-#define VAR_FLOATS(bm, bn) CMAX (STAGE_FLOATS (bm, bn), EPI_FLOATS (bm, bn))
+#define SPLIT_STAGES_FLOATS(bn) (2 * (bn) * 48)                 // two stages of SplitStage<bn>
+#define VAR_FLOATS(bm, bn) CMAX (SPLIT_STAGES_FLOATS (bn), EPI_FLOATS (bm, bn))
 #define GEMM_SMEM_FLOATS CMAX (CMAX (VAR_FLOATS (VAR0_BM, VAR0_BN), VAR_FLOATS (VAR1_BM, VAR1_BN)), \
                                CMAX (VAR_FLOATS (VAR2_BM, VAR2_BN), STAGE_FLOATS (128, KATTN_BN)))
 #define GEMM_SMEM_BYTES (GEMM_SMEM_FLOATS * 4)
@@ -103,7 +90,6 @@ __device__ __forceinline__ float gld1 (const float *p) { return *(const float __
 // Offsets are in floats from the start of the matrix.  In modes 1 and 2 the buffer descriptor bounds-checks
 // them in hardware (out-of-range loads return 0, out-of-range stores are dropped); mode 0 relies on the slack
 // every allocation carries for the few floats an edge tile reads past a row.
-typedef uint32_t u32x4 __attribute__ ((ext_vector_type (4)));
 #define CPOL_SC1 16
 template <int COH> struct ActView
 {
@@ -217,43 +203,7 @@ __device__ __forceinline__ float4 act4 (float4 v, int act)
 // while the matrix cores work on slice i.
 // ---------------------------------------------------------------------------------------------
 
-// Rows are K-contiguous in memory: weights [M][Kp], matmul / 1x1-conv activations, Q and K rows.
-template <int ROWS> struct RowLoader
-{
-    static constexpr int R = ROWS / 32;
-    // One uniform base pointer plus 32-bit byte offsets: global loads with a scalar base address need one
-    // vector register per row instead of a 64-bit pointer.
-    const char *base;
-    uint32_t off[R], chunk, row0;
-    // `rows` x `ld` floats at `p`, rows padded so that a tile never runs past them
-    __device__ __forceinline__ void init (const float *p, uint32_t first_row, uint32_t rows, uint32_t ld, uint32_t tid)
-    {
-        (void)rows;
-        chunk = tid & 7; row0 = tid >> 3;
-        base = reinterpret_cast<const char *> (p);
-        #pragma unroll
-        for (int i = 0; i < R; i++) off[i] = ((first_row + row0 + 32u * i) * ld + chunk * 4u) * 4u;
-    }
-    __device__ __forceinline__ void load (int it, float4 (&v)[R])
-    {
-        #pragma unroll
-        for (int i = 0; i < R; i++)
-        {
-            // the address space makes this a global (not flat) load whose 64-bit base stays in scalar registers
-            typedef const floatx4 __attribute__ ((address_space (1))) global_floatx4;
-            const char __attribute__ ((address_space (1))) *g = (const char __attribute__ ((address_space (1))) *)base;
-            const floatx4 x = *(global_floatx4 *)(g + (off[i] + (uint32_t)it * (GEMM_BK * 4u)));
-            v[i] = make_float4 (x[0], x[1], x[2], x[3]);
-        }
-    }
-    __device__ __forceinline__ void store (float *lds, const float4 (&v)[R])
-    {
-        #pragma unroll
-        for (int i = 0; i < R; i++) st4 (lds + (row0 + 32 * i) * LDS_ROW + chunk * 4, v[i]);
-    }
-};
-
-// Same for rows of an activation matrix (matmul / 1x1-conv operand, Q, K and probability rows).
+// Rows of Q, K and probability matrices: K-contiguous in memory.
 template <int ROWS, int COH> struct ActRowLoader
 {
     static constexpr int R = ROWS / 32;
@@ -284,6 +234,49 @@ template <int ROWS, int COH> struct ActRowLoader
     }
 };
 
+// Activation operands of contraction tiles.  A loader fetches this thread's share of one slice of ROWS rows: thread t has
+// unit t % 4 (see SLICE_K) of rows t / 4, t / 4 + 64, ...: two 16-byte pieces per row.  With ROWS = 32 the upper half of the
+// workgroup repeats the lower half's rows (the same values are written to the same places).
+template <int ROWS> struct SliceShare
+{
+    static constexpr int R = ROWS < 64 ? 1 : ROWS / 64;
+    uint32_t unit, row0;
+    __device__ __forceinline__ void init (uint32_t tid) { unit = tid & 3u; row0 = (tid >> 2) & (ROWS < 64 ? ROWS - 1u : 63u); }
+    __device__ __forceinline__ void store (char *stage, const float4 (&v)[R][2]) const
+    {
+        // (64 rows further down the same swizzle applies)
+        const uint32_t off = SplitStage<ROWS>::offset (row0, unit);
+        #pragma unroll
+        for (int i = 0; i < R; i++) SplitStage<ROWS>::write (stage, off + i * 64 * 64, split8 (v[i][0], v[i][1]));
+    }
+};
+
+// rows of an activation matrix, read in place (matmul / 1x1-conv operand)
+template <int ROWS, int COH> struct DirectLoader
+{
+    static constexpr int R = SliceShare<ROWS>::R;
+    SliceShare<ROWS> share;
+    ActView<COH> view;
+    uint32_t off[R];
+    // rows first_row.. of the view, clamped to max_row
+    __device__ __forceinline__ void init (const ActView<COH> &v, uint32_t first_row, uint32_t max_row, uint32_t ld, uint32_t tid)
+    {
+        view = v; share.init (tid);
+        #pragma unroll
+        for (int i = 0; i < R; i++)
+        {
+            uint32_t r = first_row + share.row0 + 64 * i;
+            r = r < max_row ? r : max_row;
+            off[i] = r * ld + share.unit * 4;
+        }
+    }
+    __device__ __forceinline__ void load (int it, float4 (&v)[R][2])
+    {
+        #pragma unroll
+        for (int i = 0; i < R; i++) { v[i][0] = view.ld4 (off[i] + it * SLICE_K); v[i][1] = view.ld4 (off[i] + it * SLICE_K + 16); }
+    }
+};
+
 // Implicit-GEMM activation operand of conv / FC: row n = output position (b, oh, ow); the K axis runs
 // over (kh, kw, ic) and is resolved through the layer's k-chunk table.  Replaces the reference's
 // pointer table + panel gather (prepare_input / load_im2col_ptr, reference src/tiled_kernels.c:3-159).
@@ -299,27 +292,30 @@ template <int ROWS, int COH> struct ActRowLoader
 // by which time a busy L2 had replaced it, and a 3 x 3 layer fetched its input up to nine times over the fabric.
 template <int ROWS, int COH, bool TABLE> struct ConvLoader
 {
-    static constexpr int R = ROWS / 32;
+    static constexpr int R = SliceShare<ROWS>::R;
+    SliceShare<ROWS> share;
     ActView<COH> in;
     const aspen_hip_ktab_t *ktab;
     int32_t base[R], ih0[R], iw0[R];
-    uint32_t IH, IW, chunk, row0;
+    uint32_t IH, IW;
     uint32_t KH, KW, ld0;
     uint32_t kh, kw, c;                     // tap and channel the next slice asked for starts at (!TABLE)
-    // first_it: the first K slice that will be asked for
-    __device__ __forceinline__ void init (const aspen_hip_layer_t &L, const ActView<COH> &v, uint32_t first_row, uint32_t tid, int first_it)
+    int left;                               // slices from that one to the end of the K range
+    // first_it: the first of the `count` K slices that will be asked for, in ascending order
+    __device__ __forceinline__ void init (const aspen_hip_layer_t &L, const ActView<COH> &v, uint32_t first_row, uint32_t tid, int first_it, int count)
     {
         in = v; IH = L.IH; IW = L.IW;
-        chunk = tid & 7; row0 = tid >> 3;
+        share.init (tid);
         if (TABLE) ktab = L.ktab;
         else
         {
             KH = L.KH; KW = L.KW; ld0 = L.ld0;
             kh = kw = c = 0;
+            left = count;
             if (first_it)
             {
                 const uint32_t taps = KH * KW, block = (uint32_t)first_it / taps, tap = (uint32_t)first_it - block * taps;
-                c = block * GEMM_BK;
+                c = block * SLICE_K;
                 kh = tap / KW; kw = tap - kh * KW;
             }
         }
@@ -327,7 +323,7 @@ template <int ROWS, int COH, bool TABLE> struct ConvLoader
         #pragma unroll
         for (int i = 0; i < R; i++)
         {
-            uint32_t n = first_row + row0 + 32 * i;
+            uint32_t n = first_row + share.row0 + 64 * i;
             n = n < L.N ? n : L.N - 1;
             uint32_t b = fast_div (n, L.div_ohw), rem = n - b * ohw, oh = fast_div (rem, L.div_ow), ow = rem - oh * L.OW;
             ih0[i] = (int32_t)(oh * L.stride) - (int32_t)L.pad;
@@ -335,37 +331,37 @@ template <int ROWS, int COH, bool TABLE> struct ConvLoader
             base[i] = ((int32_t)(b * L.IH) + ih0[i]) * (int32_t)L.IW * (int32_t)L.ld0 + iw0[i] * (int32_t)L.ld0;
         }
     }
-    __device__ __forceinline__ void load (int it, float4 (&v)[R])
+    __device__ __forceinline__ void load (int it, float4 (&v)[R][2])
     {
-        aspen_hip_ktab_t e;
         if (TABLE)
         {
             typedef unsigned int uintx2 __attribute__ ((ext_vector_type (2)));
-            const uintx2 raw = *(const uintx2 __attribute__ ((address_space (1))) *)(ktab + it * 8 + chunk);
-            e.offset = (int32_t)raw[0]; e.kh = (uint16_t)(raw[1] & 0xffffu); e.kw = (uint16_t)(raw[1] >> 16);
+            #pragma unroll
+            for (int q = 0; q < 2; q++)
+            {
+                const uintx2 raw = *(const uintx2 __attribute__ ((address_space (1))) *)(ktab + it * 8 + share.unit + 4 * q);
+                const int32_t kh_ = (int32_t)(raw[1] & 0xffffu), kw_ = (int32_t)(raw[1] >> 16);
+                #pragma unroll
+                for (int i = 0; i < R; i++)
+                {
+                    const bool ok = (uint32_t)(ih0[i] + kh_) < IH && (uint32_t)(iw0[i] + kw_) < IW;
+                    v[i][q] = in.ld4_if ((uint32_t)(base[i] + (int32_t)raw[0]), ok);
+                }
+            }
+            return;
         }
-        else
-        {
-            // Slices are asked for in ascending order from the one init was told, so the position is stepped, not
-            // divided out, and `it` is not looked at.  (The K loops ask for the last slice once more than they need
-            // and drop the answer: that request is one step past the K axis, i.e. the first tap again at the channels
-            // behind the last block: the 128 bytes that follow the pixel's channel run, which exist for every pixel
-            // but the matrix's last, where they lie in the slack behind the allocation.)
-            e.offset = (int32_t)((kh * IW + kw) * ld0 + c + chunk * 4);
-            e.kh = (uint16_t)kh; e.kw = (uint16_t)kw;
-            if (++kw == KW) { kw = 0; if (++kh == KH) { kh = 0; c += GEMM_BK; } }
-        }
+        // Slices are asked for in ascending order from the one init was told, so the position is stepped, not divided
+        // out, and `it` is not looked at.  It stays on the last slice: the K loops ask for that one again behind the end
+        // of the K range and drop the answer.
+        const int32_t offset = (int32_t)((kh * IW + kw) * ld0 + c + share.unit * 4);
         #pragma unroll
         for (int i = 0; i < R; i++)
         {
-            const bool ok = (uint32_t)(ih0[i] + (int32_t)e.kh) < IH && (uint32_t)(iw0[i] + (int32_t)e.kw) < IW;
-            v[i] = in.ld4_if ((uint32_t)(base[i] + e.offset), ok);
+            const bool ok = (uint32_t)(ih0[i] + (int32_t)kh) < IH && (uint32_t)(iw0[i] + (int32_t)kw) < IW;
+            v[i][0] = in.ld4_if ((uint32_t)(base[i] + offset), ok);
+            v[i][1] = in.ld4_if ((uint32_t)(base[i] + offset + 16), ok);
         }
-    }
-    __device__ __forceinline__ void store (float *lds, const float4 (&v)[R])
-    {
-        #pragma unroll
-        for (int i = 0; i < R; i++) st4 (lds + (row0 + 32 * i) * LDS_ROW + chunk * 4, v[i]);
+        if (--left > 0) { if (++kw == KW) { kw = 0; if (++kh == KH) { kh = 0; c += SLICE_K; } } }
     }
 };
 
@@ -378,20 +374,21 @@ template <int ROWS, int COH, bool TABLE> struct ConvLoader
 // every other convolution runs, stays as it is.
 template <int ROWS, int COH> struct Dense3Loader
 {
-    static constexpr int R = ROWS / 32;
+    static constexpr int R = SliceShare<ROWS>::R;
+    SliceShare<ROWS> share;
     ActView<COH> in;
     const aspen_hip_ktab_t *ktab;
     int32_t base[R], ih0[R], iw0[R];
-    uint32_t IH, IW, chunk, row0;
+    uint32_t IH, IW;
     __device__ __forceinline__ void init (const aspen_hip_layer_t &L, const ActView<COH> &v, uint32_t first_row, uint32_t tid)
     {
         in = v; ktab = L.ktab; IH = L.IH; IW = L.IW;
-        chunk = tid & 7; row0 = tid >> 3;
+        share.init (tid);
         const uint32_t ohw = L.OH * L.OW;
         #pragma unroll
         for (int i = 0; i < R; i++)
         {
-            uint32_t n = first_row + row0 + 32 * i;
+            uint32_t n = first_row + share.row0 + 64 * i;
             n = n < L.N ? n : L.N - 1;
             uint32_t b = fast_div (n, L.div_ohw), rem = n - b * ohw, oh = fast_div (rem, L.div_ow), ow = rem - oh * L.OW;
             ih0[i] = (int32_t)(oh * L.stride) - (int32_t)L.pad;
@@ -399,27 +396,26 @@ template <int ROWS, int COH> struct Dense3Loader
             base[i] = ((int32_t)(b * L.IH) + ih0[i]) * (int32_t)L.IW * (int32_t)L.ld0 + iw0[i] * (int32_t)L.ld0;
         }
     }
-    __device__ __forceinline__ void load (int it, float4 (&v)[R])
+    __device__ __forceinline__ void load (int it, float4 (&v)[R][2])
     {
         typedef unsigned int uintx4 __attribute__ ((ext_vector_type (4)));
-        const uint32_t kc = (uint32_t)it * 8 + chunk, sel = kc - 3 * ((kc * 43u) >> 7);        // kc % 3 for kc < 128
-        const uintx4 raw = *(const uintx4 __attribute__ ((address_space (1))) *)(ktab + 2 * kc);
         #pragma unroll
-        for (int i = 0; i < R; i++)
+        for (int q = 0; q < 2; q++)
         {
-            const bool oka = (uint32_t)(ih0[i] + (int32_t)(raw[1] & 0xffffu)) < IH && (uint32_t)(iw0[i] + (int32_t)(raw[1] >> 16)) < IW;
-            const bool okb = (uint32_t)(ih0[i] + (int32_t)(raw[3] & 0xffffu)) < IH && (uint32_t)(iw0[i] + (int32_t)(raw[3] >> 16)) < IW;
-            const float4 a = in.ld4_if ((uint32_t)(base[i] + (int32_t)raw[0]), oka), b = in.ld4_if ((uint32_t)(base[i] + (int32_t)raw[2]), okb);
-            v[i].x = sel == 0 ? a.x : sel == 1 ? a.y : a.z;
-            v[i].y = sel == 0 ? a.y : sel == 1 ? a.z : b.x;
-            v[i].z = sel == 0 ? a.z : sel == 1 ? b.x : b.y;
-            v[i].w = sel == 0 ? b.x : sel == 1 ? b.y : b.z;
+            const uint32_t kc = (uint32_t)it * 8 + share.unit + 4 * q, sel = kc - 3 * ((kc * 43u) >> 7);        // kc % 3 for kc < 128
+            const uintx4 raw = *(const uintx4 __attribute__ ((address_space (1))) *)(ktab + 2 * kc);
+            #pragma unroll
+            for (int i = 0; i < R; i++)
+            {
+                const bool oka = (uint32_t)(ih0[i] + (int32_t)(raw[1] & 0xffffu)) < IH && (uint32_t)(iw0[i] + (int32_t)(raw[1] >> 16)) < IW;
+                const bool okb = (uint32_t)(ih0[i] + (int32_t)(raw[3] & 0xffffu)) < IH && (uint32_t)(iw0[i] + (int32_t)(raw[3] >> 16)) < IW;
+                const float4 a = in.ld4_if ((uint32_t)(base[i] + (int32_t)raw[0]), oka), b = in.ld4_if ((uint32_t)(base[i] + (int32_t)raw[2]), okb);
+                v[i][q].x = sel == 0 ? a.x : sel == 1 ? a.y : a.z;
+                v[i][q].y = sel == 0 ? a.y : sel == 1 ? a.z : b.x;
+                v[i][q].z = sel == 0 ? a.z : sel == 1 ? b.x : b.y;
+                v[i][q].w = sel == 0 ? b.x : sel == 1 ? b.y : b.z;
+            }
         }
-    }
-    __device__ __forceinline__ void store (float *lds, const float4 (&v)[R])
-    {
-        #pragma unroll
-        for (int i = 0; i < R; i++) st4 (lds + (row0 + 32 * i) * LDS_ROW + chunk * 4, v[i]);
     }
 };
 
@@ -665,44 +661,37 @@ __device__ __forceinline__ void gemm_core (ALoader &al, BLoader &bl, int kbase, 
 //   n = wn0 + 32 i + 8 (v / 4) + 4 (lane / 32) + v % 4,   m = wm0 + 32 j + lane % 32
 #define ACC_N(wn0, i, v, lane) ((wn0) + 32 * (i) + 8 * ((v) >> 2) + 4 * ((lane) >> 5) + ((v) & 3))
 
-struct NoStats { __device__ __forceinline__ void operator() (const float4 (&)[2]) const {} };
+struct NoStats { template <class V> __device__ __forceinline__ void operator() (const V &) const {} };
 
 // A layer norm folded into a matmul tile (aspen_hip_layer_t.norm_fold), second half: the K loop has left every thread
-// the sum and the sum of squares of its eight-th of two columns' K axis (thread t: columns t / 8 and t / 8 + 32, the
-// ActRowLoader's assignment).  The eight threads of a column add up, one of them writes the column's mean and
-// 1 / sqrt (variance + eps) behind the stage in LDS, and every lane corrects its sixteen sums:
+// the sum and the sum of squares of its quarter of one column's K axis (thread t: column t / 4, the SliceShare
+// assignment).  The four threads of a column add up, one of them writes the column's mean and
+// 1 / sqrt (variance + eps) behind the stages in LDS, and every lane corrects its sixteen sums:
 // acc = rstd[n] * (acc - mean[n] * rowsum[m]).  Same arithmetic for mean and variance as tile_layernorm.
-#define NORM_FOLD_STATS_OFFSET (128 * LDS_ROW)      // floats: behind the two operand blocks of the stage
+#define NORM_FOLD_STATS_OFFSET SPLIT_STAGES_FLOATS (VAR2_BN)      // floats
 template <int COH>
-__device__ __forceinline__ void norm_fold_finish (const aspen_hip_layer_t &L, floatx16 &acc, float (&cs)[2], float (&cq)[2], float *smem,
+__device__ __forceinline__ void norm_fold_finish (const aspen_hip_layer_t &L, floatx16 &acc, float cs, float cq, float *smem,
     uint32_t tid, uint32_t m0, uint32_t n0, uint32_t wm0, uint32_t wn0)
 {
+    static_assert (NORM_FOLD_STATS_OFFSET + 2 * VAR2_BN <= GEMM_SMEM_FLOATS, "column statistics fit behind the stages");
     const uint32_t lane = tid & 63;
     #pragma unroll
-    for (int o = 1; o < 8; o <<= 1)
-    {
-        #pragma unroll
-        for (int i = 0; i < 2; i++) { cs[i] += __shfl_xor (cs[i], o, 64); cq[i] += __shfl_xor (cq[i], o, 64); }
-    }
+    for (int o = 1; o < 4; o <<= 1) { cs += __shfl_xor (cs, o, 64); cq += __shfl_xor (cq, o, 64); }
     float *st = smem + NORM_FOLD_STATS_OFFSET;
-    if ((tid & 7u) == 0)
+    if ((tid & 3u) == 0)
     {
-        #pragma unroll
-        for (int i = 0; i < 2; i++)
+        const float mean = cs / (float)L.K;
+        const float var = cq / (float)L.K - mean * mean;
+        const uint32_t n = tid >> 2;
+        const float rstd = 1.0f / sqrtf (var + 1e-6f);
+        st[2 * n] = mean; st[2 * n + 1] = rstd;
+        // (row 0 of the layer that was asked to: the pairs go to memory as well, for a fused shortcut that needs the
+        // normalised matrix nobody writes any more)
+        if (L.norm_stats != nullptr && m0 == 0 && n0 + n < L.N)
         {
-            const float mean = cs[i] / (float)L.K;
-            const float var = cq[i] / (float)L.K - mean * mean;
-            const uint32_t n = (tid >> 3) + 32 * i;
-            const float rstd = 1.0f / sqrtf (var + 1e-6f);
-            st[2 * n] = mean; st[2 * n + 1] = rstd;
-            // (row 0 of the layer that was asked to: the pairs go to memory as well, for a fused shortcut that needs the
-            // normalised matrix nobody writes any more)
-            if (L.norm_stats != nullptr && m0 == 0 && n0 + n < L.N)
-            {
-                ActView<COH> sv;
-                sv.init (L.norm_stats, L.N, 2);
-                sv.st1 (2 * (n0 + n), mean); sv.st1 (2 * (n0 + n) + 1, rstd);
-            }
+            ActView<COH> sv;
+            sv.init (L.norm_stats, L.N, 2);
+            sv.st1 (2 * (n0 + n), mean); sv.st1 (2 * (n0 + n) + 1, rstd);
         }
     }
     // (the row sums are weights: requested before the barrier)
@@ -787,6 +776,93 @@ __device__ __forceinline__ void gemm_core_single_block (ALoader &al, BLoader &bl
 }
 
 
+// ---------------------------------------------------------------------------------------------
+// K loop of the contraction tiles.  Workgroup tile = (WM x 32) weight rows x BN activation rows; WM x WN wavefronts, each
+// owning 32 x (BN / WN) of it.  The activation row is the matrix instruction's row index and the weight row its column, so each
+// accumulator register holds 32 consecutive output channels of one output column: stores are 128-byte coalesced.
+//   weights      memory -> registers, in fragment order (WeightFragments); a step's registers are asked for again, one slice
+//                ahead, as soon as the step's matrix instructions have been issued
+//   activations  memory -> registers, two slices ahead -> split into three terms -> one of two LDS stages, a slice ahead ->
+//                fragments.  Every value is split once per tile (5.5 vector instructions) and read by WM wavefronts.
+// One barrier per slice: it publishes the stage written during the slice and frees the one read.
+// Per slice of a 128 x 64 tile a wavefront issues 24 matrix instructions (768 cycles), 44 vector instructions for the split, 12
+// fragment reads and 3 + 6 + 2 stores and requests.  1024 x 100 352 x 1024 as one launch: 205 TFLOP/s (64 x 64: 163,
+// 64 x 128: 181; requests one slice ahead instead of two 200; the wavefronts 2 x 2, every weight fetched by two of
+// them, 186); the single-precision matrix instruction's own limit is 157.
+// `ready` runs between the first request for the weights and the first one for the activations: a
+// kernel that starts tiles before their parents have finished (see the ordered mode of the persistent kernel) waits
+// there, with the tile's set-up done and its first weights on their way.
+// `before_last_slice` runs right before the last slice: the place to request what the epilogue
+// will need from memory, with the operand registers free and a whole slice of arithmetic to hide the latency.
+// `stats` sees every K slice of the activation operand once, as the registers it passes through on its way into LDS
+// (a folded layer norm's column sums, see norm_fold_finish).
+// ---------------------------------------------------------------------------------------------
+template <int BN, int WM, int WN, bool RAW, class BLoader, class Hook, class Ready, class Stats = NoStats>
+__device__ __forceinline__ void split_core (const void *weights, uint32_t first_block, uint32_t total_slices, BLoader &bl, int kbase, int kiters, char *smem,
+    floatx16 (&acc)[BN / WN / 32], bool phases, Hook before_last_slice, Ready ready, Stats stats = Stats ())
+{
+    static_assert (WM * WN == 4, "four wavefronts");
+    typedef SplitStage<BN> Stage;
+    constexpr int TN = BN / WN / 32, GROUPS = 2 * TN;
+    if (phases) tile_phase_lap (12);
+    const uint32_t tid = tile_thread (), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane (tid >> 6);
+    WeightFragments<RAW> w;
+    w.init (weights, first_block + wave % WM, total_slices, lane);
+    w.load (kbase, 0); w.load (kbase, 1);
+    ready ();
+    float4 areg[2][BLoader::R][2];          // slice it is fetched into set it % 2
+    const int last = kbase + kiters - 1;
+    bl.load (kbase, areg[0]);
+    bl.load (min (kbase + 1, last), areg[1]);
+    const uint32_t row = (wave / WM) * (BN / WN) + (lane & 31);
+    const uint32_t foff[2] = {Stage::offset (row, lane >> 5), Stage::offset (row, 2 + (lane >> 5))};
+    floatx16 lo[TN];
+    #pragma unroll
+    for (int i = 0; i < TN; i++)
+        #pragma unroll
+        for (int v = 0; v < 16; v++) { acc[i][v] = 0.f; lo[i][v] = 0.f; }
+    auto refill = [&] (int set, uint32_t stage) { bl.share.store (smem + stage, areg[set]); stats (areg[set]); };
+    refill (0, 0);
+    bl.load (min (kbase + 2, last), areg[0]);
+    lds_barrier ();
+    if (phases) tile_phase_lap (8);
+    __builtin_amdgcn_s_setprio (0);
+    // slice `it` (relative to kbase) sits in LDS at `stage`; MORE: the next one is split into the other stage meanwhile (from
+    // register set `set`, which then takes the slice two after it)
+    auto slice = [&] (int it, uint32_t stage, int set, auto more)
+    {
+        constexpr bool MORE = decltype (more)::value;
+        split8_t frag[2];
+        frag[0] = Stage::read (smem + stage, foff[0]);
+        #pragma unroll
+        for (int g = 0; g < GROUPS; g++)
+        {
+            const int step = g / TN, i = g % TN;
+            if (g + 1 < GROUPS) frag[(g + 1) & 1] = Stage::read (smem + stage, foff[(g + 1) / TN] + ((g + 1) % TN) * 32 * 64);
+            if (MORE && g == 0)
+            {
+                refill (set, stage ^ Stage::BYTES);
+                bl.load (min (kbase + it + 3, last), areg[set]);
+            }
+            split_mfma (frag[g & 1], w.operand (step), acc[i], lo[i]);
+            if (MORE && i == TN - 1) w.load (kbase + it + 1, step);
+        }
+        if (MORE) lds_barrier ();
+    };
+    int it = 0;
+    for (; it + 2 < kiters; it += 2) { slice (it, 0, 1, std::true_type ()); slice (it + 1, Stage::BYTES, 0, std::true_type ()); }
+    uint32_t stage = 0;
+    if (it + 1 < kiters) { slice (it, 0, 1, std::true_type ()); it++; stage = Stage::BYTES; }
+    before_last_slice ();
+    slice (it, stage, 0, std::false_type ());
+    __builtin_amdgcn_s_setprio (TILE_PRIO);
+    #pragma unroll
+    for (int i = 0; i < TN; i++)
+        #pragma unroll
+        for (int v = 0; v < 16; v++) acc[i][v] += lo[i][v];
+    lds_barrier ();          // the caller reuses the stages (epilogue)
+}
+
 // Shortcut fused into a contraction epilogue: fuse_out = fuse_act (v + fuse_in) for the (up to) four
 // channels m .. m+3 of column n; `left` = channels of the matrix from m on.  Same arithmetic, in the same
 // order, as a residual tile reading the stored v would do.
@@ -818,26 +894,28 @@ __device__ __forceinline__ void fused_shortcut (const aspen_hip_layer_t &L, cons
 // of the thread's pieces of a fused shortcut's operand (a tile has at most 128 columns: 8 pieces per thread)
 struct shortcut_prefetch_t { float4 s[8]; float4 bias; bool have, have_shortcut; };
 
-template <int BM, int BN, int WM, int WN, int DEPTH, int COH, unsigned FEAT, class Descriptor, class Ready>
+template <int BM, int BN, int WM, int WN, int COH, unsigned FEAT, class Descriptor, class Ready>
 __device__ __forceinline__ void contraction_mainloop (const aspen_hip_layer_t &L, Descriptor descriptor, uint32_t tn, uint32_t tm, int slice, float *smem, shortcut_prefetch_t &pre, Ready ready)
 {
-    constexpr int TM = BM / WM / 32, TN = BN / WN / 32;
-    constexpr bool SINGLE = TM * TN == 1 && BM == VAR2_BM && BN == VAR2_BN;     // the hand-scheduled loop of the 64 x 64 shape
+    static_assert (BM == WM * WEIGHT_BLOCK_ROWS, "one block of weight rows per wavefront");
+    constexpr int TN = BN / WN / 32;
+    constexpr bool SMALL = BM == VAR2_BM && BN == VAR2_BN, RAW = BM == VAR4_BM && BN == VAR4_BN;      // (the tall shape's weights stay floats in memory)
     const uint32_t tid = tile_thread (), lane = tid & 63, wave = tid >> 6;
     const uint32_t m0 = tm * BM, n0 = tn * BN;
-    floatx16 acc[TN][TM];
+    floatx16 acc[TN];
     ActView<COH> in;
     // (the operands' addresses come from loads of their own: taken from `L` they are parts of an 8-register piece of
     // the descriptor, which the compiler then keeps alive, spills and restores as a whole around every K slice)
     in.init (descriptor ().in0, L.in0_columns, L.ld0);
-    int kbase = 0, kiters = (int)(L.Kp / GEMM_BK);
+    const int total = (int)(L.Kp / SLICE_K);
+    int kbase = 0, kiters = total;
     if (slice >= 0)
     {
         kbase = slice * (int)L.kiters_per_split;
         kiters = min ((int)L.kiters_per_split, kiters - kbase);
     }
-    RowLoader<BM> al;
-    al.init (descriptor ().weight, m0, (L.M + 127u) / 128u * 128u, L.Kp, tid);
+    const void *weights = descriptor ().weight;
+    char *stages = reinterpret_cast<char *> (smem);
     // a fused shortcut's other operand comes from memory another XCD may have written: the first pieces this
     // thread will need in the epilogue (see contraction_epilogue for the thread -> piece mapping) are
     // requested under the last K slice
@@ -862,27 +940,26 @@ __device__ __forceinline__ void contraction_mainloop (const aspen_hip_layer_t &L
     };
     if (L.direct == ASPEN_HIP_OPERAND_DIRECT)
     {
-        ActRowLoader<BN, COH> bl;
-        bl.init (in, n0, L.N - 1, L.ld0, 0, tid);
-        if constexpr (SINGLE && (FEAT & TILES_NORM) != 0)
+        DirectLoader<BN, COH> bl;
+        bl.init (in, n0, L.N - 1, L.ld0, tid);
+        if constexpr (SMALL && (FEAT & TILES_NORM) != 0)
         {
             // (kernels for transformer graphs: the column sums a folded layer norm needs are gathered in every such tile,
             // sixteen additions and multiplications per K slice, and used where the layer asks for them)
-            float cs[2] = {0.f, 0.f}, cq[2] = {0.f, 0.f};
-            auto stats = [&] (const float4 (&b)[2])
+            float cs = 0.f, cq = 0.f;
+            auto stats = [&] (const float4 (&b)[1][2])
             {
                 #pragma unroll
                 for (int i = 0; i < 2; i++)
                 {
-                    cs[i] += (b[i].x + b[i].y) + (b[i].z + b[i].w);
-                    cq[i] += (b[i].x * b[i].x + b[i].y * b[i].y) + (b[i].z * b[i].z + b[i].w * b[i].w);
+                    cs += (b[0][i].x + b[0][i].y) + (b[0][i].z + b[0][i].w);
+                    cq += (b[0][i].x * b[0][i].x + b[0][i].y * b[0][i].y) + (b[0][i].z * b[0][i].z + b[0][i].w * b[0][i].w);
                 }
             };
-            gemm_core_single_block<DEPTH> (al, bl, kbase, kiters, smem, acc, COH != 0, fetch_shortcut, ready, stats);
-            if (L.norm_fold) norm_fold_finish<COH> (L, acc[0][0], cs, cq, smem, tid, m0, n0, (wave % 2) * 32, (wave / 2) * 32);
+            split_core<BN, WM, WN, RAW> (weights, tm * WM, total, bl, kbase, kiters, stages, acc, COH != 0, fetch_shortcut, ready, stats);
+            if (L.norm_fold) norm_fold_finish<COH> (L, acc[0], cs, cq, smem, tid, m0, n0, (wave % 2) * 32, (wave / 2) * 32);
         }
-        else if constexpr (SINGLE) gemm_core_single_block<DEPTH> (al, bl, kbase, kiters, smem, acc, COH != 0, fetch_shortcut, ready);
-        else gemm_core<BM, BN, WM, WN, DEPTH> (al, bl, kbase, kiters, smem, acc, COH != 0, fetch_shortcut, ready);
+        else split_core<BN, WM, WN, RAW> (weights, tm * WM, total, bl, kbase, kiters, stages, acc, COH != 0, fetch_shortcut, ready);
     }
     else if constexpr ((FEAT & TILES_GATHER) != 0)
     {
@@ -891,35 +968,33 @@ __device__ __forceinline__ void contraction_mainloop (const aspen_hip_layer_t &L
         {
             Dense3Loader<BN, COH> bl;
             bl.init (L, in, n0, tid);
-            if constexpr (SINGLE) gemm_core_single_block<DEPTH> (al, bl, kbase, kiters, smem, acc, COH != 0, fetch_shortcut, ready);
-            else gemm_core<BM, BN, WM, WN, DEPTH> (al, bl, kbase, kiters, smem, acc, COH != 0, fetch_shortcut, ready);
+            split_core<BN, WM, WN, RAW> (weights, tm * WM, total, bl, kbase, kiters, stages, acc, COH != 0, fetch_shortcut, ready);
         }
-        else if (SINGLE && L.IC % GEMM_BK != 0)
+        else if (SMALL && L.IC % SLICE_K != 0)
         {
-            if constexpr (SINGLE)
+            if constexpr (SMALL)
             {
                 ConvLoader<BN, COH, true> bl;
-                bl.init (L, in, n0, tid, kbase);
-                gemm_core_single_block<DEPTH> (al, bl, kbase, kiters, smem, acc, COH != 0, fetch_shortcut, ready);
+                bl.init (L, in, n0, tid, kbase, kiters);
+                split_core<BN, WM, WN, RAW> (weights, tm * WM, total, bl, kbase, kiters, stages, acc, COH != 0, fetch_shortcut, ready);
             }
         }
         else
         {
             ConvLoader<BN, COH, false> bl;
-            bl.init (L, in, n0, tid, kbase);
-            if constexpr (SINGLE) gemm_core_single_block<DEPTH> (al, bl, kbase, kiters, smem, acc, COH != 0, fetch_shortcut, ready);
-            else gemm_core<BM, BN, WM, WN, DEPTH> (al, bl, kbase, kiters, smem, acc, COH != 0, fetch_shortcut, ready);
+            bl.init (L, in, n0, tid, kbase, kiters);
+            split_core<BN, WM, WN, RAW> (weights, tm * WM, total, bl, kbase, kiters, stages, acc, COH != 0, fetch_shortcut, ready);
         }
     }
     if (COH) tile_phase_lap (9);
-    const uint32_t wm0 = (wave % WM) * (BM / WM), wn0 = (wave / WM) * (BN / WN);
+    const uint32_t wm0 = (wave % WM) * 32, wn0 = (wave / WM) * (BN / WN);
     if (slice >= 0)
     {
         // split-K: the raw sums go straight from the accumulators to this slice's block of the output tile, in the
         // accumulators' own layout (splitk_gather reads them back the same way): four 16-byte stores per lane, each
         // instruction 1 KB in one piece; no bias, no activation, no bounds, nothing to stage through LDS.  Only the
         // 64 x 64 and the 128 x 32 shape (one accumulator block per wavefront either way) are ever cut along K.
-        if constexpr (TM * TN == 1)
+        if constexpr (TN == 1)
         {
             const aspen_hip_layer_t L = descriptor ();
             const uint32_t tiles = L.tiles_m * L.tiles_n;
@@ -928,7 +1003,7 @@ __device__ __forceinline__ void contraction_mainloop (const aspen_hip_layer_t &L
             const uint32_t base = ((uint32_t)slice * tiles + tn * L.tiles_m + tm) * SPLITK_TILE_FLOATS + tid * 4;
             #pragma unroll
             for (int q = 0; q < 4; q++)
-                part.st4 (base + q * 4 * WG_THREADS, make_float4 (acc[0][0][4 * q], acc[0][0][4 * q + 1], acc[0][0][4 * q + 2], acc[0][0][4 * q + 3]));
+                part.st4 (base + q * 4 * WG_THREADS, make_float4 (acc[0][4 * q], acc[0][4 * q + 1], acc[0][4 * q + 2], acc[0][4 * q + 3]));
         }
         return;
     }
@@ -936,12 +1011,10 @@ __device__ __forceinline__ void contraction_mainloop (const aspen_hip_layer_t &L
     // [column][channel] for contraction_epilogue.
     constexpr int TROW = BM + 8;            // (4 * TROW) % 64 == 32: the two half-waves hit disjoint banks
     #pragma unroll
-    for (int j = 0; j < TM; j++)
+    for (int i = 0; i < TN; i++)
         #pragma unroll
-        for (int i = 0; i < TN; i++)
-            #pragma unroll
-            for (int v = 0; v < 16; v++)
-                smem[ACC_N (wn0, i, v, lane) * TROW + wm0 + 32 * j + (lane & 31)] = acc[i][j][v];
+        for (int v = 0; v < 16; v++)
+            smem[ACC_N (wn0, i, v, lane) * TROW + wm0 + (lane & 31)] = acc[i][v];
     __syncthreads ();
 }
 
@@ -1955,27 +2028,26 @@ __device__ __forceinline__ void narrow_gather_finish (const aspen_hip_layer_t &L
 }
 
 // Returns the thread's piece of the tile's sums over the K slices [kbase, kbase + kiters).
-// PF > 0 (kernels that start a tile before its parents have finished, with PF * 16 KB of LDS per workgroup): the
+// PF > 0 (kernels that start a tile before its parents have finished, with PF * 24 KB of LDS per workgroup): the
 // weights of a wavefront's first PF slices are requested BEFORE `ready ()`, straight from memory into LDS
 // (buffer_load ... lds: lane l's 16 bytes land at block + 16 l, so a lane later reads back exactly the fragment it
-// asked for; LDS serves as a per-lane buffer that costs no registers), and the activations of the first NARROW_B_WINDOW
-// of them are all requested together right after it, the rest as the window's registers come free: a tile of up to PF
-// slices per wavefront pays for one trip to memory after its parents have finished.  Slices beyond PF (and all slices when PF = 0) go through registers, two in flight.
-#define NARROW_PF_SLICES 4
-#define NARROW_B_WINDOW 4           // slices of activations in flight in registers
-#define NARROW_PF_SMEM_BYTES (4 * NARROW_PF_SLICES * 4 * 1024)
+// asked for; LDS serves as a per-lane buffer that costs no registers), and the activations of those slices are all
+// requested together right after it: a tile of up to PF slices per wavefront pays for one trip to memory after its
+// parents have finished.  Slices beyond PF (and all slices when PF = 0) go through registers, two in flight.
+#define NARROW_PF_SLICES 3
+#define NARROW_PF_SMEM_BYTES (4 * NARROW_PF_SLICES * SPLIT_SLICE_BYTES)
 template <int COH, int PF, class Descriptor, class Ready>
 __device__ __forceinline__ float4 narrow_mainloop (const aspen_hip_layer_t &L, Descriptor descriptor, uint32_t tn, uint32_t tm, int kbase, int kiters,
     float *smem, Ready ready)
 {
     const uint32_t tid = tile_thread (), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane (tid >> 6);
-    const uint32_t row = lane & 31, khalf = (lane >> 5) * 4;
+    const uint32_t row = lane & 31, unit0 = (lane >> 5) * 4;       // the lane's units of a slice start at floats unit0 (step 0) and 8 + unit0 (step 1)
     // this wavefront's share of the slices: a contiguous quarter
     const int per = (kiters + 3) >> 2, w0 = min ((int)wave * per, kiters), cnt = min (per, kiters - w0), first = kbase + w0;
-    // weights: one uniform base, 32-bit byte offsets
-    const float *wptr = descriptor ().weight;
-    const char __attribute__ ((address_space (1))) *wbase = (const char __attribute__ ((address_space (1))) *)wptr;
-    const uint32_t aoff = (((tm * VAR3_BM + row) * L.Kp) + (uint32_t)first * GEMM_BK + khalf) * 4u;
+    const uint32_t total = L.Kp / SLICE_K;
+    WeightFragments<false> w0r, w1r;
+    w0r.init (descriptor ().weight, tm, total, lane);
+    w1r = w0r;
     ActView<COH> in;
     in.init (descriptor ().in0, L.in0_columns, L.ld0);
     const bool direct = L.direct == ASPEN_HIP_OPERAND_DIRECT;
@@ -1985,128 +2057,113 @@ __device__ __forceinline__ float4 narrow_mainloop (const aspen_hip_layer_t &L, D
     // tap / channel the first slice starts at (stepped from there, as ConvLoader does)
     int32_t bbase, ih0 = 0, iw0 = 0;
     uint32_t kh = 0, kw = 0, c = 0;
-    if (direct) bbase = (int32_t)(n * L.ld0 + (uint32_t)first * GEMM_BK + khalf);
+    if (direct) bbase = (int32_t)(n * L.ld0 + (uint32_t)first * SLICE_K + unit0);
     else
     {
         const uint32_t ohw = L.OH * L.OW;
         const uint32_t b = fast_div (n, L.div_ohw), rem = n - b * ohw, oh = fast_div (rem, L.div_ow), ow = rem - oh * L.OW;
         ih0 = (int32_t)(oh * L.stride) - (int32_t)L.pad;
         iw0 = (int32_t)(ow * L.stride) - (int32_t)L.pad;
-        bbase = ((int32_t)(b * L.IH) + ih0) * (int32_t)L.IW * (int32_t)L.ld0 + iw0 * (int32_t)L.ld0 + (int32_t)khalf;
+        bbase = ((int32_t)(b * L.IH) + ih0) * (int32_t)L.IW * (int32_t)L.ld0 + iw0 * (int32_t)L.ld0 + (int32_t)unit0;
         // (K order: channel block, kh, kw, channel in block; see ConvLoader)
         const uint32_t taps = L.KH * L.KW, block = (uint32_t)first / taps, tap = (uint32_t)first - block * taps;
-        c = block * GEMM_BK;
+        c = block * SLICE_K;
         kh = tap / L.KW; kw = tap - kh * L.KW;
     }
     const uint32_t IH = L.IH, IW = L.IW, KH = L.KH, KW = L.KW, ld0 = L.ld0;
-    auto load_a = [&] (int i, float4 (&a)[4])
-    {
-        #pragma unroll
-        for (int sub = 0; sub < 4; sub++)
-        {
-            const floatx4 x = *(const floatx4 __attribute__ ((address_space (1))) *)(wbase + (aoff + (uint32_t)i * (GEMM_BK * 4u) + (uint32_t)sub * 32u));
-            a[sub] = make_float4 (x[0], x[1], x[2], x[3]);
-        }
-    };
-    // slices are asked for in ascending order: the tap position is stepped
+    // a slice's four pieces in unit order: floats +0, +16 (step 0), +8, +24 (step 1); slices are asked for in ascending
+    // order: the tap position is stepped
     auto load_b = [&] (int i, float4 (&bv)[4])
     {
         if (direct)
         {
             #pragma unroll
-            for (int sub = 0; sub < 4; sub++) bv[sub] = in.ld4 ((uint32_t)(bbase + i * GEMM_BK + sub * 8));
+            for (int q = 0; q < 4; q++) bv[q] = in.ld4 ((uint32_t)(bbase + i * SLICE_K + (q & 1) * 16 + (q >> 1) * 8));
         }
         else
         {
             const int32_t off = (int32_t)((kh * IW + kw) * ld0 + c);
             const bool ok = (uint32_t)(ih0 + (int32_t)kh) < IH && (uint32_t)(iw0 + (int32_t)kw) < IW;
             #pragma unroll
-            for (int sub = 0; sub < 4; sub++) bv[sub] = in.ld4_if ((uint32_t)(bbase + off + sub * 8), ok);
-            if (++kw == KW) { kw = 0; if (++kh == KH) { kh = 0; c += GEMM_BK; } }
+            for (int q = 0; q < 4; q++) bv[q] = in.ld4_if ((uint32_t)(bbase + off + (q & 1) * 16 + (q >> 1) * 8), ok);
+            if (++kw == KW) { kw = 0; if (++kh == KH) { kh = 0; c += SLICE_K; } }
         }
     };
-    floatx16 acc;
+    floatx16 acc, lo;
     #pragma unroll
-    for (int v = 0; v < 16; v++) acc[v] = 0.f;
-    auto mfmas = [&] (const float4 (&a)[4], const float4 (&bv)[4])
-    {
-        #pragma unroll
-        for (int sub = 0; sub < 4; sub++)
-        {
-            acc = __builtin_amdgcn_mfma_f32_32x32x2f32 (bv[sub].x, a[sub].x, acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_32x32x2f32 (bv[sub].y, a[sub].y, acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_32x32x2f32 (bv[sub].z, a[sub].z, acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_32x32x2f32 (bv[sub].w, a[sub].w, acc, 0, 0, 0);
-        }
-    };
-    constexpr uint32_t REGION = PF > 0 ? PF * 1024u : (uint32_t)(VAR3_BN * NARROW_ROW);     // floats of LDS per wavefront
+    for (int v = 0; v < 16; v++) acc[v] = lo[v] = 0.f;
+    constexpr uint32_t REGION = CMAX (PF * SPLIT_SLICE_BYTES / 4u, (uint32_t)(VAR3_BN * NARROW_ROW));     // floats of LDS per wavefront
     float *mine = smem + wave * REGION;
     int done = 0;       // slices of this wavefront's share that are finished
-    float4 a0[4], a1[4], b0[4], b1[4];
+    float4 b0[4], b1[4];
     if constexpr (PF > 0)
     {
-        const uint32_t Mp = (L.M + 127u) / 128u * 128u;
-        const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc ((void *)wptr, 0, (int)(Mp * L.Kp * 4u), 0x00020000);
+        const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc ((void *)w0r.base, 0, (int)(total * SPLIT_SLICE_BYTES), 0x00020000);
         #pragma unroll
         for (int i = 0; i < PF; i++)
             if (i < cnt)
             {
                 #pragma unroll
-                for (int sub = 0; sub < 4; sub++)
-                    __builtin_amdgcn_raw_ptr_buffer_load_lds (wr, (__attribute__ ((address_space (3))) void *)(mine + (i * 4 + sub) * 256), 16,
-                        (int)(aoff + (uint32_t)i * (GEMM_BK * 4u) + (uint32_t)sub * 32u), 0, 0, 0);
+                for (int q = 0; q < 6; q++)
+                    __builtin_amdgcn_raw_ptr_buffer_load_lds (wr, (__attribute__ ((address_space (3))) void *)(mine + (i * 6 + q) * 256), 16,
+                        (int)(lane * 16u), (int)((uint32_t)(first + i) * SPLIT_SLICE_BYTES + (uint32_t)q * 1024u), 0, 0);
             }
         ready ();
         // one straight-line body per number of prefetched slices (wave-uniform): every activation request is issued
         // before the first fragment is read back, so the slices' trips to memory overlap
         auto body = [&] (auto count)
         {
-            constexpr int C = decltype (count)::value, W = C < NARROW_B_WINDOW ? C : NARROW_B_WINDOW;
-            float4 bq[W][4];
+            constexpr int C = decltype (count)::value;
+            float4 bq[C][4];
             #pragma unroll
-            for (int i = 0; i < W; i++) load_b (i, bq[i]);
+            for (int i = 0; i < C; i++) load_b (i, bq[i]);
             #pragma unroll
             for (int i = 0; i < C; i++)
-            {
-                float4 af[4];
                 #pragma unroll
-                for (int sub = 0; sub < 4; sub++) af[sub] = ld4 (mine + (i * 4 + sub) * 256 + lane * 4);
-                mfmas (af, bq[i % W]);
-                if (i + W < C) load_b (i + W, bq[i % W]);       // the window moves on: this slice's registers take the slice W ahead
-            }
+                for (int step = 0; step < 2; step++)
+                {
+                    split8_t wf;
+                    const float *f = mine + (i * 6 + step * 3) * 256 + lane * 4;
+                    wf.h = *reinterpret_cast<const u32x4 *> (f); wf.m = *reinterpret_cast<const u32x4 *> (f + 256); wf.l = *reinterpret_cast<const u32x4 *> (f + 512);
+                    split_mfma (split8 (bq[i][2 * step], bq[i][2 * step + 1]), wf, acc, lo);
+                }
         };
-        static_assert (PF == 4, "one case per prefetched slice count");
+        static_assert (PF == 3, "one case per prefetched slice count");
         const int pre = __builtin_amdgcn_readfirstlane (min (cnt, PF));
-        if (pre == 4) body (std::integral_constant<int, 4> ());
-        else if (pre == 3) body (std::integral_constant<int, 3> ());
+        if (pre == 3) body (std::integral_constant<int, 3> ());
         else if (pre == 2) body (std::integral_constant<int, 2> ());
         else if (pre == 1) body (std::integral_constant<int, 1> ());
         done = min (cnt, PF);
-        if (done < cnt) { load_a (done, a0); load_b (done, b0); }
-        if (done + 1 < cnt) { load_a (done + 1, a1); load_b (done + 1, b1); }
+        if (done < cnt) { w0r.load (first + done, 0); w0r.load (first + done, 1); load_b (done, b0); }
+        if (done + 1 < cnt) { w1r.load (first + done + 1, 0); w1r.load (first + done + 1, 1); load_b (done + 1, b1); }
     }
     else
     {
         // two slices in flight: set 0 holds the even, set 1 the odd ones of this wavefront's share
-        if (cnt > 0) load_a (0, a0);
-        if (cnt > 1) load_a (1, a1);
+        if (cnt > 0) { w0r.load (first, 0); w0r.load (first, 1); }
+        if (cnt > 1) { w1r.load (first + 1, 0); w1r.load (first + 1, 1); }
         ready ();
         if (cnt > 0) load_b (0, b0);
         if (cnt > 1) load_b (1, b1);
     }
+    auto mfmas = [&] (const WeightFragments<false> &w, const float4 (&bv)[4])
+    {
+        #pragma unroll
+        for (int step = 0; step < 2; step++) split_mfma (split8 (bv[2 * step], bv[2 * step + 1]), w.operand (step), acc, lo);
+    };
     for (int i = done; i < cnt; i += 2)
     {
-        mfmas (a0, b0);
-        if (i + 2 < cnt) { load_a (i + 2, a0); load_b (i + 2, b0); }
+        mfmas (w0r, b0);
+        if (i + 2 < cnt) { w0r.load (first + i + 2, 0); w0r.load (first + i + 2, 1); load_b (i + 2, b0); }
         if (i + 1 < cnt)
         {
-            mfmas (a1, b1);
-            if (i + 3 < cnt) { load_a (i + 3, a1); load_b (i + 3, b1); }
+            mfmas (w1r, b1);
+            if (i + 3 < cnt) { w1r.load (first + i + 3, 0); w1r.load (first + i + 3, 1); load_b (i + 3, b1); }
         }
     }
     // the four wavefronts' sums meet in LDS: [wave][column][NARROW_ROW] (a wavefront's own region, which it has read empty)
     #pragma unroll
-    for (int v = 0; v < 16; v++) mine[ACC_N (0, 0, v, lane) * NARROW_ROW + row] = acc[v];
+    for (int v = 0; v < 16; v++) mine[ACC_N (0, 0, v, lane) * NARROW_ROW + row] = acc[v] + lo[v];
     __syncthreads ();
     const narrow_piece_t pc = narrow_piece (tid);
     float4 sum = ld4 (smem + pc.n * NARROW_ROW + pc.c);
@@ -2239,23 +2296,16 @@ __device__ __forceinline__ bool run_tile (Descriptor descriptor, uint32_t t, boo
             {
                 if (row_rep) __syncthreads ();      // the previous row tile's epilogue has read the stage this one refills
                 tm = tm * reps + row_rep;
-                if (more_rows) *more_rows = row_rep + 1 < reps;
+                if (more_rows) *more_rows = row_rep + 1 < reps && (tm + 1) * VAR0_BM < L.M;      // (row tiles that lie wholly behind the last row have no weights)
             }
             const auto ready_first = [&] () { if (row_rep == 0) ready (); };
-            contraction_mainloop<VAR0_BM, VAR0_BN, 2, 2, VAR0_DEPTH, COH, FEAT> (L, descriptor, tn, tm, -1, smem, pre, ready_first);
+            contraction_mainloop<VAR0_BM, VAR0_BN, 4, 1, COH, FEAT> (L, descriptor, tn, tm, -1, smem, pre, ready_first);
             c4_log2 = 5; bn = VAR0_BN;
         }
-        else if ((FEAT & TILES_WIDE) && L.variant == ASPEN_HIP_GEMM_WIDE) { contraction_mainloop<VAR1_BM, VAR1_BN, 2, 2, VAR1_DEPTH, COH, FEAT> (L, descriptor, tn, tm, -1, smem, pre, ready); bn = VAR1_BN; }
-        else if ((FEAT & TILES_TALL) && L.variant == ASPEN_HIP_GEMM_TALL) { contraction_mainloop<VAR4_BM, VAR4_BN, 4, 1, VAR4_DEPTH, COH, FEAT> (L, descriptor, tn, tm, slice, smem, pre, ready); c4_log2 = 5; bn = VAR4_BN; }
-        else if (FEAT & TILES_SMALL)
-        {
-            // two K slices in flight for the matmul layers of transformers, one for convolutional networks (see VAR2_DEPTH)
-            bool deep = false;
-            if constexpr ((FEAT & TILES_NORM) != 0) deep = (FEAT & TILES_GATHER) == 0 || L.type == MATMUL_LAYER;
-            if constexpr ((FEAT & TILES_NORM) != 0) { if (deep) contraction_mainloop<VAR2_BM, VAR2_BN, 2, 2, VAR2_DEPTH, COH, FEAT> (L, descriptor, tn, tm, slice, smem, pre, ready); }
-            if constexpr ((FEAT & TILES_GATHER) != 0) { if (!deep) contraction_mainloop<VAR2_BM, VAR2_BN, 2, 2, 1, COH, FEAT> (L, descriptor, tn, tm, slice, smem, pre, ready); }
-        }
-        
+        else if ((FEAT & TILES_WIDE) && L.variant == ASPEN_HIP_GEMM_WIDE) { contraction_mainloop<VAR1_BM, VAR1_BN, 2, 2, COH, FEAT> (L, descriptor, tn, tm, -1, smem, pre, ready); bn = VAR1_BN; }
+        else if ((FEAT & TILES_TALL) && L.variant == ASPEN_HIP_GEMM_TALL) { contraction_mainloop<VAR4_BM, VAR4_BN, 4, 1, COH, FEAT> (L, descriptor, tn, tm, slice, smem, pre, ready); c4_log2 = 5; bn = VAR4_BN; }
+        else if (FEAT & TILES_SMALL) contraction_mainloop<VAR2_BM, VAR2_BN, 2, 2, COH, FEAT> (L, descriptor, tn, tm, slice, smem, pre, ready);
+
         const aspen_hip_layer_t E = descriptor ();
         if (slice >= 0)
         {

@@ -85,6 +85,14 @@ void apu_load_dnn_data_from_file (aspen_dnn_t *dnn, char *input_path)
     aspen_load_weight_file (dnn, input_path);
 }
 
+static void free_device (aspen_layer_t *L)
+{
+    aspen_hip_free (L->d_weight); aspen_hip_free (L->d_weight_raw); aspen_hip_free (L->d_bias); aspen_hip_free (L->d_ktab);
+    aspen_hip_free (L->d_weight_ln); aspen_hip_free (L->d_bias_ln); aspen_hip_free (L->d_rowsum_ln);
+    L->d_weight = NULL; L->d_weight_raw = NULL; L->d_bias = NULL; L->d_ktab = NULL;
+    L->d_weight_ln = NULL; L->d_bias_ln = NULL; L->d_rowsum_ln = NULL;
+}
+
 void apu_destroy_dnn (aspen_dnn_t *dnn)
 {
     if (dnn == NULL) return;
@@ -97,7 +105,7 @@ void apu_destroy_dnn (aspen_dnn_t *dnn)
     {
         aspen_layer_t *L = &dnn->layers[i];
         free (L->weight.data); free (L->bias.data);
-        aspen_hip_free (L->d_weight); aspen_hip_free (L->d_bias); aspen_hip_free (L->d_ktab);
+        free_device (L);
     }
     free (dnn->layers);
     free (dnn);
@@ -137,11 +145,8 @@ static void ochw_to_ohwc (const float *src, float *dst, unsigned int O, unsigned
 static void invalidate_device (aspen_layer_t *L)
 {
     /* device graphs that were built from these buffers must not run again as they are */
-    if ((L->d_weight || L->d_bias || L->d_ktab) && L->dnn != NULL) L->dnn->dev_generation++;
-    aspen_hip_free (L->d_weight); aspen_hip_free (L->d_bias); aspen_hip_free (L->d_ktab);
-    aspen_hip_free (L->d_weight_ln); aspen_hip_free (L->d_bias_ln); aspen_hip_free (L->d_rowsum_ln);
-    L->d_weight = NULL; L->d_bias = NULL; L->d_ktab = NULL;
-    L->d_weight_ln = NULL; L->d_bias_ln = NULL; L->d_rowsum_ln = NULL;
+    if ((L->d_weight || L->d_weight_raw || L->d_bias || L->d_ktab) && L->dnn != NULL) L->dnn->dev_generation++;
+    free_device (L);
     /* (a layer norm's parameters are part of what the matmul layers behind it hold folded in) */
     if (L->type == LAYERNORM_LAYER && L->dnn != NULL)
         for (unsigned int i = 0; i < L->dnn->num_layers; i++)
@@ -338,8 +343,8 @@ unsigned int aspen_layer_kiters (const aspen_layer_t *L)
 }
 
 /* Uploads weight / bias / k-chunk table of one layer for a parent whose column stride is parent_ld
-   floats.  Idempotent; re-run after the weights changed. */
-int aspen_layer_to_device (aspen_layer_t *L, unsigned int parent_ld)
+   floats; raw: the weights as the tall tile shape reads them.  Idempotent; re-run after the weights changed. */
+int aspen_layer_to_device (aspen_layer_t *L, unsigned int parent_ld, int raw)
 {
     if (L->type == YOLO_LAYER)
     {
@@ -348,8 +353,10 @@ int aspen_layer_to_device (aspen_layer_t *L, unsigned int parent_ld)
         return aspen_hip_h2d (L->d_weight, L->anchors, 6 * sizeof (float));
     }
     if (L->weight.data == NULL) return 0;
-    if (L->d_weight != NULL && L->dev_in_ld == parent_ld) return 0;
-    invalidate_device (L);
+    float **weight = raw ? &L->d_weight_raw : &L->d_weight;
+    const int known = L->d_bias != NULL && L->dev_in_ld == parent_ld;      /* bias and table are there, perhaps the other form of the weights */
+    if (known && *weight != NULL) return 0;
+    if (!known) invalidate_device (L);
     const unsigned int *p = L->params;
     if (L->type == LAYERNORM_LAYER)
     {
@@ -367,8 +374,7 @@ int aspen_layer_to_device (aspen_layer_t *L, unsigned int parent_ld)
     const int dense3 = aspen_layer_dense3 (L);
     const unsigned int icp = dense3 ? 3 : round_up (ic, 4);
     const unsigned int kp = round_up (taps * icp, 32);
-    const unsigned int mp = round_up (L->gemm_m, 128);
-    float *staged = calloc ((size_t)mp * kp, sizeof (float));
+    float *staged = calloc ((size_t)L->gemm_m * kp, sizeof (float));
     if (staged == NULL) return -1;
     /* K order on the device.  Channel counts that are multiples of the K slice width: (channel block of 32, tap, channel
        in block), the order the kernels' stepping loader walks (consecutive slices are the taps of one channel block, whose
@@ -383,10 +389,10 @@ int aspen_layer_to_device (aspen_layer_t *L, unsigned int parent_ld)
                 for (unsigned int c = 0; c < ic; c += 32)
                     memcpy (staged + (size_t)m * kp + ((size_t)(c / 32) * taps + t) * 32, src + c, 32 * sizeof (float));
         }
-    L->d_weight = aspen_hip_alloc ((size_t)mp * kp * sizeof (float));
-    int rc = L->d_weight ? aspen_hip_h2d (L->d_weight, staged, (size_t)mp * kp * sizeof (float)) : -1;
+    *weight = aspen_hip_upload_weights (staged, L->gemm_m, kp, raw);
+    int rc = *weight == NULL ? -1 : 0;
     free (staged);
-    if (rc) return rc;
+    if (rc || known) return rc;
     L->d_bias = aspen_hip_alloc (L->gemm_m * sizeof (float));
     if (!L->d_bias || aspen_hip_h2d (L->d_bias, L->bias.data, L->gemm_m * sizeof (float))) return -1;
     if (dense3)
@@ -439,8 +445,8 @@ int aspen_layer_norm_fold_to_device (aspen_layer_t *L, const aspen_layer_t *norm
     if (L->d_weight_ln != NULL) return 0;
     if (L->type != MATMUL_LAYER || norm->type != LAYERNORM_LAYER || L->weight.data == NULL || norm->weight.data == NULL
         || norm->gemm_m != L->gemm_k) return -1;
-    const unsigned int M = L->gemm_m, K = L->gemm_k, kp = round_up (K, 32), mp = round_up (M, 128);
-    float *staged = calloc ((size_t)mp * kp, sizeof (float)), *bias = calloc (M, sizeof (float)), *rowsum = calloc (M, sizeof (float));
+    const unsigned int M = L->gemm_m, K = L->gemm_k, kp = round_up (K, 32);
+    float *staged = calloc ((size_t)M * kp, sizeof (float)), *bias = calloc (M, sizeof (float)), *rowsum = calloc (M, sizeof (float));
     int rc = -1;
     if (staged != NULL && bias != NULL && rowsum != NULL)
     {
@@ -459,12 +465,11 @@ int aspen_layer_norm_fold_to_device (aspen_layer_t *L, const aspen_layer_t *norm
             rowsum[m] = (float)rs;
             bias[m] = (float)((L->bias.data != NULL ? (double)L->bias.data[m] : 0.0) + sh);
         }
-        L->d_weight_ln = aspen_hip_alloc ((size_t)mp * kp * sizeof (float));
+        L->d_weight_ln = aspen_hip_upload_weights (staged, M, kp, 0);
         L->d_bias_ln = aspen_hip_alloc (M * sizeof (float));
         L->d_rowsum_ln = aspen_hip_alloc (M * sizeof (float));
         if (L->d_weight_ln && L->d_bias_ln && L->d_rowsum_ln)
-            rc = aspen_hip_h2d (L->d_weight_ln, staged, (size_t)mp * kp * sizeof (float))
-                || aspen_hip_h2d (L->d_bias_ln, bias, M * sizeof (float)) || aspen_hip_h2d (L->d_rowsum_ln, rowsum, M * sizeof (float));
+            rc = aspen_hip_h2d (L->d_bias_ln, bias, M * sizeof (float)) || aspen_hip_h2d (L->d_rowsum_ln, rowsum, M * sizeof (float));
     }
     free (staged); free (bias); free (rowsum);
     return rc;

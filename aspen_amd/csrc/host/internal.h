@@ -39,7 +39,8 @@ struct aspen_layer_t
     unsigned int gemm_m, gemm_k;              /* rows / contraction length of `weight` */
     float anchors[6];                         /* YOLO layers: (width, height) of the layer's three anchor boxes */
     /* device copies, created on first use */
-    float *d_weight, *d_bias;
+    float *d_weight, *d_bias;                 /* (contraction layers: weights in the kernels' order, see aspen_hip_upload_weights) */
+    float *d_weight_raw;                      /* the same as floats, for graphs that run the layer in the tall tile shape */
     aspen_hip_ktab_t *d_ktab;
     /* matmul layers whose parent is a layer norm that the engine folds into them (see fold_layernorms in nasm.c):
        weights with the norm's scale multiplied into their K axis, bias plus the weights applied to the norm's shift,
@@ -153,7 +154,7 @@ struct dse_group_t
 aspen_dnn_t *aspen_parse_cfg (const char *path);
 int aspen_layer_validate (aspen_dnn_t *dnn, aspen_layer_t *layer);
 /* dnn.c */
-int aspen_layer_to_device (aspen_layer_t *layer, unsigned int parent_ld);
+int aspen_layer_to_device (aspen_layer_t *layer, unsigned int parent_ld, int raw);
 int aspen_load_weight_file (aspen_dnn_t *dnn, const char *path);
 int aspen_layer_norm_fold_to_device (aspen_layer_t *L, const aspen_layer_t *norm);
 int aspen_layer_dense3 (const aspen_layer_t *layer);            /* three input channels: dense K axis on the device */

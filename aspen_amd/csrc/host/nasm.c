@@ -899,7 +899,7 @@ int aspen_nasm_to_device (nasm_t *nasm)
     {
         nasm_ldata_t *ld = &nasm->ldata_arr[l];
         if (ld->parent_ldata_idx[PARENT_0] < 0) continue;
-        if (aspen_layer_to_device (ld->layer, nasm->ldata_arr[ld->parent_ldata_idx[PARENT_0]].out_mat_stride)) return -1;
+        if (aspen_layer_to_device (ld->layer, nasm->ldata_arr[ld->parent_ldata_idx[PARENT_0]].out_mat_stride, is_contraction (ld->layer->type) && ld->variant == ASPEN_HIP_GEMM_TALL)) return -1;
         if (ld->folded_norm >= 0 && aspen_layer_norm_fold_to_device (ld->layer, nasm->ldata_arr[ld->folded_norm].layer)) return -1;
     }
     return 0;
@@ -935,7 +935,7 @@ int aspen_nasm_fill_device_layers (nasm_t *nasm, aspen_hip_layer_t *dst, uint32_
             const nasm_ldata_t *pl = &nasm->ldata_arr[ld->parent_ldata_idx[PARENT_1]];
             d->in1 = nasm->d_arena + pl->out_mat_offset; d->ld1 = pl->out_mat_stride;
         }
-        d->weight = L->d_weight; d->bias = L->d_bias; d->ktab = L->d_ktab;
+        d->weight = is_contraction (L->type) && ld->variant == ASPEN_HIP_GEMM_TALL ? L->d_weight_raw : L->d_weight; d->bias = L->d_bias; d->ktab = L->d_ktab;
         d->K = L->gemm_k; d->Kp = L->dev_kp;
         d->IH = p[IN_H]; d->IW = p[IN_W]; d->IC = p[IN_C]; d->OH = p[OUT_H]; d->OW = p[OUT_W];
         d->KH = p[WEIGHT_H]; d->KW = p[WEIGHT_W]; d->stride = p[STRIDE]; d->pad = p[PADDING];

@@ -189,7 +189,7 @@ static int rebuild_graph (rpool_t *rp)
                 if (cursor[i] < g->num_ninst) { roots[nroots++] = base[i] + cursor[i]++; progress = 1; }
             }
         }
-        rp->graph = aspen_hip_graph_create (L, layers, nl, np, co, ci, ninst, roots, nroots);
+        rp->graph = aspen_hip_graph_create_prepared (L, layers, nl, np, co, ci, ninst, roots, nroots);
         if (rp->graph == NULL) rc = -1;
         else
         {

@@ -59,8 +59,8 @@ enum { ASPEN_HIP_ATTENTION_FUSED = 1 };
    builder asks aspen_hip_tile_shapes for the numbers instead of assuming them. */
 enum { ASPEN_HIP_GEMM_LARGE = 0, ASPEN_HIP_GEMM_WIDE = 1, ASPEN_HIP_GEMM_SMALL = 2, ASPEN_HIP_GEMM_NARROW = 3, ASPEN_HIP_GEMM_TALL = 4, ASPEN_HIP_NUM_GEMM_VARIANTS };
 /* shapes[2*v] = rows, shapes[2*v+1] = columns of GEMM variant v = 0..2; shapes[6] = queries per K-attention
-   tile; shapes[7] = queries per V-attention tile; shapes[8] = workgroups per compute unit the
-   kernels are built for; shapes[9], shapes[10] = rows, columns of variant 3; shapes[11], shapes[12] = of variant 4.  Pure
+   tile; shapes[7] = queries per V-attention tile; shapes[8] = workgroups per compute unit that
+   every kernel leaves room for; shapes[9], shapes[10] = rows, columns of variant 3; shapes[11], shapes[12] = of variant 4.  Pure
    constants: callable without a GPU. */
 void aspen_hip_tile_shapes (uint32_t shapes[13]);
 
@@ -163,6 +163,12 @@ int aspen_hip_dense_device_to_host (float *dst_host, const float *src, uint32_t 
    calibration point for a profiler's HBM byte counters. */
 int aspen_hip_copy (void *dst, const void *src, size_t bytes);
 
+/* ---- weights --------------------------------------------------------------------------------- */
+/* Device copy of a contraction layer's weights in the order the kernels read them, from M rows of Kp floats on the host
+   (Kp a multiple of 32; K order as for aspen_hip_layer_t.weight).  raw = 0: each float as three bfloat16 terms that add up to it exactly (6
+   bytes), for every tile shape but TALL; raw = 1: floats, for TALL.  NULL on failure; released with aspen_hip_free. */
+void *aspen_hip_upload_weights (const float *rows, uint32_t M, uint32_t Kp, int raw);
+
 /* ---- graph ----------------------------------------------------------------------------------- */
 /* Uploads a tile graph.  ninst_layer[i] = layer of tile i; num_parents[i] = its dependency count;
    children of tile i are child_idx[child_off[i] .. child_off[i+1]).  roots = tiles with no parent
@@ -170,6 +176,11 @@ int aspen_hip_copy (void *dst, const void *src, size_t bytes);
    aspen_hip_layer_t.splits) all carry the same child list, and a child counts the whole group as
    ONE parent: whichever member finishes last releases it.  (reference: ninst_t, include/nasm.h:50-66) */
 aspen_hip_graph_t *aspen_hip_graph_create (const aspen_hip_layer_t *layers, uint32_t num_layers,
+    const uint32_t *ninst_layer, const uint32_t *num_parents, const uint32_t *child_off,
+    const uint32_t *child_idx, uint32_t num_ninst, const uint32_t *roots, uint32_t num_roots);
+/* The same for layers whose `weight` (contraction layers) is an aspen_hip_upload_weights copy, which several graphs may
+   share.  aspen_hip_graph_create makes such copies of the row-major weights it is given and keeps them with the graph. */
+aspen_hip_graph_t *aspen_hip_graph_create_prepared (const aspen_hip_layer_t *layers, uint32_t num_layers,
     const uint32_t *ninst_layer, const uint32_t *num_parents, const uint32_t *child_off,
     const uint32_t *child_idx, uint32_t num_ninst, const uint32_t *roots, uint32_t num_roots);
 void aspen_hip_graph_destroy (aspen_hip_graph_t *graph);

@@ -1076,3 +1076,57 @@ def test_weights_reloaded_between_runs_are_used_by_the_next_run(gpu, mode, tmp_p
         assert H.rel_l2(want2[-1], want[-1]) > 1e-2           # the two weight sets do give different results
     finally:
         net.close()
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 1, 32), (31, 33, 64), (63, 65, 96), (64, 64, 128), (65, 63, 160), (129, 127, 1056), (300, 200, 4096)])
+def test_three_term_products_keep_single_precision(gpu, M, N, K):
+    """Every float enters a contraction as three bfloat16 terms that add up to it, six of the nine partial products are
+    summed in single precision (the other three are below 2^-25 of the product), so an output differs from the exact sum by at
+    most (roundings of the running sums) x 2^-24 x sum |a b|: one rounding per 16 K positions in each of the two running sums
+    (the matrix core may round its 16-term sums once more), the dropped products and the last additions.  Magnitudes
+    over 2^-20 .. 2^20 and all K remainders of the two-slice loop."""
+    import ctypes as C
+    L = api.lib()
+    rng = np.random.default_rng(M * 1000003 + N * 1009 + K)
+    A = (rng.standard_normal((M, K)) * 2.0 ** rng.integers(-20, 21, (M, K))).astype(np.float32)
+    B = (rng.standard_normal((N, K)) * 2.0 ** rng.integers(-20, 21, (N, K))).astype(np.float32)
+    ldc = -(-M // 4) * 4
+    bufs = [L.aspen_hip_alloc(x) for x in (A.nbytes, B.nbytes, N * ldc * 4)]
+    try:
+        assert all(bufs)
+        assert L.aspen_hip_h2d(bufs[0], A.ctypes.data_as(C.c_void_p), A.nbytes) == 0
+        assert L.aspen_hip_h2d(bufs[1], B.ctypes.data_as(C.c_void_p), B.nbytes) == 0
+        assert L.aspen_hip_sgemm(M, N, K, bufs[0], K, bufs[1], K, bufs[2], ldc, None, 0) == 0
+        out = np.zeros((N, ldc), dtype=np.float32)
+        assert L.aspen_hip_d2h(out.ctypes.data_as(C.c_void_p), bufs[2], out.nbytes) == 0
+    finally:
+        for b in bufs:
+            L.aspen_hip_free(b)
+    A64, B64 = A.astype(np.float64), B.astype(np.float64)
+    exact, scale = B64 @ A64.T, np.abs(B64) @ np.abs(A64).T
+    bound = (2 * (K // 16) + 4) * 2.0 ** -24 * scale
+    assert np.all(np.abs(out[:, :M] - exact) <= bound), np.max(np.abs(out[:, :M] - exact) / bound)
+    assert np.all(out[:, M:] == 0)
+
+
+@pytest.mark.parametrize("mode", [api.MODE_LAYERS, api.MODE_DATAFLOW], ids=["layers", "dataflow"])
+def test_row_groups_end_at_the_last_row_tile(gpu, mode):
+    """320 output channels under the 128 x 64 shape in groups of two row tiles: the second group's second row tile lies wholly
+    behind the last row (and behind the padded weights) and must not run."""
+    from oracle import cpu
+    cfg = ("[net]\nheight=64\nwidth=64\nchannels=64\n\n"
+           "[convolutional]\nfilters=320\nsize=1\nstride=1\npad=0\nactivation=relu\n\n"
+           "[convolutional]\nfilters=64\nsize=1\nstride=1\npad=0\nactivation=relu\n\n")
+    layers = M.parse_cfg(cfg)
+    tens = M.synth_weights(layers, 62, "he")
+    x = (M.synth_input(layers, 62, 32, 0, "token_ids") * 2.0 - 1.0).astype(np.float32)
+    outs = cpu.run_network(layers, tens, x, 32, 0)
+    net = H.GpuNet(cfg, tens, 32, 0, min_ninst=2048, mode=mode)
+    try:
+        net.run(x)
+        assert net.nasm.info(1)["tile_H"] == 256
+        for l in (1, 2):
+            err = H.rel_l2(net.layer(l), outs[l])
+            assert err <= H.REL_L2_TOL, f"layer {l}: rel L2 {err:.3g}"
+    finally:
+        net.close()
