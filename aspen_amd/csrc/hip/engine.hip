@@ -617,6 +617,7 @@ static unsigned graph_features (const aspen_hip_layer_t *layers, uint32_t num_la
             if (L.variant == ASPEN_HIP_GEMM_NARROW) { f |= TILES_NARROW; break; }      // (brings its own operand loaders)
             f |= L.variant == ASPEN_HIP_GEMM_LARGE ? TILES_LARGE : L.variant == ASPEN_HIP_GEMM_WIDE ? TILES_WIDE : L.variant == ASPEN_HIP_GEMM_TALL ? TILES_TALL : TILES_SMALL;
             if (L.direct != ASPEN_HIP_OPERAND_DIRECT) f |= TILES_GATHER;
+            if (L.direct == ASPEN_HIP_OPERAND_DENSE3 && L.variant == ASPEN_HIP_GEMM_WIDE) f |= TILES_DENSE_WIDE;
             break;
         case K_ATTENTION_LAYER: case V_ATTENTION_LAYER: f |= TILES_ATTENTION; break;
         case LAYERNORM_LAYER: case SOFTMAX_LAYER: f |= TILES_NORM; break;

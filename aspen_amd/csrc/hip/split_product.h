@@ -58,12 +58,13 @@ __device__ __forceinline__ void split_mfma (const split8_t &a, const split8_t &b
 {
     const bf16x8 ah = __builtin_bit_cast (bf16x8, a.h), am = __builtin_bit_cast (bf16x8, a.m), al = __builtin_bit_cast (bf16x8, a.l);
     const bf16x8 bh = __builtin_bit_cast (bf16x8, b.h), bm = __builtin_bit_cast (bf16x8, b.m), bl = __builtin_bit_cast (bf16x8, b.l);
-    hi = __builtin_amdgcn_mfma_f32_32x32x16_bf16 (ah, bh, hi, 0, 0, 0);
+    // (neighbouring instructions share an operand: 1 % at the power limit over an order that changes both)
     lo = __builtin_amdgcn_mfma_f32_32x32x16_bf16 (al, bh, lo, 0, 0, 0);
-    lo = __builtin_amdgcn_mfma_f32_32x32x16_bf16 (ah, bl, lo, 0, 0, 0);
-    lo = __builtin_amdgcn_mfma_f32_32x32x16_bf16 (am, bm, lo, 0, 0, 0);
+    hi = __builtin_amdgcn_mfma_f32_32x32x16_bf16 (ah, bh, hi, 0, 0, 0);
     lo = __builtin_amdgcn_mfma_f32_32x32x16_bf16 (am, bh, lo, 0, 0, 0);
+    lo = __builtin_amdgcn_mfma_f32_32x32x16_bf16 (am, bm, lo, 0, 0, 0);
     lo = __builtin_amdgcn_mfma_f32_32x32x16_bf16 (ah, bm, lo, 0, 0, 0);
+    lo = __builtin_amdgcn_mfma_f32_32x32x16_bf16 (ah, bl, lo, 0, 0, 0);
 }
 
 // Order of the K axis inside a slice of 32 (both operands have to agree, the sum does not care): a lane of a matrix

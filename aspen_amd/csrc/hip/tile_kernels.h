@@ -280,8 +280,8 @@ template <int ROWS, int COH> struct DirectLoader
 // Implicit-GEMM activation operand of conv / FC: row n = output position (b, oh, ow); the K axis runs
 // over (kh, kw, ic) and is resolved through the layer's k-chunk table.  Replaces the reference's
 // pointer table + panel gather (prepare_input / load_im2col_ptr, reference src/tiled_kernels.c:3-159).
-// TABLE: the K axis is resolved through the layer's k-chunk table (channel counts that are not multiples of the slice
-// width, where a slice straddles taps; 64 x 64 tiles only, the host's tile policy sees to that).  Otherwise a whole
+// TableLoader: the K axis is resolved through the layer's k-chunk table (channel counts that are not multiples of the slice
+// width, where a slice straddles taps; 64 x 64 tiles only, the host's tile policy sees to that).  StepLoader: a whole
 // slice belongs to one tap, found with a few scalar operations: fetching the table entry instead puts a dependent
 // memory access in front of the operand loads of every slice.  Two loaders, not one with a branch: with both
 // paths in one K loop the compiler waits for ALL outstanding loads wherever they join.
@@ -290,7 +290,78 @@ template <int ROWS, int COH> struct DirectLoader
 // slice mostly re-reads what the previous one or the one KW before it fetched, while it is still in the caches; with
 // the taps outermost (the reference's order) a tap's data came round again only after a whole pass over the channels,
 // by which time a busy L2 had replaced it, and a 3 x 3 layer fetched its input up to nine times over the fabric.
-template <int ROWS, int COH, bool TABLE> struct ConvLoader
+// An operand read in place (matmul, 1x1 convolution) is the stepping form with a window of one tap over images of one
+// pixel, and shares its K loop: code the persistent kernel's instruction cache holds once.
+template <int ROWS, int COH> struct StepLoader
+{
+    static constexpr int R = SliceShare<ROWS>::R;
+    SliceShare<ROWS> share;
+    ActView<COH> in;
+    int32_t base[R], ih0[R], iw0[R];
+    uint32_t IH, IW;
+    uint32_t KH, KW, ld0;
+    uint32_t kh, kw, c;                     // tap and channel the next slice asked for starts at
+    int left;                               // slices from that one to the end of the K range
+    // first_it: the first of the `count` K slices that will be asked for, in ascending order
+    __device__ __forceinline__ void init (const aspen_hip_layer_t &L, const ActView<COH> &v, uint32_t first_row, uint32_t tid, int first_it, int count)
+    {
+        in = v; ld0 = L.ld0;
+        share.init (tid);
+        left = count; kh = kw = 0;
+        if (L.direct == ASPEN_HIP_OPERAND_DIRECT)
+        {
+            IH = IW = KH = KW = 1;
+            c = (uint32_t)first_it * SLICE_K;
+            #pragma unroll
+            for (int i = 0; i < R; i++)
+            {
+                const uint32_t n = first_row + share.row0 + 64 * i;
+                ih0[i] = iw0[i] = 0;
+                base[i] = (int32_t)((n < L.N ? n : L.N - 1) * ld0 + share.unit * 4);
+            }
+            return;
+        }
+        IH = L.IH; IW = L.IW; KH = L.KH; KW = L.KW; c = 0;
+        if (first_it)
+        {
+            const uint32_t taps = KH * KW, block = (uint32_t)first_it / taps, tap = (uint32_t)first_it - block * taps;
+            c = block * SLICE_K;
+            kh = tap / KW; kw = tap - kh * KW;
+        }
+        const uint32_t ohw = L.OH * L.OW;
+        #pragma unroll
+        for (int i = 0; i < R; i++)
+        {
+            uint32_t n = first_row + share.row0 + 64 * i;
+            n = n < L.N ? n : L.N - 1;
+            uint32_t b = fast_div (n, L.div_ohw), rem = n - b * ohw, oh = fast_div (rem, L.div_ow), ow = rem - oh * L.OW;
+            ih0[i] = (int32_t)(oh * L.stride) - (int32_t)L.pad;
+            iw0[i] = (int32_t)(ow * L.stride) - (int32_t)L.pad;
+            base[i] = ((int32_t)(b * L.IH) + ih0[i]) * (int32_t)L.IW * (int32_t)L.ld0 + iw0[i] * (int32_t)L.ld0 + (int32_t)share.unit * 4;
+        }
+    }
+    // Slices are asked for in ascending order from the one init was told, so the position is stepped, not divided
+    // out, and `it` is not looked at.  It stays on the last slice: the K loops ask for that one again behind the end
+    // of the K range and drop the answer.
+    __device__ __forceinline__ void load (int it, float4 (&v)[R][2])
+    {
+        const int32_t offset = (int32_t)((kh * IW + kw) * ld0 + c);
+        #pragma unroll
+        for (int i = 0; i < R; i++)
+        {
+            const bool ok = (uint32_t)(ih0[i] + (int32_t)kh) < IH && (uint32_t)(iw0[i] + (int32_t)kw) < IW;
+            v[i][0] = in.ld4_if ((uint32_t)(base[i] + offset), ok);
+            v[i][1] = in.ld4_if ((uint32_t)(base[i] + offset + 16), ok);
+        }
+        // (selects, no branches: the K loop around it stays one block)
+        left--;
+        const uint32_t kw1 = kw + 1 == KW ? 0u : kw + 1, kh1 = kw1 ? kh : kh + 1, kh2 = kh1 == KH ? 0u : kh1, c1 = kh1 == KH ? c + SLICE_K : c;
+        kw = left > 0 ? kw1 : kw; kh = left > 0 ? kh2 : kh; c = left > 0 ? c1 : c;
+    }
+};
+
+// The same through the k-chunk table.
+template <int ROWS, int COH> struct TableLoader
 {
     static constexpr int R = SliceShare<ROWS>::R;
     SliceShare<ROWS> share;
@@ -298,27 +369,10 @@ template <int ROWS, int COH, bool TABLE> struct ConvLoader
     const aspen_hip_ktab_t *ktab;
     int32_t base[R], ih0[R], iw0[R];
     uint32_t IH, IW;
-    uint32_t KH, KW, ld0;
-    uint32_t kh, kw, c;                     // tap and channel the next slice asked for starts at (!TABLE)
-    int left;                               // slices from that one to the end of the K range
-    // first_it: the first of the `count` K slices that will be asked for, in ascending order
-    __device__ __forceinline__ void init (const aspen_hip_layer_t &L, const ActView<COH> &v, uint32_t first_row, uint32_t tid, int first_it, int count)
+    __device__ __forceinline__ void init (const aspen_hip_layer_t &L, const ActView<COH> &v, uint32_t first_row, uint32_t tid)
     {
-        in = v; IH = L.IH; IW = L.IW;
+        in = v; IH = L.IH; IW = L.IW; ktab = L.ktab;
         share.init (tid);
-        if (TABLE) ktab = L.ktab;
-        else
-        {
-            KH = L.KH; KW = L.KW; ld0 = L.ld0;
-            kh = kw = c = 0;
-            left = count;
-            if (first_it)
-            {
-                const uint32_t taps = KH * KW, block = (uint32_t)first_it / taps, tap = (uint32_t)first_it - block * taps;
-                c = block * SLICE_K;
-                kh = tap / KW; kw = tap - kh * KW;
-            }
-        }
         const uint32_t ohw = L.OH * L.OW;
         #pragma unroll
         for (int i = 0; i < R; i++)
@@ -333,40 +387,24 @@ template <int ROWS, int COH, bool TABLE> struct ConvLoader
     }
     __device__ __forceinline__ void load (int it, float4 (&v)[R][2])
     {
-        if (TABLE)
-        {
-            typedef unsigned int uintx2 __attribute__ ((ext_vector_type (2)));
-            #pragma unroll
-            for (int q = 0; q < 2; q++)
-            {
-                const uintx2 raw = *(const uintx2 __attribute__ ((address_space (1))) *)(ktab + it * 8 + share.unit + 4 * q);
-                const int32_t kh_ = (int32_t)(raw[1] & 0xffffu), kw_ = (int32_t)(raw[1] >> 16);
-                #pragma unroll
-                for (int i = 0; i < R; i++)
-                {
-                    const bool ok = (uint32_t)(ih0[i] + kh_) < IH && (uint32_t)(iw0[i] + kw_) < IW;
-                    v[i][q] = in.ld4_if ((uint32_t)(base[i] + (int32_t)raw[0]), ok);
-                }
-            }
-            return;
-        }
-        // Slices are asked for in ascending order from the one init was told, so the position is stepped, not divided
-        // out, and `it` is not looked at.  It stays on the last slice: the K loops ask for that one again behind the end
-        // of the K range and drop the answer.
-        const int32_t offset = (int32_t)((kh * IW + kw) * ld0 + c + share.unit * 4);
+        typedef unsigned int uintx2 __attribute__ ((ext_vector_type (2)));
         #pragma unroll
-        for (int i = 0; i < R; i++)
+        for (int q = 0; q < 2; q++)
         {
-            const bool ok = (uint32_t)(ih0[i] + (int32_t)kh) < IH && (uint32_t)(iw0[i] + (int32_t)kw) < IW;
-            v[i][0] = in.ld4_if ((uint32_t)(base[i] + offset), ok);
-            v[i][1] = in.ld4_if ((uint32_t)(base[i] + offset + 16), ok);
+            const uintx2 raw = *(const uintx2 __attribute__ ((address_space (1))) *)(ktab + it * 8 + share.unit + 4 * q);
+            const int32_t kh = (int32_t)(raw[1] & 0xffffu), kw = (int32_t)(raw[1] >> 16);
+            #pragma unroll
+            for (int i = 0; i < R; i++)
+            {
+                const bool ok = (uint32_t)(ih0[i] + kh) < IH && (uint32_t)(iw0[i] + kw) < IW;
+                v[i][q] = in.ld4_if ((uint32_t)(base[i] + (int32_t)raw[0]), ok);
+            }
         }
-        if (--left > 0) { if (++kw == KW) { kw = 0; if (++kh == KH) { kh = 0; c += SLICE_K; } } }
     }
 };
 
 // Implicit-GEMM operand of a convolution over THREE input channels (a network's first layer on RGB images) with a
-// dense K axis: K order (tap, channel) without the padding to four channels per tap that ConvLoader's layout has
+// dense K axis: K order (tap, channel) without the padding to four channels per tap that TableLoader's layout has
 // (ASPEN_HIP_OPERAND_DENSE3; the stem of ResNet-50 contracts 160 instead of 224, VGG-16's first layer 32 instead of
 // 64).  A chunk of four K positions spans two pixels: both are fetched (16 bytes each, the pixels of the matrix keep
 // their padded fourth float) and the chunk is put together from the last channels of the first and the first
@@ -500,13 +538,14 @@ struct NoHook { __device__ __forceinline__ void operator() () const {} };
 // cache, and a transformer graph has no use for the convolution loaders' K loops, nor a ResNet for the attention tiles.
 enum : unsigned
 {
-    TILES_GATHER = 1u,          // contraction operands gathered through ConvLoader (convolutions, FC layers over images)
+    TILES_GATHER = 1u,          // contraction operands gathered through StepLoader (convolutions, FC layers over images)
     TILES_LARGE = 2u, TILES_WIDE = 4u, TILES_SMALL = 8u,       // contraction tile shapes
     TILES_ATTENTION = 16u, TILES_NORM = 32u /* layernorm, softmax */, TILES_POOL = 64u, TILES_YOLO = 128u /* yolo, append */,
     TILES_RESIDUAL = 256u,
     TILES_NARROW = 512u,        // the 32 x 32 contraction tile of latency-bound graphs
     TILES_TALL = 1024u,         // the 128 x 32 contraction tile of weight-streaming layers
-    TILES_ALL = 2047u,
+    TILES_DENSE_WIDE = 2048u,   // the dense three-channel operand under the 64 x 128 shape (the host library's graphs take 64 x 64 for it)
+    TILES_ALL = 4095u,
     TILES_CONVNET = TILES_GATHER | TILES_LARGE | TILES_WIDE | TILES_SMALL | TILES_POOL | TILES_RESIDUAL,
     TILES_TRANSFORMER = TILES_SMALL | TILES_ATTENTION | TILES_NORM | TILES_RESIDUAL
 };
@@ -785,6 +824,10 @@ __device__ __forceinline__ void gemm_core_single_block (ALoader &al, BLoader &bl
 //   activations  memory -> registers, two slices ahead -> split into three terms -> one of two LDS stages, a slice ahead ->
 //                fragments.  Every value is split once per tile (5.5 vector instructions) and read by WM wavefronts.
 // One barrier per slice: it publishes the stage written during the slice and frees the one read.
+// The loop exists once per shape and operand kind, and each copy counts: the kernel for convolutional networks was 101 KB with nine of
+// them (reading in place apart from stepping, the three-channel and table operands under two shapes) and is 73 KB with five:
+// ResNet-50 batch 32 2.24 -> 2.10 ms, batch 8 of YOLO-v3 4.63 -> 4.42 (the instruction cache holds 64 KB).  A rolled loop (one slice per trip, requests one
+// slice ahead) saves another 9 KB and is slower where few workgroups share a compute unit: BERT-base 3 x 75 1.00 -> 1.07 ms.
 // Per slice of a 128 x 64 tile a wavefront issues 24 matrix instructions (768 cycles), 44 vector instructions for the split, 12
 // fragment reads and 3 + 6 + 2 stores and requests.  1024 x 100 352 x 1024 as one launch: 205 TFLOP/s (64 x 64: 163,
 // 64 x 128: 181; requests one slice ahead instead of two 200; the wavefronts 2 x 2, every weight fetched by two of
@@ -803,17 +846,19 @@ __device__ __forceinline__ void split_core (const void *weights, uint32_t first_
 {
     static_assert (WM * WN == 4, "four wavefronts");
     typedef SplitStage<BN> Stage;
-    constexpr int TN = BN / WN / 32, GROUPS = 2 * TN;
+    // AHEAD: slices of activations in flight from memory (two register sets of 8 R do not fit beside the wide shape's sums: its loops
+    // spilled)
+    constexpr int TN = BN / WN / 32, GROUPS = 2 * TN, AHEAD = BLoader::R > 1 ? 1 : 2;
     if (phases) tile_phase_lap (12);
     const uint32_t tid = tile_thread (), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane (tid >> 6);
     WeightFragments<RAW> w;
     w.init (weights, first_block + wave % WM, total_slices, lane);
     w.load (kbase, 0); w.load (kbase, 1);
     ready ();
-    float4 areg[2][BLoader::R][2];          // slice it is fetched into set it % 2
+    float4 areg[AHEAD][BLoader::R][2];          // slice it is fetched into set it % AHEAD
     const int last = kbase + kiters - 1;
     bl.load (kbase, areg[0]);
-    bl.load (min (kbase + 1, last), areg[1]);
+    if (AHEAD > 1) bl.load (min (kbase + 1, last), areg[AHEAD - 1]);
     const uint32_t row = (wave / WM) * (BN / WN) + (lane & 31);
     const uint32_t foff[2] = {Stage::offset (row, lane >> 5), Stage::offset (row, 2 + (lane >> 5))};
     floatx16 lo[TN];
@@ -823,12 +868,12 @@ __device__ __forceinline__ void split_core (const void *weights, uint32_t first_
         for (int v = 0; v < 16; v++) { acc[i][v] = 0.f; lo[i][v] = 0.f; }
     auto refill = [&] (int set, uint32_t stage) { bl.share.store (smem + stage, areg[set]); stats (areg[set]); };
     refill (0, 0);
-    bl.load (min (kbase + 2, last), areg[0]);
+    bl.load (min (kbase + AHEAD, last), areg[0]);
     lds_barrier ();
     if (phases) tile_phase_lap (8);
     __builtin_amdgcn_s_setprio (0);
     // slice `it` (relative to kbase) sits in LDS at `stage`; MORE: the next one is split into the other stage meanwhile (from
-    // register set `set`, which then takes the slice two after it)
+    // register set `set`, which then takes the slice AHEAD after it)
     auto slice = [&] (int it, uint32_t stage, int set, auto more)
     {
         constexpr bool MORE = decltype (more)::value;
@@ -842,7 +887,7 @@ __device__ __forceinline__ void split_core (const void *weights, uint32_t first_
             if (MORE && g == 0)
             {
                 refill (set, stage ^ Stage::BYTES);
-                bl.load (min (kbase + it + 3, last), areg[set]);
+                bl.load (min (kbase + it + 1 + AHEAD, last), areg[set]);
             }
             split_mfma (frag[g & 1], w.operand (step), acc[i], lo[i]);
             if (MORE && i == TN - 1) w.load (kbase + it + 1, step);
@@ -850,9 +895,9 @@ __device__ __forceinline__ void split_core (const void *weights, uint32_t first_
         if (MORE) lds_barrier ();
     };
     int it = 0;
-    for (; it + 2 < kiters; it += 2) { slice (it, 0, 1, std::true_type ()); slice (it + 1, Stage::BYTES, 0, std::true_type ()); }
+    for (; it + 2 < kiters; it += 2) { slice (it, 0, AHEAD - 1, std::true_type ()); slice (it + 1, Stage::BYTES, 0, std::true_type ()); }
     uint32_t stage = 0;
-    if (it + 1 < kiters) { slice (it, 0, 1, std::true_type ()); it++; stage = Stage::BYTES; }
+    if (it + 1 < kiters) { slice (it, 0, AHEAD - 1, std::true_type ()); it++; stage = Stage::BYTES; }
     before_last_slice ();
     slice (it, stage, 0, std::false_type ());
     __builtin_amdgcn_s_setprio (TILE_PRIO);
@@ -938,52 +983,55 @@ __device__ __forceinline__ void contraction_mainloop (const aspen_hip_layer_t &L
                 if (r0 + u * STEP < rows) pre.s[u] = fin.ld4 ((n0 + r0 + u * STEP) * L.fuse_ld_in + m0 + c);
         }
     };
-    if (L.direct == ASPEN_HIP_OPERAND_DIRECT)
+    const auto loop = [&] (auto &bl, auto stats) { split_core<BN, WM, WN, RAW> (weights, tm * WM, total, bl, kbase, kiters, stages, acc, COH != 0, fetch_shortcut, ready, stats); };
+    if constexpr ((FEAT & TILES_GATHER) == 0 || (SMALL && (FEAT & TILES_NORM) != 0))
     {
-        DirectLoader<BN, COH> bl;
-        bl.init (in, n0, L.N - 1, L.ld0, tid);
-        if constexpr (SMALL && (FEAT & TILES_NORM) != 0)
+        if ((FEAT & TILES_GATHER) == 0 || L.norm_fold)
         {
-            // (kernels for transformer graphs: the column sums a folded layer norm needs are gathered in every such tile,
-            // sixteen additions and multiplications per K slice, and used where the layer asks for them)
-            float cs = 0.f, cq = 0.f;
-            auto stats = [&] (const float4 (&b)[1][2])
+            DirectLoader<BN, COH> bl;
+            bl.init (in, n0, L.N - 1, L.ld0, tid);
+            if constexpr (SMALL && (FEAT & TILES_NORM) != 0)
             {
-                #pragma unroll
-                for (int i = 0; i < 2; i++)
+                // (kernels for transformer graphs: the column sums a folded layer norm needs are gathered in every such tile,
+                // sixteen additions and multiplications per K slice, and used where the layer asks for them)
+                float cs = 0.f, cq = 0.f;
+                loop (bl, [&] (const float4 (&b)[1][2])
                 {
-                    cs += (b[0][i].x + b[0][i].y) + (b[0][i].z + b[0][i].w);
-                    cq += (b[0][i].x * b[0][i].x + b[0][i].y * b[0][i].y) + (b[0][i].z * b[0][i].z + b[0][i].w * b[0][i].w);
-                }
-            };
-            split_core<BN, WM, WN, RAW> (weights, tm * WM, total, bl, kbase, kiters, stages, acc, COH != 0, fetch_shortcut, ready, stats);
-            if (L.norm_fold) norm_fold_finish<COH> (L, acc[0], cs, cq, smem, tid, m0, n0, (wave % 2) * 32, (wave / 2) * 32);
+                    #pragma unroll
+                    for (int i = 0; i < 2; i++)
+                    {
+                        cs += (b[0][i].x + b[0][i].y) + (b[0][i].z + b[0][i].w);
+                        cq += (b[0][i].x * b[0][i].x + b[0][i].y * b[0][i].y) + (b[0][i].z * b[0][i].z + b[0][i].w * b[0][i].w);
+                    }
+                });
+                if (L.norm_fold) norm_fold_finish<COH> (L, acc[0], cs, cq, smem, tid, m0, n0, (wave % 2) * 32, (wave / 2) * 32);
+            }
+            else loop (bl, NoStats ());
         }
-        else split_core<BN, WM, WN, RAW> (weights, tm * WM, total, bl, kbase, kiters, stages, acc, COH != 0, fetch_shortcut, ready);
     }
-    else if constexpr ((FEAT & TILES_GATHER) != 0)
+    if constexpr ((FEAT & TILES_GATHER) != 0)
     {
         // (the dense three-channel layout is only used for layers of up to 64 output channels, see aspen_layer_dense3)
-        if (BM == 64 && L.direct == ASPEN_HIP_OPERAND_DENSE3)
+        if ((SMALL || (BM == 64 && (FEAT & TILES_DENSE_WIDE) != 0)) && L.direct == ASPEN_HIP_OPERAND_DENSE3)
         {
             Dense3Loader<BN, COH> bl;
             bl.init (L, in, n0, tid);
-            split_core<BN, WM, WN, RAW> (weights, tm * WM, total, bl, kbase, kiters, stages, acc, COH != 0, fetch_shortcut, ready);
+            loop (bl, NoStats ());
         }
-        else if (SMALL && L.IC % SLICE_K != 0)
+        else if (SMALL && L.direct == ASPEN_HIP_OPERAND_TABLE && L.IC % SLICE_K != 0)
         {
             if constexpr (SMALL)
             {
-                ConvLoader<BN, COH, true> bl;
-                bl.init (L, in, n0, tid, kbase, kiters);
-                split_core<BN, WM, WN, RAW> (weights, tm * WM, total, bl, kbase, kiters, stages, acc, COH != 0, fetch_shortcut, ready);
+                TableLoader<BN, COH> bl;
+                bl.init (L, in, n0, tid);
+                loop (bl, NoStats ());
             }
         }
-        else
+        else if ((FEAT & TILES_NORM) == 0 || !L.norm_fold)
         {
-            ConvLoader<BN, COH, false> bl;
+            StepLoader<BN, COH> bl;
             bl.init (L, in, n0, tid, kbase, kiters);
-            split_core<BN, WM, WN, RAW> (weights, tm * WM, total, bl, kbase, kiters, stages, acc, COH != 0, fetch_shortcut, ready);
+            loop (bl, NoStats ());
         }
     }
     if (COH) tile_phase_lap (9);
@@ -2054,7 +2102,7 @@ __device__ __forceinline__ float4 narrow_mainloop (const aspen_hip_layer_t &L, D
     uint32_t n = tn * VAR3_BN + row;
     n = n < L.N ? n : L.N - 1;
     // activation operand: DIRECT = the parent's column; else the top-left input pixel of output position n and the
-    // tap / channel the first slice starts at (stepped from there, as ConvLoader does)
+    // tap / channel the first slice starts at (stepped from there, as StepLoader does)
     int32_t bbase, ih0 = 0, iw0 = 0;
     uint32_t kh = 0, kw = 0, c = 0;
     if (direct) bbase = (int32_t)(n * L.ld0 + (uint32_t)first * SLICE_K + unit0);
@@ -2065,7 +2113,7 @@ __device__ __forceinline__ float4 narrow_mainloop (const aspen_hip_layer_t &L, D
         ih0 = (int32_t)(oh * L.stride) - (int32_t)L.pad;
         iw0 = (int32_t)(ow * L.stride) - (int32_t)L.pad;
         bbase = ((int32_t)(b * L.IH) + ih0) * (int32_t)L.IW * (int32_t)L.ld0 + iw0 * (int32_t)L.ld0 + (int32_t)unit0;
-        // (K order: channel block, kh, kw, channel in block; see ConvLoader)
+        // (K order: channel block, kh, kw, channel in block; see StepLoader)
         const uint32_t taps = L.KH * L.KW, block = (uint32_t)first / taps, tap = (uint32_t)first - block * taps;
         c = block * SLICE_K;
         kh = tap / L.KW; kw = tap - kh * L.KW;

@@ -115,7 +115,7 @@ static int set_tiles (nasm_t *nasm, nasm_ldata_t *ld)
         if (cdiv (M, bm[v]) * cdiv (N, bn[v]) < want || (N <= 64 && v == ASPEN_HIP_GEMM_WIDE)) v = ASPEN_HIP_GEMM_SMALL;
         if (nasm->small_tiles_only) v = ASPEN_HIP_GEMM_SMALL;      /* graphs bound by their dependency chains, see create_nasm */
         if (nasm->kiters_cap && aspen_layer_kiters (L) > nasm->kiters_cap) v = ASPEN_HIP_GEMM_SMALL;   /* only the small shape is cut along K */
-        if (aspen_layer_table_operand (L)) v = ASPEN_HIP_GEMM_SMALL;
+        if (aspen_layer_table_operand (L) || aspen_layer_dense3 (L)) v = ASPEN_HIP_GEMM_SMALL;     /* (their loaders exist for that shape only: code the instruction cache need not hold) */
         /* latency-bound graphs (see create_nasm): a layer that the 64 x 64 shape leaves with less than half the wanted tiles
            takes the 32 x 32 shape, whose four wavefronts split the K axis between them */
         if (nasm->narrow_tiles && v == ASPEN_HIP_GEMM_SMALL && !aspen_layer_table_operand (L) && !aspen_layer_dense3 (L)
