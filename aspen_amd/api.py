@@ -230,8 +230,11 @@ class Nasm:
         n = lib().dse_get_ldata_result(self.h, l, arr, C.byref(out))
         if n < 0:
             raise RuntimeError("dse_get_ldata_result failed")
-        a = np.ctypeslib.as_array(C.cast(out, _fp), shape=(n // 4,)).copy()
-        lib()._free(out)
+        if n < _COPY_BELOW:
+            a = np.ctypeslib.as_array(C.cast(out, _fp), shape=(n // 4,)).copy()
+            lib()._free(out)
+        else:
+            a = np.asarray(_Buffer(out.value, n // 4, lib()._free))
         return a.reshape(i["W"], i["H"]) if order is None else a
 
     def result(self, order: Optional[Sequence[int]] = None) -> np.ndarray:
@@ -241,6 +244,21 @@ class Nasm:
         if self.h:
             lib().apu_destroy_nasm(self.h)
             self.h = None
+
+
+# results from this size on keep the library's buffer instead of being copied (0.2 ms for the 6.3 MB of GPT-2's)
+_COPY_BELOW = 1 << 16
+
+
+class _Buffer:
+    """A malloc'ed block of floats that an array keeps alive; released with it."""
+
+    def __init__(self, address: int, count: int, free):
+        self._address, self._free = address, free
+        self.__array_interface__ = {"shape": (count,), "typestr": "<f4", "data": (address, False), "version": 3}
+
+    def __del__(self):
+        self._free(self._address)
 
 
 class RPool:

@@ -11,6 +11,7 @@
 #include <stdio.h>
 #include <stdlib.h>
 #include <string.h>
+#include <mutex>
 #include "tile_kernels.h"
 
 #define QUEUE_EMPTY 0xffffffffu
@@ -745,59 +746,193 @@ extern "C" int aspen_hip_zero (void *dst, size_t bytes)
     return 0;
 }
 
-// Dense <-> strided columns.  dense[c * rows + r] <-> strided[c * ld + r]; padding rows [rows, ld) are written as zeros.
-__global__ void __launch_bounds__ (WG_THREADS) spread_columns_kernel (const float *__restrict__ dense, float *__restrict__ strided, uint32_t rows, uint32_t ld, size_t n)
+// Dense columns on the host <-> strided columns on the device: dense[c * rows + r] <-> strided[c * ld + r]; padding rows
+// [rows, ld) are written as zeros.  The kernels read and write PINNED host memory themselves, in pieces that report through
+// a host word each, and the host copies between the pieces and the caller's pageable buffer while the others are on the
+// link.  hipMemcpyAsync on a pageable buffer costs some 20 us before the first byte and moves 17 GB/s to the host.
+// To the host, us, that way / this way: 4 KB 25 / 10, 0.69 MB 41 / 39, 6.3 MB 385 / 241, 22 MB 1410 / 970; to the device,
+// until work may be queued behind it: 12 KB 22 / 5, 0.6 MB 44 / 18, 6.6 MB 225 / 124.
+// Bound by the host's copy out of or into pinned memory (30 to 50 GB/s), the link behind it.
+#define PIECE_BYTES (256u << 10)                        // one host word per piece
+#define LINK_PIECES 32u                                 // pieces of the pinned ring (8 MB); a launch covers at most half of them
+#define LINK_WG_FLOATS (WG_THREADS * 16u)               // floats a workgroup moves: four 16-byte groups per thread
+#define PIECE_FLOATS (PIECE_BYTES / 4u)
+#define PIECE_WGS (PIECE_FLOATS / LINK_WG_FLOATS)
+#define CPOL_SYSTEM (1 | CPOL_SC1)                      // sc0 + sc1: past every cache, host memory is not kept on the device
+struct link_args_t
 {
-    const size_t step = (size_t)gridDim.x * blockDim.x;
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += step)
+    float *matrix;              // strided, at the column of the launch's first float
+    float *pinned;              // dense pieces, the launch's first one
+    uint32_t *words;            // host: word of the launch's first piece
+    uint32_t *arrived;          // device: workgroups of a piece that are done (zero between launches)
+    uint32_t rows, ld, r0;      // r0: row of the launch's first float (its column is 0)
+    uint32_t n;                 // floats
+    uint32_t serial, up;
+};
+__global__ void __launch_bounds__ (WG_THREADS) link_kernel (const link_args_t a)
+{
+    const uint32_t piece = blockIdx.x / PIECE_WGS;
+    const __amdgpu_buffer_rsrc_t host = __builtin_amdgcn_make_buffer_rsrc ((void *)a.pinned, 0, (int)((a.n + 3u) / 4u * 16u), 0x00020000);
+    const uint32_t e0 = blockIdx.x * LINK_WG_FLOATS + threadIdx.x * 4u;
+    uint32_t c[4], r[4];
+    #pragma unroll
+    for (uint32_t q = 0; q < 4; q++)
     {
-        const size_t c = i / ld;
-        const uint32_t r = (uint32_t)(i - c * ld);
-        strided[i] = r < rows ? dense[c * rows + r] : 0.f;
+        const uint32_t x = a.r0 + e0 + q * (WG_THREADS * 4u);
+        c[q] = x / a.rows;
+        r[q] = x - c[q] * a.rows;
     }
-}
-__global__ void __launch_bounds__ (WG_THREADS) gather_columns_kernel (const float *__restrict__ strided, float *__restrict__ dense, uint32_t rows, uint32_t ld, size_t n)
-{
-    const size_t step = (size_t)gridDim.x * blockDim.x;
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += step)
+    float v[4][4];
+    if (a.up)
     {
-        const size_t c = i / rows;
-        dense[i] = strided[c * ld + (i - c * rows)];
+        #pragma unroll
+        for (uint32_t q = 0; q < 4; q++)
+        {
+            // (past the end: zeros, not stored)
+            const u32x4 x = __builtin_amdgcn_raw_buffer_load_b128 (host, (int)((e0 + q * (WG_THREADS * 4u)) * 4u), 0, CPOL_SYSTEM);
+            #pragma unroll
+            for (int k = 0; k < 4; k++) v[q][k] = __uint_as_float (x[k]);
+        }
+    }
+    #pragma unroll
+    for (uint32_t q = 0; q < 4; q++)
+    {
+        const uint32_t e = e0 + q * (WG_THREADS * 4u);
+        #pragma unroll
+        for (uint32_t k = 0; k < 4; k++)
+        {
+            const bool in = e + k < a.n;
+            float *p = a.matrix + ((size_t)c[q] * a.ld + r[q]);
+            if (a.up && in)
+            {
+                *p = v[q][k];
+                // the column's last row: its padding too
+                if (r[q] + 1 == a.rows) for (uint32_t z = a.rows; z < a.ld; z++) p[1 + z - a.rows] = 0.f;
+            }
+            if (!a.up) v[q][k] = in ? *p : 0.f;
+            if (++r[q] == a.rows) { r[q] = 0; c[q]++; }
+        }
+    }
+    if (!a.up)
+    {
+        #pragma unroll
+        for (uint32_t q = 0; q < 4; q++)
+        {
+            // (groups past the end fall outside the descriptor; the last group's spare floats lie inside its piece)
+            const u32x4 x = {__float_as_uint (v[q][0]), __float_as_uint (v[q][1]), __float_as_uint (v[q][2]), __float_as_uint (v[q][3])};
+            __builtin_amdgcn_raw_buffer_store_b128 (x, host, (int)((e0 + q * (WG_THREADS * 4u)) * 4u), 0, CPOL_SYSTEM);
+        }
+        asm volatile ("s_waitcnt vmcnt(0)" ::: "memory");      // this wavefront's stores have been acknowledged
+    }
+    // the last workgroup of a piece raises the piece's word (upload: everyone has READ the piece, the host may refill it)
+    __syncthreads ();
+    if (threadIdx.x == 0)
+    {
+        const uint32_t wgs = min (PIECE_WGS, gridDim.x - piece * PIECE_WGS);
+        if (wgs == 1u) __hip_atomic_store (a.words + piece, a.serial, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        // (relaxed: the stores above went past the caches and have been acknowledged, so there is nothing to write back)
+        else if (__hip_atomic_fetch_add (a.arrived + piece, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == wgs - 1u)
+        {
+            __hip_atomic_store (a.arrived + piece, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store (a.words + piece, a.serial, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
     }
 }
 
-// staging buffer for the two functions below; grows on demand and lives as long as the process
-static float *g_stage = nullptr;
-static size_t g_stage_bytes = 0;
-static int stage_reserve (size_t bytes)
+// the pinned ring; lives as long as the process, used by one caller at a time
+static struct
 {
-    if (bytes <= g_stage_bytes) return 0;
-    CHECK (hipStreamSynchronize (g_stream));
-    if (g_stage) { (void)hipFree (g_stage); g_stage = nullptr; g_stage_bytes = 0; }
-    CHECK (hipMalloc ((void **)&g_stage, bytes));
-    g_stage_bytes = bytes;
+    char *pinned;
+    uint32_t *words, *arrived;
+    uint32_t serial[LINK_PIECES];       // what a piece's word holds once its last launch is done with it
+    uint32_t last_serial;
+    std::mutex lock;
+} g_link;
+static int link_reserve (void)
+{
+    if (g_link.pinned) return 0;
+    char *pinned = nullptr;
+    uint32_t *words = nullptr;
+    uint32_t *arrived = (uint32_t *)aspen_hip_alloc (LINK_PIECES * sizeof (uint32_t));
+    if (!arrived) return -1;
+    hipError_t e = hipHostMalloc ((void **)&words, LINK_PIECES * sizeof (uint32_t), hipHostMallocDefault);
+    if (e == hipSuccess) e = hipHostMalloc ((void **)&pinned, (size_t)LINK_PIECES * PIECE_BYTES, hipHostMallocDefault);
+    if (e != hipSuccess) { if (words) (void)hipHostFree (words); aspen_hip_free (arrived); return fail (e, "hipHostMalloc"); }
+    for (uint32_t i = 0; i < LINK_PIECES; i++) words[i] = 0;
+    g_link.words = words; g_link.arrived = arrived; g_link.pinned = pinned;
     return 0;
 }
-static unsigned stream_grid (size_t n)
+// returns once the piece's last launch is done with it; a stream that has ended without raising the word has failed
+static int link_wait (uint32_t piece)
 {
-    const size_t want = (n + WG_THREADS - 1) / WG_THREADS, cap = (size_t)g_num_cu * 16;
-    return (unsigned)(want < cap ? (want ? want : 1) : cap);
+    for (;;)
+    {
+        for (int spin = 0; spin < 8192; spin++)        // (a look at the stream takes the runtime several microseconds)
+        {
+            if (__atomic_load_n (&g_link.words[piece], __ATOMIC_ACQUIRE) == g_link.serial[piece]) return 0;
+            __builtin_ia32_pause ();
+        }
+        const hipError_t e = hipStreamQuery (g_stream);
+        if (e == hipErrorNotReady) continue;
+        if (e == hipSuccess && __atomic_load_n (&g_link.words[piece], __ATOMIC_ACQUIRE) == g_link.serial[piece]) return 0;
+        // the ring starts over: nothing in flight refers to it any more
+        for (uint32_t i = 0; i < LINK_PIECES; i++) g_link.serial[i] = g_link.words[i];
+        return fail (e == hipSuccess ? hipErrorUnknown : e, "transfer between host and device");
+    }
+}
+// launches the transfer of floats [e0, e0 + n) of the dense matrix through the ring's pieces from `piece` on (no wrap)
+static int link_launch (float *matrix, uint32_t ld, uint32_t rows, size_t e0, uint32_t n, uint32_t piece, bool up)
+{
+    const size_t c0 = e0 / rows;
+    link_args_t a;
+    a.matrix = matrix + c0 * ld; a.pinned = (float *)(g_link.pinned + (size_t)piece * PIECE_BYTES);
+    a.words = g_link.words + piece; a.arrived = g_link.arrived + piece;
+    a.rows = rows; a.ld = ld; a.r0 = (uint32_t)(e0 - c0 * rows); a.n = n; a.up = up;
+    g_link.last_serial = g_link.last_serial + 1u ? g_link.last_serial + 1u : 1u;
+    a.serial = g_link.last_serial;
+    const uint32_t pieces = (n + PIECE_FLOATS - 1) / PIECE_FLOATS;
+    hipLaunchKernelGGL (link_kernel, dim3 ((n + LINK_WG_FLOATS - 1) / LINK_WG_FLOATS), dim3 (WG_THREADS), 0, g_stream, a);
+    CHECK (hipGetLastError ());
+    for (uint32_t i = 0; i < pieces; i++) g_link.serial[piece + i] = a.serial;
+    return 0;
 }
 
-extern "C" int aspen_hip_dense_host_to_device (float *dst, uint32_t ld, const float *src_host, uint32_t rows, size_t columns)
+// `wait`: return only when the matrix is complete; else work enqueued on the library's stream afterwards sees it
+static int dense_to_device (float *dst, uint32_t ld, const float *src_host, uint32_t rows, size_t columns, bool wait)
 {
     if (aspen_hip_init ()) return -1;
     if (!dst || !src_host || rows == 0 || ld < rows) { snprintf (g_err, sizeof (g_err), "dense_host_to_device: bad arguments"); return -1; }
     if (columns == 0) return 0;
-    if (ld == rows) return aspen_hip_h2d (dst, src_host, (size_t)rows * columns * sizeof (float));
-    const size_t bytes = (size_t)rows * columns * sizeof (float);
-    if (stage_reserve (bytes)) return -1;
-    CHECK (hipMemcpyAsync (g_stage, src_host, bytes, hipMemcpyHostToDevice, g_stream));
-    const size_t n = (size_t)ld * columns;
-    hipLaunchKernelGGL (spread_columns_kernel, dim3 (stream_grid (n)), dim3 (WG_THREADS), 0, g_stream, g_stage, dst, rows, ld, n);
-    CHECK (hipGetLastError ());
-    CHECK (hipStreamSynchronize (g_stream));       // the caller may reuse its buffer, and the next call the staging buffer
+    const std::lock_guard<std::mutex> guard (g_link.lock);
+    if (link_reserve ()) return -1;
+    // The host copies a launch's pieces while the previous launch's travel: short launches first, so that the link starts
+    // early, longer ones for large matrices (a launch costs the host about 3 us, a piece's copy 8).
+    const size_t total = (size_t)rows * columns;
+    const uint32_t longest = total >= 32u * (size_t)PIECE_FLOATS ? 8u : total >= 8u * (size_t)PIECE_FLOATS ? 4u : 1u;
+    uint32_t piece = 0, want = 1;
+    for (size_t e = 0; e < total;)
+    {
+        const uint32_t room = min (want, LINK_PIECES - piece);
+        const uint32_t n = (uint32_t)(total - e < (size_t)room * PIECE_FLOATS ? total - e : (size_t)room * PIECE_FLOATS), pieces = (n + PIECE_FLOATS - 1) / PIECE_FLOATS;
+        for (uint32_t i = 0; i < pieces; i++) if (link_wait (piece + i)) return -1;
+        memcpy (g_link.pinned + (size_t)piece * PIECE_BYTES, src_host + e, (size_t)n * sizeof (float));
+        const int rc = link_launch (dst, ld, rows, e, n, piece, true);
+        if (rc) return rc;
+        piece = (piece + pieces) % LINK_PIECES;
+        want = min (2 * want, longest);
+        e += n;
+    }
+    if (wait) CHECK (hipStreamSynchronize (g_stream));
     return 0;
+}
+
+extern "C" int aspen_hip_dense_host_to_device (float *dst, uint32_t ld, const float *src_host, uint32_t rows, size_t columns)
+{
+    return dense_to_device (dst, ld, src_host, rows, columns, true);
+}
+extern "C" int aspen_hip_dense_host_to_device_ordered (float *dst, uint32_t ld, const float *src_host, uint32_t rows, size_t columns)
+{
+    return dense_to_device (dst, ld, src_host, rows, columns, false);
 }
 
 extern "C" int aspen_hip_dense_device_to_host (float *dst_host, const float *src, uint32_t ld, uint32_t rows, size_t columns)
@@ -805,14 +940,37 @@ extern "C" int aspen_hip_dense_device_to_host (float *dst_host, const float *src
     if (aspen_hip_init ()) return -1;
     if (!dst_host || !src || rows == 0 || ld < rows) { snprintf (g_err, sizeof (g_err), "dense_device_to_host: bad arguments"); return -1; }
     if (columns == 0) return 0;
-    if (ld == rows) return aspen_hip_d2h (dst_host, src, (size_t)rows * columns * sizeof (float));
-    const size_t bytes = (size_t)rows * columns * sizeof (float), n = (size_t)rows * columns;
-    if (stage_reserve (bytes)) return -1;
-    hipLaunchKernelGGL (gather_columns_kernel, dim3 (stream_grid (n)), dim3 (WG_THREADS), 0, g_stream, src, g_stage, rows, ld, n);
-    CHECK (hipGetLastError ());
-    CHECK (hipMemcpyAsync (dst_host, g_stage, bytes, hipMemcpyDeviceToHost, g_stream));
-    CHECK (hipStreamSynchronize (g_stream));
+    const std::lock_guard<std::mutex> guard (g_link.lock);
+    if (link_reserve ()) return -1;
+    // half a ring per launch: while the host copies one half out, the other one travels
+    constexpr uint32_t HALF = LINK_PIECES / 2u;
+    const size_t total = (size_t)rows * columns, batch = (size_t)HALF * PIECE_FLOATS, batches = (total + batch - 1) / batch;
+    const auto floats = [&] (size_t b) { return total - b * batch < batch ? total - b * batch : batch; };
+    const auto launch = [&] (size_t b)
+    {
+        const uint32_t first = (uint32_t)(b & 1) * HALF;
+        for (uint32_t i = 0; i < HALF; i++) if (link_wait (first + i)) return -1;      // (an upload may still be reading)
+        return link_launch ((float *)src, ld, rows, b * batch, (uint32_t)floats (b), first, false);
+    };
+    for (size_t b = 0; b < 2 && b < batches; b++) { const int rc = launch (b); if (rc) return rc; }
+    for (size_t b = 0; b < batches; b++)
+    {
+        const size_t n = floats (b);
+        uint32_t piece = (uint32_t)(b & 1) * HALF;
+        for (size_t e = 0; e < n; e += PIECE_FLOATS, piece++)
+        {
+            if (link_wait (piece)) return -1;
+            memcpy (dst_host + b * batch + e, g_link.pinned + (size_t)piece * PIECE_BYTES, (n - e < PIECE_FLOATS ? n - e : PIECE_FLOATS) * sizeof (float));
+        }
+        if (b + 2 < batches) { const int rc = launch (b + 2); if (rc) return rc; }
+    }
     return 0;
+}
+
+static unsigned stream_grid (size_t n)
+{
+    const size_t want = (n + WG_THREADS - 1) / WG_THREADS, cap = (size_t)g_num_cu * 16;
+    return (unsigned)(want < cap ? (want ? want : 1) : cap);
 }
 
 // plain streaming copy; also the yardstick the HBM byte counters of a profiler are calibrated with (its traffic is
@@ -1537,8 +1695,9 @@ extern "C" int aspen_hip_graph_wait_group (aspen_hip_graph_t *g, uint32_t group)
     if (!g || group >= g->num_groups || !g->last_run_dataflow) return -1;
     for (;;)
     {
-        // the word is written by the device into pinned host memory: a few hundred polls between two looks at the stream
-        for (int spin = 0; spin < 256; spin++)
+        // the word is written by the device into pinned host memory: some thousand polls between two looks at the stream, which
+        // take the runtime several microseconds
+        for (int spin = 0; spin < 8192; spin++)
         {
             if (__atomic_load_n (&g->h_abort[HOST_DONE_WORD + group], __ATOMIC_ACQUIRE) == g->run_serial) return 0;
             __builtin_ia32_pause ();

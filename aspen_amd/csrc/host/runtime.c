@@ -58,11 +58,13 @@ void rpool_add_nasm_raw_input (rpool_t *rpool, nasm_t *nasm, void *input_data)
         /* dense columns -> strided columns of layer 0 (reference copy_buffer_to_ldata_out_mat, src/apu_nasm.c:809) */
         const nasm_ldata_t *ld = &nasm->ldata_arr[0];
         const size_t H = ld->out_mat_dims[OUT_H], W = ld->out_mat_dims[OUT_W];
-        aspen_hip_sync ();
-        /* one contiguous transfer, then a kernel that spreads the columns to the matrix's stride: a strided
+        /* a kernel spreads the columns to the matrix's stride: a strided
            copy of millions of 12-byte columns (3-channel images) is orders of magnitude slower, and
-           repacking on the host costs more than the transfer */
-        const int rc = aspen_hip_dense_host_to_device (nasm->d_arena + ld->out_mat_offset, ld->out_mat_stride, input_data, (uint32_t)H, W);
+           repacking on the host costs more than the transfer.  Runs before and behind it are ordered by the stream
+           (in a pool whose last run has not been collected a read-out could take the second stream: that one waits) */
+        if (rpool->running) aspen_hip_sync ();
+        const int rc = (rpool->running ? aspen_hip_dense_host_to_device : aspen_hip_dense_host_to_device_ordered)
+            (nasm->d_arena + ld->out_mat_offset, ld->out_mat_stride, input_data, (uint32_t)H, W);
         if (rc) ERROR_PRTF ("ERROR: rpool_add_nasm_raw_input: input upload failed: %s\n", aspen_hip_last_error ());
     }
     nasm->armed = 1;
@@ -413,7 +415,7 @@ static ssize_t get_ldata_output (nasm_t *nasm, unsigned int ldata_idx, LAYER_PAR
             free (raw);
         }
     }
-    else    /* padding rows stripped on the device, one contiguous transfer */
+    else    /* padding rows stripped on the device */
         rc = aspen_hip_dense_device_to_host (dense, nasm->d_arena + ld->out_mat_offset, ld->out_mat_stride, (uint32_t)H, W);
     if (rc)
     {

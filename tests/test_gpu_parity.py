@@ -1130,3 +1130,34 @@ def test_row_groups_end_at_the_last_row_tile(gpu, mode):
             assert err <= H.REL_L2_TOL, f"layer {l}: rel L2 {err:.3g}"
     finally:
         net.close()
+
+
+@pytest.mark.parametrize("rows,ld,columns", [(1, 1, 1), (3, 4, 7), (3, 4, 21846), (85, 96, 3086), (64, 64, 1024), (65535, 65536, 2), (1000, 1024, 1), (7, 32, 400001)])
+def test_matrices_travel_whole_in_both_directions(gpu, rows, ld, columns):
+    """Dense host columns to strided device columns and back, bit for bit and with zeroed padding: pieces of 65536 floats,
+    launches of up to sixteen pieces, two of them in flight (the last case goes round the pinned ring)."""
+    import ctypes as C
+    L = api.lib()
+    L.aspen_hip_dense_host_to_device_ordered.argtypes = L.aspen_hip_dense_host_to_device.argtypes = [C.c_void_p, C.c_uint32, C.c_void_p, C.c_uint32, C.c_size_t]
+    L.aspen_hip_dense_device_to_host.argtypes = [C.c_void_p, C.c_void_p, C.c_uint32, C.c_uint32, C.c_size_t]
+    p = lambda a: a.ctypes.data_as(C.c_void_p)
+    guard = 64
+    d = L.aspen_hip_alloc((ld * columns + guard) * 4)
+    assert d
+    try:
+        for rep, up in enumerate((L.aspen_hip_dense_host_to_device, L.aspen_hip_dense_host_to_device_ordered, L.aspen_hip_dense_host_to_device_ordered)):
+            x = np.random.default_rng(rows * 7 + columns + rep).integers(0, 2 ** 32, rows * columns, dtype=np.uint32)
+            full = np.full(ld * columns + guard, 0xabcdef01, dtype=np.uint32)
+            assert L.aspen_hip_h2d(d, p(full), full.nbytes) == 0
+            sent = x.copy()
+            assert up(d, ld, p(sent), rows, columns) == 0
+            sent[:] = 0                                  # the source may be reused at once
+            back = np.zeros(rows * columns + guard, dtype=np.uint32)
+            assert L.aspen_hip_dense_device_to_host(p(back), d, ld, rows, columns) == 0
+            assert np.array_equal(back[:-guard], x) and not back[-guard:].any()
+            assert L.aspen_hip_d2h(p(full), d, full.nbytes) == 0
+            cols = full[:ld * columns].reshape(columns, ld)
+            assert np.array_equal(cols[:, :rows].ravel(), x) and not cols[:, rows:].any()
+            assert (full[ld * columns:] == 0xabcdef01).all()
+    finally:
+        L.aspen_hip_free(d)
