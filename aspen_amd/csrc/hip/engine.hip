@@ -1686,7 +1686,9 @@ extern "C" int aspen_hip_graph_sync (aspen_hip_graph_t *g)
 extern "C" int aspen_hip_graph_group_done (aspen_hip_graph_t *g, uint32_t group)
 {
     if (!g || group >= g->num_groups || !g->last_run_dataflow) return -1;
-    return __atomic_load_n (&g->h_abort[HOST_DONE_WORD + group], __ATOMIC_ACQUIRE) == g->run_serial ? 1 : 0;
+    if (__atomic_load_n (&g->h_abort[HOST_DONE_WORD + group], __ATOMIC_ACQUIRE) != g->run_serial) return 0;
+    // (an ordered run that was given up still runs its tiles through and raises the words; the abort word was raised before)
+    return g->last_run_ordered && __atomic_load_n (&g->h_abort[0], __ATOMIC_ACQUIRE) != 0 ? 0 : 1;
 }
 
 extern "C" int aspen_hip_graph_wait_group (aspen_hip_graph_t *g, uint32_t group)
