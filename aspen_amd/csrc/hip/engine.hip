@@ -521,7 +521,7 @@ __device__ __forceinline__ void wait_until_ready ()
 }
 
 template <int COH, unsigned FEAT, bool ORDERED = false>
-__global__ void __launch_bounds__ (WG_THREADS, WG_PER_CU) dataflow_kernel (dataflow_args_t args)
+__global__ void __launch_bounds__ (WG_THREADS, (FEAT & TILES_DEEP) ? 2 : WG_PER_CU) dataflow_kernel (dataflow_args_t args)
 {
     extern __shared__ __align__ (16) float smem[];
     if (threadIdx.x == 0)
@@ -602,7 +602,7 @@ static const void *const dataflow_kernels[NUM_KERNEL_VARIANTS][2] = {
 static const unsigned ordered_variant_tiles[NUM_ORDERED_VARIANTS] = {TILES_CONVNET | TILES_YOLO | TILES_NARROW, TILES_CONVNET | TILES_TALL, TILES_TRANSFORMER, TILES_ALL};
 static const void *const ordered_kernels[NUM_ORDERED_VARIANTS] = {
     (const void *)dataflow_kernel<2, TILES_CONVNET | TILES_YOLO | TILES_NARROW, true>, (const void *)dataflow_kernel<2, TILES_CONVNET | TILES_TALL, true>,
-    (const void *)dataflow_kernel<2, TILES_TRANSFORMER, true>, (const void *)dataflow_kernel<2, TILES_ALL, true>};
+    (const void *)dataflow_kernel<2, TILES_TRANSFORMER | TILES_DEEP, true>, (const void *)dataflow_kernel<2, TILES_ALL, true>};
 
 // The tile kinds a graph contains, as TILES_* bits.
 static unsigned graph_features (const aspen_hip_layer_t *layers, uint32_t num_layers)
@@ -1538,10 +1538,8 @@ extern "C" int aspen_hip_run_dataflow (aspen_hip_graph_t *g, uint32_t workgroups
             // by default two per compute unit (one tile computes, the next is prepared); without the prefetch buffers three
             // from an estimated parallelism of 350 and four from 600 on (YOLO-v3 batch 1, 409: 1.30 / 1.25 / 1.26 ms with
             // two / three / four; ResNet-50 batch 4, 335: 0.72 / 0.76 / 0.76; VGG-16 batch 4, 766: 1.51 / 1.40 / 1.34)
-            // (transformer graphs, whose kernel fits three times: two below 600; BERT-base 8 x 128, 519: 1.96 / 2.00 ms with
-            // two / three, 16 x 128, 1024: 3.49 / 3.33)
-            const double three_from = (g->features & TILES_ATTENTION) ? 600.0 : 350.0;
-            const uint32_t per_cu = !small_lds || g->parallelism < three_from ? 2u : g->parallelism < 600.0 ? 3u : 4u;
+            // (the kernel of transformer graphs fits twice, see TILES_DEEP)
+            const uint32_t per_cu = !small_lds || g->parallelism < 350.0 ? 2u : g->parallelism < 600.0 ? 3u : 4u;
             if (workgroups_requested == 0) workgroups = per_cu * (uint32_t)g_num_cu < (uint32_t)fit ? per_cu * (uint32_t)g_num_cu : (uint32_t)fit;
             if (workgroups > (uint32_t)fit) workgroups = (uint32_t)fit;
         }

@@ -83,28 +83,29 @@ __device__ __forceinline__ void split_mfma (const split8_t &a, const split8_t &b
 #define SPLIT_SLICE_BYTES 6144u
 #define RAW_SLICE_BYTES 4096u
 
-template <bool RAW> struct WeightFragments
+// SETS: register sets, i.e. slices of weights in flight.
+template <bool RAW, int SETS = 1> struct WeightFragments
 {
     static constexpr uint32_t SLICE = RAW ? RAW_SLICE_BYTES : SPLIT_SLICE_BYTES, PARTS = RAW ? 2 : 3;
     typedef const char __attribute__ ((address_space (1))) *bytes_t;
     bytes_t base;               // of the wavefront's row block (uniform)
     uint32_t lane16;
-    u32x4 f[2][PARTS];          // [step]
+    u32x4 f[SETS][2][PARTS];    // [set][step]
     __device__ __forceinline__ void init (const void *w, uint32_t block, uint32_t slices, uint32_t lane)
     {
         base = (bytes_t)w + (uint64_t)block * ((uint64_t)slices * SLICE);
         lane16 = lane * 16u;
     }
-    __device__ __forceinline__ void load (int it, int step)
+    __device__ __forceinline__ void load (int it, int step, int set = 0)
     {
         const bytes_t p = base + ((uint32_t)it * SLICE + (uint32_t)step * (SLICE / 2));
         #pragma unroll
-        for (uint32_t q = 0; q < PARTS; q++) f[step][q] = *(const u32x4 __attribute__ ((address_space (1))) *)(p + (lane16 + q * 1024u));
+        for (uint32_t q = 0; q < PARTS; q++) f[set][step][q] = *(const u32x4 __attribute__ ((address_space (1))) *)(p + (lane16 + q * 1024u));
     }
-    __device__ __forceinline__ split8_t operand (int step) const
+    __device__ __forceinline__ split8_t operand (int step, int set = 0) const
     {
-        if constexpr (RAW) return split8 (__builtin_bit_cast (float4, f[step][0]), __builtin_bit_cast (float4, f[step][1]));
-        else return {f[step][0], f[step][1], f[step][2]};
+        if constexpr (RAW) return split8 (__builtin_bit_cast (float4, f[set][step][0]), __builtin_bit_cast (float4, f[set][step][1]));
+        else return {f[set][step][0], f[set][step][1], f[set][step][2]};
     }
 };
 

@@ -545,6 +545,15 @@ enum : unsigned
     TILES_NARROW = 512u,        // the 32 x 32 contraction tile of latency-bound graphs
     TILES_TALL = 1024u,         // the 128 x 32 contraction tile of weight-streaming layers
     TILES_DENSE_WIDE = 2048u,   // the dense three-channel operand under the 64 x 128 shape (the host library's graphs take 64 x 64 for it)
+    // No tile kind: 64 x 64 tiles keep four K slices of both operands in flight, four slices to a trip through the loop, in the
+    // 249 registers per lane that two workgroups per compute unit leave.  For the ordered kernel of transformer graphs, which
+    // runs two of them: its levels are a few hundred tiles of 24 slices, one or two per compute unit, and with one slice of
+    // weights and two of activations in flight a slice took 0.42 us for 0.17 us of matrix instructions.  BERT-base 8 x 128
+    // 1.81 -> 1.67 ms, 3 x 75 1.01 -> 0.95, GPT-2 4 x 512 3.23 -> 3.03; with four slices of weights and two of activations 1.71,
+    // 1.00 and 3.05; with the loop left from its middle instead of copies of the last slices behind it 1.78, 1.03 and 3.17.
+    // Convolutional graphs run three workgroups per unit and lose with two (YOLO-v3 batch 1 1.10 -> 1.16 ms, ResNet-50
+    // batch 11 1.02 -> 1.27).
+    TILES_DEEP = 4096u,
     TILES_ALL = 4095u,
     TILES_CONVNET = TILES_GATHER | TILES_LARGE | TILES_WIDE | TILES_SMALL | TILES_POOL | TILES_RESIDUAL,
     TILES_TRANSFORMER = TILES_SMALL | TILES_ATTENTION | TILES_NORM | TILES_RESIDUAL
@@ -815,13 +824,35 @@ __device__ __forceinline__ void gemm_core_single_block (ALoader &al, BLoader &bl
 }
 
 
+// f (0) .. f (COUNT - 1) with the index as a constant
+template <int FIRST, int COUNT, class F> __device__ __forceinline__ void slice_run (F f)
+{
+    f (std::integral_constant<int, FIRST> ());
+    if constexpr (FIRST + 1 < COUNT) slice_run<FIRST + 1, COUNT> (f);
+}
+// the first `left` (1 .. COUNT) of them, the last one as f (index, false)
+template <int FIRST, int COUNT, class F> __device__ __forceinline__ void last_slices (int left, F f)
+{
+    constexpr std::integral_constant<int, FIRST> turn;
+    if constexpr (FIRST + 1 < COUNT)
+    {
+        if (left > FIRST + 1)
+        {
+            f (turn, std::true_type ());
+            last_slices<FIRST + 1, COUNT> (left, f);
+            return;
+        }
+    }
+    f (turn, std::false_type ());
+}
+
 // ---------------------------------------------------------------------------------------------
 // K loop of the contraction tiles.  Workgroup tile = (WM x 32) weight rows x BN activation rows; WM x WN wavefronts, each
 // owning 32 x (BN / WN) of it.  The activation row is the matrix instruction's row index and the weight row its column, so each
 // accumulator register holds 32 consecutive output channels of one output column: stores are 128-byte coalesced.
-//   weights      memory -> registers, in fragment order (WeightFragments); a step's registers are asked for again, one slice
+//   weights      memory -> registers, in fragment order (WeightFragments); a step's registers are asked for again, SETS slices
 //                ahead, as soon as the step's matrix instructions have been issued
-//   activations  memory -> registers, two slices ahead -> split into three terms -> one of two LDS stages, a slice ahead ->
+//   activations  memory -> registers, AHEAD slices ahead -> split into three terms -> one of two LDS stages, a slice ahead ->
 //                fragments.  Every value is split once per tile (5.5 vector instructions) and read by WM wavefronts.
 // One barrier per slice: it publishes the stage written during the slice and frees the one read.
 // The loop exists once per shape and operand kind, and each copy counts: the kernel for convolutional networks was 101 KB with nine of
@@ -840,25 +871,25 @@ __device__ __forceinline__ void gemm_core_single_block (ALoader &al, BLoader &bl
 // `stats` sees every K slice of the activation operand once, as the registers it passes through on its way into LDS
 // (a folded layer norm's column sums, see norm_fold_finish).
 // ---------------------------------------------------------------------------------------------
-template <int BN, int WM, int WN, bool RAW, class BLoader, class Hook, class Ready, class Stats = NoStats>
+template <int BN, int WM, int WN, bool RAW, int SETS, int AHEAD, class BLoader, class Hook, class Ready, class Stats = NoStats>
 __device__ __forceinline__ void split_core (const void *weights, uint32_t first_block, uint32_t total_slices, BLoader &bl, int kbase, int kiters, char *smem,
     floatx16 (&acc)[BN / WN / 32], bool phases, Hook before_last_slice, Ready ready, Stats stats = Stats ())
 {
     static_assert (WM * WN == 4, "four wavefronts");
     typedef SplitStage<BN> Stage;
-    // AHEAD: slices of activations in flight from memory (two register sets of 8 R do not fit beside the wide shape's sums: its loops
-    // spilled)
-    constexpr int TN = BN / WN / 32, GROUPS = 2 * TN, AHEAD = BLoader::R > 1 ? 1 : 2;
+    constexpr int TN = BN / WN / 32, GROUPS = 2 * TN, TRIP = CMAX (2, CMAX (SETS, AHEAD));
+    static_assert (TRIP % 2 == 0 && TRIP % SETS == 0 && TRIP % AHEAD == 0, "a trip through the loop ends on the sets it began with");
     if (phases) tile_phase_lap (12);
     const uint32_t tid = tile_thread (), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane (tid >> 6);
-    WeightFragments<RAW> w;
+    const int last = kbase + kiters - 1;
+    WeightFragments<RAW, SETS> w;
     w.init (weights, first_block + wave % WM, total_slices, lane);
-    w.load (kbase, 0); w.load (kbase, 1);
+    #pragma unroll
+    for (int s = 0; s < SETS; s++) { w.load (min (kbase + s, last), 0, s); w.load (min (kbase + s, last), 1, s); }
     ready ();
     float4 areg[AHEAD][BLoader::R][2];          // slice it is fetched into set it % AHEAD
-    const int last = kbase + kiters - 1;
-    bl.load (kbase, areg[0]);
-    if (AHEAD > 1) bl.load (min (kbase + 1, last), areg[AHEAD - 1]);
+    #pragma unroll
+    for (int s = 0; s < AHEAD; s++) bl.load (min (kbase + s, last), areg[s]);
     const uint32_t row = (wave / WM) * (BN / WN) + (lane & 31);
     const uint32_t foff[2] = {Stage::offset (row, lane >> 5), Stage::offset (row, 2 + (lane >> 5))};
     floatx16 lo[TN];
@@ -872,11 +903,12 @@ __device__ __forceinline__ void split_core (const void *weights, uint32_t first_
     lds_barrier ();
     if (phases) tile_phase_lap (8);
     __builtin_amdgcn_s_setprio (0);
-    // slice `it` (relative to kbase) sits in LDS at `stage`; MORE: the next one is split into the other stage meanwhile (from
-    // register set `set`, which then takes the slice AHEAD after it)
-    auto slice = [&] (int it, uint32_t stage, int set, auto more)
+    // slice `it` (relative to kbase), the `turn`th of its trip, sits in LDS; MORE: the next one is split into the other stage
+    // meanwhile (its registers then take the slice AHEAD after it)
+    auto slice = [&] (int it, uint32_t stage, auto turn, auto more)
     {
         constexpr bool MORE = decltype (more)::value;
+        constexpr int TURN = decltype (turn)::value, SET = (TURN + 1) % AHEAD, WSET = TURN % SETS;
         split8_t frag[2];
         frag[0] = Stage::read (smem + stage, foff[0]);
         #pragma unroll
@@ -886,20 +918,32 @@ __device__ __forceinline__ void split_core (const void *weights, uint32_t first_
             if (g + 1 < GROUPS) frag[(g + 1) & 1] = Stage::read (smem + stage, foff[(g + 1) / TN] + ((g + 1) % TN) * 32 * 64);
             if (MORE && g == 0)
             {
-                refill (set, stage ^ Stage::BYTES);
-                bl.load (min (kbase + it + 1 + AHEAD, last), areg[set]);
+                refill (SET, stage ^ Stage::BYTES);
+                bl.load (min (kbase + it + 1 + AHEAD, last), areg[SET]);
             }
-            split_mfma (frag[g & 1], w.operand (step), acc[i], lo[i]);
-            if (MORE && i == TN - 1) w.load (kbase + it + 1, step);
+            split_mfma (frag[g & 1], w.operand (step, WSET), acc[i], lo[i]);
+            if (MORE && i == TN - 1) w.load (SETS > 1 ? min (kbase + it + SETS, last) : kbase + it + 1, step, WSET);
         }
         if (MORE) lds_barrier ();
     };
+    constexpr auto stage_of = [] (int turn) { return turn % 2 ? Stage::BYTES : 0u; };
     int it = 0;
-    for (; it + 2 < kiters; it += 2) { slice (it, 0, AHEAD - 1, std::true_type ()); slice (it + 1, Stage::BYTES, 0, std::true_type ()); }
-    uint32_t stage = 0;
-    if (it + 1 < kiters) { slice (it, 0, AHEAD - 1, std::true_type ()); it++; stage = Stage::BYTES; }
-    before_last_slice ();
-    slice (it, stage, 0, std::false_type ());
+    for (; it + TRIP < kiters; it += TRIP) slice_run<0, TRIP> ([&] (auto turn) { slice (it + decltype (turn)::value, stage_of (decltype (turn)::value), turn, std::true_type ()); });
+    // the last 1 .. TRIP slices
+    if constexpr (TRIP == 2)
+    {
+        constexpr std::integral_constant<int, 0> turn;
+        uint32_t stage = 0;
+        if (it + 1 < kiters) { slice (it, 0, turn, std::true_type ()); it++; stage = Stage::BYTES; }
+        before_last_slice ();
+        slice (it, stage, turn, std::false_type ());
+    }
+    else
+        last_slices<0, TRIP> (kiters - it, [&] (auto turn, auto more)
+        {
+            if constexpr (!decltype (more)::value) before_last_slice ();
+            slice (it + decltype (turn)::value, stage_of (decltype (turn)::value), turn, more);
+        });
     __builtin_amdgcn_s_setprio (TILE_PRIO);
     #pragma unroll
     for (int i = 0; i < TN; i++)
@@ -983,7 +1027,11 @@ __device__ __forceinline__ void contraction_mainloop (const aspen_hip_layer_t &L
                 if (r0 + u * STEP < rows) pre.s[u] = fin.ld4 ((n0 + r0 + u * STEP) * L.fuse_ld_in + m0 + c);
         }
     };
-    const auto loop = [&] (auto &bl, auto stats) { split_core<BN, WM, WN, RAW> (weights, tm * WM, total, bl, kbase, kiters, stages, acc, COH != 0, fetch_shortcut, ready, stats); };
+    // (one slice of activations in flight under the wide shape: a second register set does not fit beside its sums, its loops
+    // spilled; four, and as many of weights, in kernels compiled for two workgroups per compute unit, see TILES_DEEP)
+    constexpr bool DEEP = SMALL && (FEAT & TILES_DEEP) != 0;
+    constexpr int SETS = DEEP ? 4 : 1, AHEAD = SliceShare<BN>::R > 1 ? 1 : DEEP ? 4 : 2;
+    const auto loop = [&] (auto &bl, auto stats) { split_core<BN, WM, WN, RAW, SETS, AHEAD> (weights, tm * WM, total, bl, kbase, kiters, stages, acc, COH != 0, fetch_shortcut, ready, stats); };
     if constexpr ((FEAT & TILES_GATHER) == 0 || (SMALL && (FEAT & TILES_NORM) != 0))
     {
         if ((FEAT & TILES_GATHER) == 0 || L.norm_fold)
