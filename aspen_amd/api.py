@@ -122,6 +122,7 @@ def lib() -> C.CDLL:
         "aspen_hip_sgemm_static": (C.c_int, [C.c_uint32, C.c_uint32, C.c_uint32, _vp, C.c_uint32, _vp, C.c_uint32, _vp,
                                              C.c_uint32, _vp, C.c_int]),
         "aspen_hip_sgemm_static_max_bytes": (C.c_size_t, []),
+        "aspen_hip_release_workspaces": (None, []),
     }
     for name, (res, args) in sig.items():
         fn = getattr(L, name)

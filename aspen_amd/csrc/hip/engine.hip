@@ -582,7 +582,8 @@ __global__ void __launch_bounds__ (WG_THREADS, (FEAT & TILES_DEEP) ? 2 : WG_PER_
     }
 }
 
-__global__ void sgemm_kernel (const aspen_hip_layer_t L);       // defined with aspen_hip_sgemm_static
+template <unsigned FEAT> __global__ void product_kernel (const aspen_hip_layer_t L);       // defined with aspen_hip_sgemm
+static const void *const product_kernels[3] = {(const void *)product_kernel<TILES_LARGE>, (const void *)product_kernel<TILES_SMALL>, (const void *)product_kernel<TILES_NARROW>};
 
 // The persistent kernel's variants, smallest first: [variant][0] coherent loads, [1] cached loads.  A graph runs on the
 // first variant that has all its tile kinds, see graph_features.
@@ -648,7 +649,7 @@ extern "C" int aspen_hip_init (void)
     CHECK (hipStreamCreate (&g_side_stream));
     for (int i = 0; i < NUM_EVENTS; i++) CHECK (hipEventCreate (&g_events[i]));
     CHECK (hipFuncSetAttribute ((const void *)layer_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, GEMM_SMEM_BYTES));
-    CHECK (hipFuncSetAttribute ((const void *)sgemm_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, GEMM_SMEM_BYTES));
+    for (const void *k : product_kernels) CHECK (hipFuncSetAttribute (k, hipFuncAttributeMaxDynamicSharedMemorySize, GEMM_SMEM_BYTES));
     for (int v = 0; v < NUM_KERNEL_VARIANTS; v++)
         for (int coh = 0; coh < 2; coh++)
             CHECK (hipFuncSetAttribute (dataflow_kernels[v][coh], hipFuncAttributeMaxDynamicSharedMemorySize, GEMM_SMEM_BYTES));
@@ -1774,6 +1775,52 @@ extern "C" int aspen_hip_event_elapsed_ms (int a, int b, float *ms)
     return 0;
 }
 
+// One contraction tile per workgroup, the descriptor in the kernel-argument segment; compiled for one tile shape each (with
+// all of them in one kernel its loops spilled: 1000 x 3137 x 1152 85 us a call that allocates nothing, now 74).  Contiguous tile
+// ranges per XCD, as in layer_kernel: workgroups that share activation columns meet in one L2.
+template <unsigned FEAT> __global__ void __launch_bounds__ (WG_THREADS, WG_PER_CU) product_kernel (const aspen_hip_layer_t L)
+{
+    extern __shared__ __align__ (16) float smem[];
+    const uint32_t nt = gridDim.x, bid = blockIdx.x, xcd = bid & 7, local = bid >> 3, chunk = nt >> 3, rem = nt & 7;
+    run_tile<0, FEAT> ([&] () { return uniform_layer (L); }, xcd * chunk + (xcd < rem ? xcd : rem) + local, false, smem, [] () { return (uint32_t *)nullptr; });
+}
+
+// C = act (A B + bias) with A already in the order the tiles read; on the library's stream.
+static int launch_product (uint32_t M, uint32_t N, uint32_t K, const float *arranged, const float *B, uint32_t ldb, float *C, uint32_t ldc, const float *bias, int act)
+{
+    aspen_hip_layer_t L;
+    memset (&L, 0, sizeof (L));
+    const uint32_t cu = (uint32_t)g_num_cu;
+    const auto tiles = [&] (uint32_t bm, uint32_t bn) { return (uint64_t)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
+    const uint64_t small = tiles (VAR2_BM, VAR2_BN), large = tiles (VAR0_BM, VAR0_BN);
+    // us with 128 x 64 / 64 x 64 / 32 x 32 tiles on 256 compute units (whole calls): 1000 x 3137 x 1152 76 / 82 / 140, 2048 x 2048 x 1024
+    // 73 / 81 / 160, 3000 x 700 x 2048 (264 large tiles) 111 / 108 / 163, 512 x 2048 x 768 (256 small ones) 41 / 35 / 43,
+    // 64 x 8192 x 1024 (128) 45 / 36 / 34, 256 x 1024 x 512 (64) 32 / 27 / 24, 64 x 64 x 3072 (1) 94 / 64 / 42: the large shape from five
+    // workgroups for four units on, the one that splits K over its wavefronts where small tiles leave half of the units idle
+    const int v = 4 * large >= 5 * (uint64_t)cu ? 0 : 2 * small <= cu ? 2 : 1;
+    static const struct { int variant; uint32_t bm, bn; } shape[3] = {{ASPEN_HIP_GEMM_LARGE, VAR0_BM, VAR0_BN}, {ASPEN_HIP_GEMM_SMALL, VAR2_BM, VAR2_BN}, {ASPEN_HIP_GEMM_NARROW, VAR3_BM, VAR3_BN}};
+    L.type = MATMUL_LAYER; L.act = act; L.variant = shape[v].variant; L.direct = ASPEN_HIP_OPERAND_DIRECT;
+    L.M = M; L.N = N; L.ld = ldc; L.tile_m = shape[v].bm; L.tile_n = shape[v].bn;
+    L.tiles_m = (M + L.tile_m - 1) / L.tile_m; L.tiles_n = (N + L.tile_n - 1) / L.tile_n; L.num_ninst = L.tiles_m * L.tiles_n; L.splits = 1;
+    L.K = K; L.Kp = K; L.ld0 = ldb; L.out = C; L.in0 = B; L.weight = arranged; L.bias = bias;
+    fill_derived (L);
+    void *args[] = {&L};
+    CHECK (hipLaunchKernel (product_kernels[v], dim3 (L.num_ninst), dim3 (WG_THREADS), args, GEMM_SMEM_BYTES, g_stream));
+    return 0;
+}
+
+// Where aspen_hip_sgemm arranges A: kept between calls up to a limit (allocating and clearing it, and a descriptor, cost 90 us a
+// call), for one caller at a time; a call that finds it taken, on another device or beyond the limit allocates its own.
+#define PRODUCT_KEEP_BYTES ((size_t)96 << 20)
+static struct { void *p; size_t bytes; int device; std::mutex lock; } g_product;
+
+extern "C" void aspen_hip_release_workspaces (void)
+{
+    const std::lock_guard<std::mutex> guard (g_product.lock);
+    if (g_product.p) (void)hipFree (g_product.p);
+    g_product.p = nullptr; g_product.bytes = 0;
+}
+
 extern "C" int aspen_hip_sgemm (uint32_t M, uint32_t N, uint32_t K, const float *A, uint32_t lda, const float *B,
     uint32_t ldb, float *C, uint32_t ldc, const float *bias, int act)
 {
@@ -1781,24 +1828,31 @@ extern "C" int aspen_hip_sgemm (uint32_t M, uint32_t N, uint32_t K, const float 
     if (K == 0 || K % GEMM_BK || lda % 4 || ldb % 4 || ldc % 4 || lda < K || ldb < K || ldc < M)
     { snprintf (g_err, sizeof (g_err), "sgemm: K must be a multiple of 32, strides multiples of 4"); return -1; }
     // A in the order the tiles read their weights, rows padded with zeros
-    float *Ap = (float *)aspen_hip_alloc (arranged_bytes (M, K, false));
-    if (!Ap) return -1;
-    if (arrange_weights (Ap, A, lda, M, K, false)) { aspen_hip_free (Ap); return -1; }
-    aspen_hip_layer_t L;
-    memset (&L, 0, sizeof (L));
-    L.type = MATMUL_LAYER; L.act = act; L.variant = ASPEN_HIP_GEMM_SMALL; L.direct = 1;
-    L.M = M; L.N = N; L.ld = ldc; L.tile_m = 64; L.tile_n = 64;
-    L.tiles_m = (M + 63) / 64; L.tiles_n = (N + 63) / 64; L.num_ninst = L.tiles_m * L.tiles_n; L.splits = 1;
-    L.K = K; L.Kp = K; L.ld0 = ldb; L.out = C; L.in0 = B; L.weight = Ap; L.bias = bias;
-    fill_derived (L);
-    aspen_hip_layer_t *dL = upload (&L, 1);
-    if (!dL) { aspen_hip_free (Ap); return -1; }
-    hipLaunchKernelGGL (layer_kernel, dim3 (L.num_ninst), dim3 (WG_THREADS), GEMM_SMEM_BYTES, g_stream, dL, 0u, 0u, (uint32_t *)nullptr);      // no split-K: the arrival counters are not touched
-    hipError_t e = hipGetLastError ();
-    if (e == hipSuccess) e = hipStreamSynchronize (g_stream);
-    aspen_hip_free (dL); aspen_hip_free (Ap);
+    const size_t bytes = arranged_bytes (M, K, false);
+    std::unique_lock<std::mutex> kept (g_product.lock, std::try_to_lock);
+    int device = -1;
+    CHECK (hipGetDevice (&device));
+    if (kept.owns_lock () && (bytes > PRODUCT_KEEP_BYTES || (g_product.p && g_product.device != device))) kept.unlock ();
+    float *Ap = nullptr;
+    if (!kept.owns_lock ()) Ap = (float *)aspen_hip_alloc (bytes);
+    else
+    {
+        if (bytes > g_product.bytes)
+        {
+            if (g_product.p) (void)hipFree (g_product.p);       // (nothing in flight reads it: every call waits for its kernels)
+            g_product.p = aspen_hip_alloc (bytes);
+            g_product.bytes = g_product.p ? bytes : 0;
+            g_product.device = device;
+        }
+        Ap = (float *)g_product.p;
+    }
+    if (!Ap && bytes) return -1;
+    int rc = arrange_weights (Ap, A, lda, M, K, false);
+    if (!rc) rc = launch_product (M, N, K, Ap, B, ldb, C, ldc, bias, act);
+    const hipError_t e = hipStreamSynchronize (g_stream);
+    if (!kept.owns_lock ()) aspen_hip_free (Ap);
     if (e != hipSuccess) return fail (e, "sgemm launch");
-    return 0;
+    return rc;
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -1830,13 +1884,6 @@ static float *scratch_for_current_device (void)
     return g_scratch_ptr[dev];
 }
 
-// one contraction tile per workgroup, the descriptor in the kernel-argument segment
-__global__ void __launch_bounds__ (WG_THREADS, WG_PER_CU) sgemm_kernel (const aspen_hip_layer_t L)
-{
-    extern __shared__ __align__ (16) float smem[];
-    run_tile<0> ([&] () { return uniform_layer (L); }, blockIdx.x, false, smem, [] () { return (uint32_t *)nullptr; });
-}
-
 extern "C" size_t aspen_hip_sgemm_static_max_bytes (void) { return SGEMM_SCRATCH_BYTES; }
 
 extern "C" int aspen_hip_sgemm_static (uint32_t M, uint32_t N, uint32_t K, const float *A, uint32_t lda, const float *B,
@@ -1859,14 +1906,5 @@ extern "C" int aspen_hip_sgemm_static (uint32_t M, uint32_t N, uint32_t K, const
     float *Ap = scratch_for_current_device ();
     if (!Ap) return -1;
     if (arrange_weights (Ap, A, lda, M, K, false)) return -1;
-    aspen_hip_layer_t L;
-    memset (&L, 0, sizeof (L));
-    L.type = MATMUL_LAYER; L.act = act; L.variant = ASPEN_HIP_GEMM_SMALL; L.direct = 1;
-    L.M = M; L.N = N; L.ld = ldc; L.tile_m = VAR2_BM; L.tile_n = VAR2_BN;
-    L.tiles_m = (M + VAR2_BM - 1) / VAR2_BM; L.tiles_n = (N + VAR2_BN - 1) / VAR2_BN; L.num_ninst = L.tiles_m * L.tiles_n; L.splits = 1;
-    L.K = K; L.Kp = K; L.ld0 = ldb; L.out = C; L.in0 = B; L.weight = Ap; L.bias = bias;
-    fill_derived (L);
-    hipLaunchKernelGGL (sgemm_kernel, dim3 (L.num_ninst), dim3 (WG_THREADS), GEMM_SMEM_BYTES, g_stream, L);
-    CHECK (hipGetLastError ());
-    return 0;
+    return launch_product (M, N, K, Ap, B, ldb, C, ldc, bias, act);
 }

@@ -484,5 +484,6 @@ ssize_t dse_get_nasm_result (nasm_t *nasm, LAYER_PARAMS *order, void **out_ptr)
 
 void aspen_flush_dynamic_memory (void)
 {
-    /* activations live in per-nasm arenas that are freed with the nasm; there is no allocator cache to flush */
+    /* activations live in per-nasm arenas that are freed with the nasm; what the library keeps is the plain product's workspace */
+    aspen_hip_release_workspaces ();
 }

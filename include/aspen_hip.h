@@ -295,7 +295,9 @@ void aspen_hip_divider_for (uint32_t d, uint32_t out[2]);
 
 /* ---- plain SGEMM seam (reference include/kernels.h:15-33 on device pointers) -------------------- */
 /* C[n*ldc + m] = act(bias[m] + sum_k A[m*lda + k] * B[n*ldb + k]); A row-major [M][K] (not packed),
-   lda/ldb/ldc multiples of 4, K a multiple of 32. */
+   lda/ldb/ldc multiples of 4, K a multiple of 32.  The arranged copy of A lives in device memory the library keeps
+   between calls (up to 96 MB); release_workspaces gives it back. */
+void aspen_hip_release_workspaces (void);
 int aspen_hip_sgemm (uint32_t M, uint32_t N, uint32_t K, const float *A, uint32_t lda, const float *B,
     uint32_t ldb, float *C, uint32_t ldc, const float *bias, int act);
 
@@ -303,7 +305,7 @@ int aspen_hip_sgemm (uint32_t M, uint32_t N, uint32_t K, const float *A, uint32_
    hipMalloc).  No counterpart in the reference.  It runs on the library's own stream (it cannot be recorded into a
    caller's stream capture) and the first call initialises the library (stream, events, kernel attributes: call
    aspen_hip_init beforehand where that matters).  It calls no hipMalloc / hipFree:
-   the zero-padded staging copy of A that aspen_hip_sgemm allocates per call lives in a static device array of
+   the zero-padded staging copy of A that aspen_hip_sgemm allocates lives in a static device array of
    aspen_hip_sgemm_static_max_bytes () bytes (8 MiB per GPU, held until the process ends), so
    roundup (M, 128) * K * 4 must not exceed that; larger problems are refused with a message.  Asynchronous on
    the library's stream: C is complete after aspen_hip_sync ().  All calls on a GPU share the one staging

@@ -1161,3 +1161,37 @@ def test_matrices_travel_whole_in_both_directions(gpu, rows, ld, columns):
             assert (full[ld * columns:] == 0xabcdef01).all()
     finally:
         L.aspen_hip_free(d)
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 1, 32), (33, 31, 3072), (31, 2049, 96), (513, 1025, 64), (65, 8100, 32), (1031, 2570, 96), (2050, 1285, 160)])
+def test_plain_product_over_its_tile_shapes(gpu, M, N, K):
+    """32 x 32 tiles (K split over the wavefronts, also fewer slices than wavefronts), 64 x 64 and 128 x 64 tiles, as the sizes
+    choose them, edges off every tile; with bias and activation, both entry points, bit for bit alike.  Per output at most one
+    rounding per 16 K positions in each of the two running sums, a few for the additions behind them, 2^-24 each of the sum of magnitudes."""
+    import ctypes as C
+    L = api.lib()
+    rng = np.random.default_rng(M * 31 + N * 17 + K)
+    A, B = rng.standard_normal((M, K)).astype(np.float32), rng.standard_normal((N, K)).astype(np.float32)
+    bias = rng.standard_normal(M).astype(np.float32)
+    ldc = -(-M // 4) * 4
+    bufs = [L.aspen_hip_alloc(x) for x in (A.nbytes, B.nbytes, N * ldc * 4, bias.nbytes)]
+    outs = []
+    try:
+        assert all(bufs)
+        for d, h in zip((bufs[0], bufs[1], bufs[3]), (A, B, bias)):
+            assert L.aspen_hip_h2d(d, h.ctypes.data, h.nbytes) == 0
+        for call in (L.aspen_hip_sgemm, L.aspen_hip_sgemm_static, L.aspen_hip_sgemm):
+            out = np.zeros((N, ldc), dtype=np.float32)
+            assert L.aspen_hip_h2d(bufs[2], out.ctypes.data, out.nbytes) == 0
+            assert call(M, N, K, bufs[0], K, bufs[1], K, bufs[2], ldc, bufs[3], api.RELU) == 0, L.aspen_hip_last_error()
+            assert L.aspen_hip_d2h(out.ctypes.data, bufs[2], out.nbytes) == 0
+            outs.append(out)
+            L.aspen_hip_release_workspaces()
+    finally:
+        for b in bufs:
+            L.aspen_hip_free(b)
+    A64, B64 = A.astype(np.float64), B.astype(np.float64)
+    exact = np.maximum(B64 @ A64.T + bias, 0)
+    bound = (2 * (K // 16) + 8) * 2.0 ** -24 * (np.abs(B64) @ np.abs(A64).T + np.abs(bias))
+    assert np.all(np.abs(outs[0][:, :M] - exact) <= bound)
+    assert np.array_equal(outs[0], outs[1]) and np.array_equal(outs[0], outs[2]) and not outs[0][:, M:].any()
