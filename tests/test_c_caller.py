@@ -24,7 +24,7 @@ def build_caller(out_dir):
     return exe
 
 
-@pytest.mark.skipif(not os.path.isdir(REFERENCE), reason="the reference tree is not mounted here")
+@pytest.mark.skipif(not os.path.isfile(os.path.join(REFERENCE, "main.c")), reason="the reference tree is not mounted here")
 def test_reference_callers_compile_against_the_header():
     """reference main.c and examples/*/aspen_*.c include only aspen.h; every function, type, enumerator and
     system facility they use must come through include/aspen.h."""
