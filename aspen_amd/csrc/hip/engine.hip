@@ -582,7 +582,8 @@ __global__ void __launch_bounds__ (WG_THREADS, (FEAT & TILES_DEEP) ? 2 : WG_PER_
     }
 }
 
-template <unsigned FEAT> __global__ void product_kernel (const aspen_hip_layer_t L);       // defined with aspen_hip_sgemm
+// defined with aspen_hip_sgemm (the bounds stand here too: instantiated below, the kernels have those of this declaration)
+template <unsigned FEAT> __global__ void __launch_bounds__ (WG_THREADS, WG_PER_CU) product_kernel (const aspen_hip_layer_t L);
 static const void *const product_kernels[3] = {(const void *)product_kernel<TILES_LARGE>, (const void *)product_kernel<TILES_SMALL>, (const void *)product_kernel<TILES_NARROW>};
 
 // The persistent kernel's variants, smallest first: [variant][0] coherent loads, [1] cached loads.  A graph runs on the
