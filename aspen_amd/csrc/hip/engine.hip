@@ -117,10 +117,12 @@ __global__ void __launch_bounds__ (WG_THREADS, WG_PER_CU) layer_kernel (const as
     const uint32_t t = first_tile + xcd * chunk + (xcd < rem ? xcd : rem) + local;
     bool more_rows;
     uint32_t row_rep = 0;
+    const auto address = [=] () { return layers + l; };
+    const layer_at<decltype (address)> descriptor {address};
     do
     {
         more_rows = false;
-        run_tile<0> ([=] () { return scalar_layer (layers + l); }, t, false, smem, [=] () { return arrivals; }, NoHook (), row_rep++, &more_rows);
+        run_tile<0> (descriptor, t, false, smem, [=] () { return arrivals; }, NoHook (), row_rep++, &more_rows);
     } while (more_rows);
 }
 
@@ -555,7 +557,8 @@ __global__ void __launch_bounds__ (WG_THREADS, (FEAT & TILES_DEEP) ? 2 : WG_PER_
         }
         // the layer's descriptor goes from memory into scalar registers (it is shared by all tiles of the layer
         // and by all workgroups, so it sits in the scalar cache or in L2)
-        const auto descriptor = [] () { return scalar_layer (s_sched.a.layers + s_sched.layer); };
+        const auto address = [] () { return s_sched.a.layers + s_sched.layer; };
+        const layer_at<decltype (address)> descriptor {address};
         bool complete, more_rows = false;
         const auto ready = [] () { if constexpr (ORDERED) wait_until_ready (); };
         if (!(s_sched.a.flags & ASPEN_HIP_FLAG_SKIP_TILES))
@@ -1040,7 +1043,7 @@ __global__ void __launch_bounds__ (WG_THREADS) arrange_weights_kernel (const flo
         if (RAW) { *reinterpret_cast<float4 *> (d) = a; *reinterpret_cast<float4 *> (d + 1024) = b; }
         else
         {
-            const split8_t f = split8 (a, b);
+            const split8_t f = split8_weights (a, b);
             *reinterpret_cast<u32x4 *> (d) = f.h; *reinterpret_cast<u32x4 *> (d + 1024) = f.m; *reinterpret_cast<u32x4 *> (d + 2048) = f.l;
         }
     }
@@ -1783,7 +1786,10 @@ template <unsigned FEAT> __global__ void __launch_bounds__ (WG_THREADS, WG_PER_C
 {
     extern __shared__ __align__ (16) float smem[];
     const uint32_t nt = gridDim.x, bid = blockIdx.x, xcd = bid & 7, local = bid >> 3, chunk = nt >> 3, rem = nt & 7;
-    run_tile<0, FEAT> ([&] () { return uniform_layer (L); }, xcd * chunk + (xcd < rem ? xcd : rem) + local, false, smem, [] () { return (uint32_t *)nullptr; });
+    // (L is the only argument: it lies where the argument segment begins)
+    const auto address = [] () { return (const aspen_hip_layer_t *)__builtin_amdgcn_kernarg_segment_ptr (); };
+    const layer_at<decltype (address)> descriptor {address};
+    run_tile<0, FEAT> (descriptor, xcd * chunk + (xcd < rem ? xcd : rem) + local, false, smem, [] () { return (uint32_t *)nullptr; });
 }
 
 // C = act (A B + bias) with A already in the order the tiles read; on the library's stream.

@@ -14,8 +14,10 @@
 // Speed: a v_mfma_f32_32x32x16_bf16 does eight times the work of a v_mfma_f32_32x32x2_f32 in half its cycles, so six of them take 3 / 8
 // of the time.  In practice both are limited by power: a large product reaches 154 TFLOP/s with the single-precision
 // instruction (98 % of its peak) and 205-212 with this scheme.
-// The range is float's own (bfloat16 has the same exponent): terms of inputs below 2^-110 lose low bits, inputs within 0.4 %
-// of the largest float round to infinity, and an infinite input makes its products NaN.
+// The range is float's own (bfloat16 has the same exponent) with two edges.  Terms below bfloat16's smallest number, 2^-133, do not
+// exist: an input below 2^-110 enters with an absolute error of up to 2^-134.  And infinities, NaNs and floats within 0.2 % of the
+// largest one, whose h rounds to infinity, leave no finite sum (inf - inf in m, inf times a zero term): the tiles look
+// for sums that are not finite and compute those again from the floats themselves (single_precision_block in tile_kernels.h).
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -51,6 +53,38 @@ __device__ __forceinline__ split8_t split8 (float4 a, float4 b)
         s.h[q] = h; s.m[q] = m; s.l[q] = bf16_pair (u, v);
     }
     return s;
+}
+
+// The terms of weights, which the kernels have nothing else of: join2 gets every float back that is not below 2^-110.  An infinity or a
+// NaN is its own h with m = l = 0, a finite float never rounds up to infinity (the largest bfloat16 and the rest instead).
+__device__ __forceinline__ split8_t split8_weights (float4 a, float4 b)
+{
+    split8_t s = split8 (a, b);
+    const float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+    #pragma unroll
+    for (int q = 0; q < 4; q++)
+    {
+        uint32_t h = s.h[q], drop = 0;
+        #pragma unroll
+        for (int e = 0; e < 2; e++)
+        {
+            const uint32_t half = e ? 0xffff0000u : 0xffffu;
+            if ((h & 0x7f807f80u & half) != (0x7f807f80u & half)) continue;
+            if (fabsf (x[2 * q + e]) < INFINITY) h = (h & ~half) | (((h & 0x80008000u) | 0x7f7f7f7fu) & half);
+            else drop |= half;
+        }
+        if (h == s.h[q] && drop == 0) continue;
+        float u = x[2 * q] - bf16_low (h), v = x[2 * q + 1] - bf16_high (h);
+        const uint32_t m = bf16_pair (u, v);
+        u -= bf16_low (m); v -= bf16_high (m);
+        s.h[q] = h; s.m[q] = m & ~drop; s.l[q] = bf16_pair (u, v) & ~drop;
+    }
+    return s;
+}
+// the two floats of one register of each term (m + l is the rest of the float behind h, exact; so is the sum of all)
+__device__ __forceinline__ floatx2 join2 (uint32_t h, uint32_t m, uint32_t l)
+{
+    return (floatx2){bf16_low (h) + (bf16_low (m) + bf16_low (l)), bf16_high (h) + (bf16_high (m) + bf16_high (l))};
 }
 
 // hi += leading products, lo += the five small ones, of 32 x 32 x 16: rows of the result = rows of `a`, columns = rows of `b`

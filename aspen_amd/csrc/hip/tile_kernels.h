@@ -952,6 +952,132 @@ __device__ __forceinline__ void split_core (const void *weights, uint32_t first_
     lds_barrier ();          // the caller reuses the stages (epilogue)
 }
 
+// A wave-uniform copy of a layer descriptor in scalar registers.  Every value derived from the descriptor must
+// be known to be uniform: otherwise buffer descriptors get rebuilt in a per-lane "waterfall" loop around each
+// access and all tile-level control flow runs on the vector unit.
+//
+// scalar_layer reads a descriptor in device memory through the scalar data cache (read-only use: descriptors
+// are written by the host before the launch and never by a kernel), 64 dwords in a handful of wide scalar
+// loads straight into scalar registers.  `g` must be the same for all lanes.
+__device__ __forceinline__ aspen_hip_layer_t scalar_layer (const aspen_hip_layer_t *g)
+{
+    constexpr int W = sizeof (aspen_hip_layer_t) / 4;
+    static_assert (sizeof (aspen_hip_layer_t) % 4 == 0, "descriptor is a whole number of dwords");
+    const uint64_t p = (uint64_t)g;
+    // (the builtin returns int: without the casts the low half would be sign-extended over the high one)
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane ((uint32_t)p), hi = (uint32_t)__builtin_amdgcn_readfirstlane ((uint32_t)(p >> 32));
+    uint64_t up = ((uint64_t)hi << 32) | (uint64_t)lo;
+    // Every call loads afresh: the compiler may not merge the loads of two calls (and so keep all 64 dwords in
+    // registers from the first use of a descriptor to the last), because it cannot see that `up` is unchanged.
+    asm volatile ("" : "+s" (up));
+    const uint32_t __attribute__ ((address_space (4))) *src = (const uint32_t __attribute__ ((address_space (4))) *)up;
+    uint32_t w[W];
+    #pragma unroll
+    for (int i = 0; i < W; i++) w[i] = src[i];
+    aspen_hip_layer_t L;
+    __builtin_memcpy (&L, w, sizeof (aspen_hip_layer_t));
+    return L;
+}
+// How a tile asks for its layer's descriptor: `address ()` says where it lies (for all lanes the same).
+template <class Address> struct layer_at
+{
+    Address address;
+    __device__ __forceinline__ aspen_hip_layer_t operator() () const { return scalar_layer (address ()); }
+};
+
+// Sums that three terms cannot form (operands that are not finite, or whose h rounds to infinity; sums beyond the largest
+// float): one wavefront's 32 x 32 block over the slices [kbase, kbase + kiters) from the floats themselves, every lane reading
+// its operands straight from memory in fragment order, on the single-precision matrix instruction.  Nothing else comes
+// here, so it is written for size: one slice at a time, the operand's address from scratch for each.
+// n: the lane's activation row, `block`: the wavefront's block of weight rows.
+// A real function: inlined, its registers pushed the convolutional kernels' prefetched shortcuts out to scratch.
+template <bool RAW, int COH, bool GATHER, bool TABLES>
+__device__ __noinline__ floatx16 single_precision_block (const aspen_hip_layer_t *layer, uint32_t block, uint32_t n, int kbase, int kiters)
+{
+    const aspen_hip_layer_t L = scalar_layer (layer);
+    block = __builtin_amdgcn_readfirstlane (block); kbase = __builtin_amdgcn_readfirstlane (kbase); kiters = __builtin_amdgcn_readfirstlane (kiters);
+    const uint32_t lane = tile_thread () & 63, unit0 = lane >> 5, total = L.Kp / SLICE_K;
+    n = min (n, L.N - 1);
+    ActView<COH> in;
+    in.init (L.in0, L.in0_columns, L.ld0);
+    WeightFragments<RAW> w;
+    w.init (L.weight, block, total, lane);
+    int32_t base = (int32_t)(n * L.ld0), ih0 = 0, iw0 = 0;
+    const bool direct = !GATHER || L.direct == ASPEN_HIP_OPERAND_DIRECT;
+    if (!direct)
+    {
+        const uint32_t ohw = L.OH * L.OW, b = fast_div (n, L.div_ohw), rem = n - b * ohw, oh = fast_div (rem, L.div_ow), ow = rem - oh * L.OW;
+        ih0 = (int32_t)(oh * L.stride) - (int32_t)L.pad;
+        iw0 = (int32_t)(ow * L.stride) - (int32_t)L.pad;
+        base = ((int32_t)(b * L.IH) + ih0) * (int32_t)L.IW * (int32_t)L.ld0 + iw0 * (int32_t)L.ld0;
+    }
+    const auto inside = [&] (uint32_t kh, uint32_t kw) { return (uint32_t)(ih0 + (int32_t)kh) < L.IH && (uint32_t)(iw0 + (int32_t)kw) < L.IW; };
+    floatx16 acc;
+    #pragma unroll
+    for (int v = 0; v < 16; v++) acc[v] = 0.f;
+    #pragma unroll 1
+    for (int it = kbase; it < kbase + kiters; it++)
+    {
+        float4 x[2][2];
+        w.load (it, 0); w.load (it, 1);
+        uint32_t offset = (uint32_t)it * SLICE_K;
+        bool ok = true;
+        if (!direct && !(TABLES && (L.direct == ASPEN_HIP_OPERAND_DENSE3 || L.IC % SLICE_K != 0)))
+        {
+            const uint32_t taps = L.KH * L.KW, channels = (uint32_t)it / taps, tap = (uint32_t)it - channels * taps, kh = tap / L.KW, kw = tap - kh * L.KW;
+            offset = (kh * L.IW + kw) * L.ld0 + channels * SLICE_K;
+            ok = inside (kh, kw);
+        }
+        #pragma unroll
+        for (int q = 0; q < 4; q++)
+        {
+            const uint32_t unit = unit0 + (q & 2), chunk = unit + 4 * (q & 1);      // step q / 2; four floats: chunk of the slice's eight
+            float4 &d = x[q >> 1][q & 1];
+            if (TABLES && !direct && L.direct == ASPEN_HIP_OPERAND_DENSE3)
+            {
+                const uint32_t kc = (uint32_t)it * 8 + chunk, sel = kc % 3u;
+                const aspen_hip_ktab_t e0 = L.ktab[2 * kc], e1 = L.ktab[2 * kc + 1];
+                const float4 a = in.ld4_if ((uint32_t)(base + e0.offset), inside (e0.kh, e0.kw)), b = in.ld4_if ((uint32_t)(base + e1.offset), inside (e1.kh, e1.kw));
+                d.x = sel == 0 ? a.x : sel == 1 ? a.y : a.z;
+                d.y = sel == 0 ? a.y : sel == 1 ? a.z : b.x;
+                d.z = sel == 0 ? a.z : sel == 1 ? b.x : b.y;
+                d.w = sel == 0 ? b.x : sel == 1 ? b.y : b.z;
+            }
+            else if (TABLES && !direct && L.IC % SLICE_K != 0)
+            {
+                const aspen_hip_ktab_t e = L.ktab[(uint32_t)it * 8 + chunk];
+                d = in.ld4_if ((uint32_t)(base + e.offset), inside (e.kh, e.kw));
+            }
+            else d = in.ld4_if ((uint32_t)base + offset + chunk * 4, ok);
+        }
+        #pragma unroll
+        for (int step = 0; step < 2; step++)
+        {
+            float wf[8];
+            #pragma unroll
+            for (int q = 0; q < 4; q++)
+            {
+                if constexpr (RAW) { const floatx4 r = __builtin_bit_cast (floatx4, w.f[0][step][q >> 1]); wf[2 * q] = r[2 * (q & 1)]; wf[2 * q + 1] = r[2 * (q & 1) + 1]; }
+                else { const floatx2 r = join2 (w.f[0][step][0][q], w.f[0][step][1][q], w.f[0][step][2][q]); wf[2 * q] = r[0]; wf[2 * q + 1] = r[1]; }
+            }
+            const float xf[8] = {x[step][0].x, x[step][0].y, x[step][0].z, x[step][0].w, x[step][1].x, x[step][1].y, x[step][1].z, x[step][1].w};
+            #pragma unroll
+            for (int k = 0; k < 8; k++) acc = __builtin_amdgcn_mfma_f32_32x32x2f32 (xf[k], wf[k], acc, 0, 0, 0);
+        }
+    }
+    return acc;
+}
+
+// true for a wavefront one of whose sums is not finite (elementwise_maximum passes NaNs on: eight v_maximum3_f32; sixteen
+// multiply-adds with zero took 1 % of BERT-base 8 x 128)
+__device__ __forceinline__ bool sums_not_finite (const floatx16 &acc)
+{
+    float most[2] = {0.f, 0.f};
+    #pragma unroll
+    for (int v = 0; v < 16; v += 2) most[(v >> 1) & 1] = __builtin_elementwise_maximum (__builtin_elementwise_maximum (most[(v >> 1) & 1], fabsf (acc[v])), fabsf (acc[v + 1]));
+    return __builtin_expect (__any (!(__builtin_elementwise_maximum (most[0], most[1]) < INFINITY)), 0);
+}
+
 // Shortcut fused into a contraction epilogue: fuse_out = fuse_act (v + fuse_in) for the (up to) four
 // channels m .. m+3 of column n; `left` = channels of the matrix from m on.  Same arithmetic, in the same
 // order, as a residual tile reading the stored v would do.
@@ -1032,6 +1158,7 @@ __device__ __forceinline__ void contraction_mainloop (const aspen_hip_layer_t &L
     constexpr bool DEEP = SMALL && (FEAT & TILES_DEEP) != 0;
     constexpr int SETS = DEEP ? 4 : 1, AHEAD = SliceShare<BN>::R > 1 ? 1 : DEEP ? 4 : 2;
     const auto loop = [&] (auto &bl, auto stats) { split_core<BN, WM, WN, RAW, SETS, AHEAD> (weights, tm * WM, total, bl, kbase, kiters, stages, acc, COH != 0, fetch_shortcut, ready, stats); };
+    float cs = 0.f, cq = 0.f;
     if constexpr ((FEAT & TILES_GATHER) == 0 || (SMALL && (FEAT & TILES_NORM) != 0))
     {
         if ((FEAT & TILES_GATHER) == 0 || L.norm_fold)
@@ -1042,7 +1169,6 @@ __device__ __forceinline__ void contraction_mainloop (const aspen_hip_layer_t &L
             {
                 // (kernels for transformer graphs: the column sums a folded layer norm needs are gathered in every such tile,
                 // sixteen additions and multiplications per K slice, and used where the layer asks for them)
-                float cs = 0.f, cq = 0.f;
                 loop (bl, [&] (const float4 (&b)[1][2])
                 {
                     #pragma unroll
@@ -1052,7 +1178,6 @@ __device__ __forceinline__ void contraction_mainloop (const aspen_hip_layer_t &L
                         cq += (b[0][i].x * b[0][i].x + b[0][i].y * b[0][i].y) + (b[0][i].z * b[0][i].z + b[0][i].w * b[0][i].w);
                     }
                 });
-                if (L.norm_fold) norm_fold_finish<COH> (L, acc[0], cs, cq, smem, tid, m0, n0, (wave % 2) * 32, (wave / 2) * 32);
             }
             else loop (bl, NoStats ());
         }
@@ -1082,8 +1207,24 @@ __device__ __forceinline__ void contraction_mainloop (const aspen_hip_layer_t &L
             loop (bl, NoStats ());
         }
     }
-    if (COH) tile_phase_lap (9);
     const uint32_t wm0 = (wave % WM) * 32, wn0 = (wave / WM) * (BN / WN);
+    const auto again = [&] (int i) { return single_precision_block<RAW, COH, (FEAT & TILES_GATHER) != 0, BM == 64> (descriptor.address (), tm * WM + wave % WM, n0 + wn0 + 32 * i + (lane & 31), kbase, kiters); };
+    bool redo = sums_not_finite (acc[0]);
+    if constexpr (TN == 1)
+    {
+        if (redo)
+        {
+            const floatx16 x = again (0);
+            #pragma unroll
+            for (int v = 0; v < 16; v++) acc[0][v] = fabsf (acc[0][v]) < INFINITY ? acc[0][v] : x[v];
+        }
+    }
+    else redo |= sums_not_finite (acc[1]);
+    if constexpr (SMALL && (FEAT & TILES_NORM) != 0)
+    {
+        if (L.norm_fold) norm_fold_finish<COH> (L, acc[0], cs, cq, smem, tid, m0, n0, wm0, wn0);
+    }
+    if (COH) tile_phase_lap (9);
     if (slice >= 0)
     {
         // split-K: the raw sums go straight from the accumulators to this slice's block of the output tile, in the
@@ -1111,6 +1252,23 @@ __device__ __forceinline__ void contraction_mainloop (const aspen_hip_layer_t &L
         #pragma unroll
         for (int v = 0; v < 16; v++)
             smem[ACC_N (wn0, i, v, lane) * TROW + wm0 + (lane & 31)] = acc[i][v];
+    if constexpr (TN > 1)
+    {
+        if (redo)           // (every lane puts right what it has just parked)
+        {
+            #pragma unroll 1
+            for (int i = 0; i < TN; i++)
+            {
+                const floatx16 x = again (i);
+                #pragma unroll
+                for (int v = 0; v < 16; v++)
+                {
+                    float *sum = smem + ACC_N (wn0, i, v, lane) * TROW + wm0 + (lane & 31);
+                    if (!(fabsf (*sum) < INFINITY)) *sum = x[v];
+                }
+            }
+        }
+    }
     __syncthreads ();
 }
 
@@ -1973,45 +2131,6 @@ __device__ __forceinline__ void tile_fused_attention (const aspen_hip_layer_t &L
 // (reference src/dse.c:39-79).  `t` = tile index inside the layer, row-tile fastest
 // (reference src/apu_nasm.c:1218-1224).
 // ---------------------------------------------------------------------------------------------
-// A wave-uniform copy of a layer descriptor in scalar registers.  Every value derived from the descriptor must
-// be known to be uniform: otherwise buffer descriptors get rebuilt in a per-lane "waterfall" loop around each
-// access and all tile-level control flow runs on the vector unit.
-//
-// scalar_layer reads a descriptor in device memory through the scalar data cache (read-only use: descriptors
-// are written by the host before the launch and never by a kernel), 64 dwords in a handful of wide scalar
-// loads straight into scalar registers.  `g` must be the same for all lanes.
-__device__ __forceinline__ aspen_hip_layer_t scalar_layer (const aspen_hip_layer_t *g)
-{
-    constexpr int W = sizeof (aspen_hip_layer_t) / 4;
-    static_assert (sizeof (aspen_hip_layer_t) % 4 == 0, "descriptor is a whole number of dwords");
-    const uint64_t p = (uint64_t)g;
-    // (the builtin returns int: without the casts the low half would be sign-extended over the high one)
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane ((uint32_t)p), hi = (uint32_t)__builtin_amdgcn_readfirstlane ((uint32_t)(p >> 32));
-    uint64_t up = ((uint64_t)hi << 32) | (uint64_t)lo;
-    // Every call loads afresh: the compiler may not merge the loads of two calls (and so keep all 64 dwords in
-    // registers from the first use of a descriptor to the last), because it cannot see that `up` is unchanged.
-    asm volatile ("" : "+s" (up));
-    const uint32_t __attribute__ ((address_space (4))) *src = (const uint32_t __attribute__ ((address_space (4))) *)up;
-    uint32_t w[W];
-    #pragma unroll
-    for (int i = 0; i < W; i++) w[i] = src[i];
-    aspen_hip_layer_t L;
-    __builtin_memcpy (&L, w, sizeof (aspen_hip_layer_t));
-    return L;
-}
-// uniform_layer does the same for a descriptor the compiler already holds (a kernel argument).
-__device__ __forceinline__ aspen_hip_layer_t uniform_layer (const aspen_hip_layer_t &Lg)
-{
-    constexpr int W = sizeof (aspen_hip_layer_t) / 4;
-    uint32_t w[W];
-    __builtin_memcpy (w, &Lg, sizeof (aspen_hip_layer_t));
-    #pragma unroll
-    for (int i = 0; i < W; i++) w[i] = __builtin_amdgcn_readfirstlane (w[i]);
-    aspen_hip_layer_t L;
-    __builtin_memcpy (&L, w, sizeof (aspen_hip_layer_t));
-    return L;
-}
-
 // Counts this workgroup's arrival in its split-K group; true for the last of the `splits` members.  The
 // group's (write-through) stores must have been acknowledged before an arrival is counted: the last
 // one reads them.  The counter only ever grows by `splits` per run, so it needs no reset between runs.
@@ -2259,7 +2378,15 @@ __device__ __forceinline__ float4 narrow_mainloop (const aspen_hip_layer_t &L, D
     }
     // the four wavefronts' sums meet in LDS: [wave][column][NARROW_ROW] (a wavefront's own region, which it has read empty)
     #pragma unroll
-    for (int v = 0; v < 16; v++) mine[ACC_N (0, 0, v, lane) * NARROW_ROW + row] = acc[v] + lo[v];
+    for (int v = 0; v < 16; v++) acc[v] += lo[v];
+    if (sums_not_finite (acc))
+    {
+        const floatx16 x = single_precision_block<false, COH, true, false> (descriptor.address (), tm, tn * VAR3_BN + row, first, cnt);
+        #pragma unroll
+        for (int v = 0; v < 16; v++) acc[v] = fabsf (acc[v]) < INFINITY ? acc[v] : x[v];
+    }
+    #pragma unroll
+    for (int v = 0; v < 16; v++) mine[ACC_N (0, 0, v, lane) * NARROW_ROW + row] = acc[v];
     __syncthreads ();
     const narrow_piece_t pc = narrow_piece (tid);
     float4 sum = ld4 (smem + pc.n * NARROW_ROW + pc.c);
@@ -2339,8 +2466,8 @@ __device__ __forceinline__ void finish_tile (const aspen_hip_layer_t &L, uint32_
     contraction_epilogue<COH, true> (L, tn, t - tn * L.tiles_m, smem, tall ? 5 : 4, tall ? VAR4_BN : VAR2_BN, pre);
 }
 
-// Runs tile t of the layer.  `descriptor ()` yields a wave-uniform copy of the layer's descriptor (scalar_layer /
-// uniform_layer); a contraction tile asks for it a second time behind its K loop, so that what only the
+// Runs tile t of the layer.  `descriptor ()` yields a wave-uniform copy of the layer's descriptor (layer_at);
+// a contraction tile asks for it a second time behind its K loop, so that what only the
 // epilogue needs does not occupy scalar registers while the loop runs.  `arrivals ()` yields the graph's array of zero-initialised counters, one per
 // tile (used at the index of a split-K group's first tile); it is a callable so that the pointer is
 // fetched where it is needed instead of occupying registers while the tile runs.  Returns false for

@@ -165,6 +165,11 @@ int aspen_hip_dense_device_to_host (float *dst_host, const float *src, uint32_t 
    calibration point for a profiler's HBM byte counters. */
 int aspen_hip_copy (void *dst, const void *src, size_t bytes);
 
+/* ---- contraction arithmetic ------------------------------------------------------------------ */
+/* Convolutions, fully connected and matmul layers and the plain products below sum in single precision over operands split
+   into three bfloat16 terms.  Range: float's own.  Infinities, NaNs and sums beyond the largest float come out as in float
+   arithmetic (RELU and LEAKY_RELU, x > 0 ? x : ..., make a NaN 0 and keep it, as the reference's do); an operand below 2^-110
+   in magnitude enters with an absolute error of up to 2^-134. */
 /* ---- weights --------------------------------------------------------------------------------- */
 /* Device copy of a contraction layer's weights in the order the kernels read them, from M rows of Kp floats on the host
    (Kp a multiple of 32; K order as for aspen_hip_layer_t.weight).  raw = 0: each float as three bfloat16 terms that add up to it exactly (6
