@@ -80,7 +80,7 @@ struct aspen_hip_graph_t
     uint32_t default_workgroups;    // grid of a dataflow run when the caller names none, see graph_parallelism
     double parallelism;             // average parallelism of the tile graph, see graph_parallelism
     int cached_loads;       // 1: no cache line of an activation is shared by two producer tiles
-    void **d_arranged;              // per layer: the graph's own arranged copy of its weights, or NULL (see graph_create)
+    const float **row_weights;      // per layer: the caller's row-major weights, NULL where they are arranged already (see arrange_row_weights)
     unsigned long long *d_trace;    // [2*tile] start, [2*tile+1] end time stamps (allocated on first traced run)
     uint32_t *h_abort;              // pinned host word the persistent kernel raises when it gives this graph's run up
 };
@@ -1276,8 +1276,8 @@ static double graph_parallelism (const aspen_hip_layer_t *layers, const uint32_t
 
 static bool is_contraction (const aspen_hip_layer_t &L) { return (L.type == CONV_LAYER || L.type == FC_LAYER || L.type == MATMUL_LAYER) && L.num_ninst != 0; }
 
-// prepared: the contraction layers' weights come from aspen_hip_upload_weights; else they are row-major floats, and the
-// graph makes and owns the arranged copies
+// prepared: the contraction layers' weights come from aspen_hip_upload_weights; else they are row-major floats that stay the
+// caller's, and the graph owns the buffers every run arranges them in (arrange_row_weights)
 static aspen_hip_graph_t *graph_create (const aspen_hip_layer_t *layers, uint32_t num_layers,
     const uint32_t *ninst_layer, const uint32_t *num_parents, const uint32_t *child_off,
     const uint32_t *child_idx, uint32_t num_ninst, const uint32_t *roots, uint32_t num_roots, bool prepared)
@@ -1353,16 +1353,15 @@ static aspen_hip_graph_t *graph_create (const aspen_hip_layer_t *layers, uint32_
     for (uint32_t l = 0; l < num_layers; l++) fill_derived (g->h_layers[l]);
     if (!prepared)
     {
-        g->d_arranged = (void **)calloc (num_layers ? num_layers : 1, sizeof (void *));
-        bool ok = g->d_arranged != nullptr;
+        g->row_weights = (const float **)calloc (num_layers ? num_layers : 1, sizeof (float *));
+        bool ok = g->row_weights != nullptr;
         for (uint32_t l = 0; l < num_layers && ok; l++)
         {
             aspen_hip_layer_t &L = g->h_layers[l];
             if (!is_contraction (L)) continue;
-            const bool raw = L.variant == ASPEN_HIP_GEMM_TALL;
-            g->d_arranged[l] = aspen_hip_alloc (arranged_bytes (L.M, L.Kp, raw));
-            ok = g->d_arranged[l] && arrange_weights (g->d_arranged[l], L.weight, L.Kp, L.M, L.Kp, raw) == 0;
-            L.weight = (const float *)g->d_arranged[l];
+            void *arranged = aspen_hip_alloc (arranged_bytes (L.M, L.Kp, L.variant == ASPEN_HIP_GEMM_TALL));
+            ok = arranged != nullptr;
+            if (ok) { g->row_weights[l] = L.weight; L.weight = (const float *)arranged; }
         }
         if (!ok) { aspen_hip_graph_destroy (g); return nullptr; }
     }
@@ -1451,8 +1450,8 @@ extern "C" void aspen_hip_graph_destroy (aspen_hip_graph_t *g)
 {
     if (!g) return;
     (void)hipStreamSynchronize (g_stream);
-    for (uint32_t l = 0; g->d_arranged && l < g->num_layers; l++) aspen_hip_free (g->d_arranged[l]);
-    free (g->d_arranged);
+    for (uint32_t l = 0; g->row_weights && l < g->num_layers; l++) if (g->row_weights[l]) aspen_hip_free ((void *)g->h_layers[l].weight);
+    free (g->row_weights);
     aspen_hip_free (g->d_layers); aspen_hip_free (g->d_ninst_layer); aspen_hip_free (g->d_num_parents);
     aspen_hip_free (g->d_child_off); aspen_hip_free (g->d_child_idx); aspen_hip_free (g->d_roots); aspen_hip_free (g->d_ninst_home); aspen_hip_free (g->d_root_pos);
     aspen_hip_free (g->d_child_rec); aspen_hip_free (g->d_dep); aspen_hip_free (g->d_queue); aspen_hip_free (g->d_ran); aspen_hip_free (g->d_arrivals); aspen_hip_free (g->d_state); aspen_hip_free (g->d_prof); aspen_hip_free (g->d_trace); aspen_hip_free (g->d_group_sinks); aspen_hip_free (g->d_dep_spread);
@@ -1475,9 +1474,22 @@ static void launch_layer (const aspen_hip_graph_t *g, uint32_t l)
         hipLaunchKernelGGL (finish_kernel, dim3 (L.tiles_m * L.tiles_n), dim3 (WG_THREADS), EPI_FLOATS (VAR2_BM, VAR2_BN) * sizeof (float), g_stream, g->d_layers, l);
 }
 
+// The weights of a graph whose caller keeps them as rows, in the kernels' order, in front of a run: they are read as they are
+// when the run starts (2.5 times their bytes moved; graphs from aspen_hip_graph_create_prepared have nothing to do).
+static int arrange_row_weights (const aspen_hip_graph_t *g, uint32_t first_layer, uint32_t last_layer)
+{
+    for (uint32_t l = first_layer; g->row_weights && l <= last_layer; l++)
+    {
+        const aspen_hip_layer_t &L = g->h_layers[l];
+        if (g->row_weights[l] && arrange_weights ((void *)L.weight, g->row_weights[l], L.Kp, L.M, L.Kp, L.variant == ASPEN_HIP_GEMM_TALL)) return -1;
+    }
+    return 0;
+}
+
 extern "C" int aspen_hip_run_layers (aspen_hip_graph_t *g, uint32_t first_layer, uint32_t last_layer)
 {
     if (!g || first_layer > last_layer || last_layer >= g->num_layers) { snprintf (g_err, sizeof (g_err), "run_layers: bad range"); return -1; }
+    if (arrange_row_weights (g, first_layer, last_layer)) return -1;
     g->last_run_dataflow = 0;
     for (uint32_t l = first_layer; l <= last_layer; l++)
     {
@@ -1493,6 +1505,7 @@ extern "C" int aspen_hip_run_dataflow (aspen_hip_graph_t *g, uint32_t workgroups
 {
     if (!g) { snprintf (g_err, sizeof (g_err), "run_dataflow: null graph"); return -1; }
     if (g->num_ninst == 0) return 0;
+    if (arrange_row_weights (g, 0, g->num_layers - 1)) return -1;
     const uint32_t workgroups_requested = workgroups;
     if (workgroups == 0) workgroups = g->default_workgroups;
     if (workgroups > QUEUE_SLACK) workgroups = QUEUE_SLACK;         // every waiting workgroup must find a "leave" entry within its queue
@@ -1645,6 +1658,7 @@ extern "C" double aspen_hip_graph_parallelism (const aspen_hip_graph_t *g) { ret
 extern "C" int aspen_hip_profile_layers (aspen_hip_graph_t *g, uint32_t iters, float *ms_per_layer)
 {
     if (!g || !ms_per_layer || iters == 0) return -1;
+    if (g->num_layers && arrange_row_weights (g, 0, g->num_layers - 1)) return -1;
     for (uint32_t l = 0; l < g->num_layers; l++)
     {
         const aspen_hip_layer_t &L = g->h_layers[l];

@@ -186,7 +186,8 @@ aspen_hip_graph_t *aspen_hip_graph_create (const aspen_hip_layer_t *layers, uint
     const uint32_t *ninst_layer, const uint32_t *num_parents, const uint32_t *child_off,
     const uint32_t *child_idx, uint32_t num_ninst, const uint32_t *roots, uint32_t num_roots);
 /* The same for layers whose `weight` (contraction layers) is an aspen_hip_upload_weights copy, which several graphs may
-   share.  aspen_hip_graph_create makes such copies of the row-major weights it is given and keeps them with the graph. */
+   share.  A graph from aspen_hip_graph_create reads its callers' row-major weights anew in front of every run, into buffers of
+   its own (6 bytes per weight): it is the slower and larger of the two by these. */
 aspen_hip_graph_t *aspen_hip_graph_create_prepared (const aspen_hip_layer_t *layers, uint32_t num_layers,
     const uint32_t *ninst_layer, const uint32_t *num_parents, const uint32_t *child_off,
     const uint32_t *child_idx, uint32_t num_ninst, const uint32_t *roots, uint32_t num_roots);

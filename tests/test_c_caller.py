@@ -16,10 +16,10 @@ CALLER_SRC = os.path.join(ROOT, "tests", "c", "caller.c")
 REFERENCE = "/root/reference"
 
 
-def build_caller(out_dir):
+def build_caller(out_dir, src=CALLER_SRC):
     exe = os.path.join(str(out_dir), "caller")
     lib_dir = os.path.dirname(api.LIB_PATH)
-    subprocess.check_call(["gcc", "-O1", "-Wall", "-Wextra", "-Werror", "-I", INCLUDE, CALLER_SRC, "-o", exe,
+    subprocess.check_call(["gcc", "-O1", "-Wall", "-Wextra", "-Werror", "-I", INCLUDE, src, "-o", exe,
                            "-L", lib_dir, "-laspen_amd", f"-Wl,-rpath,{lib_dir}", "-Wl,-rpath,/opt/rocm/lib", "-lm"])
     return exe
 
@@ -90,3 +90,13 @@ def test_c_caller_runs_a_network_and_matches_the_reference_fixture(gpu, tmp_path
     got = np.fromfile(out_path, dtype=np.float32).reshape(want.shape)
     assert H.rel_l2(got, want) <= H.REL_L2_TOL
     assert (got.argmax(1) == want.argmax(1)).all()
+
+
+@pytest.mark.gpu
+def test_c_caller_changes_the_weights_of_its_own_graph(gpu, tmp_path):
+    """A graph built by its caller (aspen_hip_graph_create) reads the weights where the caller keeps them: weights written between
+    two runs are those of the next run, with either engine and for every layout the kernels want them in."""
+    exe = build_caller(tmp_path, os.path.join(ROOT, "tests", "c", "graph_caller.c"))
+    print("running", exe, flush=True)
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0 and r.stdout.endswith("ok\n"), r.stdout[-2000:] + r.stderr[-2000:]
