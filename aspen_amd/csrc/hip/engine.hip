@@ -1036,7 +1036,12 @@ __global__ void __launch_bounds__ (WG_THREADS) arrange_weights_kernel (const flo
         if (row < M)
         {
             const float *src = rows + (size_t)row * ld + (size_t)slice * SLICE_K + unit * 4u;
-            a = gld4 (src); b = gld4 (src + 16);
+            if (((uintptr_t)rows & 15u) == 0) { a = gld4 (src); b = gld4 (src + 16); }
+            else        // (the plain product's A may begin anywhere; its strides are multiples of four floats)
+            {
+                a = make_float4 (gld1 (src), gld1 (src + 1), gld1 (src + 2), gld1 (src + 3));
+                b = make_float4 (gld1 (src + 16), gld1 (src + 17), gld1 (src + 18), gld1 (src + 19));
+            }
         }
         constexpr uint32_t SLICE = WeightFragments<RAW>::SLICE;
         char *d = dst + bs * SLICE + step * (SLICE / 2) + lane * 16u;

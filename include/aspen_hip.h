@@ -301,8 +301,9 @@ void aspen_hip_divider_for (uint32_t d, uint32_t out[2]);
 
 /* ---- plain SGEMM seam (reference include/kernels.h:15-33 on device pointers) -------------------- */
 /* C[n*ldc + m] = act(bias[m] + sum_k A[m*lda + k] * B[n*ldb + k]); A row-major [M][K] (not packed),
-   lda/ldb/ldc multiples of 4, K a multiple of 32.  The arranged copy of A lives in device memory the library keeps
-   between calls (up to 96 MB); release_workspaces gives it back. */
+   lda/ldb/ldc multiples of 4, K a multiple of 32; A may begin at any float.  The arranged copy of A lives in device memory the
+   library keeps between calls (up to 96 MB; a call that finds it in use by another host thread takes its own);
+   release_workspaces gives it back. */
 void aspen_hip_release_workspaces (void);
 int aspen_hip_sgemm (uint32_t M, uint32_t N, uint32_t K, const float *A, uint32_t lda, const float *B,
     uint32_t ldb, float *C, uint32_t ldc, const float *bias, int act);
