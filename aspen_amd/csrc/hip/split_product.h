@@ -4,8 +4,9 @@
 // all three terms are exact (each rounding to nearest takes eight bits and a sign off the rest; the rest of the second
 // fits a bfloat16 whole).  A product of two floats is then nine products of bfloat16 terms, each of them exact in the
 // matrix core's single-precision sum.  Six are computed:
-//     a b = ah bh  +  (ah bm + am bh)  +  (ah bl + al bh + am bm)      left out: am bl + al bm + al bl < 2^-25 |a b|
-// i.e. less than half of what rounding ONE float product to a float may cost.  The leading products are summed in one
+//     a b = ah bh  +  (ah bm + am bh)  +  (ah bl + al bh + am bm)      left out: am bl + al bm + al bl < 2^-24 |a b|
+// (|m| <= 2^-8 |x|, |l| <= 2^-17 |x|), i.e. at worst what rounding ONE float product to a float may cost, 0.09 of that in the root mean
+// square over mantissas.  The leading products are summed in one
 // accumulator and the five small ones in another, added at the end: the large sum is then rounded once per 16 K positions
 // instead of once per two (v_mfma_f32_32x32x2_f32), the small sum's roundings do not count at its size, and the result is closer to the
 // exact one than the single-precision matrix instruction's (relative to a 64-bit sum, 2-norm over 128 x 128 results, inputs

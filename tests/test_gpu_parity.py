@@ -1081,7 +1081,7 @@ def test_weights_reloaded_between_runs_are_used_by_the_next_run(gpu, mode, tmp_p
 @pytest.mark.parametrize("M,N,K", [(1, 1, 32), (31, 33, 64), (63, 65, 96), (64, 64, 128), (65, 63, 160), (129, 127, 1056), (300, 200, 4096)])
 def test_three_term_products_keep_single_precision(gpu, M, N, K):
     """Every float enters a contraction as three bfloat16 terms that add up to it, six of the nine partial products are
-    summed in single precision (the other three are below 2^-25 of the product), so an output differs from the exact sum by at
+    summed in single precision (the other three are below 2^-24 of the product together), so an output differs from the exact sum by at
     most (roundings of the running sums) x 2^-24 x sum |a b|: one rounding per 16 K positions in each of the two running sums
     (the matrix core may round its 16-term sums once more), the dropped products and the last additions.  Magnitudes
     over 2^-20 .. 2^20 and all K remainders of the two-slice loop."""

@@ -186,3 +186,20 @@ def test_products_of_the_smallest_operands(gpu, m, n, k):
         err = np.abs(got - b @ a.T)
         print("worst", (m, n, k), swap, np.max(err / (bound + lost)), np.max(err / bound), flush=True)
         assert np.all(err <= bound + lost)
+
+
+@pytest.mark.parametrize("m,n,k", [(40, 37, 32), (33, 31, 3072), (513, 1025, 64), (1031, 2570, 96)])
+def test_products_whose_dropped_terms_add_up(gpu, m, n, k):
+    """Operands of one sign whose mantissa leaves the most in the three partial products that are not computed: 0.991 x 2^-24 of
+    every product, all in one direction (1 + 2^-8 - 2^-17 + 2^-23 has 0.98), next to one rounding per 16 K positions of the leading sum,
+    2^-7 of that for the small sum, and the addition of the two: 2^-24 of the sum each."""
+    worst = np.uint32(0x3f807fc0).view(np.float32)
+    rng = np.random.default_rng(k)
+    A = (worst * 2.0 ** rng.integers(-3, 4, (m, k))).astype(np.float32)
+    B = (worst * 2.0 ** rng.integers(-3, 4, (n, k))).astype(np.float32)
+    a, b = A.astype(np.float64), B.astype(np.float64)
+    exact = b @ a.T
+    for entry in (api.lib().aspen_hip_sgemm, api.lib().aspen_hip_sgemm_static):
+        error = np.max(np.abs(product(entry, A, B, np.zeros(m, dtype=np.float32), 0) - exact) / exact)
+        print("worst", (m, n, k), error * 2.0 ** 24, flush=True)
+        assert error <= (k // 16 * (1 + 2.0 ** -7) + 2) * 2.0 ** -24
