@@ -198,9 +198,9 @@ __device__ __forceinline__ float4 act4 (float4 v, int act)
 }
 
 // ---------------------------------------------------------------------------------------------
-// Operand loaders.  A loader fetches this thread's share of one GEMM_BK-wide K slice into registers
-// (load) and later parks it in LDS as [row][LDS_ROW] (store), so the global loads of slice i+1 fly
-// while the matrix cores work on slice i.
+// Operand loaders.  A loader fetches this thread's share of one K slice into registers (load) and later parks it in LDS
+// (store), so the global loads of later slices fly while the matrix cores work on this one: attention tiles as
+// [row][LDS_ROW] floats, contraction tiles as three terms (SliceShare).
 // ---------------------------------------------------------------------------------------------
 
 // Rows of Q, K and probability matrices: K-contiguous in memory.
@@ -408,7 +408,7 @@ template <int ROWS, int COH> struct TableLoader
 // (ASPEN_HIP_OPERAND_DENSE3; the stem of ResNet-50 contracts 160 instead of 224, VGG-16's first layer 32 instead of
 // 64).  A chunk of four K positions spans two pixels: both are fetched (16 bytes each, the pixels of the matrix keep
 // their padded fourth float) and the chunk is put together from the last channels of the first and the first
-// channels of the second; chunk index % 3 says how many of each.  A loader of its own so that ConvLoader's code, which
+// channels of the second; chunk index % 3 says how many of each.  A loader of its own so that StepLoader's code, which
 // every other convolution runs, stays as it is.
 template <int ROWS, int COH> struct Dense3Loader
 {
@@ -493,10 +493,10 @@ template <int COH> struct TransLoader64
 };
 
 // ---------------------------------------------------------------------------------------------
-// fp32 MFMA core.  Workgroup tile = BM weight rows x BN activation rows; WM x WN wavefronts, each
-// owning (BM/WM) x (BN/WN) built from 32x32 v_mfma_f32_32x32x2_f32 blocks.  The activation row is
-// the MFMA row index and the weight row the MFMA column, so each accumulator register holds 32
-// consecutive output channels of one output column: stores are 128-byte coalesced.
+// fp32 MFMA core of the attention tiles (contraction tiles: split_core below).  Workgroup tile = BM rows of the first operand x
+// BN rows of the second; WM x WN wavefronts, each owning (BM/WM) x (BN/WN) built from 32x32 v_mfma_f32_32x32x2_f32
+// blocks.  The second operand's row is the MFMA row index and the first one's the MFMA column, so each
+// accumulator register holds 32 consecutive rows of one output column: stores are 128-byte coalesced.
 // One LDS stage; the K slice after the staged one waits in registers.
 // ---------------------------------------------------------------------------------------------
 // LDS-only barrier: waits for this wave's LDS traffic, not for global loads still in flight.
@@ -517,14 +517,8 @@ __device__ __forceinline__ void lds_barrier ()
 
 // Instruction-group hints for the machine scheduler (masks of __builtin_amdgcn_sched_group_barrier)
 #define SG_MFMA 0x008
-#define SG_VMEM_READ 0x020
 #define SG_DS_READ 0x100
-#define SG_DS_WRITE 0x200
 
-// DEPTH = number of K slices in flight from memory (register sets): 1 = the slice after the staged one
-// waits in registers; 2 = the two slices after it do.  A slice cannot take less than the memory latency
-// divided by DEPTH, and when a compute unit runs fewer workgroups than it could hold (a graph bound by its
-// dependency chains) nothing else hides that latency; the second set costs 4 registers per 32 operand rows.
 // Instruction-arbiter priority of a wavefront everywhere but inside a K loop.  The workgroups of a compute unit share
 // its matrix pipeline; the ones in a K loop can keep it busy by themselves, while a workgroup in a tile's set-up,
 // first operand fetch, epilogue or scheduling step is on the graph's critical path with a handful of instructions:
@@ -534,7 +528,7 @@ __device__ __forceinline__ void lds_barrier ()
 struct NoHook { __device__ __forceinline__ void operator() () const {} };
 
 // What a kernel that runs tiles is compiled for.  The persistent kernel exists in a few variants that leave out the
-// tile kinds a graph does not contain: four workgroups in different phases share a compute unit's 64 KB instruction
+// tile kinds a graph does not contain: three workgroups in different phases share a compute unit's 64 KB instruction
 // cache, and a transformer graph has no use for the convolution loaders' K loops, nor a ResNet for the attention tiles.
 enum : unsigned
 {
@@ -558,17 +552,9 @@ enum : unsigned
     TILES_CONVNET = TILES_GATHER | TILES_LARGE | TILES_WIDE | TILES_SMALL | TILES_POOL | TILES_RESIDUAL,
     TILES_TRANSFORMER = TILES_SMALL | TILES_ATTENTION | TILES_NORM | TILES_RESIDUAL
 };
-// `before_last_slice` runs right before the MFMAs of the last K slice: the place to request what the epilogue
-// will need from memory, with the operand registers free and a whole slice of arithmetic to hide the latency.
-// `ready` runs between the first request for the weight operand and the first request for the activation operand: a
-// kernel that starts tiles before their parents have finished (see the ordered mode of the persistent kernel) waits
-// there, with the tile's set-up done and its first weights on their way.
-template <int BM, int BN, int WM, int WN, int DEPTH, class ALoader, class BLoader, class Hook = NoHook, class Ready = NoHook>
-__device__ __forceinline__ void gemm_core (ALoader &al, BLoader &bl, int kbase, int kiters, float *smem,
-    floatx16 (&acc)[BN / WN / 32][BM / WM / 32], bool phases = false, Hook before_last_slice = Hook (), Ready ready = Ready ())
+template <int BM, int BN, int WM, int WN, class ALoader, class BLoader>
+__device__ __forceinline__ void gemm_core (ALoader &al, BLoader &bl, int kbase, int kiters, float *smem, floatx16 (&acc)[BN / WN / 32][BM / WM / 32])
 {
-    static_assert (DEPTH == 1 || DEPTH == 2, "one or two register sets");
-    if (phases) tile_phase_lap (12);
     constexpr int TM = BM / WM / 32, TN = BN / WN / 32;
     constexpr int KK = GEMM_BK / 8;
     const uint32_t tid = tile_thread (), lane = tid & 63, wave = tid >> 6;
@@ -613,14 +599,11 @@ __device__ __forceinline__ void gemm_core (ALoader &al, BLoader &bl, int kbase, 
             }
     };
 
-    // register set s holds slice it with (it - first) % DEPTH == s
-    float4 areg[DEPTH][ALoader::R], breg[DEPTH][BLoader::R];
-    al.load (kbase, areg[0]); ready (); bl.load (kbase, breg[0]);
-    if (DEPTH == 2 && kiters > 1) { al.load (kbase + 1, areg[DEPTH - 1]); bl.load (kbase + 1, breg[DEPTH - 1]); }
-    al.store (smem, areg[0]); bl.store (smem + BM * LDS_ROW, breg[0]);
-    if (kiters > DEPTH) { al.load (kbase + DEPTH, areg[0]); bl.load (kbase + DEPTH, breg[0]); }
+    float4 areg[ALoader::R], breg[BLoader::R];      // the slice after the staged one
+    al.load (kbase, areg); bl.load (kbase, breg);
+    al.store (smem, areg); bl.store (smem + BM * LDS_ROW, breg);
+    if (kiters > 1) { al.load (kbase + 1, areg); bl.load (kbase + 1, breg); }
     lds_barrier ();
-    if (phases) tile_phase_lap (8);
     __builtin_amdgcn_s_setprio (0);
     read_frags (0, 0);
 
@@ -628,14 +611,12 @@ __device__ __forceinline__ void gemm_core (ALoader &al, BLoader &bl, int kbase, 
     //   sub-steps 0 .. KK-2: the fragments of sub-step s+1 are fetched between the two halves of the
     //   MFMAs of sub-step s, so they have arrived even if the compiler waits for ALL LDS traffic before s+1;
     //   last sub-step: once every wave holds its last fragments (barrier), the next slice (waiting in
-    //   registers) overwrites the stage and the slice DEPTH after it is requested from memory into the
+    //   registers) overwrites the stage and the one after it is requested from memory into the
     //   registers just freed, all under the first half of the sub-step's MFMAs; after the second barrier the
     //   first fragments of the new slice are fetched under the second half.
     // The scheduling-group hints pin that order; left alone, the compiler fetches each fragment right
     // before its use and the LDS latency shows.
-    // `set` (a literal at every call, so that the register arrays are indexed statically) = the register set
-    // that holds slice it + 1.
-    auto slice = [&] (int it, int set)
+    for (int it = 0; it + 1 < kiters; it++)
     {
         #pragma unroll
         for (int kk = 0; kk + 1 < KK; kk++)
@@ -650,15 +631,8 @@ __device__ __forceinline__ void gemm_core (ALoader &al, BLoader &bl, int kbase, 
         __builtin_amdgcn_sched_barrier (0);
         lds_barrier ();
         __builtin_amdgcn_sched_barrier (0);
-        al.store (smem, areg[set]); bl.store (smem + BM * LDS_ROW, breg[set]);
-        if (DEPTH == 2)
-        {
-            // always issued (the last slices are requested again and never used): a request inside a branch makes
-            // the compiler lose count of what is in flight, and it then waits for everything before every store
-            const int nxt = kbase + min (it + 1 + DEPTH, kiters - 1);
-            al.load (nxt, areg[set]); bl.load (nxt, breg[set]);
-        }
-        else if (it + 1 + DEPTH < kiters) { al.load (kbase + it + 1 + DEPTH, areg[set]); bl.load (kbase + it + 1 + DEPTH, breg[set]); }
+        al.store (smem, areg); bl.store (smem + BM * LDS_ROW, breg);
+        if (it + 2 < kiters) { al.load (kbase + it + 2, areg); bl.load (kbase + it + 2, breg); }
         mfma_half ((KK - 1) & 1, 0);
         __builtin_amdgcn_sched_barrier (0);
         lds_barrier ();
@@ -667,18 +641,8 @@ __device__ __forceinline__ void gemm_core (ALoader &al, BLoader &bl, int kbase, 
         mfma_half ((KK - 1) & 1, 1);
         __builtin_amdgcn_sched_group_barrier (SG_DS_READ, TM + TN, 0);
         __builtin_amdgcn_sched_group_barrier (SG_MFMA, 2 * TM * TN, 0);
-    };
-    if (DEPTH == 1)
-        for (int it = 0; it + 1 < kiters; it++) slice (it, 0);
-    else
-    {
-        // slice it + 1 sits in set (it + 1) % 2: two slices per trip keep the set a literal
-        int it = 0;
-        for (; it + 2 < kiters; it += 2) { slice (it, DEPTH - 1); slice (it + 1, 0); }
-        if (it + 1 < kiters) slice (it, DEPTH - 1);
     }
     // last slice: nothing left to stage
-    before_last_slice ();
     #pragma unroll
     for (int kk = 0; kk < KK; kk++)
     {
@@ -693,18 +657,6 @@ __device__ __forceinline__ void gemm_core (ALoader &al, BLoader &bl, int kbase, 
     lds_barrier ();          // the caller reuses the stage (epilogue)
 }
 
-// The same for the 64 x 64 shape, whose four waves own ONE 32 x 32 block each, scheduled by hand for a
-// workgroup that has its compute unit (nearly) to itself -- the normal case for these tiles: they are the
-// short tiles of layers cut along K, and in a graph bound by its dependency chains only one or two
-// workgroups per compute unit are inside a K loop at any time.  Then nothing but this wave's own instruction
-// order hides the slice boundary (two barriers, the LDS refill, the next requests): in gemm_core the matrix
-// pipeline drains there, 16 MFMAs of 64 cycles each took ~1600 cycles per slice.
-// Here the fragments of all four sub-steps of a slice are resident (8 registers each, affordable with one
-// accumulator block), so every piece of boundary work sits between two MFMAs that do not depend on it:
-//   M00 M01 M02 |X| M03 wA M10 wB M11 gA M12 gB M13 M20 |Y| M21 r0 M22 r1 M23 M30 r2 M31 M32 M33 r3
-// Mij = MFMA on K pair j of sub-step i; X = barrier "everyone holds this slice's fragments", wA / wB = next
-// slice registers -> LDS, gA / gB = requests for the slice DEPTH ahead, Y = barrier "refill visible",
-// ri = fragments of sub-step i of the next slice (its buffer was released by Mi3).
 // Accumulator register v of MFMA block (i, j) holds output (row n, channel m):
 //   n = wn0 + 32 i + 8 (v / 4) + 4 (lane / 32) + v % 4,   m = wm0 + 32 j + lane % 32
 #define ACC_N(wn0, i, v, lane) ((wn0) + 32 * (i) + 8 * ((v) >> 2) + 4 * ((lane) >> 5) + ((v) & 3))
@@ -754,16 +706,22 @@ __device__ __forceinline__ void norm_fold_finish (const aspen_hip_layer_t &L, fl
     }
 }
 
-template <int DEPTH, class ALoader, class BLoader, class Hook = NoHook, class Ready = NoHook, class Stats = NoStats>
-__device__ __forceinline__ void gemm_core_single_block (ALoader &al, BLoader &bl, int kbase, int kiters, float *smem,
-    floatx16 (&accs)[1][1], bool phases = false, Hook before_last_slice = Hook (), Ready ready = Ready (), Stats stats = Stats ())
+// The same for 64 x 64 products, whose four waves own ONE 32 x 32 block each, scheduled by hand for a
+// workgroup that has its compute unit (nearly) to itself: in a graph bound by its dependency chains only one or two
+// workgroups per compute unit are inside a K loop at any time.  Then nothing but this wave's own instruction
+// order hides the slice boundary (two barriers, the LDS refill, the next requests): in gemm_core the matrix
+// pipeline drains there, 16 MFMAs of 64 cycles each took ~1600 cycles per slice.
+// Here the fragments of all four sub-steps of a slice are resident (8 registers each, affordable with one
+// accumulator block), so every piece of boundary work sits between two MFMAs that do not depend on it:
+//   M00 M01 M02 |X| M03 wA M10 wB M11 gA M12 gB M13 M20 |Y| M21 r0 M22 r1 M23 M30 r2 M31 M32 M33 r3
+// Mij = MFMA on K pair j of sub-step i; X = barrier "everyone holds this slice's fragments", wA / wB = next
+// slice registers -> LDS, gA / gB = requests for the slice after it, Y = barrier "refill visible",
+// ri = fragments of sub-step i of the next slice (its buffer was released by Mi3).
+template <class ALoader, class BLoader>
+__device__ __forceinline__ void gemm_core_single_block (ALoader &al, BLoader &bl, int kbase, int kiters, float *smem, floatx16 (&accs)[1][1])
 {
-    // `stats` sees every K slice of the activation operand once, as the registers it passes through on its way into LDS
-    // (a folded layer norm's column sums, see norm_fold_finish)
-    static_assert (DEPTH == 1 || DEPTH == 2, "one or two register sets");
     static_assert (ALoader::R == 2 && BLoader::R == 2 && GEMM_BK == 32, "64 x 64 tile, four sub-steps");
     constexpr int BM = 64;
-    if (phases) tile_phase_lap (12);
     const uint32_t tid = tile_thread (), lane = tid & 63, wave = tid >> 6;
     const uint32_t wm0 = (wave % 2) * 32, wn0 = (wave / 2) * 32;
     const float *afrag = smem + wm0 * LDS_ROW + (lane & 31) * LDS_ROW + (lane >> 5) * 4;
@@ -775,43 +733,28 @@ __device__ __forceinline__ void gemm_core_single_block (ALoader &al, BLoader &bl
 #define SB __builtin_amdgcn_sched_barrier (0)
 #define RD(i) do { fa[i] = ld4 (afrag + (i) * 8); fb[i] = ld4 (bfrag + (i) * 8); SB; } while (0)
 #define MF(i, c) do { acc = __builtin_amdgcn_mfma_f32_32x32x2f32 (fb[i].c, fa[i].c, acc, 0, 0, 0); SB; } while (0)
-    float4 areg[DEPTH][2], breg[DEPTH][2];
-    al.load (kbase, areg[0]); ready (); bl.load (kbase, breg[0]);
-    if (DEPTH == 2 && kiters > 1) { al.load (kbase + 1, areg[DEPTH - 1]); bl.load (kbase + 1, breg[DEPTH - 1]); }
-    al.store (smem, areg[0]); bl.store (smem + BM * LDS_ROW, breg[0]); stats (breg[0]);
-    if (kiters > DEPTH) { al.load (kbase + DEPTH, areg[0]); bl.load (kbase + DEPTH, breg[0]); }
+    float4 areg[2], breg[2];        // the slice after the staged one
+    al.load (kbase, areg); bl.load (kbase, breg);
+    al.store (smem, areg); bl.store (smem + BM * LDS_ROW, breg);
+    if (kiters > 1) { al.load (kbase + 1, areg); bl.load (kbase + 1, breg); }
     lds_barrier ();
-    if (phases) tile_phase_lap (8);
     __builtin_amdgcn_s_setprio (0);
     SB; RD (0); RD (1); RD (2); RD (3);
-    // `set` (a literal at every call) = the register set that holds slice it + 1
-    auto slice = [&] (int it, int set)
+    for (int it = 0; it + 1 < kiters; it++)
     {
-        // requests are always issued (the last slices are asked for again and never used): a request inside a
-        // branch makes the compiler lose count of what is in flight, and it then waits for everything
-        const int nxt = kbase + (DEPTH == 2 ? min (it + 1 + DEPTH, kiters - 1) : it + 2);
         SB; MF (0, x); MF (0, y); MF (0, z);
         lds_barrier (); SB;
-        MF (0, w); al.store (smem, areg[set]); SB;
-        MF (1, x); bl.store (smem + BM * LDS_ROW, breg[set]); stats (breg[set]); SB;
-        MF (1, y); if (DEPTH == 2 || it + 2 < kiters) al.load (nxt, areg[set]); SB;
-        MF (1, z); if (DEPTH == 2 || it + 2 < kiters) bl.load (nxt, breg[set]); SB;
+        MF (0, w); al.store (smem, areg); SB;
+        MF (1, x); bl.store (smem + BM * LDS_ROW, breg); SB;
+        MF (1, y); if (it + 2 < kiters) al.load (kbase + it + 2, areg); SB;
+        MF (1, z); if (it + 2 < kiters) bl.load (kbase + it + 2, breg); SB;
         MF (1, w); MF (2, x);
         lds_barrier (); SB;
         MF (2, y); RD (0);
         MF (2, z); RD (1);
         MF (2, w); MF (3, x); RD (2);
         MF (3, y); MF (3, z); MF (3, w); RD (3);
-    };
-    if (DEPTH == 1)
-        for (int it = 0; it + 1 < kiters; it++) slice (it, 0);
-    else
-    {
-        int it = 0;
-        for (; it + 2 < kiters; it += 2) { slice (it, DEPTH - 1); slice (it + 1, 0); }
-        if (it + 1 < kiters) slice (it, DEPTH - 1);
     }
-    before_last_slice ();
     SB;
     MF (0, x); MF (0, y); MF (0, z); MF (0, w); MF (1, x); MF (1, y); MF (1, z); MF (1, w);
     MF (2, x); MF (2, y); MF (2, z); MF (2, w); MF (3, x); MF (3, y); MF (3, z); MF (3, w);
@@ -1906,7 +1849,7 @@ __device__ __forceinline__ void tile_k_attention (const aspen_hip_layer_t &L, ui
     {
         ActRowLoader<BM, COH> al; al.init (Kmat, b * S + k0, b * S + S - 1, L.ld1, h * L.hd, tid);
         ActRowLoader<BN, COH> bl; bl.init (Q, b * S + q0, b * S + S - 1, L.ld0, h * L.hd, tid);
-        gemm_core<BM, BN, WM, WN, 1> (al, bl, 0, kiters, smem, acc);
+        gemm_core<BM, BN, WM, WN> (al, bl, 0, kiters, smem, acc);
     };
     // exponential of one score; reference order of operations: mask with -1e10, scale, exp, no max subtraction.
     // The hardware exponential (2^(x log2 e), about 1e-6 relative for scores of a few units against libm's expf, two
@@ -2011,7 +1954,7 @@ __device__ __forceinline__ void tile_v_attention (const aspen_hip_layer_t &L, ui
     floatx16 acc[TN][TM];
     TransLoader64<COH> al; al.init (V, b * S * L.ld1 + m0, L.ld1, L.tile_m, S, tid);
     ActRowLoader<BN, COH> bl; bl.init (P, prow + q0, prow + S - 1, L.ld0, 0, tid);   // P's stride is a multiple of 32 with zero padding
-    gemm_core<BM, BN, WM, WN, 1> (al, bl, 0, (int)((S + GEMM_BK - 1) / GEMM_BK), smem, acc);
+    gemm_core<BM, BN, WM, WN> (al, bl, 0, (int)((S + GEMM_BK - 1) / GEMM_BK), smem, acc);
     const uint32_t mm = wm0 + (lane & 31);
     if (mm < L.tile_m)
         #pragma unroll
@@ -2072,7 +2015,7 @@ __device__ __forceinline__ void tile_fused_attention (const aspen_hip_layer_t &L
         {
             ActRowLoader<64, COH> al; al.init (Kmat, b * S + k0, b * S + S - 1, L.ld1, h * hd, tid);
             ActRowLoader<BQ, COH> bl; bl.init (Q, b * S + q0, b * S + S - 1, L.ld0, h * hd, tid);
-            gemm_core_single_block<1> (al, bl, 0, kiters, smem, sacc);          // ends with a barrier: the stage is free
+            gemm_core_single_block (al, bl, 0, kiters, smem, sacc);          // ends with a barrier: the stage is free
         }
         #pragma unroll
         for (int v = 0; v < 16; v++)
@@ -2153,13 +2096,12 @@ __device__ __forceinline__ bool splitk_arrived_last (uint32_t *counter, uint32_t
 // network): a layer of a few dozen 64 x 64 tiles with long K loops becomes a few hundred short ones, so that a
 // dependency level keeps every compute unit busy for one or two microseconds instead of a quarter of them for
 // eight.  Throughput per workgroup does not matter here, so there is nothing to share between wavefronts and
-// nothing is staged through LDS: a lane reads its operands from memory in the layout the matrix instruction wants
-// (row = lane % 32, four consecutive K values at (lane / 32) * 4 of every 8: v_mfma_f32_32x32x2_f32 pairs the two
-// half-waves' values, and both operands use the same pairing, so the K order inside a slice is immaterial), the
-// K loop has no barrier, and the four partial sums meet in LDS once.  A layer can additionally be cut along K across
-// workgroups (`slice` >= 0) exactly like the 64 x 64 shape, with blocks of 32 x 32 sums in the threads' own order.
-// Operands: weights [.][Kp]; activations read in place (DIRECT) or gathered by stepping through the taps (a
-// convolution or FC layer over channels that are a multiple of the slice width).
+// no operand is staged for another wavefront: a lane reads its weights as the fragments they are laid out in
+// (WeightFragments) and its activations as the floats of its row's units (row = lane % 32, see SLICE_K), splits these
+// itself, the K loop has no barrier, and the four partial sums meet in LDS once.  A layer can additionally be cut along K
+// across workgroups (`slice` >= 0) exactly like the 64 x 64 shape, with blocks of 32 x 32 sums in the threads' own order.
+// Activations are read in place (DIRECT) or gathered by stepping through the taps (a convolution or FC layer over
+// channels that are a multiple of the slice width).
 // ---------------------------------------------------------------------------------------------
 #define VAR3_BM 32
 #define VAR3_BN 32
