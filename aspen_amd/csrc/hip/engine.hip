@@ -523,7 +523,7 @@ __device__ __forceinline__ void wait_until_ready ()
 }
 
 template <int COH, unsigned FEAT, bool ORDERED = false>
-__global__ void __launch_bounds__ (WG_THREADS, (FEAT & TILES_DEEP) ? 2 : WG_PER_CU) dataflow_kernel (dataflow_args_t args)
+__global__ void __launch_bounds__ (WG_THREADS, (FEAT & TILES_DEEP) ? DEEP_WG_PER_CU : WG_PER_CU) dataflow_kernel (dataflow_args_t args)
 {
     extern __shared__ __align__ (16) float smem[];
     if (threadIdx.x == 0)
@@ -601,13 +601,27 @@ static const void *const dataflow_kernels[NUM_KERNEL_VARIANTS][2] = {
     {(const void *)dataflow_kernel<1, TILES_ALL>, (const void *)dataflow_kernel<2, TILES_ALL>}};
 
 // Ordered mode (see aspen_hip_run_dataflow), cached loads only: for convolutional networks, for those with weight-streaming
-// layers (VGG-16 at small batches), for transformer graphs, and with every tile kind.
-#define NUM_ORDERED_VARIANTS 4
+// layers (VGG-16 at small batches), for transformer graphs (two, see ordered_variant), and with every tile kind.
+enum { ORDERED_CONVNET, ORDERED_TALL, ORDERED_TRANSFORMER_DEEP, ORDERED_TRANSFORMER, ORDERED_ALL, NUM_ORDERED_VARIANTS };
 #define ORDERED_SMEM_BYTES CMAX (GEMM_SMEM_BYTES, NARROW_PF_SMEM_BYTES)       // the narrow tiles' weight prefetch buffers
-static const unsigned ordered_variant_tiles[NUM_ORDERED_VARIANTS] = {TILES_CONVNET | TILES_YOLO | TILES_NARROW, TILES_CONVNET | TILES_TALL, TILES_TRANSFORMER, TILES_ALL};
+static const unsigned ordered_variant_tiles[NUM_ORDERED_VARIANTS] = {TILES_CONVNET | TILES_YOLO | TILES_NARROW, TILES_CONVNET | TILES_TALL,
+    TILES_TRANSFORMER, TILES_TRANSFORMER, TILES_ALL};
 static const void *const ordered_kernels[NUM_ORDERED_VARIANTS] = {
     (const void *)dataflow_kernel<2, TILES_CONVNET | TILES_YOLO | TILES_NARROW, true>, (const void *)dataflow_kernel<2, TILES_CONVNET | TILES_TALL, true>,
-    (const void *)dataflow_kernel<2, TILES_TRANSFORMER | TILES_DEEP, true>, (const void *)dataflow_kernel<2, TILES_ALL, true>};
+    (const void *)dataflow_kernel<2, TILES_TRANSFORMER | TILES_DEEP, true>, (const void *)dataflow_kernel<2, TILES_TRANSFORMER, true>,
+    (const void *)dataflow_kernel<2, TILES_ALL, true>};
+// Below this estimated parallelism a transformer graph's levels leave a compute unit one or two tiles, which pay for four slices
+// in flight each; above it a third workgroup per unit is worth more.  Two deep / three plain ones, us: BERT-base 1 x 128 (135) 868 /
+// 918, 3 x 75 (197) 946 / 1005, 4 x 128 (339) 1110 / 1119; GPT-2 1 x 512 (388) 1374 / 1326, 2 x 256 (388) 1238 / 1162, BERT-base 8 x 128
+// (533) 1595 / 1489, 16 x 128 (1065) 2913 / 2735, GPT-2 4 x 512 (878) 2996 / 2865.
+#define DEEP_BELOW 350.0
+
+static int ordered_variant (const aspen_hip_graph_t *g)
+{
+    int v = 0;
+    while (v + 1 < NUM_ORDERED_VARIANTS && (g->features & ~ordered_variant_tiles[v]) != 0) v++;
+    return v == ORDERED_TRANSFORMER_DEEP && g->parallelism >= DEEP_BELOW ? ORDERED_TRANSFORMER : v;
+}
 
 // The tile kinds a graph contains, as TILES_* bits.
 static unsigned graph_features (const aspen_hip_layer_t *layers, uint32_t num_layers)
@@ -681,7 +695,7 @@ extern "C" void aspen_hip_tile_shapes (uint32_t shapes[13])
 {
     shapes[11] = VAR4_BM; shapes[12] = VAR4_BN;
     shapes[0] = VAR0_BM; shapes[1] = VAR0_BN; shapes[2] = VAR1_BM; shapes[3] = VAR1_BN; shapes[4] = VAR2_BM; shapes[5] = VAR2_BN;
-    shapes[6] = KATTN_BN; shapes[7] = VATTN_BN; shapes[8] = 2; shapes[9] = VAR3_BM; shapes[10] = VAR3_BN;
+    shapes[6] = KATTN_BN; shapes[7] = VATTN_BN; shapes[8] = DEEP_WG_PER_CU; shapes[9] = VAR3_BM; shapes[10] = VAR3_BN;
 }
 
 extern "C" int aspen_hip_device_info (int *num_cu, int *clock_khz, size_t *mem_bytes, char *name, int name_len)
@@ -1536,16 +1550,15 @@ extern "C" int aspen_hip_run_dataflow (aspen_hip_graph_t *g, uint32_t workgroups
     // reports 1e30 for a graph that is not listed that way)
     if (!g->cached_loads || xcd_queues || g->num_ninst > (1u << 20) || g->parallelism > 1e29) ordered = false;
     size_t ordered_smem = ORDERED_SMEM_BYTES;
+    const int ov = ordered_variant (g);
     if (ordered)
     {
         // tiles are assigned to workgroups beforehand: every workgroup of the grid must be running
         // (graphs without 32 x 32 tiles need no weight prefetch buffers: their workgroups take the LDS of any other tile, and
-        // twice as many fit a compute unit)
+        // three instead of two fit a compute unit)
         static int fits[NUM_ORDERED_VARIANTS][2];
         static bool fits_known[NUM_ORDERED_VARIANTS][2];
         const int small_lds = (g->features & TILES_NARROW) == 0;
-        int ov = 0;         // (the variant the launch below takes)
-        while (ov + 1 < NUM_ORDERED_VARIANTS && (g->features & ~ordered_variant_tiles[ov]) != 0) ov++;
         if (!fits_known[ov][small_lds])
         {
             int o = 0;
@@ -1558,12 +1571,10 @@ extern "C" int aspen_hip_run_dataflow (aspen_hip_graph_t *g, uint32_t workgroups
         if (fit < 1) ordered = false;
         else
         {
-            // by default two per compute unit (one tile computes, the next is prepared); without the prefetch buffers three
-            // from an estimated parallelism of 350 and four from 600 on (YOLO-v3 batch 1, 409: 1.30 / 1.25 / 1.26 ms with
-            // two / three / four; ResNet-50 batch 4, 335: 0.72 / 0.76 / 0.76; VGG-16 batch 4, 766: 1.51 / 1.40 / 1.34)
-            // (the kernel of transformer graphs fits twice, see TILES_DEEP)
-            const uint32_t per_cu = !small_lds || g->parallelism < 350.0 ? 2u : g->parallelism < 600.0 ? 3u : 4u;
-            if (workgroups_requested == 0) workgroups = per_cu * (uint32_t)g_num_cu < (uint32_t)fit ? per_cu * (uint32_t)g_num_cu : (uint32_t)fit;
+            // by default all that fit: two or three tiles of a unit compute, wait for their parents or are prepared.  Two / three per
+            // unit, us: ResNet-50 batch 2 (estimated parallelism 179) 628 / 626, 4 (338) 686 / 676, 6 (489) 809 / 746, YOLO-v3 batch 1 (419)
+            // 1171 / 1096, VGG-16 batch 1 (728) 598 / 514
+            if (workgroups_requested == 0) workgroups = (uint32_t)fit;
             if (workgroups > (uint32_t)fit) workgroups = (uint32_t)fit;
         }
     }
@@ -1640,12 +1651,7 @@ extern "C" int aspen_hip_run_dataflow (aspen_hip_graph_t *g, uint32_t workgroups
     CHECK (hipEventRecord (g_events[NUM_EVENTS - 2], g_stream));
     {
         const void *kernel = dataflow_kernels[g->variant][g->cached_loads ? 1 : 0];
-        if (ordered)
-        {
-            int v = 0;
-            while (v + 1 < NUM_ORDERED_VARIANTS && (g->features & ~ordered_variant_tiles[v]) != 0) v++;
-            kernel = ordered_kernels[v];
-        }
+        if (ordered) kernel = ordered_kernels[ov];
         g->last_run_ordered = ordered;
         void *kernel_args[] = {&a};
         CHECK (hipLaunchKernel (kernel, dim3 (workgroups), dim3 (WG_THREADS), kernel_args, ordered ? ordered_smem : GEMM_SMEM_BYTES, g_stream));

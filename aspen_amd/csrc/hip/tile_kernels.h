@@ -31,6 +31,7 @@ __device__ void tile_phase_lap (int which);
 #define VAR0_BM 128
 #define VAR0_BN 64
 #define WG_PER_CU 3
+#define DEEP_WG_PER_CU 2          // of the kernels compiled with TILES_DEEP
 #define KATTN_BN 32            // queries per K-attention tile
 #define VATTN_BN 64            // queries per V-attention tile
 #define VAR1_BM 64
@@ -540,13 +541,12 @@ enum : unsigned
     TILES_TALL = 1024u,         // the 128 x 32 contraction tile of weight-streaming layers
     TILES_DENSE_WIDE = 2048u,   // the dense three-channel operand under the 64 x 128 shape (the host library's graphs take 64 x 64 for it)
     // No tile kind: 64 x 64 tiles keep four K slices of both operands in flight, four slices to a trip through the loop, in the
-    // 249 registers per lane that two workgroups per compute unit leave.  For the ordered kernel of transformer graphs, which
-    // runs two of them: its levels are a few hundred tiles of 24 slices, one or two per compute unit, and with one slice of
-    // weights and two of activations in flight a slice took 0.42 us for 0.17 us of matrix instructions.  BERT-base 8 x 128
-    // 1.81 -> 1.67 ms, 3 x 75 1.01 -> 0.95, GPT-2 4 x 512 3.23 -> 3.03; with four slices of weights and two of activations 1.71,
-    // 1.00 and 3.05; with the loop left from its middle instead of copies of the last slices behind it 1.78, 1.03 and 3.17.
-    // Convolutional graphs run three workgroups per unit and lose with two (YOLO-v3 batch 1 1.10 -> 1.16 ms, ResNet-50
-    // batch 11 1.02 -> 1.27).
+    // 252 registers per lane that two workgroups per compute unit leave.  For the ordered kernel of transformer graphs of little
+    // parallelism: their levels are a few hundred tiles of 24 slices, one or two per compute unit, and with one slice of
+    // weights and two of activations in flight a slice took 0.42 us for 0.17 us of matrix instructions (see DEEP_BELOW for both
+    // sides).  With four slices of weights and two of activations BERT-base 3 x 75 took 1.00 ms instead of 0.95; with the
+    // loop left from its middle instead of copies of the last slices behind it 1.03.  Convolutional graphs lose with it (YOLO-v3
+    // batch 1 1.10 -> 1.16 ms, ResNet-50 batch 11 1.02 -> 1.27).
     TILES_DEEP = 4096u,
     TILES_ALL = 4095u,
     TILES_CONVNET = TILES_GATHER | TILES_LARGE | TILES_WIDE | TILES_SMALL | TILES_POOL | TILES_RESIDUAL,

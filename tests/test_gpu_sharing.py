@@ -1,5 +1,5 @@
 """What several graphs, calls and host threads share: the device copies of a model's weights, the plain product's kept
-workspace, the pinned ring that inputs and results travel through."""
+workspace, the pinned ring that inputs and results travel through; kernels between which a graph's size decides."""
 import ctypes as C
 import os
 import tempfile
@@ -164,3 +164,35 @@ def test_two_graphs_of_one_model_hold_a_layer_in_either_form(gpu, monkeypatch, m
         pool.destroy()
         nasm.destroy()
         big.close()
+
+
+@pytest.mark.parametrize("batch", [1, 4, 5, 9])
+def test_ordered_transformer_graphs_on_either_side_of_the_deep_kernel(gpu, batch):
+    """Two blocks of BERT-base, 128 tokens each: an estimated parallelism of 339 with four sequences, just below the limit up to which
+    the kernel with four slices in flight runs, and above it with five.  The sums are formed in one order everywhere, so
+    the persistent kernel agrees with one launch per layer to a rounding or two per layer: ten layers deep, 2^-24 each, 2^-20 in all."""
+    cfg = M.bert_cfg(2, 768, 12, 3072)
+    layers = M.parse_cfg(cfg)
+    tens = M.synth_weights(layers, 91, "gpt")
+    x = M.synth_input(layers, 91, batch, 128, "embeddings")
+    api.lib().aspen_keep_layer_outputs(0)
+    try:
+        net = H.GpuNet(cfg, tens, batch, 128, min_ninst=192, mode=api.MODE_LAYERS)
+        dse = api.DseGroup(1, api.MODE_DATAFLOW)
+        dse.set_rpool(net.rpool)
+        try:
+            net.run(x)
+            last = net.nasm.num_ldata - 1
+            want = net.layer(last).copy()
+            for _ in range(3):
+                net.rpool.reset_nasm(net.nasm)
+                dse.run()
+                dse.wait(net.nasm)
+                dse.stop()
+                assert H.rel_l2(net.layer(last), want) <= 2.0 ** -20
+            assert net.rpool.run_stats() == {"executed": net.nasm.num_ninst, "double_runs": 0, "aborted": 0}
+        finally:
+            dse.destroy()
+            net.close()
+    finally:
+        api.lib().aspen_keep_layer_outputs(1)
