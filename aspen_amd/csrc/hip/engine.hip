@@ -1358,9 +1358,10 @@ static aspen_hip_graph_t *graph_create (const aspen_hip_layer_t *layers, uint32_
         for (int i = NUM_KERNEL_VARIANTS - 2; i >= 0 && !all_tiles; i--) if ((g->features & ~kernel_variant_tiles[i]) == 0) g->variant = i;
         const uint32_t resident = (uint32_t)g_variant_wg[g->variant][g->cached_loads ? 1 : 0];      // of the variant this graph runs on
         uint32_t per_cu = resident;
-        // measured on 256 compute units (ResNet-50 batch 1 / 32, VGG-16, BERT, GPT-2): one more workgroup per
-        // unit pays once the average parallelism grows by another two tiles per unit
-        if (par < 2.0 * g_num_cu * resident) per_cu = (uint32_t)(par / (2.0 * g_num_cu)) + 1;
+        // ready-queue runs with one / two / three workgroups per unit on 256 units, us: ResNet-50 batch 1 (average parallelism 92) 629 / 676 /
+        // 714, BERT-base 3 x 75 (197) 1269 / 1315 / 1354, ResNet-50 batch 4 (338) 891 / 824 / 839, YOLO-v3 batch 1 (419) 1575 / 1392 /
+        // 1400, BERT-base 8 x 128 (533) 2228 / 1770 / 1837, ResNet-50 batch 8 (645) 1357 / 976 / 933, GPT-2 4 x 512 (878) 4095 / 3179 / 3102
+        if (par < 2.3 * g_num_cu) per_cu = par < g_num_cu ? 1u : 2u;
         if (per_cu > resident) per_cu = resident;
         g->default_workgroups = per_cu * (uint32_t)g_num_cu;
         if (getenv ("ASPEN_GPU_VERBOSE"))
@@ -1586,10 +1587,10 @@ extern "C" int aspen_hip_run_dataflow (aspen_hip_graph_t *g, uint32_t workgroups
     }
     uint32_t nq_mask = (xcd_queues && workgroups % NUM_QUEUES == 0) ? (NUM_QUEUES >> nq_shift) - 1u : 0u;
     // By default a graph that fills the device (every compute unit holds as many workgroups as fit) runs on TWO queues,
-    // one per half of the XCDs: tiles that read the same activations then meet in one of four L2s instead of eight (a
-    // tenth less memory traffic on the convolutional networks), and two pools of 512 workgroups balance as well as one of
-    // 1024 (same run time; four and eight queues cost 1 % and 3 %).  Smaller grids keep one queue: their runs are bound by
-    // dependency chains, and every restriction on who may take a ready tile lengthens those.
+    // one per half of the XCDs: tiles that read the same activations then meet in one of four L2s instead of eight.  One / two /
+    // four / eight queues, us: ResNet-50 batch 32 2166 / 2111 / 2074 / 2117, VGG-16 batch 32 5507 / 5497 / 5487 / 5589, YOLO-v3
+    // batch 8 4161 / 4110 / 4108 / 4145, ResNet-50 + VGG-16 4250 / 4220 / 4212 / 4330.  Smaller grids keep one queue: their runs
+    // are bound by dependency chains, and every restriction on who may take a ready tile lengthens those.
     if (!xcd_queues && !one_queue_env && !ordered && workgroups % NUM_QUEUES == 0
         && workgroups >= (uint32_t)g_variant_wg[g->variant][g->cached_loads ? 1 : 0] * (uint32_t)g_num_cu)
     { nq_shift = 2u; nq_mask = (NUM_QUEUES >> nq_shift) - 1u; }
@@ -1804,8 +1805,8 @@ extern "C" int aspen_hip_event_elapsed_ms (int a, int b, float *ms)
     return 0;
 }
 
-// One contraction tile per workgroup, the descriptor in the kernel-argument segment; compiled for one tile shape each (with
-// all of them in one kernel its loops spilled: 1000 x 3137 x 1152 85 us a call that allocates nothing, now 74).  Contiguous tile
+// One contraction tile per workgroup, the descriptor in the kernel-argument segment; compiled for one tile shape each (all of them
+// in one kernel spill: 1000 x 3137 x 1152 85 us a call that allocates nothing, 62 this way).  Contiguous tile
 // ranges per XCD, as in layer_kernel: workgroups that share activation columns meet in one L2.
 template <unsigned FEAT> __global__ void __launch_bounds__ (WG_THREADS, WG_PER_CU) product_kernel (const aspen_hip_layer_t L)
 {
@@ -1825,10 +1826,11 @@ static int launch_product (uint32_t M, uint32_t N, uint32_t K, const float *arra
     const uint32_t cu = (uint32_t)g_num_cu;
     const auto tiles = [&] (uint32_t bm, uint32_t bn) { return (uint64_t)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
     const uint64_t small = tiles (VAR2_BM, VAR2_BN), large = tiles (VAR0_BM, VAR0_BN);
-    // us with 128 x 64 / 64 x 64 / 32 x 32 tiles on 256 compute units (whole calls): 1000 x 3137 x 1152 76 / 82 / 140, 2048 x 2048 x 1024
-    // 73 / 81 / 160, 3000 x 700 x 2048 (264 large tiles) 111 / 108 / 163, 512 x 2048 x 768 (256 small ones) 41 / 35 / 43,
-    // 64 x 8192 x 1024 (128) 45 / 36 / 34, 256 x 1024 x 512 (64) 32 / 27 / 24, 64 x 64 x 3072 (1) 94 / 64 / 42: the large shape from five
-    // workgroups for four units on, the one that splits K over its wavefronts where small tiles leave half of the units idle
+    // us with 128 x 64 / 64 x 64 / 32 x 32 tiles on 256 compute units (whole calls): 1000 x 3137 x 1152 (400 large tiles) 68 / 83 / 116,
+    // 2048 x 2048 x 1024 (512) 68 / 80 / 136, 2000 x 1400 x 1024 (352) 61 / 62 / 100, 3000 x 700 x 2048 (264) 96 / 100 / 146, 512 x 2048 x 768
+    // (256 small ones) 36 / 34 / 37, 64 x 8192 x 1024 (128) 39 / 36 / 30, 256 x 1024 x 512 (64) 29 / 27 / 22, 64 x 64 x 3072 (1) 78 / 66 / 38: the
+    // large shape from five workgroups for four units on, the one that splits K over its wavefronts where small tiles leave
+    // half of the units idle
     const int v = 4 * large >= 5 * (uint64_t)cu ? 0 : 2 * small <= cu ? 2 : 1;
     static const struct { int variant; uint32_t bm, bn; } shape[3] = {{ASPEN_HIP_GEMM_LARGE, VAR0_BM, VAR0_BN}, {ASPEN_HIP_GEMM_SMALL, VAR2_BM, VAR2_BN}, {ASPEN_HIP_GEMM_NARROW, VAR3_BM, VAR3_BN}};
     L.type = MATMUL_LAYER; L.act = act; L.variant = shape[v].variant; L.direct = ASPEN_HIP_OPERAND_DIRECT;
@@ -1890,11 +1892,11 @@ extern "C" int aspen_hip_sgemm (uint32_t M, uint32_t N, uint32_t K, const float 
 // ------------------------------------------------------------------------------------------------
 // SGEMM that allocates nothing (for callers that cannot call hipMalloc: tight serving loops, harnesses that
 // forbid it).  It launches on the library's own stream, so it cannot join a caller's stream capture, and the first
-// call on a device performs the library's one-time initialisation (stream and event creation, kernel attributes).  aspen_hip_sgemm stages A into a zero-padded copy it allocates and frees per call; here that
-// staging copy lives in a file-scope device array, and the layer descriptor travels as a kernel argument.
+// call on a device performs the library's one-time initialisation (stream and event creation, kernel attributes).  The arranged copy of A,
+// for which aspen_hip_sgemm allocates memory when what it keeps is in use or too small, lives in a file-scope device array here.
 // Each device holds its own copy of the array at its own address: the address is looked up once per device
 // with hipGetSymbolAddress and only that pointer is ever handed to kernels.  Every call on a device shares the
-// array (it keeps the previous call's contents, so the padding rows are rewritten each time): calls are ordered
+// array (it keeps the previous call's contents, so whole blocks are rewritten each time, padding rows too): calls are ordered
 // by the library's one stream; calls made concurrently from several host threads would race.
 // ------------------------------------------------------------------------------------------------
 #define SGEMM_SCRATCH_BYTES (8u << 20)

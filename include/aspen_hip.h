@@ -203,7 +203,7 @@ double aspen_hip_graph_parallelism (const aspen_hip_graph_t *graph);
    per-kernel profiling mode. */
 int aspen_hip_run_layers (aspen_hip_graph_t *graph, uint32_t first_layer, uint32_t last_layer);
 /* Barrier-free execution: re-arms the dependency counters and the ready queue, then one persistent
-   kernel of `workgroups` workgroups (0 = a whole number per compute unit, 1 to 4, sized from the graph's
+   kernel of `workgroups` workgroups (0 = a whole number per compute unit, 1 to 3, sized from the graph's
    average parallelism) pops ready tiles until all are done.
    spin_limit bounds every wait on the ready queue (0 = default); a wait that exceeds it raises the
    abort flag of THIS graph, all workgroups exit and aspen_hip_graph_sync (graph) returns ASPEN_HIP_ERR_STALLED. */
@@ -312,9 +312,9 @@ int aspen_hip_sgemm (uint32_t M, uint32_t N, uint32_t K, const float *A, uint32_
    hipMalloc).  No counterpart in the reference.  It runs on the library's own stream (it cannot be recorded into a
    caller's stream capture) and the first call initialises the library (stream, events, kernel attributes: call
    aspen_hip_init beforehand where that matters).  It calls no hipMalloc / hipFree:
-   the zero-padded staging copy of A that aspen_hip_sgemm allocates lives in a static device array of
-   aspen_hip_sgemm_static_max_bytes () bytes (8 MiB per GPU, held until the process ends), so
-   roundup (M, 128) * K * 4 must not exceed that; larger problems are refused with a message.  Asynchronous on
+   the arranged copy of A that aspen_hip_sgemm allocates lives in a static device array (12 MiB per GPU, held until the
+   process ends), and roundup (M, 128) * K * 4 must not exceed aspen_hip_sgemm_static_max_bytes () (8 MiB); larger
+   problems are refused with a message, A, B and C off a 16-byte boundary as well.  Asynchronous on
    the library's stream: C is complete after aspen_hip_sync ().  All calls on a GPU share the one staging
    array; the library's stream orders them, calls issued concurrently from several host threads would race. */
 int aspen_hip_sgemm_static (uint32_t M, uint32_t N, uint32_t K, const float *A, uint32_t lda, const float *B,
