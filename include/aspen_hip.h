@@ -156,7 +156,9 @@ int aspen_hip_zero (void *dst, size_t bytes);
    the padding rows zeroed: through a ring of pinned memory the library keeps, read by a kernel
    that spreads the columns (what the reference's copy_buffer_to_ldata_out_mat, src/apu_nasm.c:809-826, does
    on the host).  dense_device_to_host is the inverse (reference get_packed_ldata_output_colwise).  The _ordered form
-   returns as soon as src_host may be reused: work enqueued on the library's stream afterwards (a run) sees the matrix. */
+   returns as soon as src_host may be reused: work enqueued on the library's stream afterwards (a run) sees the matrix, and a failure
+   on the device is reported by a later call that waits for the stream.  One caller at a time uses the ring: host threads
+   that transfer side by side take turns. */
 int aspen_hip_dense_host_to_device (float *dst, uint32_t ld, const float *src_host, uint32_t rows, size_t columns);
 int aspen_hip_dense_host_to_device_ordered (float *dst, uint32_t ld, const float *src_host, uint32_t rows, size_t columns);
 int aspen_hip_dense_device_to_host (float *dst_host, const float *src, uint32_t ld, uint32_t rows, size_t columns);
