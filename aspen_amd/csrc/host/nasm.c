@@ -717,7 +717,7 @@ static double nasm_parallelism (const nasm_t *nasm)
 #define CHAIN_BOUND_KITERS_CAP 48
 #define ORDERED_KITERS_CAP 24
 #define LATENCY_BOUND_BELOW 128.0
-#define ORDERED_VISION_BELOW 1250.0
+#define ORDERED_VISION_BELOW 1100.0
 static nasm_t *create_nasm (aspen_dnn_t *dnn, unsigned int min_ninst, unsigned int batch, unsigned int seq)
 {
     const char *e = getenv ("ASPEN_GPU_MAX_KITERS");            /* experiments: fixed cap, 0 = none */
@@ -729,8 +729,8 @@ static nasm_t *create_nasm (aspen_dnn_t *dnn, unsigned int min_ninst, unsigned i
     if (parallelism >= CHAIN_BOUND_BELOW)
     {
         /* (convolutional graphs a little above the limit keep their tiles but still run better in the ordered mode,
-           ordered / queue in ms: ResNet-50 batch 16, 1162: 1.49 / 1.53; VGG-16 batch 2 / 4 / 16 at 1052 / 1220 / 1234:
-           0.80 / 0.91, 1.25 / 1.30, 3.94 / 4.09; from YOLO-v3 batch 8, 1271, on the queue wins: 4.76 / 4.68) */
+           ordered / queue in us: VGG-16 batch 2, 1052: 688 / 701; from ResNet-50 batch 14, 1104, on the queue wins: 1226 / 1185,
+           batch 16, 1186: 1342 / 1258, YOLO-v3 batch 3, 1142: 2025 / 1933; VGG-16 batch 4, 1246: 1005 / 1000) */
         if (seq == 0 && parallelism < ORDERED_VISION_BELOW) nasm->ordered_pref = 1;
         return nasm;
     }
@@ -743,18 +743,15 @@ static nasm_t *create_nasm (aspen_dnn_t *dnn, unsigned int min_ninst, unsigned i
     const int tr_ordered = seq > 0 && parallelism < CHAIN_BOUND_CAP_FROM;
     nasm_t *rebuilt = build_nasm (dnn, min_ninst, batch, seq, parallelism >= CHAIN_BOUND_CAP_FROM ? CHAIN_BOUND_KITERS_CAP : tr_ordered ? ORDERED_KITERS_CAP : 0, 1, narrow);
     if (rebuilt == NULL) return nasm;
-    /* The ordered mode itself pays further up than the 32 x 32 tiles do, for convolutional networks.  Measured against the
-       ready queue (ms, ordered / queue): ResNet-50 at batch 1 / 2 / 4 / 8 / 16 (parallelism 95 / 175 / 335 / 593 / 790):
-       0.45 / 0.64, 0.62 / 0.74, 0.72 / 0.88, 0.99 / 1.08, 1.47 / 1.62; YOLO-v3 at batch 1 / 2 / 4 (409 / 691 / 942): 1.24 / 1.57,
-       1.71 / 1.94, 2.69 / 2.82; VGG-16 at batch 1 / 2 / 4 / 8 (583 / 654 / 766 / 884): 0.54 / 0.64, 0.82 / 0.85, 1.24 / 1.31,
-       2.16 / 2.24.  Graphs that are not rebuilt here (1024 and up) are a tie or lose (YOLO-v3 batch 8, 1271: 4.76 / 4.68;
-       ResNet-50 batch 32: 2.56 / 2.39).  Transformer graphs win with it below 400, together with the cap of 24 K slices
-       (BERT-base, batch x tokens 8 x 128 / 4 x 128 / 8 x 64 / 2 x 384: 2.00 / 2.15, 1.38 / 1.46, 1.34 / 1.39, 1.90 / 2.08;
-       GPT-2 1 x 512 / 2 x 256 / 8 x 128: 1.59 / 1.65, 1.43 / 1.50, 2.01 / 2.10); above, the times are within a percent or two
-       of each other either way (GPT-2 4 x 512, 529: 3.56 / 3.60 on one box, 3.57 / 3.52 on another; BERT-base 16 x 128:
-       3.34 / 3.38), and the ordered mode moves far less data: a tile's workgroup, and with it the XCD whose L2 its operands
-       pass through, is fixed by the tile's index, so every XCD keeps to an eighth of a layer's weight rows.  So every
-       rebuilt graph asks for the ordered mode.  Where it matters, apu_generate_nasm times both. */
+    /* The ordered mode itself pays further up than the 32 x 32 tiles do.  Measured against the ready queue (us, ordered /
+       queue): ResNet-50 at batch 2 / 4 / 6 / 8 / 11 / 12 (parallelism 179 / 338 / 489 / 645 / 874 / 955): 625 / 772, 675 / 825,
+       746 / 900, 829 / 936, 1019 / 1046, 1090 / 1085; YOLO-v3 at batch 1 / 2 (419 / 834): 1099 / 1396, 1552 / 1618; VGG-16 at
+       batch 1 (728): 513 / 582.  Graphs that are not rebuilt here are above.  Transformer graphs, those of little
+       parallelism with the cap of 24 K slices: BERT-base, batch x tokens 3 x 75 / 4 x 128 / 8 x 128 / 16 x 128: 949 / 1268,
+       1111 / 1481, 1544 / 1781, 2837 / 2860; GPT-2 1 x 512 / 2 x 256 / 4 x 512: 1328 / 1656, 1163 / 1451, 2943 / 3140, and the ordered
+       mode moves less data: a tile's workgroup, and with it the XCD whose L2 its operands pass through, is fixed by the
+       tile's index, so every XCD keeps to an eighth of a layer's weight rows.  So every rebuilt graph asks for the
+       ordered mode.  Where it matters, apu_generate_nasm times both. */
     rebuilt->ordered_pref = 1;
     apu_destroy_nasm (nasm);
     return rebuilt;
