@@ -523,7 +523,7 @@ __device__ __forceinline__ void wait_until_ready ()
 }
 
 template <int COH, unsigned FEAT, bool ORDERED = false>
-__global__ void __launch_bounds__ (WG_THREADS, (FEAT & TILES_DEEP) ? DEEP_WG_PER_CU : WG_PER_CU) dataflow_kernel (dataflow_args_t args)
+__global__ void __launch_bounds__ (WG_THREADS, WG_PER_CU) dataflow_kernel (dataflow_args_t args)
 {
     extern __shared__ __align__ (16) float smem[];
     if (threadIdx.x == 0)
@@ -601,26 +601,21 @@ static const void *const dataflow_kernels[NUM_KERNEL_VARIANTS][2] = {
     {(const void *)dataflow_kernel<1, TILES_ALL>, (const void *)dataflow_kernel<2, TILES_ALL>}};
 
 // Ordered mode (see aspen_hip_run_dataflow), cached loads only: for convolutional networks, for those with weight-streaming
-// layers (VGG-16 at small batches), for transformer graphs (two, see ordered_variant), and with every tile kind.
-enum { ORDERED_CONVNET, ORDERED_TALL, ORDERED_TRANSFORMER_DEEP, ORDERED_TRANSFORMER, ORDERED_ALL, NUM_ORDERED_VARIANTS };
+// layers (VGG-16 at small batches), for transformer graphs, for those with 32 x 32 tiles (a few dozen tokens; on the variant with every tile
+// kind, whose attention tiles spill, BERT-base 1 x 16 took 670 us instead of 600), and with every tile kind.
+enum { ORDERED_CONVNET, ORDERED_TALL, ORDERED_TRANSFORMER, ORDERED_TRANSFORMER_NARROW, ORDERED_ALL, NUM_ORDERED_VARIANTS };
 #define ORDERED_SMEM_BYTES CMAX (GEMM_SMEM_BYTES, NARROW_PF_SMEM_BYTES)       // the narrow tiles' weight prefetch buffers
 static const unsigned ordered_variant_tiles[NUM_ORDERED_VARIANTS] = {TILES_CONVNET | TILES_YOLO | TILES_NARROW, TILES_CONVNET | TILES_TALL,
-    TILES_TRANSFORMER, TILES_TRANSFORMER, TILES_ALL};
+    TILES_TRANSFORMER, TILES_TRANSFORMER | TILES_NARROW, TILES_ALL};
 static const void *const ordered_kernels[NUM_ORDERED_VARIANTS] = {
     (const void *)dataflow_kernel<2, TILES_CONVNET | TILES_YOLO | TILES_NARROW, true>, (const void *)dataflow_kernel<2, TILES_CONVNET | TILES_TALL, true>,
-    (const void *)dataflow_kernel<2, TILES_TRANSFORMER | TILES_DEEP, true>, (const void *)dataflow_kernel<2, TILES_TRANSFORMER, true>,
+    (const void *)dataflow_kernel<2, TILES_TRANSFORMER, true>, (const void *)dataflow_kernel<2, TILES_TRANSFORMER | TILES_NARROW, true>,
     (const void *)dataflow_kernel<2, TILES_ALL, true>};
-// Below this estimated parallelism a transformer graph's levels leave a compute unit one or two tiles, which pay for four slices
-// in flight each; above it a third workgroup per unit is worth more.  Two deep / three plain ones, us: BERT-base 1 x 128 (135) 868 /
-// 918, 3 x 75 (197) 946 / 1005, 4 x 128 (339) 1110 / 1119; GPT-2 1 x 512 (388) 1374 / 1326, 2 x 256 (388) 1238 / 1162, BERT-base 8 x 128
-// (533) 1595 / 1489, 16 x 128 (1065) 2913 / 2735, GPT-2 4 x 512 (878) 2996 / 2865.
-#define DEEP_BELOW 350.0
-
 static int ordered_variant (const aspen_hip_graph_t *g)
 {
     int v = 0;
     while (v + 1 < NUM_ORDERED_VARIANTS && (g->features & ~ordered_variant_tiles[v]) != 0) v++;
-    return v == ORDERED_TRANSFORMER_DEEP && g->parallelism >= DEEP_BELOW ? ORDERED_TRANSFORMER : v;
+    return v;
 }
 
 // The tile kinds a graph contains, as TILES_* bits.
@@ -695,7 +690,7 @@ extern "C" void aspen_hip_tile_shapes (uint32_t shapes[13])
 {
     shapes[11] = VAR4_BM; shapes[12] = VAR4_BN;
     shapes[0] = VAR0_BM; shapes[1] = VAR0_BN; shapes[2] = VAR1_BM; shapes[3] = VAR1_BN; shapes[4] = VAR2_BM; shapes[5] = VAR2_BN;
-    shapes[6] = KATTN_BN; shapes[7] = VATTN_BN; shapes[8] = DEEP_WG_PER_CU; shapes[9] = VAR3_BM; shapes[10] = VAR3_BN;
+    shapes[6] = KATTN_BN; shapes[7] = VATTN_BN; shapes[8] = MIN_WG_PER_CU; shapes[9] = VAR3_BM; shapes[10] = VAR3_BN;
 }
 
 extern "C" int aspen_hip_device_info (int *num_cu, int *clock_khz, size_t *mem_bytes, char *name, int name_len)
@@ -1043,9 +1038,9 @@ __global__ void __launch_bounds__ (WG_THREADS) arrange_weights_kernel (const flo
     const size_t n = (size_t)blocks * slices * 128u, stride = (size_t)gridDim.x * blockDim.x;
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride)
     {
-        const uint32_t lane = (uint32_t)i & 63u, step = (uint32_t)(i >> 6) & 1u;
+        const uint32_t lane = (uint32_t)i & 63u, half = (uint32_t)(i >> 6) & 1u;
         const size_t bs = i >> 7, block = bs / slices;
-        const uint32_t slice = (uint32_t)(bs - block * slices), row = (uint32_t)block * WEIGHT_BLOCK_ROWS + (lane & 31u), unit = 2u * step + (lane >> 5);
+        const uint32_t slice = (uint32_t)(bs - block * slices), row = (uint32_t)block * WEIGHT_BLOCK_ROWS + 16u * half + (lane & 15u), unit = lane >> 4;
         float4 a = make_float4 (0.f, 0.f, 0.f, 0.f), b = a;
         if (row < M)
         {
@@ -1057,8 +1052,8 @@ __global__ void __launch_bounds__ (WG_THREADS) arrange_weights_kernel (const flo
                 b = make_float4 (gld1 (src + 16), gld1 (src + 17), gld1 (src + 18), gld1 (src + 19));
             }
         }
-        constexpr uint32_t SLICE = WeightFragments<RAW>::SLICE;
-        char *d = dst + bs * SLICE + step * (SLICE / 2) + lane * 16u;
+        constexpr uint32_t SLICE = WeightFragments<RAW, 2>::SLICE;
+        char *d = dst + bs * SLICE + half * (SLICE / 2) + lane * 16u;
         if (RAW) { *reinterpret_cast<float4 *> (d) = a; *reinterpret_cast<float4 *> (d + 1024) = b; }
         else
         {

@@ -12,9 +12,12 @@
 // exact one than the single-precision matrix instruction's (relative to a 64-bit sum, 2-norm over 128 x 128 results, inputs
 // normal / rectified normal: K = 64 4.8e-8 / 4.2e-8 against 1.4e-7 / 1.0e-7; K = 1024 1.8e-7 / 1.5e-7 against 5.7e-7 / 4.2e-7;
 // K = 4096 4.0e-7 / 3.2e-7 against 1.1e-6 / 8.1e-7; with one accumulator for all six products 1.0e-6 / 9.5e-7).
-// Speed: a v_mfma_f32_32x32x16_bf16 does eight times the work of a v_mfma_f32_32x32x2_f32 in half its cycles, so six of them take 3 / 8
-// of the time.  In practice both are limited by power: a large product reaches 154 TFLOP/s with the single-precision
-// instruction (98 % of its peak) and 205-212 with this scheme.
+// Speed: bfloat16 matrix instructions do sixteen times the single-precision one's work per cycle, so six products take 3 / 8 of its
+// time.  In practice both are limited by power, and a product's time is its energy.  Registers alone, every compute
+// unit, products in TFLOP/s of the floats' work (417 nominal): v_mfma_f32_32x32x16_bf16 300, v_mfma_f32_16x16x32_bf16 355 (half the
+// accumulator traffic per product); a loop that also splits, stages and fetches what a 128 x 64 tile does, 188 and 229 (a 64 x 64
+// tile's 184).  So the smaller block it is.  The sums come out the same: over 1000 x 3137 and 2048 x 2048 results, K = 32 ... 4096, both
+// instructions' errors against 64-bit sums agree to three digits.
 // The range is float's own (bfloat16 has the same exponent) with two edges.  Terms below bfloat16's smallest number, 2^-133, do not
 // exist: an input below 2^-110 enters with an absolute error of up to 2^-134.  And infinities, NaNs and floats within 0.2 % of the
 // largest one, whose h rounds to infinity, leave no finite sum (inf - inf in m, inf times a zero term): the tiles look
@@ -24,6 +27,8 @@
 #include <stdint.h>
 
 typedef float floatx16 __attribute__ ((ext_vector_type (16)));
+typedef float floatx8 __attribute__ ((ext_vector_type (8)));
+typedef float floatx4 __attribute__ ((ext_vector_type (4)));
 typedef uint32_t u32x4 __attribute__ ((ext_vector_type (4)));
 typedef __bf16 bf16x2 __attribute__ ((ext_vector_type (2)));
 typedef __bf16 bf16x8 __attribute__ ((ext_vector_type (8)));
@@ -36,6 +41,15 @@ __device__ __forceinline__ uint32_t bf16_pair (float a, float b)
 }
 __device__ __forceinline__ float bf16_low (uint32_t p) { return __builtin_bit_cast (float, p << 16); }
 __device__ __forceinline__ float bf16_high (uint32_t p) { return __builtin_bit_cast (float, p & 0xffff0000u); }
+
+// the next term of eight floats; they keep what it leaves
+__device__ __forceinline__ u32x4 take_term (float4 &a, float4 &b)
+{
+    const u32x4 t = {bf16_pair (a.x, a.y), bf16_pair (a.z, a.w), bf16_pair (b.x, b.y), bf16_pair (b.z, b.w)};
+    a.x -= bf16_low (t[0]); a.y -= bf16_high (t[0]); a.z -= bf16_low (t[1]); a.w -= bf16_high (t[1]);
+    b.x -= bf16_low (t[2]); b.y -= bf16_high (t[2]); b.z -= bf16_low (t[3]); b.w -= bf16_high (t[3]);
+    return t;
+}
 
 // the three terms of eight floats, as matrix-core operands (K positions 0 .. 7 of a lane)
 struct split8_t { u32x4 h, m, l; };
@@ -88,65 +102,83 @@ __device__ __forceinline__ floatx2 join2 (uint32_t h, uint32_t m, uint32_t l)
     return (floatx2){bf16_low (h) + (bf16_low (m) + bf16_low (l)), bf16_high (h) + (bf16_high (m) + bf16_high (l))};
 }
 
-// hi += leading products, lo += the five small ones, of 32 x 32 x 16: rows of the result = rows of `a`, columns = rows of `b`
-__device__ __forceinline__ void split_mfma (const split8_t &a, const split8_t &b, floatx16 &hi, floatx16 &lo)
+__device__ __forceinline__ floatx4 mfma_bf16 (const u32x4 &a, const u32x4 &b, const floatx4 &c)
 {
-    const bf16x8 ah = __builtin_bit_cast (bf16x8, a.h), am = __builtin_bit_cast (bf16x8, a.m), al = __builtin_bit_cast (bf16x8, a.l);
-    const bf16x8 bh = __builtin_bit_cast (bf16x8, b.h), bm = __builtin_bit_cast (bf16x8, b.m), bl = __builtin_bit_cast (bf16x8, b.l);
-    // (neighbouring instructions share an operand: 1 % at the power limit over an order that changes both)
-    lo = __builtin_amdgcn_mfma_f32_32x32x16_bf16 (al, bh, lo, 0, 0, 0);
-    hi = __builtin_amdgcn_mfma_f32_32x32x16_bf16 (ah, bh, hi, 0, 0, 0);
-    lo = __builtin_amdgcn_mfma_f32_32x32x16_bf16 (am, bh, lo, 0, 0, 0);
-    lo = __builtin_amdgcn_mfma_f32_32x32x16_bf16 (am, bm, lo, 0, 0, 0);
-    lo = __builtin_amdgcn_mfma_f32_32x32x16_bf16 (ah, bm, lo, 0, 0, 0);
-    lo = __builtin_amdgcn_mfma_f32_32x32x16_bf16 (ah, bl, lo, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16 (__builtin_bit_cast (bf16x8, a), __builtin_bit_cast (bf16x8, b), c, 0, 0, 0);
 }
-
+// hi += leading products, lo += the five small ones, of COUNT neighbouring blocks of 16 x 16 x 32: rows of the result = rows of
+// `a`, columns = rows of `b[j]`.  Neighbouring instructions share the operand of `a` and add to different sums.
+template <int COUNT>
+__device__ __forceinline__ void split_mfma (const split8_t &a, const split8_t (&b)[COUNT], floatx4 (&hi)[COUNT], floatx4 (&lo)[COUNT])
+{
+    #pragma unroll
+    for (int j = 0; j < COUNT; j++) lo[j] = mfma_bf16 (a.h, b[j].l, lo[j]);
+    #pragma unroll
+    for (int j = 0; j < COUNT; j++) hi[j] = mfma_bf16 (a.h, b[j].h, hi[j]);
+    #pragma unroll
+    for (int j = 0; j < COUNT; j++) lo[j] = mfma_bf16 (a.h, b[j].m, lo[j]);
+    #pragma unroll
+    for (int j = 0; j < COUNT; j++) lo[j] = mfma_bf16 (a.m, b[j].m, lo[j]);
+    #pragma unroll
+    for (int j = 0; j < COUNT; j++) lo[j] = mfma_bf16 (a.m, b[j].h, lo[j]);
+    #pragma unroll
+    for (int j = 0; j < COUNT; j++) lo[j] = mfma_bf16 (a.l, b[j].h, lo[j]);
+}
 // Order of the K axis inside a slice of 32 (both operands have to agree, the sum does not care): a lane of a matrix
-// instruction holds eight K positions of one row, "unit" u = 2 * step + lane / 32 (u = 0 .. 3, two instruction steps per
-// slice), and unit u stands for the slice's floats 4u .. 4u+3 and 16+4u .. 16+4u+3.  Four neighbouring threads that
-// fetch the four units of a row then read 64 contiguous bytes with each of their two 16-byte requests.
+// instruction holds eight K positions of row lane % 16, "unit" u = lane / 16, and unit u stands for the slice's floats
+// 4u .. 4u+3 and 16+4u .. 16+4u+3.  Four neighbouring threads that fetch the four units of a row then read 64 contiguous bytes
+// with each of their two 16-byte requests.
 #define SLICE_K 32
 
-// Weights on the device.  SPLIT: per block of 32 rows and slice, per step, the terms h, m, l, each as the 64 lanes' 16 bytes in a row (lane l: row
-// l % 32, unit 2 * step + l / 32): 6144 bytes that a wavefront fetches with six contiguous 1 KB requests straight into
-// the registers the matrix instructions read.  RAW: the same with the floats themselves, per step two rows of 64 x 16
+// Weights on the device.  SPLIT: per block of 32 rows and slice, per half of 16 rows, the terms h, m, l, each as the 64 lanes' 16 bytes in a
+// row (lane l: row l % 16, unit l / 16): 6144 bytes that a wavefront fetches with contiguous 1 KB requests straight into
+// the registers the matrix instructions read.  RAW: the same with the floats themselves, per half two rows of 64 x 16
 // bytes (floats 4u .. and 16+4u ..): 4096 bytes per block and slice, split in registers.  A weight belongs to one
-// wavefront of a tile (or is shared by two, from the compute unit's cache), so nothing is staged through LDS.
+// wavefront of a tile, so nothing is staged through LDS.
 // RAW is for layers that are bound by the weights' trip from memory.
 #define WEIGHT_BLOCK_ROWS 32
 #define SPLIT_SLICE_BYTES 6144u
 #define RAW_SLICE_BYTES 4096u
 
-// SETS: register sets, i.e. slices of weights in flight.
-template <bool RAW, int SETS = 1> struct WeightFragments
+// HALVES: neighbouring groups of 16 rows (2: a whole block); SETS: register sets, i.e. slices of weights in flight.
+template <bool RAW, int HALVES, int SETS = 1> struct WeightFragments
 {
     static constexpr uint32_t SLICE = RAW ? RAW_SLICE_BYTES : SPLIT_SLICE_BYTES, PARTS = RAW ? 2 : 3;
     typedef const char __attribute__ ((address_space (1))) *bytes_t;
-    bytes_t base;               // of the wavefront's row block (uniform)
+    bytes_t base;               // of the wavefront's first group of 16 rows (uniform)
     uint32_t lane16;
-    u32x4 f[SETS][2][PARTS];    // [set][step]
-    __device__ __forceinline__ void init (const void *w, uint32_t block, uint32_t slices, uint32_t lane)
+    u32x4 f[SETS][HALVES][PARTS];
+    // group: the first group of 16 rows, even where HALVES is 2
+    __device__ __forceinline__ void init (const void *w, uint32_t group, uint32_t slices, uint32_t lane)
     {
-        base = (bytes_t)w + (uint64_t)block * ((uint64_t)slices * SLICE);
+        base = (bytes_t)w + ((uint64_t)(group >> 1) * ((uint64_t)slices * SLICE) + (group & 1u) * (SLICE / 2));
         lane16 = lane * 16u;
     }
-    __device__ __forceinline__ void load (int it, int step, int set = 0)
+    __device__ __forceinline__ void load (int it, int set = 0)
     {
-        const bytes_t p = base + ((uint32_t)it * SLICE + (uint32_t)step * (SLICE / 2));
+        const bytes_t p = base + (uint32_t)it * SLICE;
         #pragma unroll
-        for (uint32_t q = 0; q < PARTS; q++) f[set][step][q] = *(const u32x4 __attribute__ ((address_space (1))) *)(p + (lane16 + q * 1024u));
+        for (uint32_t j = 0; j < HALVES; j++)
+            #pragma unroll
+            for (uint32_t q = 0; q < PARTS; q++) f[set][j][q] = *(const u32x4 __attribute__ ((address_space (1))) *)(p + (lane16 + j * (SLICE / 2) + q * 1024u));
     }
-    __device__ __forceinline__ split8_t operand (int step, int set = 0) const
+    __device__ __forceinline__ void take_second_set ()
     {
-        if constexpr (RAW) return split8 (__builtin_bit_cast (float4, f[set][step][0]), __builtin_bit_cast (float4, f[set][step][1]));
-        else return {f[set][step][0], f[set][step][1], f[set][step][2]};
+        #pragma unroll
+        for (uint32_t j = 0; j < HALVES; j++)
+            #pragma unroll
+            for (uint32_t q = 0; q < PARTS; q++) f[0][j][q] = f[1][j][q];
+    }
+    __device__ __forceinline__ split8_t operand (int half, int set = 0) const
+    {
+        if constexpr (RAW) return split8 (__builtin_bit_cast (float4, f[set][half][0]), __builtin_bit_cast (float4, f[set][half][1]));
+        else return {f[set][half][0], f[set][half][1], f[set][half][2]};
     }
 };
 
 // LDS stage of the other operand, one slice of ROWS rows: three planes (h, m, l) of ROWS x 64 bytes, the four 16-byte units
-// of a row in the order unit ^ (row / 4 % 4): a fragment read (16 neighbouring rows, the same unit, at a time) and a write (four rows whole)
-// both touch every bank once.
+// of a row in the order unit ^ (row / 4 % 4): sixteen lanes of a fragment read (16 rows, the same unit) and of a write (four rows
+// whole) both touch every bank once.
 template <int ROWS> struct SplitStage
 {
     static constexpr uint32_t PLANE = ROWS * 64u, BYTES = 3u * PLANE;

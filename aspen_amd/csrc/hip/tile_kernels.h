@@ -31,7 +31,7 @@ __device__ void tile_phase_lap (int which);
 #define VAR0_BM 128
 #define VAR0_BN 64
 #define WG_PER_CU 3
-#define DEEP_WG_PER_CU 2          // of the kernels compiled with TILES_DEEP
+#define MIN_WG_PER_CU 2           // ordered launches with the narrow tiles' prefetch buffers
 #define KATTN_BN 32            // queries per K-attention tile
 #define VATTN_BN 64            // queries per V-attention tile
 #define VAR1_BM 64
@@ -46,7 +46,8 @@ __device__ void tile_phase_lap (int which);
 #define SPLITK_TILE_FLOATS (VAR2_BM * VAR2_BN)     // one slice's sums of one output tile: a block of its own in `partial` (the tall shape has as many)
 #define CMAX(a, b) ((a) > (b) ? (a) : (b))
 #define STAGE_FLOATS(bm, bn) (((bm) + (bn)) * LDS_ROW)          // attention tiles
-#define EPI_FLOATS(bm, bn) ((bn) * ((bm) + 8))
+#define EPI_ROW(bm) ((bm) + 4)      // floats per parked column: 4 * EPI_ROW = 16 modulo 64, the quarters of a wavefront hit different banks
+#define EPI_FLOATS(bm, bn) ((bn) * EPI_ROW (bm))
 #define SPLIT_STAGES_FLOATS(bn) (2 * (bn) * 48)                 // two stages of SplitStage<bn>
 #define VAR_FLOATS(bm, bn) CMAX (SPLIT_STAGES_FLOATS (bn), EPI_FLOATS (bm, bn))
 #define GEMM_SMEM_FLOATS CMAX (CMAX (VAR_FLOATS (VAR0_BM, VAR0_BN), VAR_FLOATS (VAR1_BM, VAR1_BN)), \
@@ -69,7 +70,6 @@ __device__ __forceinline__ void st4 (float *p, float4 v) { *reinterpret_cast<flo
 // Loads from device memory through pointers the compiler cannot prove to be global (descriptor fields)
 // would be FLAT instructions, which count as LDS traffic too: every wait for an LDS fragment would
 // then also wait for them.  These go through the global address space explicitly.
-typedef float floatx4 __attribute__ ((ext_vector_type (4)));
 __device__ __forceinline__ float4 gld4 (const float *p)
 {
     const floatx4 x = *(const floatx4 __attribute__ ((address_space (1))) *)p;
@@ -243,12 +243,12 @@ template <int ROWS> struct SliceShare
     static constexpr int R = ROWS < 64 ? 1 : ROWS / 64;
     uint32_t unit, row0;
     __device__ __forceinline__ void init (uint32_t tid) { unit = tid & 3u; row0 = (tid >> 2) & (ROWS < 64 ? ROWS - 1u : 63u); }
-    __device__ __forceinline__ void store (char *stage, const float4 (&v)[R][2]) const
+    // term 0, 1, 2 = h, m, l; what is left of the values afterwards replaces them, so the terms are stored in this order
+    __device__ __forceinline__ void store_term (char *stage, float4 (&v)[R][2], int term) const
     {
-        // (64 rows further down the same swizzle applies)
-        const uint32_t off = SplitStage<ROWS>::offset (row0, unit);
+        const uint32_t off = SplitStage<ROWS>::offset (row0, unit) + term * SplitStage<ROWS>::PLANE;
         #pragma unroll
-        for (int i = 0; i < R; i++) SplitStage<ROWS>::write (stage, off + i * 64 * 64, split8 (v[i][0], v[i][1]));
+        for (int i = 0; i < R; i++) *reinterpret_cast<u32x4 *> (stage + off + i * 64 * 64) = take_term (v[i][0], v[i][1]);
     }
 };
 
@@ -519,6 +519,7 @@ __device__ __forceinline__ void lds_barrier ()
 // Instruction-group hints for the machine scheduler (masks of __builtin_amdgcn_sched_group_barrier)
 #define SG_MFMA 0x008
 #define SG_DS_READ 0x100
+#define SCHED_GROUP_MASK 0x14        // what may cross a sched_barrier: scalar arithmetic, global memory
 
 // Instruction-arbiter priority of a wavefront everywhere but inside a K loop.  The workgroups of a compute unit share
 // its matrix pipeline; the ones in a K loop can keep it busy by themselves, while a workgroup in a tile's set-up,
@@ -540,14 +541,6 @@ enum : unsigned
     TILES_NARROW = 512u,        // the 32 x 32 contraction tile of latency-bound graphs
     TILES_TALL = 1024u,         // the 128 x 32 contraction tile of weight-streaming layers
     TILES_DENSE_WIDE = 2048u,   // the dense three-channel operand under the 64 x 128 shape (the host library's graphs take 64 x 64 for it)
-    // No tile kind: 64 x 64 tiles keep four K slices of both operands in flight, four slices to a trip through the loop, in the
-    // 252 registers per lane that two workgroups per compute unit leave.  For the ordered kernel of transformer graphs of little
-    // parallelism: their levels are a few hundred tiles of 24 slices, one or two per compute unit, and with one slice of
-    // weights and two of activations in flight a slice took 0.42 us for 0.17 us of matrix instructions (see DEEP_BELOW for both
-    // sides).  With four slices of weights and two of activations BERT-base 3 x 75 took 1.00 ms instead of 0.95; with the
-    // loop left from its middle instead of copies of the last slices behind it 1.03.  Convolutional graphs lose with it (YOLO-v3
-    // batch 1 1.10 -> 1.16 ms, ResNet-50 batch 11 1.02 -> 1.27).
-    TILES_DEEP = 4096u,
     TILES_ALL = 4095u,
     TILES_CONVNET = TILES_GATHER | TILES_LARGE | TILES_WIDE | TILES_SMALL | TILES_POOL | TILES_RESIDUAL,
     TILES_TRANSFORMER = TILES_SMALL | TILES_ATTENTION | TILES_NORM | TILES_RESIDUAL
@@ -661,6 +654,10 @@ __device__ __forceinline__ void gemm_core (ALoader &al, BLoader &bl, int kbase, 
 //   n = wn0 + 32 i + 8 (v / 4) + 4 (lane / 32) + v % 4,   m = wm0 + 32 j + lane % 32
 #define ACC_N(wn0, i, v, lane) ((wn0) + 32 * (i) + 8 * ((v) >> 2) + 4 * ((lane) >> 5) + ((v) & 3))
 
+// Contraction tiles: register v of block (i, j) of a wavefront whose rows start at wm0 holds output (row n, channel m):
+//   n = 16 i + 4 (lane / 16) + v,   m = wm0 + 16 j + lane % 16
+#define BLOCK_N(i, v, lane) (16 * (i) + 4 * ((lane) >> 4) + (v))
+
 struct NoStats { template <class V> __device__ __forceinline__ void operator() (const V &) const {} };
 
 // A layer norm folded into a matmul tile (aspen_hip_layer_t.norm_fold), second half: the K loop has left every thread
@@ -670,8 +667,8 @@ struct NoStats { template <class V> __device__ __forceinline__ void operator() (
 // acc = rstd[n] * (acc - mean[n] * rowsum[m]).  Same arithmetic for mean and variance as tile_layernorm.
 #define NORM_FOLD_STATS_OFFSET SPLIT_STAGES_FLOATS (VAR2_BN)      // floats
 template <int COH>
-__device__ __forceinline__ void norm_fold_finish (const aspen_hip_layer_t &L, floatx16 &acc, float cs, float cq, float *smem,
-    uint32_t tid, uint32_t m0, uint32_t n0, uint32_t wm0, uint32_t wn0)
+__device__ __forceinline__ void norm_fold_finish (const aspen_hip_layer_t &L, floatx4 (&acc)[4][1], float cs, float cq, float *smem,
+    uint32_t tid, uint32_t m0, uint32_t n0, uint32_t wm0)
 {
     static_assert (NORM_FOLD_STATS_OFFSET + 2 * VAR2_BN <= GEMM_SMEM_FLOATS, "column statistics fit behind the stages");
     const uint32_t lane = tid & 63;
@@ -695,15 +692,17 @@ __device__ __forceinline__ void norm_fold_finish (const aspen_hip_layer_t &L, fl
         }
     }
     // (the row sums are weights: requested before the barrier)
-    const uint32_t m = min (m0 + wm0 + (lane & 31), L.M - 1);
+    const uint32_t m = min (m0 + wm0 + (lane & 15), L.M - 1);
     const float rs = gld1 (L.in1 + m);
     lds_barrier ();
     #pragma unroll
-    for (int v = 0; v < 16; v++)
-    {
-        const uint32_t n = ACC_N (wn0, 0, v, lane);
-        acc[v] = st[2 * n + 1] * (acc[v] - st[2 * n] * rs);
-    }
+    for (int i = 0; i < 4; i++)
+        #pragma unroll
+        for (int v = 0; v < 4; v++)
+        {
+            const uint32_t n = BLOCK_N (i, v, lane);
+            acc[i][0][v] = st[2 * n + 1] * (acc[i][0][v] - st[2 * n] * rs);
+        }
 }
 
 // The same for 64 x 64 products, whose four waves own ONE 32 x 32 block each, scheduled by hand for a
@@ -767,45 +766,23 @@ __device__ __forceinline__ void gemm_core_single_block (ALoader &al, BLoader &bl
 }
 
 
-// f (0) .. f (COUNT - 1) with the index as a constant
-template <int FIRST, int COUNT, class F> __device__ __forceinline__ void slice_run (F f)
-{
-    f (std::integral_constant<int, FIRST> ());
-    if constexpr (FIRST + 1 < COUNT) slice_run<FIRST + 1, COUNT> (f);
-}
-// the first `left` (1 .. COUNT) of them, the last one as f (index, false)
-template <int FIRST, int COUNT, class F> __device__ __forceinline__ void last_slices (int left, F f)
-{
-    constexpr std::integral_constant<int, FIRST> turn;
-    if constexpr (FIRST + 1 < COUNT)
-    {
-        if (left > FIRST + 1)
-        {
-            f (turn, std::true_type ());
-            last_slices<FIRST + 1, COUNT> (left, f);
-            return;
-        }
-    }
-    f (turn, std::false_type ());
-}
-
 // ---------------------------------------------------------------------------------------------
-// K loop of the contraction tiles.  Workgroup tile = (WM x 32) weight rows x BN activation rows; WM x WN wavefronts, each
-// owning 32 x (BN / WN) of it.  The activation row is the matrix instruction's row index and the weight row its column, so each
-// accumulator register holds 32 consecutive output channels of one output column: stores are 128-byte coalesced.
-//   weights      memory -> registers, in fragment order (WeightFragments); a step's registers are asked for again, SETS slices
-//                ahead, as soon as the step's matrix instructions have been issued
+// K loop of the contraction tiles.  Workgroup tile = (64 TM) weight rows x BN activation rows, the four wavefronts below each other,
+// 16 TM rows each.  The activation row is the matrix instruction's row index and the weight row its column, so each
+// accumulator register holds 16 consecutive output channels of four output columns.
+//   weights      memory -> registers, in fragment order (WeightFragments), two slices ahead.  A weight is fetched by one wavefront
+//                only: a compute unit's first-level cache delivers 64 bytes a cycle, and with the wavefronts of a 64 x 64 tile
+//                two by two, every weight fetched twice, a slice took 512 cycles of it for 384 of matrix instructions.
 //   activations  memory -> registers, AHEAD slices ahead -> split into three terms -> one of two LDS stages, a slice ahead ->
-//                fragments.  Every value is split once per tile (5.5 vector instructions) and read by WM wavefronts.
+//                fragments.  Every value is split once per tile (5.5 vector instructions) and read by all four wavefronts.
 // One barrier per slice: it publishes the stage written during the slice and frees the one read.
 // The loop exists once per shape and operand kind, and each copy counts: the kernel for convolutional networks was 101 KB with nine of
-// them (reading in place apart from stepping, the three-channel and table operands under two shapes) and is 73 KB with five:
-// ResNet-50 batch 32 2.24 -> 2.10 ms, batch 8 of YOLO-v3 4.63 -> 4.42 (the instruction cache holds 64 KB).  A rolled loop (one slice per trip, requests one
-// slice ahead) saves another 9 KB and is slower where few workgroups share a compute unit: BERT-base 3 x 75 1.00 -> 1.07 ms.
-// Per slice of a 128 x 64 tile a wavefront issues 24 matrix instructions (768 cycles), 44 vector instructions for the split, 12
-// fragment reads and 3 + 6 + 2 stores and requests.  1024 x 100 352 x 1024 as one launch: 205 TFLOP/s (64 x 64: 163,
-// 64 x 128: 181; requests one slice ahead instead of two 200; the wavefronts 2 x 2, every weight fetched by two of
-// them, 186); the single-precision matrix instruction's own limit is 157.
+// them (reading in place apart from stepping, the three-channel and table operands under two shapes) and is 80 KB with five
+// (the instruction cache holds 64 KB).
+// Per slice of a 128 x 64 tile a wavefront issues 48 matrix instructions (768 cycles), 44 vector instructions for the split, 12
+// fragment reads and 3 + 6 + 2 stores and requests.  1024 x 100 352 x 1024, the same card, with 32 x 32 blocks / this way:
+// 173 / 196 TFLOP/s (64 x 64 tiles 141 / 158).  Whole networks: VGG-16 batch 32 5.46 -> 5.13 ms, ResNet-50 batch 32 2.11 -> 1.97, YOLO-v3 batch 8
+// 4.09 -> 3.81, BERT-base 8 x 128 1.50 -> 1.41, GPT-2 4 x 512 3.02 -> 2.86.
 // `ready` runs between the first request for the weights and the first one for the activations: a
 // kernel that starts tiles before their parents have finished (see the ordered mode of the persistent kernel) waits
 // there, with the tile's set-up done and its first weights on their way.
@@ -814,84 +791,92 @@ template <int FIRST, int COUNT, class F> __device__ __forceinline__ void last_sl
 // `stats` sees every K slice of the activation operand once, as the registers it passes through on its way into LDS
 // (a folded layer norm's column sums, see norm_fold_finish).
 // ---------------------------------------------------------------------------------------------
-template <int BN, int WM, int WN, bool RAW, int SETS, int AHEAD, class BLoader, class Hook, class Ready, class Stats = NoStats>
-__device__ __forceinline__ void split_core (const void *weights, uint32_t first_block, uint32_t total_slices, BLoader &bl, int kbase, int kiters, char *smem,
-    floatx16 (&acc)[BN / WN / 32], bool phases, Hook before_last_slice, Ready ready, Stats stats = Stats ())
+template <int BN, int TM, bool RAW, int AHEAD, class BLoader, class Hook, class Ready, class Stats = NoStats>
+__device__ __forceinline__ void split_core (const void *weights, uint32_t first_group, uint32_t total_slices, BLoader &bl, int kbase, int kiters, char *smem,
+    floatx4 (&acc)[BN / 16][TM], bool phases, Hook before_last_slice, Ready ready, Stats stats = Stats ())
 {
-    static_assert (WM * WN == 4, "four wavefronts");
     typedef SplitStage<BN> Stage;
-    constexpr int TN = BN / WN / 32, GROUPS = 2 * TN, TRIP = CMAX (2, CMAX (SETS, AHEAD));
-    static_assert (TRIP % 2 == 0 && TRIP % SETS == 0 && TRIP % AHEAD == 0, "a trip through the loop ends on the sets it began with");
+    constexpr int TN = BN / 16;
+    static_assert (AHEAD == 1 || AHEAD == 2, "a trip through the loop, two slices, ends on the sets it began with");
     if (phases) tile_phase_lap (12);
     const uint32_t tid = tile_thread (), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane (tid >> 6);
     const int last = kbase + kiters - 1;
-    WeightFragments<RAW, SETS> w;
-    w.init (weights, first_block + wave % WM, total_slices, lane);
-    #pragma unroll
-    for (int s = 0; s < SETS; s++) { w.load (min (kbase + s, last), 0, s); w.load (min (kbase + s, last), 1, s); }
+    WeightFragments<RAW, TM, 2> w;
+    w.init (weights, first_group + wave * TM, total_slices, lane);
+    w.load (kbase, 0);
     ready ();
+    // (requested in the order in which the loop asks for them: where the two orders differ, the compiler's waits at the loop's head suit
+    // the worse one, and a wait inside the loop then sits out requests that were made a slice ago)
     float4 areg[AHEAD][BLoader::R][2];          // slice it is fetched into set it % AHEAD
     #pragma unroll
     for (int s = 0; s < AHEAD; s++) bl.load (min (kbase + s, last), areg[s]);
-    const uint32_t row = (wave / WM) * (BN / WN) + (lane & 31);
-    const uint32_t foff[2] = {Stage::offset (row, lane >> 5), Stage::offset (row, 2 + (lane >> 5))};
-    floatx16 lo[TN];
+    const uint32_t foff = Stage::offset (lane & 15, lane >> 4);
+    floatx4 lo[TN][TM];
     #pragma unroll
     for (int i = 0; i < TN; i++)
         #pragma unroll
-        for (int v = 0; v < 16; v++) { acc[i][v] = 0.f; lo[i][v] = 0.f; }
-    auto refill = [&] (int set, uint32_t stage) { bl.share.store (smem + stage, areg[set]); stats (areg[set]); };
-    refill (0, 0);
+        for (int j = 0; j < TM; j++) acc[i][j] = lo[i][j] = (floatx4){0.f, 0.f, 0.f, 0.f};
+    stats (areg[0]);
+    #pragma unroll
+    for (int term = 0; term < 3; term++) bl.share.store_term (smem, areg[0], term);
     bl.load (min (kbase + AHEAD, last), areg[0]);
+    w.load (min (kbase + 1, last), 1);
     lds_barrier ();
     if (phases) tile_phase_lap (8);
     __builtin_amdgcn_s_setprio (0);
-    // slice `it` (relative to kbase), the `turn`th of its trip, sits in LDS; MORE: the next one is split into the other stage
+    // slice `it` (relative to kbase), the `turn`th of its two, sits in LDS; MORE: the next one is split into the other stage
     // meanwhile (its registers then take the slice AHEAD after it)
     auto slice = [&] (int it, uint32_t stage, auto turn, auto more)
     {
         constexpr bool MORE = decltype (more)::value;
-        constexpr int TURN = decltype (turn)::value, SET = (TURN + 1) % AHEAD, WSET = TURN % SETS;
-        split8_t frag[2];
-        frag[0] = Stage::read (smem + stage, foff[0]);
+        constexpr int TURN = decltype (turn)::value, SET = (TURN + 1) % AHEAD;
+        split8_t wf[TM], frag[2];
         #pragma unroll
-        for (int g = 0; g < GROUPS; g++)
+        for (int j = 0; j < TM; j++) wf[j] = w.operand (j, TURN);
+        frag[0] = Stage::read (smem + stage, foff);
+        #pragma unroll
+        for (int g = 0; g < TN; g++)
         {
-            const int step = g / TN, i = g % TN;
-            if (g + 1 < GROUPS) frag[(g + 1) & 1] = Stage::read (smem + stage, foff[(g + 1) / TN] + ((g + 1) % TN) * 32 * 64);
-            if (MORE && g == 0)
+            if (g + 1 < TN) frag[(g + 1) & 1] = Stage::read (smem + stage, foff + (g + 1) * 16 * 64);
+            if constexpr (MORE)
             {
-                refill (SET, stage ^ Stage::BYTES);
-                bl.load (min (kbase + it + 1 + AHEAD, last), areg[SET]);
+                // the next slice's terms, spread over the fragments
+                if (g == 0) stats (areg[SET]);
+                #pragma unroll
+                for (int term = 0; term < 3; term++) if (g == min (term, TN - 1)) bl.share.store_term (smem + (stage ^ Stage::BYTES), areg[SET], term);
+                if (g == min (2, TN - 1)) bl.load (min (kbase + it + 1 + AHEAD, last), areg[SET]);
             }
-            split_mfma (frag[g & 1], w.operand (step, WSET), acc[i], lo[i]);
-            if (MORE && i == TN - 1) w.load (SETS > 1 ? min (kbase + it + SETS, last) : kbase + it + 1, step, WSET);
+            split_mfma (frag[g & 1], wf, acc[g], lo[g]);
+            // (matrix instructions and fragment reads stay in their group: left alone, the compiler sorts a whole slice's by weight term
+            // and holds every fragment at once)
+            __builtin_amdgcn_sched_barrier (SCHED_GROUP_MASK);
         }
+        if (MORE) w.load (min (kbase + it + 2, last), TURN);
         if (MORE) lds_barrier ();
     };
-    constexpr auto stage_of = [] (int turn) { return turn % 2 ? Stage::BYTES : 0u; };
     int it = 0;
-    for (; it + TRIP < kiters; it += TRIP) slice_run<0, TRIP> ([&] (auto turn) { slice (it + decltype (turn)::value, stage_of (decltype (turn)::value), turn, std::true_type ()); });
-    // the last 1 .. TRIP slices
-    if constexpr (TRIP == 2)
+    for (; it + 2 < kiters; it += 2)
     {
-        constexpr std::integral_constant<int, 0> turn;
-        uint32_t stage = 0;
-        if (it + 1 < kiters) { slice (it, 0, turn, std::true_type ()); it++; stage = Stage::BYTES; }
-        before_last_slice ();
-        slice (it, stage, turn, std::false_type ());
+        slice (it, 0, std::integral_constant<int, 0> (), std::true_type ());
+        slice (it + 1, Stage::BYTES, std::integral_constant<int, 1> (), std::true_type ());
     }
-    else
-        last_slices<0, TRIP> (kiters - it, [&] (auto turn, auto more)
-        {
-            if constexpr (!decltype (more)::value) before_last_slice ();
-            slice (it + decltype (turn)::value, stage_of (decltype (turn)::value), turn, more);
-        });
+    // the last one or two slices (one copy of the last: its weights are moved to the first set where they are in the second; a copy each
+    // made the compiler spill where the copies' sums meet)
+    constexpr std::integral_constant<int, 0> first;
+    uint32_t stage = 0;
+    if (it + 1 < kiters)
+    {
+        slice (it, 0, first, std::true_type ());
+        it++; stage = Stage::BYTES;
+        w.take_second_set ();
+    }
+    before_last_slice ();
+    slice (it, stage, first, std::false_type ());
     __builtin_amdgcn_s_setprio (TILE_PRIO);
     #pragma unroll
     for (int i = 0; i < TN; i++)
         #pragma unroll
-        for (int v = 0; v < 16; v++) acc[i][v] += lo[i][v];
+        for (int j = 0; j < TM; j++) acc[i][j] += lo[i][j];
     lds_barrier ();          // the caller reuses the stages (epilogue)
 }
 
@@ -929,95 +914,101 @@ template <class Address> struct layer_at
 };
 
 // Sums that three terms cannot form (operands that are not finite, or whose h rounds to infinity; sums beyond the largest
-// float): one wavefront's 32 x 32 block over the slices [kbase, kbase + kiters) from the floats themselves, every lane reading
-// its operands straight from memory in fragment order, on the single-precision matrix instruction.  Nothing else comes
-// here, so it is written for size: one slice at a time, the operand's address from scratch for each.
-// n: the lane's activation row, `block`: the wavefront's block of weight rows.
+// float): 16 weight rows x 32 activation rows of one wavefront over the slices [kbase, kbase + kiters) from the floats themselves,
+// every lane reading its operands straight from memory in fragment order, on the single-precision matrix instruction.  Nothing
+// else comes here, so it is written for size: one slice at a time, the operand's address from scratch for each.
+// group: the 16 weight rows; n: the lane's first activation row (row lane % 16 of the first block), the second one is n + 16.
 // A real function: inlined, its registers pushed the convolutional kernels' prefetched shortcuts out to scratch.
 template <bool RAW, int COH, bool GATHER, bool TABLES>
-__device__ __noinline__ floatx16 single_precision_block (const aspen_hip_layer_t *layer, uint32_t block, uint32_t n, int kbase, int kiters)
+__device__ __noinline__ floatx8 single_precision_block (const aspen_hip_layer_t *layer, uint32_t group, uint32_t n, int kbase, int kiters)
 {
     const aspen_hip_layer_t L = scalar_layer (layer);
-    block = __builtin_amdgcn_readfirstlane (block); kbase = __builtin_amdgcn_readfirstlane (kbase); kiters = __builtin_amdgcn_readfirstlane (kiters);
-    const uint32_t lane = tile_thread () & 63, unit0 = lane >> 5, total = L.Kp / SLICE_K;
-    n = min (n, L.N - 1);
+    group = __builtin_amdgcn_readfirstlane (group); kbase = __builtin_amdgcn_readfirstlane (kbase); kiters = __builtin_amdgcn_readfirstlane (kiters);
+    const uint32_t lane = tile_thread () & 63, unit = lane >> 4, total = L.Kp / SLICE_K;
     ActView<COH> in;
     in.init (L.in0, L.in0_columns, L.ld0);
-    WeightFragments<RAW> w;
-    w.init (L.weight, block, total, lane);
-    int32_t base = (int32_t)(n * L.ld0), ih0 = 0, iw0 = 0;
+    WeightFragments<RAW, 1> w;
+    w.init (L.weight, group, total, lane);
     const bool direct = !GATHER || L.direct == ASPEN_HIP_OPERAND_DIRECT;
-    if (!direct)
-    {
-        const uint32_t ohw = L.OH * L.OW, b = fast_div (n, L.div_ohw), rem = n - b * ohw, oh = fast_div (rem, L.div_ow), ow = rem - oh * L.OW;
-        ih0 = (int32_t)(oh * L.stride) - (int32_t)L.pad;
-        iw0 = (int32_t)(ow * L.stride) - (int32_t)L.pad;
-        base = ((int32_t)(b * L.IH) + ih0) * (int32_t)L.IW * (int32_t)L.ld0 + iw0 * (int32_t)L.ld0;
-    }
-    const auto inside = [&] (uint32_t kh, uint32_t kw) { return (uint32_t)(ih0 + (int32_t)kh) < L.IH && (uint32_t)(iw0 + (int32_t)kw) < L.IW; };
-    floatx16 acc;
-    #pragma unroll
-    for (int v = 0; v < 16; v++) acc[v] = 0.f;
+    floatx8 acc;
     #pragma unroll 1
-    for (int it = kbase; it < kbase + kiters; it++)
+    for (uint32_t i = 0; i < 2; i++)
     {
-        float4 x[2][2];
-        w.load (it, 0); w.load (it, 1);
-        uint32_t offset = (uint32_t)it * SLICE_K;
-        bool ok = true;
-        if (!direct && !(TABLES && (L.direct == ASPEN_HIP_OPERAND_DENSE3 || L.IC % SLICE_K != 0)))
+        const uint32_t c = min (n + 16 * i, L.N - 1);
+        int32_t base = (int32_t)(c * L.ld0), ih0 = 0, iw0 = 0;
+        if (!direct)
         {
-            const uint32_t taps = L.KH * L.KW, channels = (uint32_t)it / taps, tap = (uint32_t)it - channels * taps, kh = tap / L.KW, kw = tap - kh * L.KW;
-            offset = (kh * L.IW + kw) * L.ld0 + channels * SLICE_K;
-            ok = inside (kh, kw);
+            const uint32_t ohw = L.OH * L.OW, b = fast_div (c, L.div_ohw), rem = c - b * ohw, oh = fast_div (rem, L.div_ow), ow = rem - oh * L.OW;
+            ih0 = (int32_t)(oh * L.stride) - (int32_t)L.pad;
+            iw0 = (int32_t)(ow * L.stride) - (int32_t)L.pad;
+            base = ((int32_t)(b * L.IH) + ih0) * (int32_t)L.IW * (int32_t)L.ld0 + iw0 * (int32_t)L.ld0;
         }
-        #pragma unroll
-        for (int q = 0; q < 4; q++)
+        const auto inside = [&] (uint32_t kh, uint32_t kw) { return (uint32_t)(ih0 + (int32_t)kh) < L.IH && (uint32_t)(iw0 + (int32_t)kw) < L.IW; };
+        floatx4 sum = {0.f, 0.f, 0.f, 0.f};
+        #pragma unroll 1
+        for (int it = kbase; it < kbase + kiters; it++)
         {
-            const uint32_t unit = unit0 + (q & 2), chunk = unit + 4 * (q & 1);      // step q / 2; four floats: chunk of the slice's eight
-            float4 &d = x[q >> 1][q & 1];
-            if (TABLES && !direct && L.direct == ASPEN_HIP_OPERAND_DENSE3)
+            float4 x[2];
+            w.load (it);
+            uint32_t offset = (uint32_t)it * SLICE_K;
+            bool ok = true;
+            if (!direct && !(TABLES && (L.direct == ASPEN_HIP_OPERAND_DENSE3 || L.IC % SLICE_K != 0)))
             {
-                const uint32_t kc = (uint32_t)it * 8 + chunk, sel = kc % 3u;
-                const aspen_hip_ktab_t e0 = L.ktab[2 * kc], e1 = L.ktab[2 * kc + 1];
-                const float4 a = in.ld4_if ((uint32_t)(base + e0.offset), inside (e0.kh, e0.kw)), b = in.ld4_if ((uint32_t)(base + e1.offset), inside (e1.kh, e1.kw));
-                d.x = sel == 0 ? a.x : sel == 1 ? a.y : a.z;
-                d.y = sel == 0 ? a.y : sel == 1 ? a.z : b.x;
-                d.z = sel == 0 ? a.z : sel == 1 ? b.x : b.y;
-                d.w = sel == 0 ? b.x : sel == 1 ? b.y : b.z;
+                const uint32_t taps = L.KH * L.KW, channels = (uint32_t)it / taps, tap = (uint32_t)it - channels * taps, kh = tap / L.KW, kw = tap - kh * L.KW;
+                offset = (kh * L.IW + kw) * L.ld0 + channels * SLICE_K;
+                ok = inside (kh, kw);
             }
-            else if (TABLES && !direct && L.IC % SLICE_K != 0)
+            #pragma unroll
+            for (int q = 0; q < 2; q++)
             {
-                const aspen_hip_ktab_t e = L.ktab[(uint32_t)it * 8 + chunk];
-                d = in.ld4_if ((uint32_t)(base + e.offset), inside (e.kh, e.kw));
+                const uint32_t chunk = unit + 4 * q;      // four floats: chunk of the slice's eight
+                float4 &d = x[q];
+                if (TABLES && !direct && L.direct == ASPEN_HIP_OPERAND_DENSE3)
+                {
+                    const uint32_t kc = (uint32_t)it * 8 + chunk, sel = kc % 3u;
+                    const aspen_hip_ktab_t e0 = L.ktab[2 * kc], e1 = L.ktab[2 * kc + 1];
+                    const float4 a = in.ld4_if ((uint32_t)(base + e0.offset), inside (e0.kh, e0.kw)), b = in.ld4_if ((uint32_t)(base + e1.offset), inside (e1.kh, e1.kw));
+                    d.x = sel == 0 ? a.x : sel == 1 ? a.y : a.z;
+                    d.y = sel == 0 ? a.y : sel == 1 ? a.z : b.x;
+                    d.z = sel == 0 ? a.z : sel == 1 ? b.x : b.y;
+                    d.w = sel == 0 ? b.x : sel == 1 ? b.y : b.z;
+                }
+                else if (TABLES && !direct && L.IC % SLICE_K != 0)
+                {
+                    const aspen_hip_ktab_t e = L.ktab[(uint32_t)it * 8 + chunk];
+                    d = in.ld4_if ((uint32_t)(base + e.offset), inside (e.kh, e.kw));
+                }
+                else d = in.ld4_if ((uint32_t)base + offset + chunk * 4, ok);
             }
-            else d = in.ld4_if ((uint32_t)base + offset + chunk * 4, ok);
-        }
-        #pragma unroll
-        for (int step = 0; step < 2; step++)
-        {
             float wf[8];
             #pragma unroll
             for (int q = 0; q < 4; q++)
             {
-                if constexpr (RAW) { const floatx4 r = __builtin_bit_cast (floatx4, w.f[0][step][q >> 1]); wf[2 * q] = r[2 * (q & 1)]; wf[2 * q + 1] = r[2 * (q & 1) + 1]; }
-                else { const floatx2 r = join2 (w.f[0][step][0][q], w.f[0][step][1][q], w.f[0][step][2][q]); wf[2 * q] = r[0]; wf[2 * q + 1] = r[1]; }
+                if constexpr (RAW) { const floatx4 r = __builtin_bit_cast (floatx4, w.f[0][0][q >> 1]); wf[2 * q] = r[2 * (q & 1)]; wf[2 * q + 1] = r[2 * (q & 1) + 1]; }
+                else { const floatx2 r = join2 (w.f[0][0][0][q], w.f[0][0][1][q], w.f[0][0][2][q]); wf[2 * q] = r[0]; wf[2 * q + 1] = r[1]; }
             }
-            const float xf[8] = {x[step][0].x, x[step][0].y, x[step][0].z, x[step][0].w, x[step][1].x, x[step][1].y, x[step][1].z, x[step][1].w};
+            const float xf[8] = {x[0].x, x[0].y, x[0].z, x[0].w, x[1].x, x[1].y, x[1].z, x[1].w};
             #pragma unroll
-            for (int k = 0; k < 8; k++) acc = __builtin_amdgcn_mfma_f32_32x32x2f32 (xf[k], wf[k], acc, 0, 0, 0);
+            for (int k = 0; k < 8; k++) sum = __builtin_amdgcn_mfma_f32_16x16x4f32 (xf[k], wf[k], sum, 0, 0, 0);
         }
+        #pragma unroll
+        for (int v = 0; v < 4; v++) { if (i == 0) acc[v] = sum[v]; else acc[4 + v] = sum[v]; }
     }
     return acc;
 }
 
-// true for a wavefront one of whose sums is not finite (elementwise_maximum passes NaNs on: eight v_maximum3_f32; sixteen
+// true for a wavefront one of whose sums is not finite (elementwise_maximum passes NaNs on: one v_maximum3_f32 for two sums;
 // multiply-adds with zero took 1 % of BERT-base 8 x 128)
-__device__ __forceinline__ bool sums_not_finite (const floatx16 &acc)
+template <int TN, int TM>
+__device__ __forceinline__ bool sums_not_finite (const floatx4 (&acc)[TN][TM])
 {
     float most[2] = {0.f, 0.f};
     #pragma unroll
-    for (int v = 0; v < 16; v += 2) most[(v >> 1) & 1] = __builtin_elementwise_maximum (__builtin_elementwise_maximum (most[(v >> 1) & 1], fabsf (acc[v])), fabsf (acc[v + 1]));
+    for (int i = 0; i < TN; i++)
+        #pragma unroll
+        for (int j = 0; j < TM; j++)
+            #pragma unroll
+            for (int v = 0; v < 4; v += 2) most[v >> 1] = __builtin_elementwise_maximum (__builtin_elementwise_maximum (most[v >> 1], fabsf (acc[i][j][v])), fabsf (acc[i][j][v + 1]));
     return __builtin_expect (__any (!(__builtin_elementwise_maximum (most[0], most[1]) < INFINITY)), 0);
 }
 
@@ -1052,15 +1043,15 @@ __device__ __forceinline__ void fused_shortcut (const aspen_hip_layer_t &L, cons
 // of the thread's pieces of a fused shortcut's operand (a tile has at most 128 columns: 8 pieces per thread)
 struct shortcut_prefetch_t { float4 s[8]; float4 bias; bool have, have_shortcut; };
 
-template <int BM, int BN, int WM, int WN, int COH, unsigned FEAT, class Descriptor, class Ready>
+template <int BM, int BN, int COH, unsigned FEAT, class Descriptor, class Ready>
 __device__ __forceinline__ void contraction_mainloop (const aspen_hip_layer_t &L, Descriptor descriptor, uint32_t tn, uint32_t tm, int slice, float *smem, shortcut_prefetch_t &pre, Ready ready)
 {
-    static_assert (BM == WM * WEIGHT_BLOCK_ROWS, "one block of weight rows per wavefront");
-    constexpr int TN = BN / WN / 32;
+    constexpr int TM = BM / 64, TN = BN / 16;
+    static_assert (TM == 1 || TM == 2, "four wavefronts below each other, 16 or 32 rows each");
     constexpr bool SMALL = BM == VAR2_BM && BN == VAR2_BN, RAW = BM == VAR4_BM && BN == VAR4_BN;      // (the tall shape's weights stay floats in memory)
     const uint32_t tid = tile_thread (), lane = tid & 63, wave = tid >> 6;
     const uint32_t m0 = tm * BM, n0 = tn * BN;
-    floatx16 acc[TN];
+    floatx4 acc[TN][TM];
     ActView<COH> in;
     // (the operands' addresses come from loads of their own: taken from `L` they are parts of an 8-register piece of
     // the descriptor, which the compiler then keeps alive, spills and restores as a whole around every K slice)
@@ -1096,11 +1087,11 @@ __device__ __forceinline__ void contraction_mainloop (const aspen_hip_layer_t &L
                 if (r0 + u * STEP < rows) pre.s[u] = fin.ld4 ((n0 + r0 + u * STEP) * L.fuse_ld_in + m0 + c);
         }
     };
-    // (one slice of activations in flight under the wide shape: a second register set does not fit beside its sums, its loops
-    // spilled; four, and as many of weights, in kernels compiled for two workgroups per compute unit, see TILES_DEEP)
-    constexpr bool DEEP = SMALL && (FEAT & TILES_DEEP) != 0;
-    constexpr int SETS = DEEP ? 4 : 1, AHEAD = SliceShare<BN>::R > 1 ? 1 : DEEP ? 4 : 2;
-    const auto loop = [&] (auto &bl, auto stats) { split_core<BN, WM, WN, RAW, SETS, AHEAD> (weights, tm * WM, total, bl, kbase, kiters, stages, acc, COH != 0, fetch_shortcut, ready, stats); };
+    // Two slices of weights in flight; of activations two, or one where the sums take 64 registers (with two as well the large shape's loops
+    // spilled).  Four and four for 64 x 64 tiles, in a kernel for two workgroups per unit, ran BERT-base 3 x 75 in the same
+    // 938 us as this one for three.
+    constexpr int AHEAD = TM * TN > 4 ? 1 : 2;
+    const auto loop = [&] (auto &bl, auto stats) { split_core<BN, TM, RAW, AHEAD> (weights, tm * (BM / 16), total, bl, kbase, kiters, stages, acc, COH != 0, fetch_shortcut, ready, stats); };
     float cs = 0.f, cq = 0.f;
     if constexpr ((FEAT & TILES_GATHER) == 0 || (SMALL && (FEAT & TILES_NORM) != 0))
     {
@@ -1150,22 +1141,29 @@ __device__ __forceinline__ void contraction_mainloop (const aspen_hip_layer_t &L
             loop (bl, NoStats ());
         }
     }
-    const uint32_t wm0 = (wave % WM) * 32, wn0 = (wave / WM) * (BN / WN);
-    const auto again = [&] (int i) { return single_precision_block<RAW, COH, (FEAT & TILES_GATHER) != 0, BM == 64> (descriptor.address (), tm * WM + wave % WM, n0 + wn0 + 32 * i + (lane & 31), kbase, kiters); };
-    bool redo = sums_not_finite (acc[0]);
-    if constexpr (TN == 1)
+    const uint32_t wm0 = wave * 16 * TM;
+    // (columns 32 i .. of rows 16 j ..)
+    const auto again = [&] (int i, int j) { return single_precision_block<RAW, COH, (FEAT & TILES_GATHER) != 0, BM == 64> (descriptor.address (), tm * (BM / 16) + wave * TM + j, n0 + 32 * i + (lane & 15), kbase, kiters); };
+    constexpr bool FEW = TN * TM <= 4;          // the sums wait in registers meanwhile
+    const bool redo = sums_not_finite (acc);
+    if constexpr (FEW)
     {
         if (redo)
         {
-            const floatx16 x = again (0);
             #pragma unroll
-            for (int v = 0; v < 16; v++) acc[0][v] = fabsf (acc[0][v]) < INFINITY ? acc[0][v] : x[v];
+            for (int i = 0; i < TN / 2; i++)
+                #pragma unroll
+                for (int j = 0; j < TM; j++)
+                {
+                    const floatx8 x = again (i, j);
+                    #pragma unroll
+                    for (int v = 0; v < 8; v++) { const float y = acc[2 * i + (v >> 2)][j][v & 3]; acc[2 * i + (v >> 2)][j][v & 3] = fabsf (y) < INFINITY ? y : x[v]; }
+                }
         }
     }
-    else redo |= sums_not_finite (acc[1]);
     if constexpr (SMALL && (FEAT & TILES_NORM) != 0)
     {
-        if (L.norm_fold) norm_fold_finish<COH> (L, acc[0], cs, cq, smem, tid, m0, n0, wm0, wn0);
+        if (L.norm_fold) norm_fold_finish<COH> (L, acc, cs, cq, smem, tid, m0, n0, wm0);
     }
     if (COH) tile_phase_lap (9);
     if (slice >= 0)
@@ -1173,8 +1171,8 @@ __device__ __forceinline__ void contraction_mainloop (const aspen_hip_layer_t &L
         // split-K: the raw sums go straight from the accumulators to this slice's block of the output tile, in the
         // accumulators' own layout (splitk_gather reads them back the same way): four 16-byte stores per lane, each
         // instruction 1 KB in one piece; no bias, no activation, no bounds, nothing to stage through LDS.  Only the
-        // 64 x 64 and the 128 x 32 shape (one accumulator block per wavefront either way) are ever cut along K.
-        if constexpr (TN == 1)
+        // 64 x 64 and the 128 x 32 shape (four accumulator blocks per wavefront either way) are ever cut along K.
+        if constexpr (FEW)
         {
             const aspen_hip_layer_t L = descriptor ();
             const uint32_t tiles = L.tiles_m * L.tiles_n;
@@ -1183,30 +1181,32 @@ __device__ __forceinline__ void contraction_mainloop (const aspen_hip_layer_t &L
             const uint32_t base = ((uint32_t)slice * tiles + tn * L.tiles_m + tm) * SPLITK_TILE_FLOATS + tid * 4;
             #pragma unroll
             for (int q = 0; q < 4; q++)
-                part.st4 (base + q * 4 * WG_THREADS, make_float4 (acc[0][4 * q], acc[0][4 * q + 1], acc[0][4 * q + 2], acc[0][4 * q + 3]));
+                part.st4 (base + q * 4 * WG_THREADS, make_float4 (acc[q / TM][q % TM][0], acc[q / TM][q % TM][1], acc[q / TM][q % TM][2], acc[q / TM][q % TM][3]));
         }
         return;
     }
     // Epilogue through LDS (free after the last K slice): the raw accumulators are parked as
     // [column][channel] for contraction_epilogue.
-    constexpr int TROW = BM + 8;            // (4 * TROW) % 64 == 32: the two half-waves hit disjoint banks
+    constexpr int TROW = EPI_ROW (BM);
     #pragma unroll
     for (int i = 0; i < TN; i++)
         #pragma unroll
-        for (int v = 0; v < 16; v++)
-            smem[ACC_N (wn0, i, v, lane) * TROW + wm0 + (lane & 31)] = acc[i][v];
-    if constexpr (TN > 1)
+        for (int j = 0; j < TM; j++)
+            #pragma unroll
+            for (int v = 0; v < 4; v++) smem[BLOCK_N (i, v, lane) * TROW + wm0 + 16 * j + (lane & 15)] = acc[i][j][v];
+    if constexpr (!FEW)
     {
         if (redo)           // (every lane puts right what it has just parked)
         {
             #pragma unroll 1
-            for (int i = 0; i < TN; i++)
+            for (int p = 0; p < TN / 2 * TM; p++)
             {
-                const floatx16 x = again (i);
+                const int i = p / TM, j = p % TM;
+                const floatx8 x = again (i, j);
                 #pragma unroll
-                for (int v = 0; v < 16; v++)
+                for (int v = 0; v < 8; v++)
                 {
-                    float *sum = smem + ACC_N (wn0, i, v, lane) * TROW + wm0 + (lane & 31);
+                    float *sum = smem + BLOCK_N (2 * i + (v >> 2), v & 3, lane) * TROW + wm0 + 16 * j + (lane & 15);
                     if (!(fabsf (*sum) < INFINITY)) *sum = x[v];
                 }
             }
@@ -1216,14 +1216,14 @@ __device__ __forceinline__ void contraction_mainloop (const aspen_hip_layer_t &L
 }
 
 // Second part of a contraction tile of BM = 4 << c4_log2 channels by BN columns, accumulators parked in
-// LDS as [column][BM + 8]: a rolled loop adds the bias, applies the activation and writes 128-bit pieces,
+// LDS as [column][EPI_ROW (BM)]: a rolled loop adds the bias, applies the activation and writes 128-bit pieces,
 // so a wavefront covers whole 512-byte (BM = 128) / 256-byte (BM = 64) runs of a column.
 template <int COH, bool NORM = false>
 __device__ __forceinline__ void contraction_epilogue (const aspen_hip_layer_t &L, uint32_t tn, uint32_t tm, float *smem,
     uint32_t c4_log2, uint32_t BN, const shortcut_prefetch_t &pre)
 {
     const uint32_t tid = tile_thread ();
-    const uint32_t C4 = 1u << c4_log2, BM = 4u << c4_log2, TROW = BM + 8;
+    const uint32_t C4 = 1u << c4_log2, BM = 4u << c4_log2, TROW = EPI_ROW (BM);
     const uint32_t m0 = tm * BM, n0 = tn * BN;
     const int act = L.act;
     ActView<COH> out;
@@ -1354,16 +1354,16 @@ __device__ __forceinline__ void splitk_gather (const aspen_hip_layer_t &L, uint3
             { v[q].x += use ? p[j][q].x : 0.f; v[q].y += use ? p[j][q].y : 0.f; v[q].z += use ? p[j][q].z : 0.f; v[q].w += use ? p[j][q].w : 0.f; }
         }
     }
-    // (tall: 128 channels x 32 columns, the four wavefronts' blocks below each other; else 2 x 2 blocks of 64 x 64)
-    const uint32_t TROW = (tall ? VAR4_BM : VAR2_BM) + 8;
-    const uint32_t wm0 = tall ? wave * 32 : (wave % 2) * 32, wn0 = tall ? 0u : (wave / 2) * 32, m = wm0 + (lane & 31);
+    // (a wavefront's four blocks lie beside each other, of the tall shape two by two)
+    const uint32_t TROW = EPI_ROW (tall ? VAR4_BM : VAR2_BM), wm0 = wave * (tall ? 32 : 16) + (lane & 15);
     #pragma unroll
     for (int q = 0; q < 4; q++)
     {
-        smem[ACC_N (wn0, 0, 4 * q, lane) * TROW + m] = v[q].x;
-        smem[ACC_N (wn0, 0, 4 * q + 1, lane) * TROW + m] = v[q].y;
-        smem[ACC_N (wn0, 0, 4 * q + 2, lane) * TROW + m] = v[q].z;
-        smem[ACC_N (wn0, 0, 4 * q + 3, lane) * TROW + m] = v[q].w;
+        const uint32_t i = tall ? q >> 1 : q, m = wm0 + (tall ? 16 * (q & 1) : 0);
+        smem[BLOCK_N (i, 0, lane) * TROW + m] = v[q].x;
+        smem[BLOCK_N (i, 1, lane) * TROW + m] = v[q].y;
+        smem[BLOCK_N (i, 2, lane) * TROW + m] = v[q].z;
+        smem[BLOCK_N (i, 3, lane) * TROW + m] = v[q].w;
     }
     __syncthreads ();
 }
@@ -2198,57 +2198,71 @@ __device__ __forceinline__ float4 narrow_mainloop (const aspen_hip_layer_t &L, D
     float *smem, Ready ready)
 {
     const uint32_t tid = tile_thread (), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane (tid >> 6);
-    const uint32_t row = lane & 31, unit0 = (lane >> 5) * 4;       // the lane's units of a slice start at floats unit0 (step 0) and 8 + unit0 (step 1)
+    const uint32_t row = lane & 15, unit0 = (lane >> 4) * 4;       // the lane's columns are row and row + 16, its unit starts at float unit0 of a slice
     // this wavefront's share of the slices: a contiguous quarter
     const int per = (kiters + 3) >> 2, w0 = min ((int)wave * per, kiters), cnt = min (per, kiters - w0), first = kbase + w0;
     const uint32_t total = L.Kp / SLICE_K;
-    WeightFragments<false> w0r, w1r;
-    w0r.init (descriptor ().weight, tm, total, lane);
+    WeightFragments<false, 2> w0r, w1r;
+    w0r.init (descriptor ().weight, 2 * tm, total, lane);
     w1r = w0r;
     ActView<COH> in;
     in.init (descriptor ().in0, L.in0_columns, L.ld0);
     const bool direct = L.direct == ASPEN_HIP_OPERAND_DIRECT;
-    uint32_t n = tn * VAR3_BN + row;
-    n = n < L.N ? n : L.N - 1;
     // activation operand: DIRECT = the parent's column; else the top-left input pixel of output position n and the
     // tap / channel the first slice starts at (stepped from there, as StepLoader does)
-    int32_t bbase, ih0 = 0, iw0 = 0;
+    int32_t bbase[2], ih0[2] = {0, 0}, iw0[2] = {0, 0};
     uint32_t kh = 0, kw = 0, c = 0;
-    if (direct) bbase = (int32_t)(n * L.ld0 + (uint32_t)first * SLICE_K + unit0);
-    else
+    #pragma unroll
+    for (int i = 0; i < 2; i++)
     {
-        const uint32_t ohw = L.OH * L.OW;
-        const uint32_t b = fast_div (n, L.div_ohw), rem = n - b * ohw, oh = fast_div (rem, L.div_ow), ow = rem - oh * L.OW;
-        ih0 = (int32_t)(oh * L.stride) - (int32_t)L.pad;
-        iw0 = (int32_t)(ow * L.stride) - (int32_t)L.pad;
-        bbase = ((int32_t)(b * L.IH) + ih0) * (int32_t)L.IW * (int32_t)L.ld0 + iw0 * (int32_t)L.ld0 + (int32_t)unit0;
+        const uint32_t n = min (tn * VAR3_BN + row + 16 * i, L.N - 1);
+        if (direct) bbase[i] = (int32_t)(n * L.ld0 + (uint32_t)first * SLICE_K + unit0);
+        else
+        {
+            const uint32_t ohw = L.OH * L.OW;
+            const uint32_t b = fast_div (n, L.div_ohw), rem = n - b * ohw, oh = fast_div (rem, L.div_ow), ow = rem - oh * L.OW;
+            ih0[i] = (int32_t)(oh * L.stride) - (int32_t)L.pad;
+            iw0[i] = (int32_t)(ow * L.stride) - (int32_t)L.pad;
+            bbase[i] = ((int32_t)(b * L.IH) + ih0[i]) * (int32_t)L.IW * (int32_t)L.ld0 + iw0[i] * (int32_t)L.ld0 + (int32_t)unit0;
+        }
+    }
+    if (!direct)
+    {
         // (K order: channel block, kh, kw, channel in block; see StepLoader)
         const uint32_t taps = L.KH * L.KW, block = (uint32_t)first / taps, tap = (uint32_t)first - block * taps;
         c = block * SLICE_K;
         kh = tap / L.KW; kw = tap - kh * L.KW;
     }
     const uint32_t IH = L.IH, IW = L.IW, KH = L.KH, KW = L.KW, ld0 = L.ld0;
-    // a slice's four pieces in unit order: floats +0, +16 (step 0), +8, +24 (step 1); slices are asked for in ascending
+    // a slice's four pieces: floats +0, +16 of the first column and of the second; slices are asked for in ascending
     // order: the tap position is stepped
     auto load_b = [&] (int i, float4 (&bv)[4])
     {
         if (direct)
         {
             #pragma unroll
-            for (int q = 0; q < 4; q++) bv[q] = in.ld4 ((uint32_t)(bbase + i * SLICE_K + (q & 1) * 16 + (q >> 1) * 8));
+            for (int q = 0; q < 4; q++) bv[q] = in.ld4 ((uint32_t)(bbase[q >> 1] + i * SLICE_K + (q & 1) * 16));
         }
         else
         {
             const int32_t off = (int32_t)((kh * IW + kw) * ld0 + c);
-            const bool ok = (uint32_t)(ih0 + (int32_t)kh) < IH && (uint32_t)(iw0 + (int32_t)kw) < IW;
             #pragma unroll
-            for (int q = 0; q < 4; q++) bv[q] = in.ld4_if ((uint32_t)(bbase + off + (q & 1) * 16 + (q >> 1) * 8), ok);
+            for (int q = 0; q < 4; q++)
+            {
+                const bool ok = (uint32_t)(ih0[q >> 1] + (int32_t)kh) < IH && (uint32_t)(iw0[q >> 1] + (int32_t)kw) < IW;
+                bv[q] = in.ld4_if ((uint32_t)(bbase[q >> 1] + off + (q & 1) * 16), ok);
+            }
             if (++kw == KW) { kw = 0; if (++kh == KH) { kh = 0; c += SLICE_K; } }
         }
     };
-    floatx16 acc, lo;
+    floatx4 acc[2][2], lo[2][2];
     #pragma unroll
-    for (int v = 0; v < 16; v++) acc[v] = lo[v] = 0.f;
+    for (int p = 0; p < 4; p++) acc[p >> 1][p & 1] = lo[p >> 1][p & 1] = (floatx4){0.f, 0.f, 0.f, 0.f};
+    const auto products = [&] (const split8_t (&wf)[2], const float4 (&bv)[4])
+    {
+        #pragma unroll
+        for (int i = 0; i < 2; i++) split_mfma (split8 (bv[2 * i], bv[2 * i + 1]), wf, acc[i], lo[i]);
+    };
     constexpr uint32_t REGION = CMAX (PF * SPLIT_SLICE_BYTES / 4u, (uint32_t)(VAR3_BN * NARROW_ROW));     // floats of LDS per wavefront
     float *mine = smem + wave * REGION;
     int done = 0;       // slices of this wavefront's share that are finished
@@ -2276,14 +2290,16 @@ __device__ __forceinline__ float4 narrow_mainloop (const aspen_hip_layer_t &L, D
             for (int i = 0; i < C; i++) load_b (i, bq[i]);
             #pragma unroll
             for (int i = 0; i < C; i++)
+            {
+                split8_t wf[2];
                 #pragma unroll
-                for (int step = 0; step < 2; step++)
+                for (int j = 0; j < 2; j++)
                 {
-                    split8_t wf;
-                    const float *f = mine + (i * 6 + step * 3) * 256 + lane * 4;
-                    wf.h = *reinterpret_cast<const u32x4 *> (f); wf.m = *reinterpret_cast<const u32x4 *> (f + 256); wf.l = *reinterpret_cast<const u32x4 *> (f + 512);
-                    split_mfma (split8 (bq[i][2 * step], bq[i][2 * step + 1]), wf, acc, lo);
+                    const float *f = mine + (i * 6 + j * 3) * 256 + lane * 4;
+                    wf[j].h = *reinterpret_cast<const u32x4 *> (f); wf[j].m = *reinterpret_cast<const u32x4 *> (f + 256); wf[j].l = *reinterpret_cast<const u32x4 *> (f + 512);
                 }
+                products (wf, bq[i]);
+            }
         };
         static_assert (PF == 3, "one case per prefetched slice count");
         const int pre = __builtin_amdgcn_readfirstlane (min (cnt, PF));
@@ -2291,44 +2307,50 @@ __device__ __forceinline__ float4 narrow_mainloop (const aspen_hip_layer_t &L, D
         else if (pre == 2) body (std::integral_constant<int, 2> ());
         else if (pre == 1) body (std::integral_constant<int, 1> ());
         done = min (cnt, PF);
-        if (done < cnt) { w0r.load (first + done, 0); w0r.load (first + done, 1); load_b (done, b0); }
-        if (done + 1 < cnt) { w1r.load (first + done + 1, 0); w1r.load (first + done + 1, 1); load_b (done + 1, b1); }
+        if (done < cnt) { w0r.load (first + done); load_b (done, b0); }
+        if (done + 1 < cnt) { w1r.load (first + done + 1); load_b (done + 1, b1); }
     }
     else
     {
         // two slices in flight: set 0 holds the even, set 1 the odd ones of this wavefront's share
-        if (cnt > 0) { w0r.load (first, 0); w0r.load (first, 1); }
-        if (cnt > 1) { w1r.load (first + 1, 0); w1r.load (first + 1, 1); }
+        if (cnt > 0) { w0r.load (first); }
+        if (cnt > 1) { w1r.load (first + 1); }
         ready ();
         if (cnt > 0) load_b (0, b0);
         if (cnt > 1) load_b (1, b1);
     }
-    auto mfmas = [&] (const WeightFragments<false> &w, const float4 (&bv)[4])
+    auto mfmas = [&] (const WeightFragments<false, 2> &w, const float4 (&bv)[4])
     {
-        #pragma unroll
-        for (int step = 0; step < 2; step++) split_mfma (split8 (bv[2 * step], bv[2 * step + 1]), w.operand (step), acc, lo);
+        const split8_t wf[2] = {w.operand (0), w.operand (1)};
+        products (wf, bv);
     };
     for (int i = done; i < cnt; i += 2)
     {
         mfmas (w0r, b0);
-        if (i + 2 < cnt) { w0r.load (first + i + 2, 0); w0r.load (first + i + 2, 1); load_b (i + 2, b0); }
+        if (i + 2 < cnt) { w0r.load (first + i + 2); load_b (i + 2, b0); }
         if (i + 1 < cnt)
         {
             mfmas (w1r, b1);
-            if (i + 3 < cnt) { w1r.load (first + i + 3, 0); w1r.load (first + i + 3, 1); load_b (i + 3, b1); }
+            if (i + 3 < cnt) { w1r.load (first + i + 3); load_b (i + 3, b1); }
         }
     }
     // the four wavefronts' sums meet in LDS: [wave][column][NARROW_ROW] (a wavefront's own region, which it has read empty)
     #pragma unroll
-    for (int v = 0; v < 16; v++) acc[v] += lo[v];
+    for (int p = 0; p < 4; p++) acc[p >> 1][p & 1] += lo[p >> 1][p & 1];
     if (sums_not_finite (acc))
     {
-        const floatx16 x = single_precision_block<false, COH, true, false> (descriptor.address (), tm, tn * VAR3_BN + row, first, cnt);
         #pragma unroll
-        for (int v = 0; v < 16; v++) acc[v] = fabsf (acc[v]) < INFINITY ? acc[v] : x[v];
+        for (int j = 0; j < 2; j++)
+        {
+            const floatx8 x = single_precision_block<false, COH, true, false> (descriptor.address (), 2 * tm + j, tn * VAR3_BN + row, first, cnt);
+            #pragma unroll
+            for (int v = 0; v < 8; v++) { const float y = acc[v >> 2][j][v & 3]; acc[v >> 2][j][v & 3] = fabsf (y) < INFINITY ? y : x[v]; }
+        }
     }
     #pragma unroll
-    for (int v = 0; v < 16; v++) mine[ACC_N (0, 0, v, lane) * NARROW_ROW + row] = acc[v];
+    for (int p = 0; p < 4; p++)
+        #pragma unroll
+        for (int v = 0; v < 4; v++) mine[BLOCK_N (p >> 1, v, lane) * NARROW_ROW + 16 * (p & 1) + row] = acc[p >> 1][p & 1][v];
     __syncthreads ();
     const narrow_piece_t pc = narrow_piece (tid);
     float4 sum = ld4 (smem + pc.n * NARROW_ROW + pc.c);
@@ -2464,12 +2486,12 @@ __device__ __forceinline__ bool run_tile (Descriptor descriptor, uint32_t t, boo
                 if (more_rows) *more_rows = row_rep + 1 < reps && (tm + 1) * VAR0_BM < L.M;      // (row tiles that lie wholly behind the last row have no weights)
             }
             const auto ready_first = [&] () { if (row_rep == 0) ready (); };
-            contraction_mainloop<VAR0_BM, VAR0_BN, 4, 1, COH, FEAT> (L, descriptor, tn, tm, -1, smem, pre, ready_first);
+            contraction_mainloop<VAR0_BM, VAR0_BN, COH, FEAT> (L, descriptor, tn, tm, -1, smem, pre, ready_first);
             c4_log2 = 5; bn = VAR0_BN;
         }
-        else if ((FEAT & TILES_WIDE) && L.variant == ASPEN_HIP_GEMM_WIDE) { contraction_mainloop<VAR1_BM, VAR1_BN, 2, 2, COH, FEAT> (L, descriptor, tn, tm, -1, smem, pre, ready); bn = VAR1_BN; }
-        else if ((FEAT & TILES_TALL) && L.variant == ASPEN_HIP_GEMM_TALL) { contraction_mainloop<VAR4_BM, VAR4_BN, 4, 1, COH, FEAT> (L, descriptor, tn, tm, slice, smem, pre, ready); c4_log2 = 5; bn = VAR4_BN; }
-        else if (FEAT & TILES_SMALL) contraction_mainloop<VAR2_BM, VAR2_BN, 2, 2, COH, FEAT> (L, descriptor, tn, tm, slice, smem, pre, ready);
+        else if ((FEAT & TILES_WIDE) && L.variant == ASPEN_HIP_GEMM_WIDE) { contraction_mainloop<VAR1_BM, VAR1_BN, COH, FEAT> (L, descriptor, tn, tm, -1, smem, pre, ready); bn = VAR1_BN; }
+        else if ((FEAT & TILES_TALL) && L.variant == ASPEN_HIP_GEMM_TALL) { contraction_mainloop<VAR4_BM, VAR4_BN, COH, FEAT> (L, descriptor, tn, tm, slice, smem, pre, ready); c4_log2 = 5; bn = VAR4_BN; }
+        else if (FEAT & TILES_SMALL) contraction_mainloop<VAR2_BM, VAR2_BN, COH, FEAT> (L, descriptor, tn, tm, slice, smem, pre, ready);
 
         const aspen_hip_layer_t E = descriptor ();
         if (slice >= 0)
