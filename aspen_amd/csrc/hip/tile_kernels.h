@@ -1967,21 +1967,14 @@ __device__ __forceinline__ void tile_v_attention (const aspen_hip_layer_t &L, ui
             }
 }
 
-// Fused attention tile: one (batch, head) x VATTN_BN queries, scores and weighted values in one pass, the S x S
-// probability matrix never leaves the chip (reference: tiled_k_attention followed by tiled_v_attention,
-// src/tiled_kernels.c:784-1037, which round-trip it through memory).  Per block of 64 keys:
-//   e[q][key] = exp (scale * (key > q && masked ? -1e10 : K[key] . Q[q]))      (the reference's order of operations,
-//                                                                               no max subtraction)
-//   rowsum[q] += sum_key e[q][key];   O[q][ch] += sum_key e[q][key] * V[key][ch]
-// and at the end O[q][ch] / rowsum[q].  The reference divides the probabilities first and multiplies then; dividing
-// the sum of products instead differs by rounding only (1e-7 relative).  The exponentials of a key block go to LDS in
-// the layout of an activation operand (row = query, K axis = key), the transposed values are staged next to them.
-// in0 = Query, in1 = Key, fuse_in = Value (stride fuse_ld_in); one head of at most 64 channels per tile.
-// Used when nothing but the V-attention layer reads the probabilities and their matrix need not be kept.
-// ---------------------------------------------------------------------------------------------
+// Fused attention in single precision throughout, for tiles whose sums are not finite (see tile_fused_attention, which calls it
+// and says what a tile computes): the exponentials of a key block go to LDS in the layout of an activation operand (row =
+// query, K axis = key), the transposed values are staged next to them.  A real function: it runs in the place of a tile.
 template <int COH>
-__device__ __forceinline__ void tile_fused_attention (const aspen_hip_layer_t &L, uint32_t tn, uint32_t tm, float *smem)
+__device__ __noinline__ void single_precision_attention (const aspen_hip_layer_t *layer, uint32_t tn, uint32_t tm, float *smem)
 {
+    const aspen_hip_layer_t L = scalar_layer (layer);
+    tn = __builtin_amdgcn_readfirstlane (tn); tm = __builtin_amdgcn_readfirstlane (tm);
     constexpr int BQ = VATTN_BN, BKEY = 64, EROW = BKEY + 4;
     static_assert (BQ == 64, "four wavefronts, one 32 x 32 block each");
     static_assert ((64 + BQ) * LDS_ROW + BQ * EROW <= GEMM_SMEM_FLOATS, "operand stage and exponentials fit the tile's LDS");
@@ -2067,6 +2060,158 @@ __device__ __forceinline__ void tile_fused_attention (const aspen_hip_layer_t &L
             if (q < S) out.st1 ((b * S + q) * L.ld + h * hd + ch, oacc[v] / qsum[ql]);
         }
     __syncthreads ();                                    // qsum is reused by the next tile of this workgroup
+}
+
+// Fused attention tile: one (batch, head) x VATTN_BN queries, scores and weighted values in one pass, the S x S
+// probability matrix never leaves the chip (reference: tiled_k_attention followed by tiled_v_attention,
+// src/tiled_kernels.c:784-1037, which round-trip it through memory).  Per block of 64 keys:
+//   e[q][key] = exp (scale * (key > q && masked ? -1e10 : K[key] . Q[q]))      (the reference's order of operations,
+//                                                                               no max subtraction)
+//   rowsum[q] += sum_key e[q][key];   O[q][ch] += sum_key e[q][key] * V[key][ch]
+// and at the end O[q][ch] / rowsum[q].  The reference divides the probabilities first and multiplies then; dividing
+// the sum of products instead differs by rounding only (1e-7 relative).
+// Both products are formed from three bfloat16 terms like a contraction tile's.  A wavefront owns 16 queries: their fragments stay
+// in registers, keys and transposed values are staged as terms for all four.  The keys are the matrix instruction's rows, so a lane
+// holds, of its query's scores, four consecutive keys of every 16: with two such blocks side by side that is the order of a
+// fragment's unit, and the exponentials are the second product's operand where they are: no trip through LDS, no sum over
+// wavefronts.  The next block's keys and values are requested while this one is worked on.  Two barriers per block.
+// Bound by vector instructions (480 per block and lane, 264 of them the terms) beside 96 matrix instructions, and by the way to
+// memory and back for few keys.  Against both products on the single-precision instruction with the exponentials through LDS, a tile's
+// time over two blocks of 64 keys (BERT-base 3 x 75) 11.7 -> 8 us, over eight (GPT-2 4 x 512) 49 -> 34; BERT-base 1 x 16 605 ->
+// 581 us, 3 x 75 946 -> 892, 8 x 128 1450 -> 1388, GPT-2 4 x 512 2787 -> 2598.  Error against 64 bits, scores of up to 15, 16 ... 512
+// tokens: 1.4e-7 ... 3.3e-7, before 2.9e-7 ... 7.4e-7.
+// in0 = Query, in1 = Key, fuse_in = Value (stride fuse_ld_in); one head of 32 or 64 channels per tile.
+// Used when nothing but the V-attention layer reads the probabilities and their matrix need not be kept.
+// ---------------------------------------------------------------------------------------------
+template <int COH>
+__device__ __forceinline__ void tile_fused_attention (const aspen_hip_layer_t &L, const aspen_hip_layer_t *layer, uint32_t tn, uint32_t tm, float *smem)
+{
+    typedef SplitStage<64> Stage;
+    static_assert (VATTN_BN == 64 && 4 * Stage::BYTES <= GEMM_SMEM_BYTES, "16 queries to a wavefront; two slices of keys and two of values");
+    const uint32_t tid = tile_thread (), lane = tid & 63, wave = tid >> 6, unit = lane >> 4;
+    const uint32_t S = L.seq, qtiles = (S + VATTN_BN - 1) / VATTN_BN, hd = L.hd;
+    const uint32_t b = tn / qtiles, q0 = (tn - b * qtiles) * VATTN_BN, q = q0 + wave * 16 + (lane & 15), last = b * S + S - 1;
+    // a head of 32 channels runs like one of 64: its second slice is the first one's values times zero, the outputs of its channels 32 ..
+    // are not stored
+    const bool wide = hd > 32;
+    const uint32_t second = wide ? 32u : 0u;
+    char *keys = reinterpret_cast<char *> (smem), *values = keys + 2 * Stage::BYTES;
+    ActView<COH> Q, Kmat, V, out;
+    Q.init (L.in0, L.N, L.ld0); Kmat.init (L.in1, L.N, L.ld1); V.init (L.fuse_in, L.N, L.fuse_ld_in); out.init (L.out, L.N, L.ld);
+    const float scale = 1.0f / sqrtf ((float)hd);
+    const uint32_t kend = L.masked ? min (S, q0 + (uint32_t)VATTN_BN) : S;
+    // what this thread stages of a block: unit tid % 4 of key tid / 4; channels 4 c4 .. of keys 4 (tid / 16) ..  (rows behind the sequence
+    // and channels behind the head repeat the last ones: such exponentials are zero, such channels are not stored)
+    const uint32_t kr = tid >> 2, ku = tid & 3, vk = tid >> 4, c4 = tid & 15, vc = min (c4, hd / 4 - 1) * 4;
+    float4 kreg[4], vreg[4];
+    auto fetch = [&] (uint32_t k0)
+    {
+        const uint32_t ko = min (b * S + k0 + kr, last) * L.ld1 + tm * hd + ku * 4;
+        kreg[0] = Kmat.ld4 (ko); kreg[1] = Kmat.ld4 (ko + 16);
+        kreg[2] = Kmat.ld4 (ko + second); kreg[3] = Kmat.ld4 (ko + second + 16);
+        #pragma unroll
+        for (uint32_t e = 0; e < 4; e++) vreg[e] = V.ld4 (min (b * S + k0 + 4 * vk + e, last) * L.fuse_ld_in + tm * hd + vc);
+    };
+    const uint32_t qo = min (b * S + q, last) * L.ld0 + tm * hd + unit * 4;
+    float4 qreg[4];
+    qreg[0] = Q.ld4 (qo); qreg[1] = Q.ld4 (qo + 16);
+    if (wide) { qreg[2] = Q.ld4 (qo + 32); qreg[3] = Q.ld4 (qo + 48); }
+    else qreg[2] = qreg[3] = make_float4 (0.f, 0.f, 0.f, 0.f);
+    fetch (0);
+    const split8_t qf[2][1] = {{split8 (qreg[0], qreg[1])}, {split8 (qreg[2], qreg[3])}};
+    floatx4 o[4][1], olo[4][1];
+    #pragma unroll
+    for (int c = 0; c < 4; c++) o[c][0] = olo[c][0] = (floatx4){0.f, 0.f, 0.f, 0.f};
+    float part = 0.f;
+    const float exponent = scale * 1.4426950408889634f;      // exp (scale x) = 2 ^ (exponent x), the hardware's exponential
+    const uint32_t foff = Stage::offset (lane & 15, unit), koff = Stage::offset (kr, ku);
+    // eight fragments one after the other, each fetched while the one before it is multiplied
+    const auto eight = [&] (const char *stages, auto product)
+    {
+        split8_t frag[2];
+        frag[0] = Stage::read (stages, foff);
+        #pragma unroll
+        for (int f = 0; f < 8; f++)
+        {
+            if (f < 7) frag[(f + 1) & 1] = Stage::read (stages + ((f + 1) >> 2) * Stage::BYTES, foff + ((f + 1) & 3) * 16 * 64);
+            product (frag[f & 1], f >> 2, f & 3);
+            __builtin_amdgcn_sched_barrier (SCHED_GROUP_MASK | 2);
+        }
+    };
+    for (uint32_t k0 = 0; k0 < kend; k0 += 64)
+    {
+        #pragma unroll
+        for (int s = 0; s < 2; s++)
+            #pragma unroll
+            for (int term = 0; term < 3; term++) *reinterpret_cast<u32x4 *> (keys + s * Stage::BYTES + term * Stage::PLANE + koff) = take_term (kreg[2 * s], kreg[2 * s + 1]);
+        {
+            // four keys of four channels: half a unit of four rows
+            char *dst = values + (vk >> 3) * Stage::BYTES + ((vk >> 2) & 1u) * 8u;
+            float x[4][4] = {{vreg[0].x, vreg[1].x, vreg[2].x, vreg[3].x}, {vreg[0].y, vreg[1].y, vreg[2].y, vreg[3].y},
+                             {vreg[0].z, vreg[1].z, vreg[2].z, vreg[3].z}, {vreg[0].w, vreg[1].w, vreg[2].w, vreg[3].w}};
+            #pragma unroll
+            for (uint32_t e = 0; e < 4; e++)
+            {
+                char *row = dst + Stage::offset (c4 * 4 + e, vk & 3u);
+                #pragma unroll
+                for (int term = 0; term < 3; term++)
+                {
+                    const uint32_t lo2 = bf16_pair (x[e][0], x[e][1]), hi2 = bf16_pair (x[e][2], x[e][3]);
+                    x[e][0] -= bf16_low (lo2); x[e][1] -= bf16_high (lo2); x[e][2] -= bf16_low (hi2); x[e][3] -= bf16_high (hi2);
+                    *reinterpret_cast<uint2 *> (row + term * Stage::PLANE) = make_uint2 (lo2, hi2);
+                }
+            }
+        }
+        if (k0 + 64 < kend) fetch (k0 + 64);
+        lds_barrier ();
+        floatx4 sc[4][1], slo[4][1];
+        #pragma unroll
+        for (int i = 0; i < 4; i++) sc[i][0] = slo[i][0] = (floatx4){0.f, 0.f, 0.f, 0.f};
+        eight (keys, [&] (const split8_t &f, int s, int i) { split_mfma (f, qf[s], sc[i], slo[i]); });
+        if (k0 + 64 > S || (L.masked && k0 + 63 > q0))
+        {
+            // the block reaches behind the sequence or past a query of the tile
+            #pragma unroll
+            for (int i = 0; i < 4; i++)
+                #pragma unroll
+                for (int v = 0; v < 4; v++)
+                {
+                    const uint32_t key = k0 + BLOCK_N (i, v, lane);
+                    float x = sc[i][0][v] + slo[i][0][v];
+                    if (L.masked && key > q) x = -1e10f;
+                    sc[i][0][v] = key < S ? __builtin_amdgcn_exp2f (x * exponent) : 0.f;
+                }
+        }
+        else
+        {
+            #pragma unroll
+            for (int i = 0; i < 4; i++)
+                #pragma unroll
+                for (int v = 0; v < 4; v++) sc[i][0][v] = __builtin_amdgcn_exp2f ((sc[i][0][v] + slo[i][0][v]) * exponent);
+        }
+        split8_t ef[2][1];
+        #pragma unroll
+        for (int s = 0; s < 2; s++)
+        {
+            const floatx4 a = sc[2 * s][0], b = sc[2 * s + 1][0];
+            part += ((a[0] + a[1]) + (a[2] + a[3])) + ((b[0] + b[1]) + (b[2] + b[3]));
+            ef[s][0] = split8 (make_float4 (a[0], a[1], a[2], a[3]), make_float4 (b[0], b[1], b[2], b[3]));
+        }
+        eight (values, [&] (const split8_t &f, int s, int c) { split_mfma (f, ef[s], o[c], olo[c]); });
+        lds_barrier ();                                  // everyone has read the block
+    }
+    part += __shfl_xor (part, 16, 64);
+    part += __shfl_xor (part, 32, 64);
+    #pragma unroll
+    for (int c = 0; c < 4; c++) o[c][0] += olo[c][0];
+    // (scores that are not finite show in the exponentials' sum or in the outputs)
+    if (__syncthreads_or (sums_not_finite (o) || __any (!(part < INFINITY)))) { single_precision_attention<COH> (layer, tn, tm, smem); return; }
+    if (q < S)
+    {
+        #pragma unroll
+        for (uint32_t c = 0; c < 4; c++)
+            if (c < 2 || wide) out.st4 ((b * S + q) * L.ld + tm * hd + BLOCK_N (c, 0, lane), make_float4 (o[c][0][0] / part, o[c][0][1] / part, o[c][0][2] / part, o[c][0][3] / part));
+    }
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -2520,7 +2665,7 @@ __device__ __forceinline__ bool run_tile (Descriptor descriptor, uint32_t t, boo
         if constexpr ((FEAT & TILES_ATTENTION) != 0)
         {
             ready ();
-            if (L.direct == ASPEN_HIP_ATTENTION_FUSED) tile_fused_attention<COH> (L, tn, tm, smem);
+            if (L.direct == ASPEN_HIP_ATTENTION_FUSED) tile_fused_attention<COH> (L, descriptor.address (), tn, tm, smem);
             else tile_v_attention<COH> (L, tn, tm, smem);
         }
         break;

@@ -203,3 +203,64 @@ def test_products_whose_dropped_terms_add_up(gpu, m, n, k):
         error = np.max(np.abs(product(entry, A, B, np.zeros(m, dtype=np.float32), 0) - exact) / exact)
         print("worst", (m, n, k), error * 2.0 ** 24, flush=True)
         assert error <= (k // 16 * (1 + 2.0 ** -7) + 2) * 2.0 ** -24
+
+
+@pytest.mark.parametrize("mode,flags", [(api.MODE_LAYERS, 0), (api.MODE_DATAFLOW, QUEUE), (api.MODE_DATAFLOW, ORDERED)], ids=["layers", "queue", "ordered"])
+@pytest.mark.parametrize("masked", [False, True], ids=["full", "causal"])
+@pytest.mark.parametrize("hidden,seq", [(64, 1), (128, 63), (128, 64), (64, 65), (128, 130)])
+def test_fused_attention_of_infinite_and_largest_operands(gpu, engine_flags, hidden, seq, masked, mode, flags):
+    """One block of two heads of 32 or 64 channels (a fused tile: 64 queries and 64 keys at a time) over three sequences.  The first
+    is ordinary.  In the second one key has +-3e38 in a channel in which some queries hold the same: scores of -inf, whose
+    exponential is zero, and of +inf, whose is infinite.  In the third one token's values are infinite.  Expected: the layer's
+    formula in 64 bits over the Query, Key and Value the device computed, scores rounded to float; the three-term products
+    and the hardware's exponential (2^-22 of scores of a few units) stay within 1e-5 of the row's largest value."""
+    engine_flags(flags)
+    cfg = M.bert_cfg(1, hidden, 2, hidden)
+    if masked:
+        cfg = cfg.replace("[attention_k]", "[attention_k]\nmasked=1")
+    layers = M.parse_cfg(cfg)
+    a = next(L for L in layers if L["type"] == "attn_k")
+    assert bool(a["masked"]) == masked
+    qi, ki, vi = a["p0"], a["p1"], layers[a["idx"] + 1]["p1"]
+    tens = M.synth_weights(layers, 5, "gpt")
+    w = {(i, k): t for i, k, t in tens}
+    for i in (qi, ki, vi):
+        w[i, "WEIGHT"][:] *= 5
+        w[i, "WEIGHT"][:, :3] = 0
+    c, t, batch = 7, seq // 3, 3
+    w[ki, "WEIGHT"][c] = w[qi, "WEIGHT"][c] = 0
+    w[ki, "BIAS"][c] = w[qi, "BIAS"][c] = 0
+    w[ki, "WEIGHT"][c, 0] = w[qi, "WEIGHT"][c, 1] = 3e38
+    w[vi, "WEIGHT"][5, 2] = 3e38
+    x = M.synth_input(layers, 6, batch, seq, "embeddings").reshape(batch, seq, hidden) * 20
+    x[:, :, :3] = 0
+    x[1, t, 0] = 1
+    x[1, seq // 2:, 1] = -1
+    x[1, -1, 1] = 1 if seq > 1 else -1
+    x[2, t, 2] = 1e30
+    api.lib().aspen_keep_layer_outputs(0)
+    try:
+        net = H.GpuNet(cfg, tens, batch, seq, min_ninst=8, mode=mode)
+        try:
+            assert net.nasm.info(a["idx"] + 1)["fused_attention"] >= 0
+            net.run(np.ascontiguousarray(x, dtype=np.float32))
+            q, k, v = (net.layer(i).reshape(batch, seq, 2, hidden // 2).astype(np.float64) for i in (qi, ki, vi))
+            got = net.layer(a["idx"] + 1).reshape(batch, seq, 2, hidden // 2)
+        finally:
+            net.close()
+    finally:
+        api.lib().aspen_keep_layer_outputs(1)
+    with np.errstate(all="ignore"):
+        scores = np.einsum("bqhc,bkhc->bhqk", q, k).astype(np.float32)
+        if masked:
+            scores = np.where(np.arange(seq)[None, :] > np.arange(seq)[:, None], np.float32(-1e10), scores)
+        e = np.exp((scores * np.float32(1 / np.sqrt(hidden // 2))).astype(np.float64)).transpose(0, 2, 3, 1)[..., None]
+        weighted = e * v[:, None]
+        if masked:      # blocks of 64 keys behind all of a tile's queries are not computed
+            weighted[:, np.arange(seq)[None, :] // 64 > np.arange(seq)[:, None] // 64] = 0
+        want = weighted.sum(2) / e.sum(2)
+    assert np.isinf(v).any() and np.isfinite(want[0]).all()
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isposinf(got), np.isposinf(want)) and np.array_equal(np.isneginf(got), np.isneginf(want))
+    finite = np.isfinite(want)
+    most = np.max(np.abs(np.where(finite, want, 0)), axis=-1, keepdims=True)
+    assert np.max(np.abs(np.where(finite, got, 0) - np.where(finite, want, 0)) / np.maximum(most, 1e-30)) <= 1e-5
