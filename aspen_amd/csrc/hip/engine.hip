@@ -522,8 +522,17 @@ __device__ __forceinline__ void wait_until_ready ()
     if ((a.flags & ASPEN_HIP_FLAG_PROFILE) && threadIdx.x == 0) { const unsigned long long t = wall_clock64 (); s_sched.ticks[5] += t - s_sched.p0; s_sched.p0 = t; }
 }
 
+// Ordered kernels whose only shapes are 64 x 64 and 128 x 32 tiles fit four workgroups per compute unit, 128 registers, and need half the
+// LDS.  Their graphs are bound by latency, which a fourth tile per unit hides: see ORDERED_SMALL.
+static constexpr int ordered_wg_per_cu (unsigned tiles) { return (tiles & (TILES_LARGE | TILES_WIDE | TILES_NARROW | TILES_ATTENTION)) == 0 ? 4 : WG_PER_CU; }
+// LDS of an ordered launch; narrow: the graph has 32 x 32 tiles, which prefetch weights into it
+static constexpr size_t ordered_lds (unsigned tiles, bool narrow)
+{
+    return narrow ? CMAX (GEMM_SMEM_BYTES, NARROW_PF_SMEM_BYTES) : ordered_wg_per_cu (tiles) == 4 ? CMAX (VAR_FLOATS (VAR2_BM, VAR2_BN), VAR_FLOATS (VAR4_BM, VAR4_BN)) * 4 : GEMM_SMEM_BYTES;
+}
+
 template <int COH, unsigned FEAT, bool ORDERED = false>
-__global__ void __launch_bounds__ (WG_THREADS, WG_PER_CU) dataflow_kernel (dataflow_args_t args)
+__global__ void __launch_bounds__ (WG_THREADS, ORDERED ? ordered_wg_per_cu (FEAT) : WG_PER_CU) dataflow_kernel (dataflow_args_t args)
 {
     extern __shared__ __align__ (16) float smem[];
     if (threadIdx.x == 0)
@@ -600,17 +609,23 @@ static const void *const dataflow_kernels[NUM_KERNEL_VARIANTS][2] = {
     {(const void *)dataflow_kernel<1, TILES_CONVNET | TILES_YOLO>, (const void *)dataflow_kernel<2, TILES_CONVNET | TILES_YOLO>},
     {(const void *)dataflow_kernel<1, TILES_ALL>, (const void *)dataflow_kernel<2, TILES_ALL>}};
 
-// Ordered mode (see aspen_hip_run_dataflow), cached loads only: for convolutional networks, for those with weight-streaming
-// layers (VGG-16 at small batches), for transformer graphs, for those with 32 x 32 tiles (a few dozen tokens; on the variant with every tile
-// kind, whose attention tiles spill, BERT-base 1 x 16 took 670 us instead of 600), and with every tile kind.
-enum { ORDERED_CONVNET, ORDERED_TALL, ORDERED_TRANSFORMER, ORDERED_TRANSFORMER_NARROW, ORDERED_ALL, NUM_ORDERED_VARIANTS };
-#define ORDERED_SMEM_BYTES CMAX (GEMM_SMEM_BYTES, NARROW_PF_SMEM_BYTES)       // the narrow tiles' weight prefetch buffers
-static const unsigned ordered_variant_tiles[NUM_ORDERED_VARIANTS] = {TILES_CONVNET | TILES_YOLO | TILES_NARROW, TILES_CONVNET | TILES_TALL,
-    TILES_TRANSFORMER, TILES_TRANSFORMER | TILES_NARROW, TILES_ALL};
+// Ordered mode (see aspen_hip_run_dataflow), cached loads only, smallest first.  Convolutional graphs that are rebuilt for it have
+// no large and no wide tiles: without those the kernel is 69 instead of 122 KB (98 with 32 x 32 tiles; the instruction cache holds
+// 64) and takes 128 registers.  us with the one for all convolutional graphs / that kernel, three workgroups per compute unit / four:
+// ResNet-50 batch 2 567 / 553 (32 x 32 tiles: two per unit), 4 636 / 615 / 595, 11 990 / 951 / 882, YOLO-v3 batch 1 1053 / 1018 / 996, 2 1496 / - / 1378,
+// VGG-16 batch 1 505 / - / 500.
+// Transformer graphs with 32 x 32 tiles (a few dozen tokens) have one because attention spills on the one with every tile
+// kind: BERT-base 1 x 16 670 / 600.
+enum { ORDERED_SMALL, ORDERED_SMALL_NARROW, ORDERED_SMALL_TALL, ORDERED_CONVNET, ORDERED_TALL, ORDERED_TRANSFORMER, ORDERED_TRANSFORMER_NARROW, ORDERED_ALL,
+    NUM_ORDERED_VARIANTS };
+static const unsigned ordered_variant_tiles[NUM_ORDERED_VARIANTS] = {TILES_SMALL_CONVNET | TILES_YOLO, TILES_SMALL_CONVNET | TILES_YOLO | TILES_NARROW,
+    TILES_SMALL_CONVNET | TILES_TALL, TILES_CONVNET | TILES_YOLO | TILES_NARROW, TILES_CONVNET | TILES_TALL, TILES_TRANSFORMER, TILES_TRANSFORMER | TILES_NARROW, TILES_ALL};
+#define ORDERED_KERNEL(tiles) (const void *)dataflow_kernel<2, tiles, true>
 static const void *const ordered_kernels[NUM_ORDERED_VARIANTS] = {
-    (const void *)dataflow_kernel<2, TILES_CONVNET | TILES_YOLO | TILES_NARROW, true>, (const void *)dataflow_kernel<2, TILES_CONVNET | TILES_TALL, true>,
-    (const void *)dataflow_kernel<2, TILES_TRANSFORMER, true>, (const void *)dataflow_kernel<2, TILES_TRANSFORMER | TILES_NARROW, true>,
-    (const void *)dataflow_kernel<2, TILES_ALL, true>};
+    ORDERED_KERNEL (TILES_SMALL_CONVNET | TILES_YOLO), ORDERED_KERNEL (TILES_SMALL_CONVNET | TILES_YOLO | TILES_NARROW), ORDERED_KERNEL (TILES_SMALL_CONVNET | TILES_TALL),
+    ORDERED_KERNEL (TILES_CONVNET | TILES_YOLO | TILES_NARROW), ORDERED_KERNEL (TILES_CONVNET | TILES_TALL), ORDERED_KERNEL (TILES_TRANSFORMER),
+    ORDERED_KERNEL (TILES_TRANSFORMER | TILES_NARROW), ORDERED_KERNEL (TILES_ALL)};
+
 static int ordered_variant (const aspen_hip_graph_t *g)
 {
     int v = 0;
@@ -629,7 +644,11 @@ static unsigned graph_features (const aspen_hip_layer_t *layers, uint32_t num_la
         switch (L.type)
         {
         case CONV_LAYER: case FC_LAYER: case MATMUL_LAYER:
-            if (L.variant == ASPEN_HIP_GEMM_NARROW) { f |= TILES_NARROW; break; }      // (brings its own operand loaders)
+            if (L.variant == ASPEN_HIP_GEMM_NARROW)      // (brings its own operand loaders; gathering for any operand that is not read in place)
+            {
+                f |= TILES_NARROW | (L.direct != ASPEN_HIP_OPERAND_DIRECT ? TILES_GATHER : 0u);
+                break;
+            }
             f |= L.variant == ASPEN_HIP_GEMM_LARGE ? TILES_LARGE : L.variant == ASPEN_HIP_GEMM_WIDE ? TILES_WIDE : L.variant == ASPEN_HIP_GEMM_TALL ? TILES_TALL : TILES_SMALL;
             if (L.direct != ASPEN_HIP_OPERAND_DIRECT) f |= TILES_GATHER;
             if (L.direct == ASPEN_HIP_OPERAND_DENSE3 && L.variant == ASPEN_HIP_GEMM_WIDE) f |= TILES_DENSE_WIDE;
@@ -667,7 +686,7 @@ extern "C" int aspen_hip_init (void)
         for (int coh = 0; coh < 2; coh++)
             CHECK (hipFuncSetAttribute (dataflow_kernels[v][coh], hipFuncAttributeMaxDynamicSharedMemorySize, GEMM_SMEM_BYTES));
     for (int v = 0; v < NUM_ORDERED_VARIANTS; v++)
-        CHECK (hipFuncSetAttribute (ordered_kernels[v], hipFuncAttributeMaxDynamicSharedMemorySize, ORDERED_SMEM_BYTES));
+        CHECK (hipFuncSetAttribute (ordered_kernels[v], hipFuncAttributeMaxDynamicSharedMemorySize, (int)ordered_lds (ordered_variant_tiles[v], (ordered_variant_tiles[v] & TILES_NARROW) != 0)));
     // how many persistent workgroups really fit a compute unit (registers, LDS), per variant: a graph's default grid
     // follows the variant it runs on
     g_resident_wg = WG_PER_CU;
@@ -1545,25 +1564,21 @@ extern "C" int aspen_hip_run_dataflow (aspen_hip_graph_t *g, uint32_t workgroups
     // (a static assignment in index order only terminates when every tile's parents have smaller indices: graph_parallelism
     // reports 1e30 for a graph that is not listed that way)
     if (!g->cached_loads || xcd_queues || g->num_ninst > (1u << 20) || g->parallelism > 1e29) ordered = false;
-    size_t ordered_smem = ORDERED_SMEM_BYTES;
-    const int ov = ordered_variant (g);
+    const int ov = ordered_variant (g), narrow = (g->features & TILES_NARROW) != 0;
+    const size_t ordered_smem = ordered_lds (ordered_variant_tiles[ov], narrow);
     if (ordered)
     {
         // tiles are assigned to workgroups beforehand: every workgroup of the grid must be running
-        // (graphs without 32 x 32 tiles need no weight prefetch buffers: their workgroups take the LDS of any other tile, and
-        // three instead of two fit a compute unit)
         static int fits[NUM_ORDERED_VARIANTS][2];
         static bool fits_known[NUM_ORDERED_VARIANTS][2];
-        const int small_lds = (g->features & TILES_NARROW) == 0;
-        if (!fits_known[ov][small_lds])
+        if (!fits_known[ov][narrow])
         {
             int o = 0;
-            CHECK (hipOccupancyMaxActiveBlocksPerMultiprocessor (&o, ordered_kernels[ov], WG_THREADS, small_lds ? GEMM_SMEM_BYTES : ORDERED_SMEM_BYTES));
-            fits[ov][small_lds] = o * g_num_cu;
-            fits_known[ov][small_lds] = true;
+            CHECK (hipOccupancyMaxActiveBlocksPerMultiprocessor (&o, ordered_kernels[ov], WG_THREADS, ordered_smem));
+            fits[ov][narrow] = o * g_num_cu;
+            fits_known[ov][narrow] = true;
         }
-        const int fit = fits[ov][small_lds];
-        ordered_smem = small_lds ? GEMM_SMEM_BYTES : ORDERED_SMEM_BYTES;
+        const int fit = fits[ov][narrow];
         if (fit < 1) ordered = false;
         else
         {

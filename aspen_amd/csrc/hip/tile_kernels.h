@@ -543,6 +543,7 @@ enum : unsigned
     TILES_DENSE_WIDE = 2048u,   // the dense three-channel operand under the 64 x 128 shape (the host library's graphs take 64 x 64 for it)
     TILES_ALL = 4095u,
     TILES_CONVNET = TILES_GATHER | TILES_LARGE | TILES_WIDE | TILES_SMALL | TILES_POOL | TILES_RESIDUAL,
+    TILES_SMALL_CONVNET = TILES_GATHER | TILES_SMALL | TILES_POOL | TILES_RESIDUAL,
     TILES_TRANSFORMER = TILES_SMALL | TILES_ATTENTION | TILES_NORM | TILES_RESIDUAL
 };
 template <int BM, int BN, int WM, int WN, class ALoader, class BLoader>
@@ -2338,7 +2339,7 @@ __device__ __forceinline__ void narrow_gather_finish (const aspen_hip_layer_t &L
 // parents have finished.  Slices beyond PF (and all slices when PF = 0) go through registers, two in flight.
 #define NARROW_PF_SLICES 3
 #define NARROW_PF_SMEM_BYTES (4 * NARROW_PF_SLICES * SPLIT_SLICE_BYTES)
-template <int COH, int PF, class Descriptor, class Ready>
+template <int COH, int PF, bool GATHER, class Descriptor, class Ready>
 __device__ __forceinline__ float4 narrow_mainloop (const aspen_hip_layer_t &L, Descriptor descriptor, uint32_t tn, uint32_t tm, int kbase, int kiters,
     float *smem, Ready ready)
 {
@@ -2352,7 +2353,7 @@ __device__ __forceinline__ float4 narrow_mainloop (const aspen_hip_layer_t &L, D
     w1r = w0r;
     ActView<COH> in;
     in.init (descriptor ().in0, L.in0_columns, L.ld0);
-    const bool direct = L.direct == ASPEN_HIP_OPERAND_DIRECT;
+    const bool direct = !GATHER || L.direct == ASPEN_HIP_OPERAND_DIRECT;
     // activation operand: DIRECT = the parent's column; else the top-left input pixel of output position n and the
     // tap / channel the first slice starts at (stepped from there, as StepLoader does)
     int32_t bbase[2], ih0[2] = {0, 0}, iw0[2] = {0, 0};
@@ -2487,7 +2488,7 @@ __device__ __forceinline__ float4 narrow_mainloop (const aspen_hip_layer_t &L, D
         #pragma unroll
         for (int j = 0; j < 2; j++)
         {
-            const floatx8 x = single_precision_block<false, COH, true, false> (descriptor.address (), 2 * tm + j, tn * VAR3_BN + row, first, cnt);
+            const floatx8 x = single_precision_block<false, COH, GATHER, false> (descriptor.address (), 2 * tm + j, tn * VAR3_BN + row, first, cnt);
             #pragma unroll
             for (int v = 0; v < 8; v++) { const float y = acc[v >> 2][j][v & 3]; acc[v >> 2][j][v & 3] = fabsf (y) < INFINITY ? y : x[v]; }
         }
@@ -2509,7 +2510,7 @@ __device__ __forceinline__ float4 narrow_mainloop (const aspen_hip_layer_t &L, D
 }
 
 // One narrow tile; returns false for a split-K member that was not the last of its group.
-template <int COH, int PF, class Descriptor, class Arrivals, class Ready>
+template <int COH, int PF, bool GATHER, class Descriptor, class Arrivals, class Ready>
 __device__ __forceinline__ bool narrow_tile (const aspen_hip_layer_t &L, Descriptor descriptor, uint32_t t, uint32_t tn, uint32_t tm, int slice, uint32_t group,
     float *smem, Arrivals arrivals, Ready ready)
 {
@@ -2539,7 +2540,7 @@ __device__ __forceinline__ bool narrow_tile (const aspen_hip_layer_t &L, Descrip
             have_sc = true;
         }
     };
-    const float4 sum = narrow_mainloop<COH, PF> (L, descriptor, tn, tm, kbase, kiters, smem, ready_then_shortcut);
+    const float4 sum = narrow_mainloop<COH, PF, GATHER> (L, descriptor, tn, tm, kbase, kiters, smem, ready_then_shortcut);
     if (COH) tile_phase_lap (9);
     if (slice < 0)
     {
@@ -2619,7 +2620,7 @@ __device__ __forceinline__ bool run_tile (Descriptor descriptor, uint32_t t, boo
         c4_log2 = 4; bn = VAR2_BN;
         if constexpr ((FEAT & TILES_NARROW) != 0)
         {
-            if (L.variant == ASPEN_HIP_GEMM_NARROW) return narrow_tile<COH, NARROW_PF> (L, descriptor, t, tn, tm, slice, group, smem, arrivals, ready);
+            if (L.variant == ASPEN_HIP_GEMM_NARROW) return narrow_tile<COH, NARROW_PF, (FEAT & TILES_GATHER) != 0> (L, descriptor, t, tn, tm, slice, group, smem, arrivals, ready);
         }
         if ((FEAT & TILES_LARGE) && L.variant == ASPEN_HIP_GEMM_LARGE)
         {
