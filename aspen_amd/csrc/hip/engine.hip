@@ -524,7 +524,10 @@ __device__ __forceinline__ void wait_until_ready ()
 
 // Ordered kernels whose only shapes are 64 x 64 and 128 x 32 tiles fit four workgroups per compute unit, 128 registers, and need half the
 // LDS.  Their graphs are bound by latency, which a fourth tile per unit hides: see ORDERED_SMALL.
-static constexpr int ordered_wg_per_cu (unsigned tiles) { return (tiles & (TILES_LARGE | TILES_WIDE | TILES_NARROW | TILES_ATTENTION)) == 0 ? 4 : WG_PER_CU; }
+static constexpr int ordered_wg_per_cu (unsigned tiles)
+{
+    return (tiles & TILES_NARROW) && tiles != TILES_ALL ? 2 : (tiles & (TILES_LARGE | TILES_WIDE | TILES_ATTENTION)) == 0 ? 4 : WG_PER_CU;
+}
 // LDS of an ordered launch; narrow: the graph has 32 x 32 tiles, which prefetch weights into it
 static constexpr size_t ordered_lds (unsigned tiles, bool narrow)
 {
@@ -619,11 +622,11 @@ static const void *const dataflow_kernels[NUM_KERNEL_VARIANTS][2] = {
 enum { ORDERED_SMALL, ORDERED_SMALL_NARROW, ORDERED_SMALL_TALL, ORDERED_CONVNET, ORDERED_TALL, ORDERED_TRANSFORMER, ORDERED_TRANSFORMER_NARROW, ORDERED_ALL,
     NUM_ORDERED_VARIANTS };
 static const unsigned ordered_variant_tiles[NUM_ORDERED_VARIANTS] = {TILES_SMALL_CONVNET | TILES_YOLO, TILES_SMALL_CONVNET | TILES_YOLO | TILES_NARROW,
-    TILES_SMALL_CONVNET | TILES_TALL, TILES_CONVNET | TILES_YOLO | TILES_NARROW, TILES_CONVNET | TILES_TALL, TILES_TRANSFORMER, TILES_TRANSFORMER | TILES_NARROW, TILES_ALL};
+    TILES_SMALL_CONVNET | TILES_TALL, TILES_CONVNET | TILES_YOLO, TILES_CONVNET | TILES_TALL, TILES_TRANSFORMER, TILES_TRANSFORMER | TILES_NARROW, TILES_ALL};
 #define ORDERED_KERNEL(tiles) (const void *)dataflow_kernel<2, tiles, true>
 static const void *const ordered_kernels[NUM_ORDERED_VARIANTS] = {
     ORDERED_KERNEL (TILES_SMALL_CONVNET | TILES_YOLO), ORDERED_KERNEL (TILES_SMALL_CONVNET | TILES_YOLO | TILES_NARROW), ORDERED_KERNEL (TILES_SMALL_CONVNET | TILES_TALL),
-    ORDERED_KERNEL (TILES_CONVNET | TILES_YOLO | TILES_NARROW), ORDERED_KERNEL (TILES_CONVNET | TILES_TALL), ORDERED_KERNEL (TILES_TRANSFORMER),
+    ORDERED_KERNEL (TILES_CONVNET | TILES_YOLO), ORDERED_KERNEL (TILES_CONVNET | TILES_TALL), ORDERED_KERNEL (TILES_TRANSFORMER),
     ORDERED_KERNEL (TILES_TRANSFORMER | TILES_NARROW), ORDERED_KERNEL (TILES_ALL)};
 
 static int ordered_variant (const aspen_hip_graph_t *g)

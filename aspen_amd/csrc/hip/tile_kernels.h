@@ -2425,6 +2425,10 @@ __device__ __forceinline__ float4 narrow_mainloop (const aspen_hip_layer_t &L, D
                     __builtin_amdgcn_raw_ptr_buffer_load_lds (wr, (__attribute__ ((address_space (3))) void *)(mine + (i * 6 + q) * 256), 16,
                         (int)(lane * 16u), (int)((uint32_t)(first + i) * SPLIT_SLICE_BYTES + (uint32_t)q * 1024u), 0, 0);
             }
+        // the two slices behind those: weights now, activations behind the others' (a wavefront that asked for them when it was through
+        // with the first three waited for memory once more)
+        if (PF < cnt) w0r.load (first + PF);
+        if (PF + 1 < cnt) w1r.load (first + PF + 1);
         ready ();
         // one straight-line body per number of prefetched slices (wave-uniform): every activation request is issued
         // before the first fragment is read back, so the slices' trips to memory overlap
@@ -2434,6 +2438,11 @@ __device__ __forceinline__ float4 narrow_mainloop (const aspen_hip_layer_t &L, D
             float4 bq[C][4];
             #pragma unroll
             for (int i = 0; i < C; i++) load_b (i, bq[i]);
+            if constexpr (C == PF)
+            {
+                if (PF < cnt) load_b (PF, b0);
+                if (PF + 1 < cnt) load_b (PF + 1, b1);
+            }
             #pragma unroll
             for (int i = 0; i < C; i++)
             {
@@ -2453,8 +2462,6 @@ __device__ __forceinline__ float4 narrow_mainloop (const aspen_hip_layer_t &L, D
         else if (pre == 2) body (std::integral_constant<int, 2> ());
         else if (pre == 1) body (std::integral_constant<int, 1> ());
         done = min (cnt, PF);
-        if (done < cnt) { w0r.load (first + done); load_b (done, b0); }
-        if (done + 1 < cnt) { w1r.load (first + done + 1); load_b (done + 1, b1); }
     }
     else
     {
