@@ -1375,9 +1375,9 @@ static aspen_hip_graph_t *graph_create (const aspen_hip_layer_t *layers, uint32_
         for (int i = NUM_KERNEL_VARIANTS - 2; i >= 0 && !all_tiles; i--) if ((g->features & ~kernel_variant_tiles[i]) == 0) g->variant = i;
         const uint32_t resident = (uint32_t)g_variant_wg[g->variant][g->cached_loads ? 1 : 0];      // of the variant this graph runs on
         uint32_t per_cu = resident;
-        // ready-queue runs with one / two / three workgroups per unit on 256 units, us: ResNet-50 batch 1 (average parallelism 92) 629 / 676 /
-        // 714, BERT-base 3 x 75 (197) 1269 / 1315 / 1354, ResNet-50 batch 4 (338) 891 / 824 / 839, YOLO-v3 batch 1 (419) 1575 / 1392 /
-        // 1400, BERT-base 8 x 128 (533) 2228 / 1770 / 1837, ResNet-50 batch 8 (645) 1357 / 976 / 933, GPT-2 4 x 512 (878) 4095 / 3179 / 3102
+        // ready-queue runs with one / two / three workgroups per unit on 256 units, us: ResNet-50 batch 1 (average parallelism 92) 640 / 677 /
+        // 705, BERT-base 3 x 75 (197) 1212 / 1228 / 1257, ResNet-50 batch 4 (338) 839 / 783 / 798, YOLO-v3 batch 1 (419) 1484 / 1339 /
+        // 1308, BERT-base 8 x 128 (533) 2232 / 1665 / 1682, ResNet-50 batch 8 (645) 1300 / 941 / 899, GPT-2 4 x 512 (878) 4104 / 2929 / 2742
         if (par < 2.3 * g_num_cu) per_cu = par < g_num_cu ? 1u : 2u;
         if (per_cu > resident) per_cu = resident;
         g->default_workgroups = per_cu * (uint32_t)g_num_cu;
@@ -1585,9 +1585,9 @@ extern "C" int aspen_hip_run_dataflow (aspen_hip_graph_t *g, uint32_t workgroups
         if (fit < 1) ordered = false;
         else
         {
-            // by default all that fit: two or three tiles of a unit compute, wait for their parents or are prepared.  Two / three per
-            // unit, us: ResNet-50 batch 2 (estimated parallelism 179) 628 / 626, 4 (338) 686 / 676, 6 (489) 809 / 746, YOLO-v3 batch 1 (419)
-            // 1171 / 1096, VGG-16 batch 1 (728) 598 / 514
+            // by default all that fit: two to four tiles of a unit compute, wait for their parents or are prepared.  Two / three / four
+            // per unit, us: ResNet-50 batch 4 (estimated parallelism 338) 620 / 614 / 595, 6 (489) 746 / 690 / 674, YOLO-v3 batch 1 (419)
+            // 1081 / 1016 / 997, VGG-16 batch 1 (728) 586 / 512 / 498, BERT-base 8 x 128 (533) 1521 / 1397 (three fit)
             if (workgroups_requested == 0) workgroups = (uint32_t)fit;
             if (workgroups > (uint32_t)fit) workgroups = (uint32_t)fit;
         }
@@ -1599,14 +1599,16 @@ extern "C" int aspen_hip_run_dataflow (aspen_hip_graph_t *g, uint32_t workgroups
         if (!g->d_dep_spread) return -1;
     }
     uint32_t nq_mask = (xcd_queues && workgroups % NUM_QUEUES == 0) ? (NUM_QUEUES >> nq_shift) - 1u : 0u;
-    // By default a graph that fills the device (every compute unit holds as many workgroups as fit) runs on TWO queues,
-    // one per half of the XCDs: tiles that read the same activations then meet in one of four L2s instead of eight.  One / two /
-    // four / eight queues, us: ResNet-50 batch 32 2166 / 2111 / 2074 / 2117, VGG-16 batch 32 5507 / 5497 / 5487 / 5589, YOLO-v3
-    // batch 8 4161 / 4110 / 4108 / 4145, ResNet-50 + VGG-16 4250 / 4220 / 4212 / 4330.  Smaller grids keep one queue: their runs
+    // By default a graph that fills the device (every compute unit holds as many workgroups as fit) runs on FOUR queues,
+    // one per pair of XCDs: tiles that read the same activations then meet in one of two L2s instead of eight.  One / two /
+    // four / eight queues, us: ResNet-50 batch 32 2023 / 1967 / 1951 / 1909, VGG-16 batch 32 5176 / 5149 / 5124 / 5137, YOLO-v3
+    // batch 8 3937 / 3844 / 3819 / 3818, ResNet-50 + VGG-16 4000 / 3910 / 3887 / 3955 (eight cannot balance two networks).  Two / four on
+    // another box: ResNet-50 batch 20 1440 / 1430, 24 1667 / 1654, 32 2014 / 1985, YOLO-v3 batch 4 2264 / 2224, 8 3847 / 3837, ResNet-50 +
+    // VGG-16 3924 / 3942, BERT-base 4 x 512 2814 / 2802, GPT-2 16 x 128 2558 / 2559.  Smaller grids keep one queue: their runs
     // are bound by dependency chains, and every restriction on who may take a ready tile lengthens those.
     if (!xcd_queues && !one_queue_env && !ordered && workgroups % NUM_QUEUES == 0
         && workgroups >= (uint32_t)g_variant_wg[g->variant][g->cached_loads ? 1 : 0] * (uint32_t)g_num_cu)
-    { nq_shift = 2u; nq_mask = (NUM_QUEUES >> nq_shift) - 1u; }
+    { nq_shift = 1u; nq_mask = (NUM_QUEUES >> nq_shift) - 1u; }
     queue_counts_t counts;
     if (nq_mask && g->root_shift != nq_shift)
     {

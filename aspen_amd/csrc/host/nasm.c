@@ -717,7 +717,7 @@ static double nasm_parallelism (const nasm_t *nasm)
 #define CHAIN_BOUND_KITERS_CAP 48
 #define ORDERED_KITERS_CAP 24
 #define LATENCY_BOUND_BELOW 128.0
-#define ORDERED_VISION_BELOW 1100.0
+#define ORDERED_VISION_BELOW 1160.0
 static nasm_t *create_nasm (aspen_dnn_t *dnn, unsigned int min_ninst, unsigned int batch, unsigned int seq)
 {
     const char *e = getenv ("ASPEN_GPU_MAX_KITERS");            /* experiments: fixed cap, 0 = none */
@@ -729,8 +729,8 @@ static nasm_t *create_nasm (aspen_dnn_t *dnn, unsigned int min_ninst, unsigned i
     if (parallelism >= CHAIN_BOUND_BELOW)
     {
         /* (convolutional graphs a little above the limit keep their tiles but still run better in the ordered mode,
-           ordered / queue in us: VGG-16 batch 2, 1052: 688 / 701; from ResNet-50 batch 14, 1104, on the queue wins: 1226 / 1185,
-           batch 16, 1186: 1342 / 1258, YOLO-v3 batch 3, 1142: 2025 / 1933; VGG-16 batch 4, 1246: 1005 / 1000) */
+           ordered / queue in us: VGG-16 batch 2, 1052: 652 / 686, ResNet-50 batch 14, 1104: 1064 / 1156, YOLO-v3 batch 3, 1142:
+           1741 / 1852; from ResNet-50 batch 16, 1186, on the queue wins: 1262 / 1206; VGG-16 batch 4, 1246: 965 / 964) */
         if (seq == 0 && parallelism < ORDERED_VISION_BELOW) nasm->ordered_pref = 1;
         return nasm;
     }
