@@ -1968,7 +1968,7 @@ __device__ __forceinline__ void tile_v_attention (const aspen_hip_layer_t &L, ui
             }
 }
 
-// Fused attention in single precision throughout, for tiles whose sums are not finite (see tile_fused_attention, which calls it
+// Fused attention in single precision throughout, for tiles whose sums are not finite or too small (see tile_fused_attention, which calls it
 // and says what a tile computes): the exponentials of a key block go to LDS in the layout of an activation operand (row =
 // query, K axis = key), the transposed values are staged next to them.  A real function: it runs in the place of a tile.
 template <int COH>
@@ -2205,8 +2205,17 @@ __device__ __forceinline__ void tile_fused_attention (const aspen_hip_layer_t &L
     part += __shfl_xor (part, 32, 64);
     #pragma unroll
     for (int c = 0; c < 4; c++) o[c][0] += olo[c][0];
-    // (scores that are not finite show in the exponentials' sum or in the outputs)
-    if (__syncthreads_or (sums_not_finite (o) || __any (!(part < INFINITY)))) { single_precision_attention<COH> (layer, tn, tm, smem); return; }
+    // Scores of +inf or NaN show in the exponentials' sum or in the outputs (one of -inf has an exponential of zero either way).
+    // Terms below 2^-133 do not exist, so an exponential below 2^-110 or such a value enters with an error of up to 2^-134: too
+    // much for a row whose exponentials are all that small (scaled scores below -76: 2.5e-3 of the result at -86) and for
+    // results below 2^-110.  What passes is within 2^-24 of the row's largest value (below 2^100, as queries and keys have to be).
+    const float least = 0x1p-110f * fmaxf (part, 1.f);
+    bool again = !(part < INFINITY) || (part > 0.f && part < 0x1p-110f * (float)S);
+    #pragma unroll
+    for (int c = 0; c < 4; c++)
+        #pragma unroll
+        for (int v = 0; v < 4; v++) again |= o[c][0][v] != 0.f && fabsf (o[c][0][v]) < least;
+    if (__syncthreads_or (sums_not_finite (o) || __any (again))) { single_precision_attention<COH> (layer, tn, tm, smem); return; }
     if (q < S)
     {
         #pragma unroll

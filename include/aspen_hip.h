@@ -171,7 +171,9 @@ int aspen_hip_copy (void *dst, const void *src, size_t bytes);
 /* Convolutions, fully connected and matmul layers and the plain products below sum in single precision over operands split
    into three bfloat16 terms.  Range: float's own.  Infinities, NaNs and sums beyond the largest float come out as in float
    arithmetic (RELU and LEAKY_RELU, x > 0 ? x : ..., make a NaN 0 and keep it, as the reference's do); an operand below 2^-110
-   in magnitude enters with an absolute error of up to 2^-134. */
+   in magnitude enters with an absolute error of up to 2^-134.  Fused attention multiplies in the same way, but forms tiles
+   whose exponentials or results are that small in single precision: its queries and keys have the two limits of a contraction's
+   operands, its exponentials and values none as long as the values stay below 2^100. */
 /* ---- weights --------------------------------------------------------------------------------- */
 /* Device copy of a contraction layer's weights in the order the kernels read them, from M rows of Kp floats on the host
    (Kp a multiple of 32; K order as for aspen_hip_layer_t.weight).  raw = 0: each float as three bfloat16 terms that add up to it exactly (6

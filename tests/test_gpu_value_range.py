@@ -264,3 +264,66 @@ def test_fused_attention_of_infinite_and_largest_operands(gpu, engine_flags, hid
     finite = np.isfinite(want)
     most = np.max(np.abs(np.where(finite, want, 0)), axis=-1, keepdims=True)
     assert np.max(np.abs(np.where(finite, got, 0) - np.where(finite, want, 0)) / np.maximum(most, 1e-30)) <= 1e-5
+
+
+@pytest.mark.parametrize("mode,flags", [(api.MODE_LAYERS, 0), (api.MODE_DATAFLOW, QUEUE), (api.MODE_DATAFLOW, ORDERED)], ids=["layers", "queue", "ordered"])
+@pytest.mark.parametrize("masked", [False, True], ids=["full", "causal"])
+@pytest.mark.parametrize("hidden,seq", [(64, 1), (128, 16), (128, 64), (64, 65), (128, 130)])
+def test_fused_attention_of_small_exponentials(gpu, engine_flags, hidden, seq, masked, mode, flags):
+    """Rows whose exponentials are all small: one block of two heads of 32 or 64 channels over five sequences whose scaled scores
+    are s = -5, -76, -80, -84 and -86 (exponentials of 2^-7 ... 2^-124; float's smallest is 2^-126).  In the first head the
+    scores of a sequence are equal (one channel of the queries and keys is not zero), so that its results are means of the
+    values, whatever the exponentials' own error: within S + 3 roundings of 2^-24 (the sums, the quotient, what the terms leave
+    out) of the row's largest value.  In the second they vary by some tenths: a score of 86 sqrt (hd) has an error of hd 2^-24 of
+    its products' magnitudes and the exponent two roundings of 2^-24 of 125, together less than 2e-4 of an exponential.  A
+    sixth sequence has ordinary scores and values of 1e-37 (the products
+    that make them lose low bits, which is no matter here)."""
+    engine_flags(flags)
+    cfg = M.bert_cfg(1, hidden, 2, hidden)
+    if masked:
+        cfg = cfg.replace("[attention_k]", "[attention_k]\nmasked=1")
+    layers = M.parse_cfg(cfg)
+    a = next(L for L in layers if L["type"] == "attn_k")
+    qi, ki, vi = a["p0"], a["p1"], layers[a["idx"] + 1]["p1"]
+    tens = M.synth_weights(layers, 5, "gpt")
+    w = {(i, k): t for i, k, t in tens}
+    hd, batch = hidden // 2, 6
+    for i in (qi, ki, vi):
+        w[i, "WEIGHT"][:, :2] = 0
+        w[i, "BIAS"][:] = 0
+        if i != vi:
+            w[i, "WEIGHT"][:hd] = 0
+            w[i, "WEIGHT"][hd:] *= 5
+            w[i, "WEIGHT"][7] = w[i, "WEIGHT"][hd + 7] = 0
+            w[i, "WEIGHT"][7, int(i == ki)] = w[i, "WEIGHT"][hd + 7, int(i == ki)] = 1
+    x = M.synth_input(layers, 6, batch, seq, "embeddings").reshape(batch, seq, hidden) * 20
+    scaled = [-5.0, -76.0, -80.0, -84.0, -86.0, 0.0]
+    x[:, :, 0] = np.array(scaled)[:, None] * np.sqrt(hd) / 8
+    x[:, :, 1] = 8
+    x[5] = 0
+    x[5, :, 2:] = M.synth_input(layers, 7, 1, seq, "embeddings").reshape(seq, hidden)[:, 2:] * 1e-34
+    api.lib().aspen_keep_layer_outputs(0)
+    try:
+        net = H.GpuNet(cfg, tens, batch, seq, min_ninst=8, mode=mode)
+        try:
+            assert net.nasm.info(a["idx"] + 1)["fused_attention"] >= 0
+            net.run(np.ascontiguousarray(x, dtype=np.float32))
+            q, k, v = (net.layer(i).reshape(batch, seq, 2, hd).astype(np.float64) for i in (qi, ki, vi))
+            got = net.layer(a["idx"] + 1).reshape(batch, seq, 2, hd)
+        finally:
+            net.close()
+    finally:
+        api.lib().aspen_keep_layer_outputs(1)
+    assert np.isfinite(got).all()
+    worst = np.zeros((batch, 2))
+    for b in range(batch):
+        for h in range(2):
+            scores = q[b, :, h] @ k[b, :, h].T / np.sqrt(hd)
+            assert np.abs(scores - scaled[b]).max() <= (1e-5 * abs(scaled[b]) if h == 0 else 1.0)
+            if masked:
+                scores = np.where(np.arange(seq)[None, :] > np.arange(seq)[:, None], -np.inf, scores)
+            e = np.exp(scores)
+            want = e @ v[b, :, h] / e.sum(-1, keepdims=True)
+            worst[b, h] = np.max(np.abs(got[b, :, h] - want) / np.max(np.abs(v[b, :, h])))
+    print("worst", (hidden, seq, masked), worst.tolist(), flush=True)
+    assert np.all(worst[:, 0] <= (seq + 3) * 2.0 ** -24) and np.all(worst[:, 1] <= 2e-4)
