@@ -647,6 +647,7 @@ static unsigned graph_features (const aspen_hip_layer_t *layers, uint32_t num_la
         switch (L.type)
         {
         case CONV_LAYER: case FC_LAYER: case MATMUL_LAYER:
+            if (L.norm_fold || L.fuse_norm_stats) f |= TILES_NORM;       // (the norm itself has no tiles then)
             if (L.variant == ASPEN_HIP_GEMM_NARROW)      // (brings its own operand loaders; gathering for any operand that is not read in place)
             {
                 f |= TILES_NARROW | (L.direct != ASPEN_HIP_OPERAND_DIRECT ? TILES_GATHER : 0u);

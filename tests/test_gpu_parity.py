@@ -386,6 +386,42 @@ def test_folded_layernorm_matches_oracle(gpu, engine_flags, monkeypatch, name, m
         api.lib().aspen_keep_layer_outputs(1)
 
 
+NORM_WITHOUT_ATTENTION = {
+    "matmul": "[layernorm]\nM=128\n\n[matmul]\nM=192\nactivation=gelu\n\n",
+    "shortcut": "[layernorm]\nM=128\n\n[matmul]\nM=192\nactivation=gelu\n\n[matmul]\nM=128\n\n[shortcut]\nfrom=-3\nM=128\n\n[matmul]\nM=64\n\n",
+}
+
+
+@pytest.mark.parametrize("mode,flags", [(api.MODE_LAYERS, QUEUE), (api.MODE_DATAFLOW, QUEUE), (api.MODE_DATAFLOW, ORDERED)], ids=["layers", "dataflow", "dataflow-ordered"])
+@pytest.mark.parametrize("name", list(NORM_WITHOUT_ATTENTION))
+def test_folded_layernorm_without_attention(gpu, engine_flags, monkeypatch, name, mode, flags):
+    """The same in a graph that has no other layer of a transformer and no layer norm with tiles of its own: the kernel it runs on
+    has to be one that folds."""
+    from oracle import cpu
+    engine_flags(flags)
+    monkeypatch.setenv("ASPEN_GPU_NARROW_TILES", "0")
+    cfg = "[net]\nM=128\nheight=1\nfilters=128\n\n[matmul]\nM=128\n\n" + NORM_WITHOUT_ATTENTION[name]
+    layers = M.parse_cfg(cfg)
+    tens, batch, seq = M.synth_weights(layers, 23, "gpt"), 3, 37
+    x = M.synth_input(layers, 23, batch, seq, "embeddings") * 10 + np.float32(0.5)
+    outs = cpu.run_network(layers, tens, x, batch, seq)
+    api.lib().aspen_keep_layer_outputs(0)
+    try:
+        net = H.GpuNet(cfg, tens, batch, seq, min_ninst=16, mode=mode)
+        try:
+            infos = [net.nasm.info(l) for l in range(net.nasm.num_ldata)]
+            assert infos[3]["folded_norm"] == 2 and infos[2]["num_ninst"] == 0
+            net.run(x.astype(np.float32))
+            for l in range(1, net.nasm.num_ldata):
+                if not infos[l]["discarded"]:
+                    err = H.rel_l2(net.layer(l), outs[l])
+                    assert err <= H.REL_L2_TOL, f"layer {l} ({layers[l]['type']}): rel L2 {err:.3g}"
+        finally:
+            net.close()
+    finally:
+        api.lib().aspen_keep_layer_outputs(1)
+
+
 def test_results_in_the_callers_dimension_order(gpu):
     """dse_get_ldata_result permutes a layer's native tensor into the order the caller names (reference
     get_ldata_output, src/apu.c:227-297): matrices of a transformer are (BATCH, MAT_N, MAT_M), attention
