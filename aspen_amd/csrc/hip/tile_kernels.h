@@ -88,23 +88,24 @@ __device__ __forceinline__ float gld1 (const float *p) { return *(const float __
 //      shared by two producer tiles (the host checks strides and tile heights): a line is first
 //      fetched after its only producer has finished, every element is written once per launch, and
 //      the caches start a launch invalidated, so a cached line can never be stale.
-// Offsets are in floats from the start of the matrix.  In modes 1 and 2 the buffer descriptor bounds-checks
-// them in hardware (out-of-range loads return 0, out-of-range stores are dropped); mode 0 relies on the slack
+// Offsets are in floats from the start of the matrix.  In modes 1 and 2 (and of mode 0 in ld4_if) the buffer descriptor bounds-checks
+// them in hardware (out-of-range loads return 0, out-of-range stores are dropped); mode 0 else relies on the slack
 // every allocation carries for the few floats an edge tile reads past a row.
 #define CPOL_SC1 16
 template <int COH> struct ActView
 {
     // COH != 0: buffer descriptor.  COH == 0: uniform base address for global loads / stores with 32-bit
     // offsets (measured: lower latency than buffer instructions, which counts when a single image runs
-    // through one launch per layer; 64-bit pointers per row instead cost that kernel enough registers
-    // to spill the weight pointers into the middle of its first loads).
+    // through one launch per layer: ResNet-50 batch 1 512 against 525 us, and transformers 1 %; 64-bit pointers per row instead cost
+    // that kernel enough registers to spill the weight pointers into the middle of its first loads), but for loads that may be
+    // left out, see ld4_if.
     __amdgpu_buffer_rsrc_t rsrc;
     char __attribute__ ((address_space (1))) *base;
     static constexpr int LOAD_POLICY = COH == 1 ? CPOL_SC1 : 0, STORE_POLICY = COH ? CPOL_SC1 : 0;
     __device__ __forceinline__ void init (const float *p, uint32_t columns, uint32_t ld)
     {
-        if (COH) rsrc = __builtin_amdgcn_make_buffer_rsrc ((void *)p, 0, (int)(columns * ld * 4u + 256u), 0x00020000);
-        else base = (char __attribute__ ((address_space (1))) *)p;
+        rsrc = __builtin_amdgcn_make_buffer_rsrc ((void *)p, 0, (int)(columns * ld * 4u + 256u), 0x00020000);
+        if (!COH) base = (char __attribute__ ((address_space (1))) *)p;
     }
     __device__ __forceinline__ float4 ld4 (uint32_t off) const
     {
@@ -112,12 +113,13 @@ template <int COH> struct ActView
         const floatx4 x = *(const floatx4 __attribute__ ((address_space (1))) *)(base + off * 4u);
         return make_float4 (x[0], x[1], x[2], x[3]);
     }
-    // ok ? ld4 (off) : zeros.  With a buffer descriptor the choice is made on the offset (one past anything the
-    // descriptor covers reads as zeros): no branch around the load, so a K loop that uses it stays one basic block.
+    // ok ? ld4 (off) : zeros.  The choice is made on the offset (one past anything the descriptor covers reads as zeros): no
+    // branch around the load, so a K loop that uses it stays one basic block.  One launch per layer, with a branch / this way:
+    // VGG-16 batch 32 7250 / 5205 us, ResNet-50 batch 32 2860 / 2595, YOLO-v3 batch 8 4530 / 4370 (the branch splits the matrix instructions' groups,
+    // which are placed by hand, and the loop's head then waits for every request in flight).
     __device__ __forceinline__ float4 ld4_if (uint32_t off, bool ok) const
     {
-        if (COH) return __builtin_bit_cast (float4, __builtin_amdgcn_raw_buffer_load_b128 (rsrc, ok ? (int)(off * 4u) : (int)0xfffffff0u, 0, LOAD_POLICY));
-        return ok ? ld4 (off) : make_float4 (0.f, 0.f, 0.f, 0.f);
+        return __builtin_bit_cast (float4, __builtin_amdgcn_raw_buffer_load_b128 (rsrc, ok ? (int)(off * 4u) : (int)0xfffffff0u, 0, LOAD_POLICY));
     }
     __device__ __forceinline__ float ld1 (uint32_t off) const
     {
