@@ -523,10 +523,10 @@ __device__ __forceinline__ void wait_until_ready ()
 }
 
 // Ordered kernels whose only shapes are 64 x 64 and 128 x 32 tiles fit four workgroups per compute unit, 128 registers, and need half the
-// LDS.  Their graphs are bound by latency, which a fourth tile per unit hides: see ORDERED_SMALL.
+// LDS.  Their graphs are bound by latency, which a fourth tile per unit hides: see ORDERED_SMALL.  Two where 32 x 32 tiles' buffers fill the LDS.
 static constexpr int ordered_wg_per_cu (unsigned tiles)
 {
-    return (tiles & TILES_NARROW) && tiles != TILES_ALL ? 2 : (tiles & (TILES_LARGE | TILES_WIDE | TILES_ATTENTION)) == 0 ? 4 : WG_PER_CU;
+    return (tiles & TILES_NARROW) ? 2 : (tiles & (TILES_LARGE | TILES_WIDE | TILES_ATTENTION)) == 0 ? 4 : WG_PER_CU;
 }
 // LDS of an ordered launch; narrow: the graph has 32 x 32 tiles, which prefetch weights into it
 static constexpr size_t ordered_lds (unsigned tiles, bool narrow)
@@ -618,21 +618,27 @@ static const void *const dataflow_kernels[NUM_KERNEL_VARIANTS][2] = {
 // ResNet-50 batch 2 567 / 553 (32 x 32 tiles: two per unit), 4 636 / 615 / 595, 11 990 / 951 / 882, YOLO-v3 batch 1 1053 / 1018 / 996, 2 1496 / - / 1378,
 // VGG-16 batch 1 505 / - / 500.
 // Transformer graphs with 32 x 32 tiles (a few dozen tokens) have one because attention spills on the one with every tile
-// kind: BERT-base 1 x 16 670 / 600.
-enum { ORDERED_SMALL, ORDERED_SMALL_NARROW, ORDERED_SMALL_TALL, ORDERED_CONVNET, ORDERED_TALL, ORDERED_TRANSFORMER, ORDERED_TRANSFORMER_NARROW, ORDERED_ALL,
-    NUM_ORDERED_VARIANTS };
+// kind: BERT-base 1 x 16 670 / 600.  Pools of networks of different kinds: 32 x 32 tiles keep two slices of weights more in registers, which
+// spills in the 168 registers of three workgroups per unit (844 registers in the kernel of every tile kind), and their buffers leave LDS
+// for two anyway; so kernels with them are built for two, the others come without.  us, one kernel of every kind / these:
+// ResNet-50 batch 1 + VGG-16 batch 2 1654 / 1164 (1227 with the attention and norm tiles in the kernel as well), + BERT-base 1 x 16 1556 / 998; BERT-base 8 x 128
+// + ResNet-50 batch 11 (no 32 x 32 tiles) 3037 / 2457, batch 4 2400 / 2041, YOLO-v3 batch 1 + VGG-16 batch 1 1932 / 1585.
+enum { ORDERED_SMALL, ORDERED_SMALL_NARROW, ORDERED_SMALL_TALL, ORDERED_CONVNET, ORDERED_CONVNET_NARROW, ORDERED_TALL, ORDERED_TRANSFORMER, ORDERED_TRANSFORMER_NARROW,
+    ORDERED_ALL, ORDERED_ALL_NARROW, NUM_ORDERED_VARIANTS };
 static const unsigned ordered_variant_tiles[NUM_ORDERED_VARIANTS] = {TILES_SMALL_CONVNET | TILES_YOLO, TILES_SMALL_CONVNET | TILES_YOLO | TILES_NARROW,
-    TILES_SMALL_CONVNET | TILES_TALL, TILES_CONVNET | TILES_YOLO, TILES_CONVNET | TILES_TALL, TILES_TRANSFORMER, TILES_TRANSFORMER | TILES_NARROW, TILES_ALL};
+    TILES_SMALL_CONVNET | TILES_TALL, TILES_CONVNET | TILES_YOLO, TILES_CONVNET | TILES_YOLO | TILES_TALL | TILES_NARROW, TILES_CONVNET | TILES_TALL, TILES_TRANSFORMER,
+    TILES_TRANSFORMER | TILES_NARROW, TILES_ALL & ~TILES_NARROW, TILES_ALL};
 #define ORDERED_KERNEL(tiles) (const void *)dataflow_kernel<2, tiles, true>
 static const void *const ordered_kernels[NUM_ORDERED_VARIANTS] = {
     ORDERED_KERNEL (TILES_SMALL_CONVNET | TILES_YOLO), ORDERED_KERNEL (TILES_SMALL_CONVNET | TILES_YOLO | TILES_NARROW), ORDERED_KERNEL (TILES_SMALL_CONVNET | TILES_TALL),
-    ORDERED_KERNEL (TILES_CONVNET | TILES_YOLO), ORDERED_KERNEL (TILES_CONVNET | TILES_TALL), ORDERED_KERNEL (TILES_TRANSFORMER),
-    ORDERED_KERNEL (TILES_TRANSFORMER | TILES_NARROW), ORDERED_KERNEL (TILES_ALL)};
+    ORDERED_KERNEL (TILES_CONVNET | TILES_YOLO), ORDERED_KERNEL (TILES_CONVNET | TILES_YOLO | TILES_TALL | TILES_NARROW), ORDERED_KERNEL (TILES_CONVNET | TILES_TALL), ORDERED_KERNEL (TILES_TRANSFORMER),
+    ORDERED_KERNEL (TILES_TRANSFORMER | TILES_NARROW), ORDERED_KERNEL (TILES_ALL & ~TILES_NARROW), ORDERED_KERNEL (TILES_ALL)};
 
+// the first that has all of the graph's tile kinds, with 32 x 32 tiles only where the graph has some (the last two between them take any graph)
 static int ordered_variant (const aspen_hip_graph_t *g)
 {
     int v = 0;
-    while (v + 1 < NUM_ORDERED_VARIANTS && (g->features & ~ordered_variant_tiles[v]) != 0) v++;
+    while (v + 1 < NUM_ORDERED_VARIANTS && ((g->features & ~ordered_variant_tiles[v]) != 0 || ((g->features ^ ordered_variant_tiles[v]) & TILES_NARROW) != 0)) v++;
     return v;
 }
 

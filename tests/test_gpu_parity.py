@@ -1,6 +1,7 @@
 """GPU parity: the HIP library (through the C ABI) against the compiled-reference fixtures and the
 CPU oracle, per layer, relative L2 <= 1e-4 and identical argmax."""
 import os
+import tempfile
 
 import numpy as np
 import pytest
@@ -420,6 +421,54 @@ def test_folded_layernorm_without_attention(gpu, engine_flags, monkeypatch, name
             net.close()
     finally:
         api.lib().aspen_keep_layer_outputs(1)
+
+
+def test_ordered_kernels_of_mixed_tile_kinds(gpu, engine_flags, monkeypatch):
+    """Combinations of tile kinds in one ordered run: 32 x 32 tiles that gather (a 3 x 3 window) in a graph with a softmax, i.e. of a
+    transformer's kinds otherwise; and pools of a network of 32 x 32 tiles, or of large and wide ones, with another network."""
+    from oracle import cpu
+    engine_flags(ORDERED)
+    conv = "[convolutional]\nfilters={}\nsize={}\nstride=1\npad={}\nactivation=relu\n\n"
+    gathering = "[net]\nheight=3\nwidth=3\nchannels=64\n\n" + conv.format(40, 3, 0) + "[softmax]\n\n"
+    narrow = "[net]\nheight=8\nwidth=8\nchannels=64\n\n" + conv.format(96, 3, 1) + conv.format(33, 1, 0)
+    large = "[net]\nheight=64\nwidth=64\nchannels=64\n\n" + conv.format(128, 3, 1) + conv.format(40, 1, 0)
+    bert = M.bert_cfg(1, 64, 2, 128)
+    for pool in ([(gathering, 37, 16, "1", (32, 32))], [(narrow, 3, 16, "1", (32, 32)), (large, 32, 16, "0", (128, 64))],
+                 [(narrow, 3, 16, "1", (32, 32)), (bert, 2, 16, "0", (64, 64))], [(bert, 2, 16, "0", (64, 64)), (large, 32, 16, "0", (128, 64))]):
+        rpool, nets = api.RPool(), []
+        dse = api.DseGroup(1, api.MODE_DATAFLOW)
+        dse.set_rpool(rpool)
+        for seed, (cfg, batch, tiles, nt, shape) in enumerate(pool):
+            monkeypatch.setenv("ASPEN_GPU_NARROW_TILES", nt)
+            layers = M.parse_cfg(cfg)
+            seq = 24 if cfg == bert else 0
+            tens = M.synth_weights(layers, 40 + seed, "gpt" if seq else "he")
+            x = M.synth_input(layers, 40 + seed, batch, seq, "embeddings")
+            path = tempfile.mktemp(suffix=".bin")
+            M.write_aspen_data(path, tens)
+            dnn = api.Dnn(cfg, path)
+            os.unlink(path)
+            nasm = api.Nasm(dnn, batch, seq, tiles)
+            info = nasm.info(1)
+            assert (info["tile_H"], info["tile_W"]) == shape, info
+            rpool.add_nasm_raw_input(nasm, x)
+            nets.append((dnn, nasm, layers, cpu.run_network(layers, tens, x, batch, seq)))
+        try:
+            dse.run()
+            for _, nasm, _, _ in nets:
+                dse.wait(nasm)
+            dse.stop()
+            assert dse.last_run_ordered()
+            for _, nasm, layers, outs in nets:
+                for l in range(1, nasm.num_ldata):
+                    err = H.rel_l2(nasm.layer_output(l), outs[l])
+                    assert err <= H.REL_L2_TOL, f"layer {l} ({layers[l]['type']}): rel L2 {err:.3g}"
+        finally:
+            dse.destroy()
+            rpool.destroy()
+            for dnn, nasm, _, _ in nets:
+                nasm.destroy()
+                dnn.destroy()
 
 
 def test_results_in_the_callers_dimension_order(gpu):
