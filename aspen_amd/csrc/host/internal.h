@@ -109,7 +109,9 @@ struct nasm_t
     int small_tiles_only;                    /* every contraction layer uses the small tile shape, see create_nasm */
     int narrow_tiles;                        /* layers short of tiles use the 32 x 32 shape, see create_nasm */
     int ordered_pref;                        /* persistent kernel in its ordered mode (no ready queue): 1 yes (graphs bound by latency, see create_nasm;
-                                                the tuner; aspen_nasm_set_ordered), 0 no, -1 the engine decides from the graph's parallelism */
+                                                the tuner; aspen_nasm_set_ordered), ORDERED_ALONE yes in a pool of its own, 0 no, -1 the engine
+                                                decides from the graph's parallelism */
+#define ORDERED_ALONE 2
     nasm_ldata_t *ldata_arr;
     unsigned int num_ldata;
     unsigned int num_ninst;

@@ -718,6 +718,7 @@ static double nasm_parallelism (const nasm_t *nasm)
 #define ORDERED_KITERS_CAP 24
 #define LATENCY_BOUND_BELOW 128.0
 #define ORDERED_VISION_BELOW 1160.0
+#define ORDERED_VISION_POOLED_BELOW 1100.0
 static nasm_t *create_nasm (aspen_dnn_t *dnn, unsigned int min_ninst, unsigned int batch, unsigned int seq)
 {
     const char *e = getenv ("ASPEN_GPU_MAX_KITERS");            /* experiments: fixed cap, 0 = none */
@@ -730,8 +731,11 @@ static nasm_t *create_nasm (aspen_dnn_t *dnn, unsigned int min_ninst, unsigned i
     {
         /* (convolutional graphs a little above the limit keep their tiles but still run better in the ordered mode,
            ordered / queue in us: VGG-16 batch 2, 1052: 652 / 686, ResNet-50 batch 14, 1104: 1064 / 1156, YOLO-v3 batch 3, 1142:
-           1741 / 1852; from ResNet-50 batch 16, 1186, on the queue wins: 1262 / 1206; VGG-16 batch 4, 1246: 965 / 964) */
-        if (seq == 0 && parallelism < ORDERED_VISION_BELOW) nasm->ordered_pref = 1;
+           1741 / 1852; from ResNet-50 batch 16, 1186, on the queue wins: 1262 / 1206; VGG-16 batch 4, 1246: 965 / 964.
+           Beside another network of its pool the nearest of them wait for the other's tiles in the index order and lose: ResNet-50 batch 14 + batch 1
+           1866 / 1687, + batch 4 1607 / 1364, + batch 11 1870 / 1784, YOLO-v3 batch 3 + ResNet-50 batch 1 2729 / 2523, + BERT-base 1 x 16
+           3115 / 2483; VGG-16 batch 2 + ResNet-50 batch 1 1161 / 1092, + BERT-base 1 x 16 1382 / 1346, but + YOLO-v3 batch 1 1712 / 2102) */
+        if (seq == 0 && parallelism < ORDERED_VISION_BELOW) nasm->ordered_pref = parallelism < ORDERED_VISION_POOLED_BELOW ? 1 : ORDERED_ALONE;
         return nasm;
     }
     /* bound by the LATENCY of its chains (one image through a deep network; the engine runs such a graph in its ordered

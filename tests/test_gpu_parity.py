@@ -471,6 +471,35 @@ def test_ordered_kernels_of_mixed_tile_kinds(gpu, engine_flags, monkeypatch):
                 dnn.destroy()
 
 
+def test_graph_that_is_ordered_only_alone_in_its_pool(gpu):
+    """A convolutional graph of 1152 equal tiles, an estimated parallelism just below the limit of 1160: alone in its pool it runs in
+    the ordered mode, beside a second one on the ready queue, and alone again when that one has gone; the same results."""
+    cfg = "[net]\nheight=64\nwidth=64\nchannels=64\n\n[convolutional]\nfilters=64\nsize=1\nstride=1\npad=0\nactivation=relu\n\n"
+    layers = M.parse_cfg(cfg)
+    tens = M.synth_weights(layers, 31, "he")
+    x = M.synth_input(layers, 31, 18, 0)
+    net = H.GpuNet(cfg, tens, 18, 0, min_ninst=1152)
+    second = api.Nasm(net.dnn, 18, 0, 1152)
+    try:
+        assert net.nasm.num_ninst == 1152
+        net.run(x)
+        assert net.dse.last_run_ordered()
+        alone = net.layer(1).copy()
+        net.rpool.add_nasm_raw_input(second, x)
+        net.run(x)
+        net.dse.wait(second)
+        assert not net.dse.last_run_ordered()
+        assert np.array_equal(net.layer(1), alone) and np.array_equal(second.layer_output(1), alone)
+        second.destroy()
+        second = None
+        net.run(x)
+        assert net.dse.last_run_ordered() and np.array_equal(net.layer(1), alone)
+    finally:
+        if second is not None:
+            second.destroy()
+        net.close()
+
+
 def test_results_in_the_callers_dimension_order(gpu):
     """dse_get_ldata_result permutes a layer's native tensor into the order the caller names (reference
     get_ldata_output, src/apu.c:227-297): matrices of a transformer are (BATCH, MAT_N, MAT_M), attention
