@@ -1829,7 +1829,12 @@ extern "C" int aspen_hip_event_elapsed_ms (int a, int b, float *ms)
 
 // One contraction tile per workgroup, the descriptor in the kernel-argument segment; compiled for one tile shape each (all of them
 // in one kernel spill: 1000 x 3137 x 1152 85 us a call that allocates nothing, 62 this way).  Contiguous tile
-// ranges per XCD, as in layer_kernel: workgroups that share activation columns meet in one L2.
+// ranges per XCD, as in layer_kernel: workgroups that share activation columns meet in one L2.  Large tiles in bands of PRODUCT_BAND rows of
+// tiles: the hundred that an XCD runs at a time then share their weights (six bytes a float) as well.  Column by column through all rows, each
+// fetched weights of its own, and from 4096 rows on a product was bound by that; rows to a band all / 12 / 8 / 6 / 4, us a call: 4096 x 8192 x
+// 3072 1343 / 958 / 957 / 948 / 953, 4096 x 4096 x 4096 910 / 658 / 658 / 651 / 645, 8192 x 8192 x 8192 8320 / 5980 / 5740 / 5550 / 5270, 2048 x 8192 x 2048 342 / 333 /
+// 333 / 333 / 331, 1000 x 3137 x 1152 66 / 66 / 66 / 66 / 66.
+#define PRODUCT_BAND 4u
 template <unsigned FEAT> __global__ void __launch_bounds__ (WG_THREADS, WG_PER_CU) product_kernel (const aspen_hip_layer_t L)
 {
     extern __shared__ __align__ (16) float smem[];
@@ -1837,7 +1842,14 @@ template <unsigned FEAT> __global__ void __launch_bounds__ (WG_THREADS, WG_PER_C
     // (L is the only argument: it lies where the argument segment begins)
     const auto address = [] () { return (const aspen_hip_layer_t *)__builtin_amdgcn_kernarg_segment_ptr (); };
     const layer_at<decltype (address)> descriptor {address};
-    run_tile<0, FEAT> (descriptor, xcd * chunk + (xcd < rem ? xcd : rem) + local, false, smem, [] () { return (uint32_t *)nullptr; });
+    uint32_t t = xcd * chunk + (xcd < rem ? xcd : rem) + local;
+    if ((FEAT & TILES_LARGE) && L.tiles_m > PRODUCT_BAND)
+    {
+        const uint32_t bands = (L.tiles_m + PRODUCT_BAND - 1) / PRODUCT_BAND, rows = (L.tiles_m + bands - 1) / bands, size = rows * L.tiles_n, band = t / size, r = t - band * size;
+        const uint32_t height = min (rows, L.tiles_m - band * rows), tn = r / height;
+        t = tn * L.tiles_m + band * rows + (r - tn * height);
+    }
+    run_tile<0, FEAT> (descriptor, t, false, smem, [] () { return (uint32_t *)nullptr; });
 }
 
 // C = act (A B + bias) with A already in the order the tiles read; on the library's stream.
@@ -1848,11 +1860,12 @@ static int launch_product (uint32_t M, uint32_t N, uint32_t K, const float *arra
     const uint32_t cu = (uint32_t)g_num_cu;
     const auto tiles = [&] (uint32_t bm, uint32_t bn) { return (uint64_t)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
     const uint64_t small = tiles (VAR2_BM, VAR2_BN), large = tiles (VAR0_BM, VAR0_BN);
-    // us with 128 x 64 / 64 x 64 / 32 x 32 tiles on 256 compute units (whole calls): 1000 x 3137 x 1152 (400 large tiles) 68 / 83 / 116,
-    // 2048 x 2048 x 1024 (512) 68 / 80 / 136, 2000 x 1400 x 1024 (352) 61 / 62 / 100, 3000 x 700 x 2048 (264) 96 / 100 / 146, 512 x 2048 x 768
-    // (256 small ones) 36 / 34 / 37, 64 x 8192 x 1024 (128) 39 / 36 / 30, 256 x 1024 x 512 (64) 29 / 27 / 22, 64 x 64 x 3072 (1) 78 / 66 / 38: the
-    // large shape from five workgroups for four units on, the one that splits K over its wavefronts where small tiles leave
-    // half of the units idle
+    // us with 128 x 64 / 64 x 64 / 32 x 32 tiles on 256 compute units (whole calls): 1000 x 3137 x 1152 (400 large tiles) 64 / 75 / 123,
+    // 2048 x 2048 x 1024 (512) 70 / 81 / 136, 1536 x 1984 x 3072 (372) 133 / 132 / -, 2048 x 1408 x 2048 (352) 99 / 104 / -, 2000 x 1400 x 1024 (352)
+    // 65 / 63 / 102, 1280 x 2048 x 1024 (320) 62 / 58 / -, 3000 x 700 x 2048 (264) 96 / 91 / 147, 512 x 2048 x 768 (256 small ones) 42 / 36 / 40,
+    // 64 x 8192 x 1024 (128) 47 / 38 / 33, 256 x 1024 x 512 (64) 34 / 29 / 25, 64 x 64 x 3072 (1) 92 / 61 / 37: the large shape from five workgroups for
+    // four units on (up to three tiles for two units either may win, by 6 % at most), the one that splits K over its wavefronts where small tiles
+    // leave half of the units idle
     const int v = 4 * large >= 5 * (uint64_t)cu ? 0 : 2 * small <= cu ? 2 : 1;
     static const struct { int variant; uint32_t bm, bn; } shape[3] = {{ASPEN_HIP_GEMM_LARGE, VAR0_BM, VAR0_BN}, {ASPEN_HIP_GEMM_SMALL, VAR2_BM, VAR2_BN}, {ASPEN_HIP_GEMM_NARROW, VAR3_BM, VAR3_BN}};
     L.type = MATMUL_LAYER; L.act = act; L.variant = shape[v].variant; L.direct = ASPEN_HIP_OPERAND_DIRECT;
