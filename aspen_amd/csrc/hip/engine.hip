@@ -602,14 +602,17 @@ template <unsigned FEAT> __global__ void __launch_bounds__ (WG_THREADS, WG_PER_C
 static const void *const product_kernels[3] = {(const void *)product_kernel<TILES_LARGE>, (const void *)product_kernel<TILES_SMALL>, (const void *)product_kernel<TILES_NARROW>};
 
 // The persistent kernel's variants, smallest first: [variant][0] coherent loads, [1] cached loads.  A graph runs on the
-// first variant that has all its tile kinds, see graph_features.
-#define NUM_KERNEL_VARIANTS 5
-static const unsigned kernel_variant_tiles[NUM_KERNEL_VARIANTS] = {TILES_TRANSFORMER, TILES_CONVNET, TILES_CONVNET | TILES_TALL, TILES_CONVNET | TILES_YOLO, TILES_ALL};
+// first variant that has all its tile kinds, see graph_features.  32 x 32 tiles of convolutional graphs have one because the one with every
+// tile kind spills 529 registers: ResNet-50 batch 1 on the queue 650 / 580 us, in a pool with batch 14 1688 / 1250, with YOLO-v3 batch 1 1733 / 1437.
+#define NUM_KERNEL_VARIANTS 6
+static const unsigned kernel_variant_tiles[NUM_KERNEL_VARIANTS] = {TILES_TRANSFORMER, TILES_CONVNET, TILES_CONVNET | TILES_TALL, TILES_CONVNET | TILES_YOLO,
+    TILES_SMALL_CONVNET | TILES_YOLO | TILES_NARROW, TILES_ALL};
 static const void *const dataflow_kernels[NUM_KERNEL_VARIANTS][2] = {
     {(const void *)dataflow_kernel<1, TILES_TRANSFORMER>, (const void *)dataflow_kernel<2, TILES_TRANSFORMER>},
     {(const void *)dataflow_kernel<1, TILES_CONVNET>, (const void *)dataflow_kernel<2, TILES_CONVNET>},
     {(const void *)dataflow_kernel<1, TILES_CONVNET | TILES_TALL>, (const void *)dataflow_kernel<2, TILES_CONVNET | TILES_TALL>},
     {(const void *)dataflow_kernel<1, TILES_CONVNET | TILES_YOLO>, (const void *)dataflow_kernel<2, TILES_CONVNET | TILES_YOLO>},
+    {(const void *)dataflow_kernel<1, TILES_SMALL_CONVNET | TILES_YOLO | TILES_NARROW>, (const void *)dataflow_kernel<2, TILES_SMALL_CONVNET | TILES_YOLO | TILES_NARROW>},
     {(const void *)dataflow_kernel<1, TILES_ALL>, (const void *)dataflow_kernel<2, TILES_ALL>}};
 
 // Ordered mode (see aspen_hip_run_dataflow), cached loads only, smallest first.  Convolutional graphs that are rebuilt for it have

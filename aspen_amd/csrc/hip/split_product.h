@@ -186,12 +186,6 @@ template <int ROWS> struct SplitStage
 {
     static constexpr uint32_t PLANE = ROWS * 64u, BYTES = 3u * PLANE;
     static __device__ __forceinline__ uint32_t offset (uint32_t row, uint32_t unit) { return row * 64u + ((unit ^ ((0u - (row >> 2)) & 3u)) * 16u); }
-    static __device__ __forceinline__ void write (char *stage, uint32_t off, const split8_t &s)
-    {
-        *reinterpret_cast<u32x4 *> (stage + off) = s.h;
-        *reinterpret_cast<u32x4 *> (stage + off + PLANE) = s.m;
-        *reinterpret_cast<u32x4 *> (stage + off + 2 * PLANE) = s.l;
-    }
     static __device__ __forceinline__ split8_t read (const char *stage, uint32_t off)
     {
         return {*reinterpret_cast<const u32x4 *> (stage + off), *reinterpret_cast<const u32x4 *> (stage + off + PLANE), *reinterpret_cast<const u32x4 *> (stage + off + 2 * PLANE)};

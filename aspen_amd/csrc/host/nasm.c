@@ -733,8 +733,8 @@ static nasm_t *create_nasm (aspen_dnn_t *dnn, unsigned int min_ninst, unsigned i
            ordered / queue in us: VGG-16 batch 2, 1052: 652 / 686, ResNet-50 batch 14, 1104: 1064 / 1156, YOLO-v3 batch 3, 1142:
            1741 / 1852; from ResNet-50 batch 16, 1186, on the queue wins: 1262 / 1206; VGG-16 batch 4, 1246: 965 / 964.
            Beside another network of its pool the nearest of them wait for the other's tiles in the index order and lose: ResNet-50 batch 14 + batch 1
-           1866 / 1687, + batch 4 1607 / 1364, + batch 11 1870 / 1784, YOLO-v3 batch 3 + ResNet-50 batch 1 2729 / 2523, + BERT-base 1 x 16
-           3115 / 2483; VGG-16 batch 2 + ResNet-50 batch 1 1161 / 1092, + BERT-base 1 x 16 1382 / 1346, but + YOLO-v3 batch 1 1712 / 2102) */
+           1863 / 1253, + batch 4 1610 / 1377, + batch 11 1888 / 1815, YOLO-v3 batch 3 + ResNet-50 batch 1 2740 / 1940, + BERT-base 1 x 16
+           3126 / 2505; VGG-16 batch 2 + ResNet-50 batch 1 1159 / 1090, + BERT-base 1 x 16 1381 / 1348, but + YOLO-v3 batch 1 1722 / 2096) */
         if (seq == 0 && parallelism < ORDERED_VISION_BELOW) nasm->ordered_pref = parallelism < ORDERED_VISION_POOLED_BELOW ? 1 : ORDERED_ALONE;
         return nasm;
     }
