@@ -1385,8 +1385,8 @@ static aspen_hip_graph_t *graph_create (const aspen_hip_layer_t *layers, uint32_
         for (int i = NUM_KERNEL_VARIANTS - 2; i >= 0 && !all_tiles; i--) if ((g->features & ~kernel_variant_tiles[i]) == 0) g->variant = i;
         const uint32_t resident = (uint32_t)g_variant_wg[g->variant][g->cached_loads ? 1 : 0];      // of the variant this graph runs on
         uint32_t per_cu = resident;
-        // ready-queue runs with one / two / three workgroups per unit on 256 units, us: ResNet-50 batch 1 (average parallelism 92) 640 / 677 /
-        // 705, BERT-base 3 x 75 (197) 1212 / 1228 / 1257, ResNet-50 batch 4 (338) 839 / 783 / 798, YOLO-v3 batch 1 (419) 1484 / 1339 /
+        // ready-queue runs with one / two / three workgroups per unit on 256 units, us: ResNet-50 batch 1 (average parallelism 92) 577 / 600 /
+        // 594, BERT-base 3 x 75 (197) 1212 / 1228 / 1257, ResNet-50 batch 4 (338) 839 / 783 / 798, YOLO-v3 batch 1 (419) 1484 / 1339 /
         // 1308, BERT-base 8 x 128 (533) 2232 / 1665 / 1682, ResNet-50 batch 8 (645) 1300 / 941 / 899, GPT-2 4 x 512 (878) 4104 / 2929 / 2742
         if (par < 2.3 * g_num_cu) per_cu = par < g_num_cu ? 1u : 2u;
         if (per_cu > resident) per_cu = resident;

@@ -7,8 +7,9 @@
 //     a b = ah bh  +  (ah bm + am bh)  +  (ah bl + al bh + am bm)      left out: am bl + al bm + al bl < 2^-24 |a b|
 // (|m| <= 2^-8 |x|, |l| <= 2^-17 |x|), i.e. at worst what rounding ONE float product to a float may cost, 0.09 of that in the root mean
 // square over mantissas.  The leading products are summed in one
-// accumulator and the five small ones in another, added at the end: the large sum is then rounded once per 16 K positions
-// instead of once per two (v_mfma_f32_32x32x2_f32), the small sum's roundings do not count at its size, and the result is closer to the
+// accumulator and the five small ones in another, added at the end: the large sum is then rounded once per 32 K positions,
+// one v_mfma_f32_16x16x32_bf16 (32 addends that make 0.75 units in the last place raise the sum; each half, 0.375, would not), instead of
+// once per two (v_mfma_f32_32x32x2_f32), the small sum's roundings do not count at its size, and the result is closer to the
 // exact one than the single-precision matrix instruction's (relative to a 64-bit sum, 2-norm over 128 x 128 results, inputs
 // normal / rectified normal: K = 64 4.8e-8 / 4.2e-8 against 1.4e-7 / 1.0e-7; K = 1024 1.8e-7 / 1.5e-7 against 5.7e-7 / 4.2e-7;
 // K = 4096 4.0e-7 / 3.2e-7 against 1.1e-6 / 8.1e-7; with one accumulator for all six products 1.0e-6 / 9.5e-7).
@@ -16,7 +17,7 @@
 // time.  In practice both are limited by power, and a product's time is its energy.  Registers alone, every compute
 // unit, products in TFLOP/s of the floats' work (417 nominal): v_mfma_f32_32x32x16_bf16 300, v_mfma_f32_16x16x32_bf16 355 (half the
 // accumulator traffic per product); a loop that also splits, stages and fetches what a 128 x 64 tile does, 188 and 229 (a 64 x 64
-// tile's 184).  So the smaller block it is.  The sums come out the same: over 1000 x 3137 and 2048 x 2048 results, K = 32 ... 4096, both
+// tile's 184; whole products of 128 x 64 tiles reach 214 to 230, see PRODUCT_BAND).  So the smaller block it is.  The sums come out the same: over 1000 x 3137 and 2048 x 2048 results, K = 32 ... 4096, both
 // instructions' errors against 64-bit sums agree to three digits.
 // The range is float's own (bfloat16 has the same exponent) with two edges.  Terms below bfloat16's smallest number, 2^-133, do not
 // exist: an input below 2^-110 enters with an absolute error of up to 2^-134.  And infinities, NaNs and floats within 0.2 % of the

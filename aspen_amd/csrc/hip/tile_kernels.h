@@ -2256,7 +2256,7 @@ __device__ __forceinline__ bool splitk_arrived_last (uint32_t *counter, uint32_t
 // dependency level keeps every compute unit busy for one or two microseconds instead of a quarter of them for
 // eight.  Throughput per workgroup does not matter here, so there is nothing to share between wavefronts and
 // no operand is staged for another wavefront: a lane reads its weights as the fragments they are laid out in
-// (WeightFragments) and its activations as the floats of its row's units (row = lane % 32, see SLICE_K), splits these
+// (WeightFragments) and its activations as the floats of its two columns' units (columns lane % 16 and 16 + lane % 16, see SLICE_K), splits these
 // itself, the K loop has no barrier, and the four partial sums meet in LDS once.  A layer can additionally be cut along K
 // across workgroups (`slice` >= 0) exactly like the 64 x 64 shape, with blocks of 32 x 32 sums in the threads' own order.
 // Activations are read in place (DIRECT) or gathered by stepping through the taps (a convolution or FC layer over

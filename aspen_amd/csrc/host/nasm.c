@@ -739,7 +739,10 @@ static nasm_t *create_nasm (aspen_dnn_t *dnn, unsigned int min_ninst, unsigned i
         return nasm;
     }
     /* bound by the LATENCY of its chains (one image through a deep network; the engine runs such a graph in its ordered
-       mode): layers short of tiles take the 32 x 32 shape */
+       mode): layers short of tiles take the 32 x 32 shape.  us with 64 x 64 / 32 x 32 tiles: BERT-base 1 x 16 (parallelism 73) 719 / 563,
+       1 x 64 (74) 789 / 625, GPT-2 4 x 16 (81) 780 / 628, ResNet-50 batch 1 (94) 514 / 398; BERT-base 1 x 100 (134) 808 / 861, 1 x 128 (135)
+       826 / 868, 2 x 64 (135) 799 / 788, GPT-2 1 x 128 (149) 799 / 781; ResNet-50 batch 2 (179) 542 / 605, BERT-base 4 x 64 (194) 875 / 920,
+       3 x 75 (197) 887 / 946, ResNet-50 batch 4 (338) 582 / 950 */
     const char *nt = getenv ("ASPEN_GPU_NARROW_TILES");
     const int narrow = nt != NULL ? atoi (nt) != 0 : parallelism < LATENCY_BOUND_BELOW;
     /* transformer graphs below the cap's limit run the ordered mode (below), where shorter tiles do pay: no tile longer
@@ -748,11 +751,11 @@ static nasm_t *create_nasm (aspen_dnn_t *dnn, unsigned int min_ninst, unsigned i
     nasm_t *rebuilt = build_nasm (dnn, min_ninst, batch, seq, parallelism >= CHAIN_BOUND_CAP_FROM ? CHAIN_BOUND_KITERS_CAP : tr_ordered ? ORDERED_KITERS_CAP : 0, 1, narrow);
     if (rebuilt == NULL) return nasm;
     /* The ordered mode itself pays further up than the 32 x 32 tiles do.  Measured against the ready queue (us, ordered /
-       queue): ResNet-50 at batch 2 / 4 / 6 / 8 / 11 / 12 (parallelism 179 / 338 / 489 / 645 / 874 / 955): 625 / 772, 675 / 825,
-       746 / 900, 829 / 936, 1019 / 1046, 1090 / 1085; YOLO-v3 at batch 1 / 2 (419 / 834): 1099 / 1396, 1552 / 1618; VGG-16 at
-       batch 1 (728): 513 / 582.  Graphs that are not rebuilt here are above.  Transformer graphs, those of little
-       parallelism with the cap of 24 K slices: BERT-base, batch x tokens 3 x 75 / 4 x 128 / 8 x 128 / 16 x 128: 949 / 1268,
-       1111 / 1481, 1544 / 1781, 2837 / 2860; GPT-2 1 x 512 / 2 x 256 / 4 x 512: 1328 / 1656, 1163 / 1451, 2943 / 3140, and the ordered
+       queue): ResNet-50 at batch 2 / 4 / 6 / 8 / 11 / 12 (parallelism 179 / 338 / 489 / 645 / 874 / 955): 542 / 714, 582 / 774,
+       662 / 855, 746 / 868, 867 / 966, 937 / 1023; YOLO-v3 at batch 1 / 2 (419 / 834): 976 / 1319, 1354 / 1472; VGG-16 at
+       batch 1 (728): 491 / 546.  Graphs that are not rebuilt here are above.  Transformer graphs, those of little
+       parallelism with the cap of 24 K slices: BERT-base, batch x tokens 3 x 75 / 4 x 128 / 8 x 128 / 16 x 128: 888 / 1199,
+       993 / 1346, 1344 / 1656, 2547 / 2514; GPT-2 1 x 512 / 2 x 256 / 4 x 512: 1088 / 1416, 1007 / 1337, 2542 / 2602, and the ordered
        mode moves less data: a tile's workgroup, and with it the XCD whose L2 its operands pass through, is fixed by the
        tile's index, so every XCD keeps to an eighth of a layer's weight rows.  So every rebuilt graph asks for the
        ordered mode.  Where it matters, apu_generate_nasm times both. */
