@@ -22,15 +22,15 @@ sys.path.insert(0, ROOT)
 
 PEAK_FP32_MFMA_TFLOPS = 157.3      # MI355X dense fp32 matrix peak
 # what the contractions could reach: a float product is six bfloat16 products on the matrix cores, dense bf16 peak 2.5 PFLOP/s
-# (limited by power, a large product reaches 205 TFLOP/s)
+# (limited by power, large products reach 214 to 230 TFLOP/s)
 PEAK_CONTRACTION_TFLOPS = 2500.0 / 6.0
 PEAK_HBM_GBS = 8000.0
 # HBM bytes per launch of the persistent kernel, measured with rocprofv3 FETCH_SIZE / WRITE_SIZE passes
 # calibrated on the library's copy kernel (summaries: profiles/dataflow_kernel_resnet50_b32_hbm_traffic.txt and
 # profiles/dataflow_kernel_vgg16_co_inference_bert_gpt2_kernel_stats_hbm_traffic.txt); valid for these tuned configurations only
-MEASURED_TRAFFIC_BYTES = {("resnet50_b32", "dataflow", 1536): 9.31e9, ("vgg16_b32", "dataflow", 1536): 24.04e9,
-                          ("co_resnet50_vgg16_b16", "dataflow", 1536): 18.49e9, ("bert_base_b8_s128", "dataflow", 192): 3.05e9,
-                          ("gpt2_b4_s512", "dataflow", 384): 10.53e9, ("resnet50_b1", "dataflow", 256): 0.466e9}
+MEASURED_TRAFFIC_BYTES = {("resnet50_b32", "dataflow", 1536): 9.51e9, ("vgg16_b32", "dataflow", 1536): 23.92e9,
+                          ("co_resnet50_vgg16_b16", "dataflow", 1536): 18.42e9, ("bert_base_b8_s128", "dataflow", 192): 3.05e9,
+                          ("gpt2_b4_s512", "dataflow", 384): 10.02e9, ("resnet50_b1", "dataflow", 256): 0.466e9}
 
 # algorithmic GEMM-class flops per unit (2*M*N*K with the reference's K: padding taps counted, full
 # S x S attention): per image for the vision nets, per token for the transformers
