@@ -1832,11 +1832,12 @@ extern "C" int aspen_hip_event_elapsed_ms (int a, int b, float *ms)
 
 // One contraction tile per workgroup, the descriptor in the kernel-argument segment; compiled for one tile shape each (all of them
 // in one kernel spill: 1000 x 3137 x 1152 85 us a call that allocates nothing, 62 this way).  Contiguous tile
-// ranges per XCD, as in layer_kernel: workgroups that share activation columns meet in one L2.  Large tiles in bands of PRODUCT_BAND rows of
-// tiles: the hundred that an XCD runs at a time then share their weights (six bytes a float) as well.  Column by column through all rows, each
-// fetched weights of its own, and from 4096 rows on a product was bound by that; rows to a band all / 12 / 8 / 6 / 4, us a call: 4096 x 8192 x
-// 3072 1343 / 958 / 957 / 948 / 953, 4096 x 4096 x 4096 910 / 658 / 658 / 651 / 645, 8192 x 8192 x 8192 8320 / 5980 / 5740 / 5550 / 5270, 2048 x 8192 x 2048 342 / 333 /
-// 333 / 333 / 331, 1000 x 3137 x 1152 66 / 66 / 66 / 66 / 66.
+// ranges per XCD, as in layer_kernel: workgroups that share activation columns meet in one L2.  Large tiles from nine rows of tiles on go in bands
+// of PRODUCT_BAND rows: the hundred that an XCD runs at a time then share their weights (six bytes a float) as well.  Column by column
+// through all rows, each fetched weights of its own, and from 4096 rows on a product was bound by that; rows to a band all / 12 / 8 / 6 / 4, us a call:
+// 4096 x 8192 x 3072 1343 / 958 / 957 / 948 / 953, 4096 x 4096 x 4096 910 / 658 / 658 / 651 / 645, 8192 x 8192 x 8192 8320 / 5980 / 5740 / 5550 / 5270, 2048 x 8192 x
+// 2048 342 / 333 / 333 / 333 / 331, 1664 x 3000 x 3072 196 / 189 / 188 / 187 / 186.  With eight rows there is nothing to gain and the divisions cost
+// (1000 x 3137 x 1152 60.0 / - / - / - / 60.8).
 #define PRODUCT_BAND 4u
 template <unsigned FEAT> __global__ void __launch_bounds__ (WG_THREADS, WG_PER_CU) product_kernel (const aspen_hip_layer_t L)
 {
@@ -1846,7 +1847,7 @@ template <unsigned FEAT> __global__ void __launch_bounds__ (WG_THREADS, WG_PER_C
     const auto address = [] () { return (const aspen_hip_layer_t *)__builtin_amdgcn_kernarg_segment_ptr (); };
     const layer_at<decltype (address)> descriptor {address};
     uint32_t t = xcd * chunk + (xcd < rem ? xcd : rem) + local;
-    if ((FEAT & TILES_LARGE) && L.tiles_m > PRODUCT_BAND)
+    if ((FEAT & TILES_LARGE) && L.tiles_m > 2 * PRODUCT_BAND)
     {
         const uint32_t bands = (L.tiles_m + PRODUCT_BAND - 1) / PRODUCT_BAND, rows = (L.tiles_m + bands - 1) / bands, size = rows * L.tiles_n, band = t / size, r = t - band * size;
         const uint32_t height = min (rows, L.tiles_m - band * rows), tn = r / height;

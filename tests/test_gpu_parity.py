@@ -1277,10 +1277,10 @@ def test_matrices_travel_whole_in_both_directions(gpu, rows, ld, columns):
         L.aspen_hip_free(d)
 
 
-@pytest.mark.parametrize("M,N,K", [(1, 1, 32), (33, 31, 3072), (31, 2049, 96), (513, 1025, 64), (65, 8100, 32), (1031, 2570, 96), (2050, 1285, 160), (577, 4100, 32), (3201, 840, 64)])
+@pytest.mark.parametrize("M,N,K", [(1, 1, 32), (33, 31, 3072), (31, 2049, 96), (513, 1025, 64), (65, 8100, 32), (1031, 2570, 96), (2050, 1285, 160), (1281, 1990, 32), (3201, 840, 64)])
 def test_plain_product_over_its_tile_shapes(gpu, M, N, K):
     """32 x 32 tiles (K split over the wavefronts, also fewer slices than wavefronts), 64 x 64 and 128 x 64 tiles, as the sizes
-    choose them, edges off every tile (of 128 x 64 ones with 9, 17, 5 and 26 rows: in bands of 3, of 4 and 1, of 3 and 2, of 4 and 2); with bias and activation, both entry points, bit for bit alike.  Per output at most one
+    choose them, edges off every tile (of 128 x 64 ones with 9, 17, 11 and 26 rows: in bands of 3, of 4 and 1, of 4 and 3, of 4 and 2); with bias and activation, both entry points, bit for bit alike.  Per output at most one
     rounding per 16 K positions in each of the two running sums, a few for the additions behind them, 2^-24 each of the sum of magnitudes."""
     import ctypes as C
     L = api.lib()
